@@ -99,14 +99,6 @@ extern "C" {
                                      bf16 tensors it costs next to nothing in accuracy (what is stored is
                                      rounded to bf16 either way).  Off unless passed.                 */
 
-#define T2FW_FLAG_TILES 32       /* decay rule, states of up to 64 x 64 that the 16-bit matrix-core kernels do not take
-                                     (fp32 tensors, other widths): fp32 matrix-core kernels in tiles of 16 steps, at the
-                                     accuracy of the exact kernels, for a checkpoint interval of 64 (a forward call without
-                                     checkpoints: any).  The backward call needs the workspace that
-                                     t2fw_lfw_workspace_bytes reports for these flags.  What the tiles cannot hold (gates
-                                     outside [0, 1], very small gates or very large values) is done by the exact recurrence
-                                     in the same call, 64 steps at a time.                            */
-
 int t2fw_abi_version(void);
 const char *t2fw_last_error(void);
 

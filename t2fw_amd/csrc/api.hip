@@ -4,7 +4,6 @@
 #include "lfw_scan.hpp"
 #include "lfw_chunk.hpp"
 #include "lfw_par.hpp"
-#include "lfw_tile.hpp"
 #include "dfw_scan.hpp"
 #include "cast.hpp"
 #include "gate.hpp"
@@ -85,25 +84,6 @@ bool chunk_shape_ok(int64_t D, int64_t K, int32_t dtype, int32_t flags) {
     return (flags & T2FW_FLAG_FORCE_SCAN) == 0 && D == 64 && K == 64 && (dtype == T2FW_F16 || dtype == T2FW_BF16);
 }
 
-// The fp32 matrix-core kernels (T2FW_FLAG_TILES) cover states of up to 64 x 64 with 64 steps between checkpoints.
-bool tile_shape_ok(int64_t D, int64_t K, int32_t dtype, int32_t flags) {
-    return (flags & T2FW_FLAG_TILES) != 0 && (flags & T2FW_FLAG_FORCE_SCAN) == 0 && D <= CH_N && K <= CH_N && dtype != T2FW_F64 &&
-           !chunk_shape_ok(D, K, dtype, flags);
-}
-// Their backward's scratch: per (row, chunk) the adjoint [64][64] fp32, two vectors of gate products, a flag and a list entry
-struct TileScratch {
-    size_t tots, flags, list, total;           // byte offsets from the start of the workspace
-};
-TileScratch tile_scratch(int64_t B, int64_t T) {
-    const size_t items = (size_t)(B * (T <= 0 ? 1 : (T + TILE_CHUNK - 1) / TILE_CHUNK));
-    TileScratch s;
-    s.tots = items * (CH_N * CH_N * 4);
-    s.flags = s.tots + items * (2 * CH_N * 4);
-    s.list = s.flags + (items * 4 + 255) / 256 * 256;
-    s.total = s.list + (items * 4 + 4 + 255) / 256 * 256;
-    return s;
-}
-
 // compute units of the current device (-1 on error)
 int compute_units() {
     int dev = 0, n = 0;
@@ -176,7 +156,6 @@ size_t backward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int3
         const size_t inner = par_ok(B, T, Cd, flags) ? par_scratch(B, T, Cd).total : 2 * row_flag_bytes(B);
         return Cd == C ? inner : dense_scratch(inner, B, T, Cd, elem_size(dtype)).total;
     }
-    if (B > 0 && C == TILE_CHUNK && tile_shape_ok(D, K, dtype, flags)) return tile_scratch(B, T).total;
     return 0;
 }
 
@@ -338,14 +317,6 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
         const bool split = 2 * chunk_rows_padded(B) <= cus;
         return chunk_forward(c, dtype, op, split, st);
     }
-    if (tile_shape_ok(D, K, dtype, flags) && (ckpt == nullptr || C == TILE_CHUNK) && T * heads < CHUNK_MAX_T && B <= 0x3fffffff) {
-        TileFwdArgs t{};
-        t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.s0 = s0;
-        t.out = out; t.next_state = next_state; t.ckpt = ckpt;
-        t.B = B; t.T = T; t.NC = a.NC;
-        t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
-        return tile_forward(t, dtype, st);
-    }
     return scan_forward(a, dtype, st);
 }
 
@@ -483,23 +454,6 @@ static int lfw_backward_rows(const void *g_out, const void *g_state, const void 
         const int op = (dtype == T2FW_F16 && (flags & T2FW_FLAG_FP16_OPERANDS)) ? 1 : 0;
         c.redo = (flags & T2FW_FLAG_NO_FIXUP) ? 0 : 1;
         return chunk_backward(c, dtype, op, st);
-    }
-    if (tile_shape_ok(D, K, dtype, flags) && C_given == TILE_CHUNK && T * heads < CHUNK_MAX_T && B * a.NC <= 0x0fffffff) {
-        const TileScratch sc = tile_scratch(B, T);
-        if (workspace == nullptr || workspace_bytes < sc.total)
-            return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", sc.total, workspace_bytes);
-        if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
-        unsigned char *const ws = static_cast<unsigned char *>(workspace);
-        TileBwdArgs t{};
-        t.g_out = g_out; t.g_state = g_state; t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.ckpt = ckpt;
-        t.d_x = d_x; t.d_f = d_f; t.d_q = d_q; t.d_k = d_k; t.d_f_key = d_f_key; t.d_s0 = d_s0;
-        t.gh = reinterpret_cast<float *>(ws);
-        t.tots = reinterpret_cast<float *>(ws + sc.tots);
-        t.flags = reinterpret_cast<int32_t *>(ws + sc.flags);
-        t.list = reinterpret_cast<int32_t *>(ws + sc.list);
-        t.B = B; t.T = T; t.NC = a.NC;
-        t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
-        return tile_backward(t, dtype, st);
     }
     a.C = C_given;
     a.NC = t2fw_lfw_num_ckpt(T, C_given);

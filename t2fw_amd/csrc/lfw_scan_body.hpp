@@ -182,11 +182,7 @@ __device__ __forceinline__ void bwd_scan_body_kg(const ScanBwdArgs &p, int64_t b
     auto el_ok = [&](int j) -> bool { return row_ok && g.k0 + j < colw; };
 
     Acc G[KPL];
-    if (p.g_end != nullptr) {
-#pragma unroll
-        for (int j = 0; j < KPL; ++j)
-            G[j] = el_ok(j) ? Acc(p.g_end[SIDE == 0 ? row * 64 + g.k0 + j : (g.k0 + j) * 64 + row]) : Acc(0);
-    } else {
+    {
         const IO *gs = (const IO *)p.g_state + b * DK;
 #pragma unroll
         for (int j = 0; j < KPL; ++j) G[j] = el_ok(j) ? to_acc(gs[st_off(j)]) : Acc(0);
@@ -340,7 +336,7 @@ __device__ __forceinline__ void bwd_scan_body_kg(const ScanBwdArgs &p, int64_t b
             }
         }
     }
-    if (SIDE == 0 && p.g_end == nullptr) {
+    if (SIDE == 0) {
         IO *ds = (IO *)p.d_s0 + b * DK;
 #pragma unroll
         for (int j = 0; j < KPL; ++j)

@@ -73,27 +73,6 @@ def _dtype_code(dtype):
         raise RuntimeError("t2fw: unsupported dtype %s" % dtype)
 
 
-# Steps from which the fp32 matrix-core kernels (four launches backward, one forward) are faster than the exact
-# per-step ones (two and one), whose time is steps times the latency of one step.  GPU time of forward + backward, exact
-# against tiles, microseconds: 64 x 64 float32, 96 rows: 30 / 27 at 16 steps, 47 / 31 at 32; 33 x 17 float16, 96 rows:
-# 25 / 27 and 39 / 31.  A forward call alone with widths of one 16-channel block wastes most of a workgroup: 4 x 4
-# float32, 1024 rows: 27 / 34 at 32 steps, 46 / 38 at 64.
-TILES_MIN_STEPS = 32
-TILES_MIN_STEPS_NARROW_FORWARD = 64
-
-
-def _tile_flags(T, D, K, C, dtype, flags, need_grad=True):
-    """``flags`` of a call whose shape the 16-bit matrix-core kernels do not take, with T2FW_FLAG_TILES added where the
-    fp32 matrix-core kernels serve it (states of up to 64 x 64, checkpoints every 64 steps); a caller's own flags stand."""
-    if flags != _lib.FLAG_AUTO or C != 64 or D > 64 or K > 64 or dtype == torch.float64:
-        return flags
-    if T < (TILES_MIN_STEPS if need_grad or D > 16 or K > 16 else TILES_MIN_STEPS_NARROW_FORWARD):
-        return flags
-    if D == 64 and K == 64 and dtype != torch.float32:
-        return flags
-    return flags | _lib.FLAG_TILES
-
-
 # ---- widths that are multiples of 64 (other than 64 x 64) as independent 64 x 64 blocks -------------------
 # The recurrence couples neither the rows of the state nor its columns: S[d, k] sees x[d], f[d], k[k], f_key[k]
 # only, and o[d] is a sum over k.  A D x K state is (D / 64) (K / 64) independent 64 x 64 recurrences -- value
@@ -218,7 +197,6 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
         return _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
     lib = _lib.load()
     C = _ckpt_interval()
-    flags = _tile_flags(T, D, K, C, value.dtype, flags, need_grad)
     dev = value.device
     nc, ws_bytes, _, regions = _sizes(B * H, T, D, K, C, code, flags)
     with _on_device(dev):
