@@ -99,6 +99,14 @@ extern "C" {
                                      bf16 tensors it costs next to nothing in accuracy (what is stored is
                                      rounded to bf16 either way).  Off unless passed.                 */
 
+#define T2FW_FLAG_EXACT_CHUNKS 32 /* decay rule, states of up to 64 x 64 that the 16-bit matrix-core kernels do not take
+                                     (fp32 tensors, other widths): the exact recurrence with the 64-step chunks of a row
+                                     side by side, for a checkpoint interval of 64 (a forward call without checkpoints:
+                                     any).  Forward and backward need the workspace that t2fw_lfw_forward_workspace_bytes
+                                     and t2fw_lfw_workspace_bytes report for these flags.  Rows with a gate of magnitude
+                                     above one are done step by step over the whole sequence in the same call.  More than
+                                     65536 rows x chunks: the flag is ignored. */
+
 int t2fw_abi_version(void);
 const char *t2fw_last_error(void);
 

@@ -4,6 +4,7 @@
 #include "lfw_scan.hpp"
 #include "lfw_chunk.hpp"
 #include "lfw_par.hpp"
+#include "lfw_xpar.hpp"
 #include "dfw_scan.hpp"
 #include "cast.hpp"
 #include "gate.hpp"
@@ -84,6 +85,33 @@ bool chunk_shape_ok(int64_t D, int64_t K, int32_t dtype, int32_t flags) {
     return (flags & T2FW_FLAG_FORCE_SCAN) == 0 && D == 64 && K == 64 && (dtype == T2FW_F16 || dtype == T2FW_BF16);
 }
 
+// The chunk-parallel exact kernels (T2FW_FLAG_EXACT_CHUNKS) cover states of up to 64 x 64 that the 16-bit matrix-core
+// kernels do not take; the scratch is bounded (16 KB per row and chunk of 64 steps, 1 GB).
+constexpr int64_t XPAR_MAX_ITEMS = 65536;
+int64_t xpar_chunks(int64_t T) { return T <= 0 ? 1 : (T + XP_CHUNK - 1) / XP_CHUNK; }
+bool xpar_ok(int64_t B, int64_t T, int64_t D, int64_t K, int32_t dtype, int32_t flags) {
+    return (flags & T2FW_FLAG_EXACT_CHUNKS) != 0 && (flags & T2FW_FLAG_FORCE_SCAN) == 0 && D <= XP_N && K <= XP_N &&
+           dtype != T2FW_F64 && !chunk_shape_ok(D, K, dtype, flags) && B > 0 && T > 0 && B <= XPAR_MAX_ITEMS &&
+           xpar_chunks(T) <= XPAR_MAX_ITEMS / B;
+}
+size_t xpar_workspace_bytes(int64_t B, int64_t T) {
+    const size_t items = (size_t)(B * xpar_chunks(T));
+    return items * (XP_N * XP_N * 4 + 2 * XP_N * 4) + (items * 4 + 255) / 256 * 256 + ((size_t)B * 16 + 255) / 256 * 256;
+}
+XparScratch xpar_scratch(void *workspace, int64_t B, int64_t T) {
+    const size_t items = (size_t)(B * xpar_chunks(T));
+    unsigned char *w = static_cast<unsigned char *>(workspace);
+    XparScratch s;
+    s.states = reinterpret_cast<float *>(w);
+    w += items * (XP_N * XP_N * 4);
+    s.tots = reinterpret_cast<float *>(w);
+    w += items * (2 * XP_N * 4);
+    s.chunk_flags = reinterpret_cast<int32_t *>(w);
+    w += (items * 4 + 255) / 256 * 256;
+    s.row_flags = reinterpret_cast<int32_t *>(w);
+    return s;
+}
+
 // compute units of the current device (-1 on error)
 int compute_units() {
     int dev = 0, n = 0;
@@ -123,8 +151,9 @@ ParScratch par_scratch(int64_t B, int64_t T, int32_t C) {
     return s;
 }
 
-size_t forward_workspace_bytes(int64_t B, int64_t D, int64_t K, int32_t dtype, int32_t flags) {
+size_t forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32_t dtype, int32_t flags) {
     if (B > 0 && chunk_shape_ok(D, K, dtype, flags)) return 2 * row_flag_bytes(B);
+    if (xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T);
     return 0;
 }
 
@@ -156,6 +185,7 @@ size_t backward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int3
         const size_t inner = par_ok(B, T, Cd, flags) ? par_scratch(B, T, Cd).total : 2 * row_flag_bytes(B);
         return Cd == C ? inner : dense_scratch(inner, B, T, Cd, elem_size(dtype)).total;
     }
+    if (C == XP_CHUNK && xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T);
     return 0;
 }
 
@@ -217,15 +247,15 @@ int64_t t2fw_lfw_num_ckpt(int64_t T, int32_t C) {
 
 size_t t2fw_lfw_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32_t C, int32_t dtype,
                                 int32_t flags) {
-    const size_t fwd = forward_workspace_bytes(B, D, K, dtype, flags);
+    const size_t fwd = forward_workspace_bytes(B, T, D, K, dtype, flags);
     const size_t bwd = backward_workspace_bytes(B, T, D, K, C, dtype, flags);
     return fwd > bwd ? fwd : bwd;
 }
 
 size_t t2fw_lfw_forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32_t C, int32_t dtype,
                                         int32_t flags) {
-    (void)T; (void)C;
-    return forward_workspace_bytes(B, D, K, dtype, flags);
+    (void)C;
+    return forward_workspace_bytes(B, T, D, K, dtype, flags);
 }
 
 int t2fw_host_workspace_device_pointer(void *host_workspace, void **device_pointer) {
@@ -298,7 +328,7 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
 
     if (chunk_shape_ok(D, K, dtype, flags) && (ckpt == nullptr || C % 32 == 0) && T * heads < CHUNK_MAX_T &&
         aligned16({x, f, q, k, f_key, s0, out, next_state, ckpt})) {
-        const size_t need = forward_workspace_bytes(B, D, K, dtype, flags);
+        const size_t need = forward_workspace_bytes(B, T, D, K, dtype, flags);
         if (workspace == nullptr || workspace_bytes < need)
             return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
@@ -316,6 +346,19 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
         if (cus < 0) return fail(T2FW_ERR_HIP, "could not read the device's compute-unit count");
         const bool split = 2 * chunk_rows_padded(B) <= cus;
         return chunk_forward(c, dtype, op, split, st);
+    }
+    if (xpar_ok(B, T, D, K, dtype, flags) && (ckpt == nullptr || C == XP_CHUNK) && T * heads < CHUNK_MAX_T) {
+        const size_t need = xpar_workspace_bytes(B, T);
+        if (workspace == nullptr || workspace_bytes < need)
+            return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+        if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
+        XparFwdArgs t{};
+        t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.s0 = s0;
+        t.out = out; t.next_state = next_state; t.ckpt = ckpt;
+        t.ws = xpar_scratch(workspace, B, T);
+        t.B = B; t.T = T; t.NC = xpar_chunks(T);
+        t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
+        return xpar_forward(t, dtype, st);
     }
     return scan_forward(a, dtype, st);
 }
@@ -454,6 +497,19 @@ static int lfw_backward_rows(const void *g_out, const void *g_state, const void 
         const int op = (dtype == T2FW_F16 && (flags & T2FW_FLAG_FP16_OPERANDS)) ? 1 : 0;
         c.redo = (flags & T2FW_FLAG_NO_FIXUP) ? 0 : 1;
         return chunk_backward(c, dtype, op, st);
+    }
+    if (C_given == XP_CHUNK && xpar_ok(B, T, D, K, dtype, flags) && T * heads < CHUNK_MAX_T) {
+        const size_t need = xpar_workspace_bytes(B, T);
+        if (workspace == nullptr || workspace_bytes < need)
+            return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+        if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
+        XparBwdArgs t{};
+        t.g_out = g_out; t.g_state = g_state; t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.ckpt = ckpt;
+        t.d_x = d_x; t.d_f = d_f; t.d_q = d_q; t.d_k = d_k; t.d_f_key = d_f_key; t.d_s0 = d_s0;
+        t.ws = xpar_scratch(workspace, B, T);
+        t.B = B; t.T = T; t.NC = a.NC;
+        t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
+        return xpar_backward(t, dtype, st);
     }
     a.C = C_given;
     a.NC = t2fw_lfw_num_ckpt(T, C_given);

@@ -45,7 +45,9 @@ __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b
     Acc S[KPL];
 #pragma unroll
     for (int j = 0; j < KPL; ++j)
-        S[j] = (row_ok && g.k0 + j < KW) ? to_acc(s0[(b * D + d) * K + col0 + g.k0 + j]) : Acc(0);
+        S[j] = !(row_ok && g.k0 + j < KW) ? Acc(0)
+               : p.s_start != nullptr     ? Acc(p.s_start[d * 64 + g.k0 + j])
+                                          : to_acc(s0[(b * D + d) * K + col0 + g.k0 + j]);
 
     // outputs of a block of steps: written, or added to what the passes over other key channels left
     auto flush = [&](int n_blk, int64_t t_blk) {
@@ -110,7 +112,7 @@ __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b
     }
     __syncthreads();
     flush(n_prev, t_prev);
-    if (row_ok) {
+    if (row_ok && next_state != nullptr) {
 #pragma unroll
         for (int j = 0; j < KPL; ++j)
             if (g.k0 + j < KW) next_state[(b * D + d) * K + col0 + g.k0 + j] = from_acc<IO>(S[j]);
@@ -182,7 +184,11 @@ __device__ __forceinline__ void bwd_scan_body_kg(const ScanBwdArgs &p, int64_t b
     auto el_ok = [&](int j) -> bool { return row_ok && g.k0 + j < colw; };
 
     Acc G[KPL];
-    {
+    if (p.g_end != nullptr) {
+#pragma unroll
+        for (int j = 0; j < KPL; ++j)
+            G[j] = el_ok(j) ? Acc(p.g_end[SIDE == 0 ? row * 64 + g.k0 + j : (g.k0 + j) * 64 + row]) : Acc(0);
+    } else {
         const IO *gs = (const IO *)p.g_state + b * DK;
 #pragma unroll
         for (int j = 0; j < KPL; ++j) G[j] = el_ok(j) ? to_acc(gs[st_off(j)]) : Acc(0);
@@ -336,7 +342,7 @@ __device__ __forceinline__ void bwd_scan_body_kg(const ScanBwdArgs &p, int64_t b
             }
         }
     }
-    if (SIDE == 0) {
+    if (SIDE == 0 && p.d_s0 != nullptr) {
         IO *ds = (IO *)p.d_s0 + b * DK;
 #pragma unroll
         for (int j = 0; j < KPL; ++j)

@@ -1,0 +1,41 @@
+// Exact per-step recurrence, chunk-parallel: states of up to 64 x 64 of any width, fp32 / fp16 / bf16 tensors
+// (lfw_xpar.hip).
+#pragma once
+
+#include "common.hpp"
+
+namespace t2fw {
+
+constexpr int XP_CHUNK = 64;           // tokens per chunk, and between checkpoints
+constexpr int XP_N = 64;               // row stride of a chunk's state in the scratch
+
+struct XparScratch {
+    float *states;                     // [B * NC][64][64]: a chunk's increment, then the state (adjoint) entering it
+    float *tots;                       // [B * NC][2][64]: a chunk's gate products, value side and key side
+    int32_t *chunk_flags;              // [B * NC]
+    int32_t *row_flags;                // [B][4]: the row is left to the recurrence over the whole sequence
+};
+
+struct XparFwdArgs {
+    const void *x, *f, *q, *k, *f_key, *s0;
+    void *out, *next_state, *ckpt;     // ckpt may be null; else one state per chunk
+    XparScratch ws;
+    int64_t B, T, NC;
+    int32_t D, K, heads;
+};
+
+struct XparBwdArgs {
+    const void *g_out, *g_state, *x, *f, *q, *k, *f_key, *ckpt;
+    void *d_x, *d_f, *d_q, *d_k, *d_f_key, *d_s0;
+    XparScratch ws;
+    int64_t B, T, NC;
+    int32_t D, K, heads;
+};
+
+int xpar_forward(const XparFwdArgs &a, int dtype, hipStream_t stream);
+int xpar_backward(const XparBwdArgs &a, int dtype, hipStream_t stream);
+// launch 3 for fp32 tensors with D = K = 64 (lfw_xpar64.hip)
+int xpar64_forward(const XparFwdArgs &a, hipStream_t stream);
+int xpar64_backward(const XparBwdArgs &a, hipStream_t stream);
+
+}  // namespace t2fw

@@ -1,0 +1,387 @@
+// Launch 3 of the chunk-parallel exact recurrence (lfw_xpar.hip) for fp32 tensors with 64 x 64 states: the same steps in
+// the same arithmetic, laid out so that almost every VALU instruction is one of the recurrence's own.
+//
+// One workgroup of four waves per (row, chunk) [backward: and side].  A lane is a row of the state (value channels;
+// key channels on the backward's key side), a wave holds 16 of the other side's channels ("columns") in registers; lane
+// l also holds the inputs of column l % 16, which DPP broadcasts within each row of 16 lanes as an operand of the
+// multiplications: neither LDS nor scalar registers carry the inputs.  A contraction over columns, S_t q_t and the like,
+// is lane-local; the four waves' shares meet in LDS, eight steps at a time.  A state element costs 4 VALU instructions
+// per step forward and 12.75 / 13.75 backward (value / key side: 3.75 + 3 to rebuild the states, the rest for the adjoint
+// and the sums), the per-step kernels' arithmetic without their cross-lane sums.
+//
+// Backward, per chunk: the states at steps 16, 32 and 48 (LDS) are rebuilt from the checkpoint, blocks of 16 steps are
+// visited last to first, and per half block the eight states are rebuilt into registers and the adjoint runs back over
+// them.  A row that is left to the recurrence over the whole sequence (lfw_xpar.hip) is walked by the workgroup of its
+// first chunk, chunk by chunk, with the state or the adjoint kept.
+//
+// B = 96, T = 1024: forward 77 us (51 us of VALU issue), backward 557 us (about 290 us of issue at two waves per SIMD: the
+// rest is waiting for a segment's inputs).  The per-step kernels over whole rows take 220 and 813 us, their bodies on
+// chunks 154 and 600 us.
+// Tried and slower: rank-one terms on v_mfma_f32_4x4x1 (forward 115 us, backward 603), column vectors in scalar registers
+// (105 and 1145: every wave misses the scalar cache once per step and array).
+#include "lfw_chunk.hpp"
+#include "lfw_scan.hpp"
+#include "lfw_xpar.hpp"
+
+namespace t2fw {
+namespace {
+
+constexpr int XW_THREADS = 256;
+constexpr int XW_COLS = 16;            // columns per wave
+constexpr int XW_SEG = 8;              // steps whose inputs, states and sums are in flight together
+
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long long)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)v >> 32));
+    return (int64_t)(((unsigned long long)hi << 32) | lo);
+}
+
+// XW_SEG steps of one array, one value per lane.  p: the array at the segment's first step (wave-uniform), c: the lane's
+// channel; steps from n on are read from the last one (and replaced by pad_steps).
+__device__ __forceinline__ void load_steps(float (&r)[XW_SEG], const float *p, int c, int64_t ts, int n) {
+#pragma unroll
+    for (int j = 0; j < XW_SEG; ++j) r[j] = (p + min(j, n - 1) * ts)[(unsigned)c];
+}
+__device__ __forceinline__ void pad_steps(float (&r)[XW_SEG], int n, float pad) {
+#pragma unroll
+    for (int j = 0; j < XW_SEG; ++j) r[j] = j < n ? r[j] : pad;
+}
+
+// lane N of each row of 16, in every lane of the row
+template <int N> __device__ __forceinline__ float bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+// The compiler folds a broadcast into a multiplication but not into a multiply-add: those are written out.  Both blocks
+// start with the two wait states that a DPP read of a register just written by the VALU needs.
+//
+// sum over the wave's columns of S times the column vector (chains of four, as the per-step kernel's lanes)
+__device__ __forceinline__ float dot(const floatx4 (&S)[4], float col) {
+    float a0, a1, a2, a3;
+    asm("s_nop 1\n"
+        "v_mul_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %4, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %1, %4, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %2, %4, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %3, %4, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %4, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %1, %4, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %2, %4, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %3, %4, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %4, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %1, %4, %18 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %2, %4, %19 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %3, %4, %20 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
+        : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3)
+        : "v"(col), "v"(S[0][0]), "v"(S[0][1]), "v"(S[0][2]), "v"(S[0][3]), "v"(S[1][0]), "v"(S[1][1]), "v"(S[1][2]), "v"(S[1][3]), "v"(S[2][0]), "v"(S[2][1]), "v"(S[2][2]), "v"(S[2][3]), "v"(S[3][0]), "v"(S[3][1]), "v"(S[3][2]), "v"(S[3][3]));
+    return (a0 + a1) + (a2 + a3);
+}
+// G += (column vector) (x) (row vector)
+__device__ __forceinline__ void add_outer(floatx4 (&G)[4], float col, float row) {
+    float g[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) g[n] = G[n / 4][n % 4];
+    asm("s_nop 1\n"
+        "v_fmac_f32_dpp %0, %16, %17 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %1, %16, %17 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %2, %16, %17 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %3, %16, %17 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %4, %16, %17 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %5, %16, %17 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %6, %16, %17 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %7, %16, %17 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %8, %16, %17 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %9, %16, %17 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %10, %16, %17 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %11, %16, %17 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %12, %16, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %13, %16, %17 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %14, %16, %17 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %15, %16, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
+        : "+v"(g[0]), "+v"(g[1]), "+v"(g[2]), "+v"(g[3]), "+v"(g[4]), "+v"(g[5]), "+v"(g[6]), "+v"(g[7]), "+v"(g[8]), "+v"(g[9]), "+v"(g[10]), "+v"(g[11]), "+v"(g[12]), "+v"(g[13]), "+v"(g[14]), "+v"(g[15])
+        : "v"(col), "v"(row));
+#pragma unroll
+    for (int n = 0; n < 16; ++n) G[n / 4][n % 4] = g[n];
+}
+
+// What follows (volatile) does not start before v is there: keeps the steps apart, whose products would not fit the
+// registers all at once.
+__device__ __forceinline__ void settle(floatx4 (&v)[4]) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+__device__ __forceinline__ void settle(float &a, float &b, float &c, float &d) {
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+
+// S <- S * (f (x) f_key) + x (x) k
+template <int Q> __device__ __forceinline__ void step4(floatx4 &out, const floatx4 &S, float ca, float cf, float ra, float rf) {
+    out[0] = fmaf(S[0], bcast<4 * Q + 0>(cf) * rf, bcast<4 * Q + 0>(ca) * ra);
+    out[1] = fmaf(S[1], bcast<4 * Q + 1>(cf) * rf, bcast<4 * Q + 1>(ca) * ra);
+    out[2] = fmaf(S[2], bcast<4 * Q + 2>(cf) * rf, bcast<4 * Q + 2>(ca) * ra);
+    out[3] = fmaf(S[3], bcast<4 * Q + 3>(cf) * rf, bcast<4 * Q + 3>(ca) * ra);
+}
+__device__ __forceinline__ void step(floatx4 (&out)[4], const floatx4 (&S)[4], float ca, float cf, float ra, float rf) {
+    step4<0>(out[0], S[0], ca, cf, ra, rf);
+    step4<1>(out[1], S[1], ca, cf, ra, rf);
+    step4<2>(out[2], S[2], ca, cf, ra, rf);
+    step4<3>(out[3], S[3], ca, cf, ra, rf);
+}
+// G *= (column vector) (x) (row vector)
+__device__ __forceinline__ void scale_outer(floatx4 (&G)[4], float col, float row) {
+    float g[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) g[n] = G[n / 4][n % 4];
+    asm("s_nop 1\n"
+        "v_mul_f32_dpp %0, %16, %0 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %1, %16, %1 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %2, %16, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %3, %16, %3 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %4, %16, %4 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %5, %16, %5 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %6, %16, %6 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %7, %16, %7 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %8, %16, %8 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %9, %16, %9 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %10, %16, %10 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %11, %16, %11 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %12, %16, %12 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %13, %16, %13 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %14, %16, %14 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %15, %16, %15 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
+        : "+v"(g[0]), "+v"(g[1]), "+v"(g[2]), "+v"(g[3]), "+v"(g[4]), "+v"(g[5]), "+v"(g[6]), "+v"(g[7]), "+v"(g[8]), "+v"(g[9]), "+v"(g[10]), "+v"(g[11]), "+v"(g[12]), "+v"(g[13]), "+v"(g[14]), "+v"(g[15])
+        : "v"(col));
+#pragma unroll
+    for (int n = 0; n < 16; ++n) G[n / 4][n % 4] = g[n] * row;
+}
+
+__device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
+    const int4 v = *reinterpret_cast<const int4 *>(ws.row_flags + 4 * b);
+    return __builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0;
+}
+
+// 16 consecutive columns of row `row` of a [64][64] state, or 16 rows of column `row` (TRANSPOSED); p, col0 wave-uniform,
+// p aligned to its elements
+struct __attribute__((packed, aligned(4))) Float4 {
+    float v[4];
+};
+template <bool TRANSPOSED> __device__ __forceinline__ void load_state(floatx4 (&S)[4], const float *p, int row, int col0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (TRANSPOSED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[q][e] = (p + (col0 + 4 * q + e) * XP_N)[(unsigned)row];
+        } else {
+            const Float4 v = *reinterpret_cast<const Float4 *>((p + col0 + 4 * q) + (unsigned)(row * XP_N));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[q][e] = v.v[e];
+        }
+    }
+}
+__device__ __forceinline__ void store_state(float *p, const floatx4 (&S)[4], int row, int col0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<Float4 *>((p + col0 + 4 * q) + (unsigned)(row * XP_N)) = Float4{{S[q][0], S[q][1], S[q][2], S[q][3]}};
+}
+
+// ---- forward --------------------------------------------------------------------------------------
+__global__ __launch_bounds__(XW_THREADS) void lfw_xpar64_fwd_kernel(XparFwdArgs p) {
+    __shared__ float part[2][XW_SEG][4][XP_N];
+    const int64_t item = blockIdx.x, b = item / p.NC;
+    const int chunk = (int)(item - b * p.NC);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col0 = XW_COLS * w;
+    const bool whole = row_left(p.ws, b);
+    if (whole && chunk != 0) return;
+    const int T = (int)p.T, t_end = whole ? T : min(T, (chunk + 1) * XP_CHUNK);
+    const int64_t ts = (int64_t)p.heads * XP_N, line0 = uniform64(row_first_token(b, p.T, p.heads)) * XP_N;
+    const float *const x = (const float *)p.x + line0, *const f = (const float *)p.f + line0;
+    const float *const k = (const float *)p.k + line0 + col0, *const fk = (const float *)p.f_key + line0 + col0;
+    const int cl = lane & 15;
+    const float *const q = (const float *)p.q + line0 + col0;
+    float *const out = (float *)p.out + line0;
+    float *const ckpt = (float *)p.ckpt;
+    floatx4 S[4];
+    load_state<false>(S, whole ? (const float *)p.s0 + b * (XP_N * XP_N) : p.ws.states + item * (XP_N * XP_N), lane, col0);
+    int buf = 0;
+    float rx[XW_SEG], rf[XW_SEG], ck[XW_SEG], cf[XW_SEG], cq[XW_SEG];
+    auto fetch = [&](int t0) {
+        const int n = t_end - t0;
+        load_steps(rx, x + t0 * ts, lane, ts, n);
+        load_steps(rf, f + t0 * ts, lane, ts, n);
+        load_steps(ck, k + t0 * ts, cl, ts, n);
+        load_steps(cf, fk + t0 * ts, cl, ts, n);
+        load_steps(cq, q + t0 * ts, cl, ts, n);
+        if (n < XW_SEG) {
+            pad_steps(rx, n, 0.f);
+            pad_steps(rf, n, 1.f);
+            pad_steps(ck, n, 0.f);
+            pad_steps(cf, n, 1.f);
+        }
+    };
+    int t0 = chunk * XP_CHUNK;
+    fetch(t0);
+    for (; t0 < t_end; t0 += XW_SEG, buf ^= 1) {
+        const int n = min(XW_SEG, t_end - t0);
+        if (ckpt != nullptr && (t0 & (XP_CHUNK - 1)) == 0)
+            store_state(ckpt + (b * p.NC + (t0 / XP_CHUNK)) * (XP_N * XP_N), S, lane, col0);
+        float cx[XW_SEG], cff[XW_SEG], kx[XW_SEG], kf[XW_SEG], kq[XW_SEG];
+#pragma unroll
+        for (int j = 0; j < XW_SEG; ++j) {
+            cx[j] = rx[j]; cff[j] = rf[j]; kx[j] = ck[j]; kf[j] = cf[j]; kq[j] = cq[j];
+        }
+        if (t0 + XW_SEG < t_end) fetch(t0 + XW_SEG);
+#pragma unroll
+        for (int j = 0; j < XW_SEG; ++j) {
+            step(S, S, kx[j], kf[j], cx[j], cff[j]);
+            part[buf][j][w][lane] = dot(S, kq[j]);
+        }
+        __syncthreads();                 // the shares of this segment are there; the other buffer is free again
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int j = w + 4 * u;
+            const float(*const s)[XP_N] = part[buf][j];
+            if (j < n) (out + (t0 + j) * ts)[(unsigned)lane] = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+        }
+    }
+    if (t_end == T) store_state((float *)p.next_state + b * (XP_N * XP_N), S, lane, col0);
+}
+
+// ---- backward -------------------------------------------------------------------------------------
+constexpr int XW_BLOCK = 2 * XW_SEG;
+struct BwdSmem {
+    float part[3][XW_SEG][4][XP_N];
+    float start[3][XW_COLS][XW_THREADS];      // states at steps 16, 32 and 48 of a chunk, lane-private
+};
+static_assert(2 * sizeof(BwdSmem) <= 160 * 1024, "two workgroups must fit the LDS of one CU");
+
+template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdArgs &p, BwdSmem &sm, int64_t b, int chunk, bool whole) {
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col0 = XW_COLS * w;
+    const int64_t ts = (int64_t)p.heads * XP_N, line0 = uniform64(row_first_token(b, p.T, p.heads)) * XP_N;
+    const float *const ra = (const float *)(SIDE ? p.k : p.x) + line0, *const rf = (const float *)(SIDE ? p.f_key : p.f) + line0;
+    const float *const ru = (const float *)(SIDE ? p.q : p.g_out) + line0;
+    const float *const ca = (const float *)(SIDE ? p.x : p.k) + line0 + col0, *const cf = (const float *)(SIDE ? p.f : p.f_key) + line0 + col0;
+    const float *const cu = (const float *)(SIDE ? p.g_out : p.q) + line0 + col0;
+    float *const d_a = (float *)(SIDE ? p.d_k : p.d_x) + line0, *const d_f = (float *)(SIDE ? p.d_f_key : p.d_f) + line0;
+    float *const d_u = (float *)p.d_q + line0;
+    const int cl = lane & 15;
+    floatx4 S[4], G[4];
+
+    // S over the eight steps from t0
+    auto advance = [&](int t0) {
+        float va[XW_SEG], vf[XW_SEG], ka[XW_SEG], kf[XW_SEG];
+        load_steps(va, ra + t0 * ts, lane, ts, XW_SEG);
+        load_steps(vf, rf + t0 * ts, lane, ts, XW_SEG);
+        load_steps(ka, ca + t0 * ts, cl, ts, XW_SEG);
+        load_steps(kf, cf + t0 * ts, cl, ts, XW_SEG);
+#pragma unroll
+        for (int j = 0; j < XW_SEG; ++j) step(S, S, ka[j], kf[j], va[j], vf[j]);
+    };
+    // The segment [t0, t0 + n): its states rebuilt from S, the adjoint back over them, the sums stored.
+    auto reverse = [&](int t0, int n) {
+        float va[XW_SEG], vf[XW_SEG], vu[XW_SEG], ka[XW_SEG], kf[XW_SEG], ku[XW_SEG];
+        load_steps(va, ra + t0 * ts, lane, ts, n);
+        load_steps(vf, rf + t0 * ts, lane, ts, n);
+        load_steps(ka, ca + t0 * ts, cl, ts, n);
+        load_steps(kf, cf + t0 * ts, cl, ts, n);
+        if (n < XW_SEG) {
+            pad_steps(va, n, 0.f);
+            pad_steps(vf, n, 1.f);
+            pad_steps(ka, n, 0.f);
+            pad_steps(kf, n, 1.f);
+        }
+        floatx4 st[XW_SEG + 1][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) st[0][q] = S[q];
+#pragma unroll
+        for (int j = 0; j < XW_SEG; ++j) {
+            settle(ka[j], kf[j], va[j], vf[j]);
+            step(st[j + 1], st[j], ka[j], kf[j], va[j], vf[j]);
+            settle(st[j + 1]);
+            if (j == XW_SEG / 2) {
+                load_steps(vu, ru + t0 * ts, lane, ts, n);
+                load_steps(ku, cu + t0 * ts, cl, ts, n);
+            }
+        }
+        pad_steps(vu, n, 0.f);
+        pad_steps(ku, n, 0.f);
+        __syncthreads();                 // the sums of the segment before have been read
+#pragma unroll
+        for (int j = XW_SEG - 1; j >= 0; --j) {
+            settle(ku[j], kf[j], vu[j], vf[j]);
+            add_outer(G, ku[j], vu[j]);      // G_t = g_t (x) q_t + ...
+            floatx4 w_[4];
+            sm.part[0][j][w][lane] = dot(G, ka[j]);                                      // d_x / d_k
+            if (SIDE == 1) sm.part[2][j][w][lane] = dot(st[j + 1], ku[j]);               // d_q
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w_[q] = G[q] * st[j][q];
+            sm.part[1][j][w][lane] = dot(w_, kf[j]);                                     // d_f / d_f_key
+            scale_outer(G, kf[j], vf[j]);
+            settle(G);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < (SIDE ? 3 : 2); ++o)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int j = w + 4 * h;
+                const float(*const s)[XP_N] = sm.part[o][j];
+                if (j < n) ((o == 0 ? d_a : o == 1 ? d_f : d_u) + (t0 + j) * ts)[(unsigned)lane] = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+            }
+    };
+
+    const float *const g_end = whole ? (const float *)p.g_state + b * (XP_N * XP_N) : p.ws.states + (b * p.NC + chunk) * (XP_N * XP_N);
+    load_state<SIDE == 1>(G, g_end, lane, col0);
+    for (int c = whole ? (int)p.NC - 1 : chunk; c >= chunk; --c) {
+        const float *const s0 = (const float *)p.ckpt + (b * p.NC + c) * (XP_N * XP_N);
+        const int tc = c * XP_CHUNK, len = (int)min((int64_t)XP_CHUNK, p.T - tc), nblk = (len + XW_BLOCK - 1) / XW_BLOCK;
+        load_state<SIDE == 1>(S, s0, lane, col0);
+        for (int blk = 1; blk < nblk; ++blk) {           // to the start of the last block
+            advance(tc + XW_BLOCK * (blk - 1));
+            advance(tc + XW_BLOCK * (blk - 1) + XW_SEG);
+#pragma unroll
+            for (int u = 0; u < XW_COLS; ++u) sm.start[blk - 1][u][tid] = S[u / 4][u % 4];
+        }
+        for (int blk = nblk - 1; blk >= 0; --blk) {
+            const int t0 = tc + XW_BLOCK * blk, n = min(XW_BLOCK, tc + len - t0);
+            for (int half = n > XW_SEG ? 1 : 0; half >= 0; --half) {
+                if (blk == 0) {
+                    load_state<SIDE == 1>(S, s0, lane, col0);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < XW_COLS; ++u) S[u / 4][u % 4] = sm.start[blk - 1][u][tid];
+                }
+                if (half) advance(t0);
+                reverse(t0 + XW_SEG * half, min(n - XW_SEG * half, XW_SEG));
+            }
+        }
+    }
+    if (SIDE == 0 && chunk == 0) store_state((float *)p.d_s0 + b * (XP_N * XP_N), G, lane, col0);
+}
+
+__global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_kernel(XparBwdArgs p) {
+    __shared__ BwdSmem sm;
+    const int64_t item = blockIdx.x >> 1, b = item / p.NC;
+    const int chunk = (int)(item - b * p.NC);
+    const bool whole = row_left(p.ws, b);
+    if (whole && chunk != 0) return;
+    if ((blockIdx.x & 1) == 0)
+        backward_side<0>(p, sm, b, chunk, whole);
+    else
+        backward_side<1>(p, sm, b, chunk, whole);
+}
+
+}  // namespace
+
+int xpar64_forward(const XparFwdArgs &a, hipStream_t stream) {
+    hipLaunchKernelGGL(lfw_xpar64_fwd_kernel, dim3((unsigned)(a.B * a.NC)), dim3(XW_THREADS), 0, stream, a);
+    return check_hip(hipGetLastError(), "lfw_xpar64_fwd_kernel launch");
+}
+
+int xpar64_backward(const XparBwdArgs &a, hipStream_t stream) {
+    hipLaunchKernelGGL(lfw_xpar64_bwd_kernel, dim3((unsigned)(2 * a.B * a.NC)), dim3(XW_THREADS), 0, stream, a);
+    return check_hip(hipGetLastError(), "lfw_xpar64_bwd_kernel launch");
+}
+
+}  // namespace t2fw

@@ -73,6 +73,26 @@ def _dtype_code(dtype):
         raise RuntimeError("t2fw: unsupported dtype %s" % dtype)
 
 
+# Where the chunk-parallel exact kernels (three launches per direction) take the place of the per-step ones (one launch
+# forward, two backward).  Forward + backward, per-step against chunk-parallel, microseconds: 96 rows of 64 x 64 float32,
+# 128 steps 180 / 192 (host-bound: the launches), 256 steps 264 / 216, 1024 steps 1005 / 673; 13 rows of 33 x 17 float16,
+# 128 steps 177 / 195, 385 steps 338 / 193.  Many rows fill the chip by themselves: 512 rows of 64 x 64, 256 steps 872 /
+# 886; 1024 rows of 16 x 16 277 / 364.
+EXACT_CHUNKS_MIN_STEPS = 224
+EXACT_CHUNKS_MAX_TILES = 1024          # rows x blocks of 16 channels
+
+
+def _exact_chunk_flags(rows, T, D, K, C, dtype, flags):
+    """``flags`` of a call that the 16-bit matrix-core kernels do not take, with FLAG_EXACT_CHUNKS added where the
+    chunk-parallel exact kernels serve it (states of up to 64 x 64, checkpoints every 64 steps); a caller's own flags
+    stand."""
+    if flags != _lib.FLAG_AUTO or C != 64 or D > 64 or K > 64 or T < EXACT_CHUNKS_MIN_STEPS or dtype == torch.float64:
+        return flags
+    if (D == 64 and K == 64 and dtype != torch.float32) or rows * -(-max(D, K) // 16) > EXACT_CHUNKS_MAX_TILES:
+        return flags
+    return flags | _lib.FLAG_EXACT_CHUNKS
+
+
 # ---- widths that are multiples of 64 (other than 64 x 64) as independent 64 x 64 blocks -------------------
 # The recurrence couples neither the rows of the state nor its columns: S[d, k] sees x[d], f[d], k[k], f_key[k]
 # only, and o[d] is a sum over k.  A D x K state is (D / 64) (K / 64) independent 64 x 64 recurrences -- value
@@ -197,6 +217,7 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
         return _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
     lib = _lib.load()
     C = _ckpt_interval()
+    flags = _exact_chunk_flags(B * H, T, D, K, C, value.dtype, flags)
     dev = value.device
     nc, ws_bytes, _, regions = _sizes(B * H, T, D, K, C, code, flags)
     with _on_device(dev):
@@ -271,7 +292,7 @@ class LFWFunction(torch.autograd.Function):
     Inputs are already gated (no sigmoid is applied here), as in the reference.
     fp16 / bf16 tensors with D = K = 64 run on the matrix-core kernels, those whose widths are other multiples
     of 64 as independent 64 x 64 blocks on the same kernels (``_block_counts`` above), everything else on the
-    exact per-step kernels; T2FW_FLAGS=1 keeps the exact kernels for every shape."""
+    exact kernels (per-step, or with the chunks of a row side by side: ``_exact_chunk_flags``); T2FW_FLAGS=1 keeps the exact kernels for every shape."""
 
     @staticmethod
     def forward(ctx, value, forget, query, key, f_key, state):

@@ -1,0 +1,89 @@
+"""The chunk-parallel exact kernels of the decay rule (T2FW_FLAG_EXACT_CHUNKS: float32 tensors, widths of up to 64)
+against the float64 oracle, at the tolerance of the per-step kernels (TOL of test_lfw_gpu).  Sizes sit on the edges of the
+kernels' pieces (8, 16 and 64 steps, 16 and 32 channels)."""
+import pytest
+import torch
+
+from tests.lfw_cases import make_config_inputs, make_reference_test_inputs
+from tests.test_lfw_gpu import NAMES, TOL, assert_close, check_all, oracle_all
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def exact_chunks(monkeypatch):
+    monkeypatch.setenv("T2FW_FLAGS", "32")
+
+
+F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
+
+
+@pytest.mark.parametrize("B,T,D,K,dtype", [
+    (1, 1, 64, 64, F32), (2, 7, 64, 64, F32), (2, 8, 64, 64, F32), (2, 9, 64, 64, F32), (2, 17, 64, 64, F32),
+    (3, 64, 64, 64, F32), (2, 65, 64, 64, F32), (2, 127, 64, 64, F32), (2, 1000, 64, 64, F32), (2, 80, 1, 1, F32),
+    (2, 80, 16, 17, F32), (1, 200, 63, 48, F32), (2, 65, 33, 64, F32), (2, 130, 64, 32, F32),
+    (2, 150, 17, 5, F16), (2, 64, 64, 49, F16), (2, 150, 31, 32, BF16),
+])
+def test_edges(B, T, D, K, dtype):
+    x, f, q, k, fk, s, go, gs = make_config_inputs(B, T, D, K, dtype, seed=T + D, in_scale=0.5, state_std=0.5, gate_mean=1.5)
+    check_all((x, f, q, k, fk, s), go, gs, dtype)
+
+
+def test_gates_down_to_one_sixty_fourth():
+    x, f, q, k, fk, s, go, gs = make_reference_test_inputs(3, 300, 64, 64, F32, seed=5)
+    check_all((x, f, q, k, fk, s), go, gs, F32)
+
+
+@pytest.mark.parametrize("what", ["zero", "tiny", "above one", "one side's product overflows", "negative", "large values"])
+@pytest.mark.parametrize("D,K,dtype", [(64, 64, F32), (20, 40, F32), (20, 40, BF16)])
+def test_unusual_gates_and_values(what, D, K, dtype):
+    """One row of three is out of the ordinary; gates above one send it through the whole sequence step by step."""
+    x, f, q, k, fk, s, go, gs = make_config_inputs(3, 150, D, K, dtype, seed=3, in_scale=0.5, state_std=0.5)
+    if what == "zero":
+        f[1, 70, 3] = 0
+        fk[1, 5, 7] = 0
+        fk[2, 149, 0] = 0
+    elif what == "tiny":
+        f[1, 64:80] = 2.0 ** -20
+    elif what == "above one":
+        fk[1, 100, 2] = 1.25
+    elif what == "one side's product overflows":
+        f[1, :, :] = 2.0 ** -6
+        fk[1, :, :] = 2.0 ** 5
+    elif what == "negative":
+        f[0, 30, 1] = -0.5
+    else:
+        x[1, 90] *= 2.0 ** 42
+    check_all((x, f, q, k, fk, s), go, gs, dtype)
+
+
+def test_nan_stays_in_its_row():
+    from t2fw_amd import LFWFunction
+    ins = [t.cuda() for t in make_config_inputs(3, 150, 64, 64, F32, seed=4)[:6]]
+    ref = LFWFunction.apply(*ins)
+    ins[0][1, 70, 5] = float("nan")
+    out, nxt = LFWFunction.apply(*ins)
+    for a, r in ((out, ref[0]), (nxt, ref[1])):
+        assert torch.equal(a[[0, 2]], r[[0, 2]])
+    assert torch.isnan(out[1, 70:, 5]).all()
+    # the row now runs step by step from its first state: the same terms, chunk states rounded in another order (both
+    # orders are within TOL[F32] of the exact sums)
+    assert_close(out[1, :70], ref[0][1, :70].cpu(), F32, "outputs before the NaN", tol=TOL[F32])
+
+
+def test_head_strided_tensors():
+    from t2fw_amd import LFWHeadsFunction
+    B, T, H = 2, 100, 3
+    heads = lambda t: t.view(B, H, T, -1).transpose(1, 2).contiguous().cuda()
+    rows = lambda t: t.transpose(1, 2).reshape(B * H, T, -1)
+    for D, K in ((64, 64), (40, 24)):
+        x, f, q, k, fk, s, go, gs = make_config_inputs(B * H, T, D, K, F32, seed=9, in_scale=0.5, state_std=0.5)
+        st = lambda t: t.view(B, H, D, K).contiguous().cuda()
+        ins = [heads(t).requires_grad_() for t in (x, f, q, k, fk)] + [st(s).requires_grad_()]
+        out, nxt = LFWHeadsFunction.apply(*ins)
+        grads = torch.autograd.grad([out, nxt], ins, [heads(go), st(gs)])
+        r_out, r_nxt, r_grads = oracle_all((x, f, q, k, fk, s), go, gs)
+        assert_close(rows(out), r_out, F32, "outputs", tol=TOL[F32])
+        assert_close(nxt.reshape(B * H, D, K), r_nxt, F32, "next_state", tol=TOL[F32])
+        for n, g, r in zip(NAMES, grads, r_grads):
+            assert_close(g.reshape(B * H, D, K) if n == "d_state" else rows(g), r, F32, n, tol=TOL[F32])
