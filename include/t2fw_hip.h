@@ -259,6 +259,22 @@ int t2fw_cast(const void *const *src, void *const *dst, const int64_t *n, int32_
               int32_t src_dtype, int32_t dst_dtype, void *stream);
 
 /*
+ * Strided copies of 64-element vectors, up to T2FW_BLOCK_COPY_MAX arrays of one dtype (f32 / f16 / bf16) in one launch:
+ *   dst[i0][i1][i2][i3][0..63] = sum over t < terms of src[i0 stride[0] + .. + i3 stride[3] + t term_stride + 0..63]
+ * dst is dense, strides are in elements (0 repeats), sums are carried in fp32 and rounded once.  What tensors whose
+ * widths are multiples of 64 need to run as independent 64 x 64 blocks, and to put the results together again.  No
+ * counterpart in the reference (one kernel serves every width there, lfw_kernel.cu:105-121).
+ */
+#define T2FW_BLOCK_COPY_MAX 8
+typedef struct t2fw_block_copy_desc {
+    const void *src;
+    void *dst;
+    int64_t size[4], stride[4];
+    int64_t terms, term_stride;
+} t2fw_block_copy_desc;
+int t2fw_block_copy(const t2fw_block_copy_desc *arrays, int32_t count, int32_t dtype, void *stream);
+
+/*
  * Sigmoid gating of both forget gates in one launch: f = sigmoid(f_logit) [n_f elements],
  * f_key = sigmoid(fk_logit) [n_fk elements]; outputs may alias the inputs.  The reference leaves
  * the non-linearity to the caller (functional_lfw.py:25-30); dtype f32 / f16 / bf16.

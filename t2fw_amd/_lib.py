@@ -27,6 +27,12 @@ FLAG_EXACT_CHUNKS = 32
 
 _vp, _i64, _i32, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_size_t
 
+
+class BlockCopyDesc(ctypes.Structure):
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("size", _i64 * 4), ("stride", _i64 * 4),
+                ("terms", _i64), ("term_stride", _i64)]
+
+
 # name -> (restype, argtypes); mirrors include/t2fw_hip.h one to one
 SIGNATURES = {
     "t2fw_abi_version": (ctypes.c_int, []),
@@ -44,6 +50,7 @@ SIGNATURES = {
     "t2fw_lfw_backward_heads": (ctypes.c_int, [_vp] * 15 + [_i64] * 5 + [_i32] * 3 + [_vp, _sz, _vp]),
     "t2fw_lfw_step": (ctypes.c_int, [_vp] * 8 + [_i64] * 3 + [_i32, _vp]),
     "t2fw_cast": (ctypes.c_int, [ctypes.POINTER(ctypes.c_void_p)] * 2 + [ctypes.POINTER(ctypes.c_int64), _i32, _i32, _i32, _vp]),
+    "t2fw_block_copy": (ctypes.c_int, [_vp, _i32, _i32, _vp]),
     "t2fw_gate_forward": (ctypes.c_int, [_vp] * 4 + [_i64] * 2 + [_i32, _vp]),
     "t2fw_gate_backward": (ctypes.c_int, [_vp] * 6 + [_i64] * 2 + [_i32, _vp]),
     "t2fw_dfw_forward": (ctypes.c_int, [_vp] * 7 + [_i64] * 4 + [_i32, _i32, _vp]),
@@ -87,6 +94,34 @@ def ptr(t):
 
 def current_stream_handle(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+def block_plan(*arrays):
+    """The descriptors of one t2fw_block_copy launch without their addresses, as bytes (callers keep one per shape).
+    Array: (sizes, strides) or (sizes, strides, terms, term stride), outermost first, at most four sizes."""
+    plan = (BlockCopyDesc * len(arrays))()
+    for d, (sizes, strides, *sum_) in zip(plan, arrays):
+        assert len(sizes) == len(strides) <= 4
+        lead = 4 - len(sizes)
+        d.size[:] = [1] * lead + list(sizes)
+        d.stride[:] = [0] * lead + list(strides)
+        d.terms, d.term_stride = sum_ if sum_ else (1, 0)
+    return bytes(plan)
+
+
+def block_copy(plan, srcs, dsts):
+    """One launch of t2fw_block_copy on the current stream: dsts[i] from srcs[i] as ``plan`` (block_plan) says.
+    Tensors in host memory (no kernel of this library takes them) are copied by torch."""
+    n = len(srcs)
+    descs = (BlockCopyDesc * n).from_buffer_copy(plan)
+    for d, s, t in zip(descs, srcs, dsts):
+        d.src, d.dst = s.data_ptr(), t.data_ptr()
+    if not srcs[0].is_cuda:
+        for d, s, t in zip(descs, srcs, dsts):
+            view = s.as_strided((*d.size, d.terms, 64), (*d.stride, d.term_stride, 1))
+            t.view(view.shape[:4] + (64,)).copy_(view.sum(dim=4))
+        return
+    check(load().t2fw_block_copy(descs, n, DTYPE_CODE[srcs[0].dtype], current_stream_handle(srcs[0].device)))
 
 
 def cast_tensors(srcs, dsts, stream):

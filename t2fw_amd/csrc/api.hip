@@ -6,6 +6,7 @@
 #include "lfw_par.hpp"
 #include "lfw_xpar.hpp"
 #include "dfw_scan.hpp"
+#include "blocks.hpp"
 #include "cast.hpp"
 #include "gate.hpp"
 #include "lfw_step.hpp"
@@ -639,6 +640,33 @@ int t2fw_cast(const void *const *src, void *const *dst, const int64_t *n, int32_
         a.src[i] = src[i]; a.dst[i] = dst[i]; a.n[i] = n[i];
     }
     return cast_tensors(a, src_dtype, dst_dtype, static_cast<hipStream_t>(stream));
+}
+
+int t2fw_block_copy(const t2fw_block_copy_desc *arrays, int32_t count, int32_t dtype, void *stream) {
+    const size_t es = elem_size(dtype);
+    if (es == 0) return fail(T2FW_ERR_BAD_DTYPE, "unknown dtype code %d", dtype);
+    if (count < 0 || count > T2FW_BLOCK_COPY_MAX)
+        return fail(T2FW_ERR_BAD_SHAPE, "t2fw_block_copy takes 0 to %d arrays, got %d", T2FW_BLOCK_COPY_MAX, count);
+    if (count > 0 && arrays == nullptr) return fail(T2FW_ERR_NULL_POINTER, "null array list");
+    BlockCopyArgs a{};
+    for (int i = 0; i < count; ++i) {
+        const t2fw_block_copy_desc &d = arrays[i];
+        long double vectors = 1;
+        for (int m = 0; m < 4; ++m) {
+            if (d.size[m] < 0) return fail(T2FW_ERR_BAD_SHAPE, "sizes must be non-negative");
+            if (d.stride[m] < 0 || d.stride[m] % 64 != 0) return fail(T2FW_ERR_BAD_SHAPE, "strides must be multiples of 64");
+            vectors *= (long double)d.size[m];
+        }
+        if (d.terms < 1 || d.term_stride < 0 || d.term_stride % 64 != 0)
+            return fail(T2FW_ERR_BAD_SHAPE, "at least one term, its stride a multiple of 64");
+        if (vectors == 0) continue;
+        if (vectors > 2147483647.0L) return fail(T2FW_ERR_UNSUPPORTED, "t2fw_block_copy: more than 2^31 vectors");
+        const NamedPtr ptrs[] = {{"src", d.src}, {"dst", d.dst}};
+        const int rc = check_ptrs(ptrs, 2, es);
+        if (rc) return rc;
+        a.a[a.count++] = d;
+    }
+    return a.count == 0 ? T2FW_OK : block_copy(a, dtype, static_cast<hipStream_t>(stream));
 }
 
 int t2fw_gate_forward(const void *f_logit, const void *fk_logit, void *f, void *f_key, int64_t n_f, int64_t n_fk,

@@ -2,6 +2,7 @@
 ``DFWFunction.apply(query, key, value, state)`` (t2fw/functional_dfw.py:29-65), backed by the
 HIP kernels in libt2fw_hip.so.  As in the reference, backward consumes the per-step deltas
 and the final state saved by forward (t2fw/functional_dfw.py:46-51)."""
+import functools
 import os
 
 import torch
@@ -69,36 +70,43 @@ def _value_block_count(value, query):
     return D // 64
 
 
-def _rows_of_value_blocks(t, nd):          # [B,T,64 nd] -> [B nd,T,64]
-    B, T = t.shape[:2]
-    return t.view(B, T, nd, 64).permute(0, 2, 1, 3).reshape(B * nd, T, 64).contiguous()
-
-
-def _rows_repeated(t, nd):                 # [B,T,M] -> [B nd,T,M]
-    B, T, M = t.shape
-    return t.unsqueeze(1).expand(B, nd, T, M).reshape(B * nd, T, M).contiguous()
-
-
-def _value_blocks_from_rows(t, nd):        # [B nd,T,64] -> [B,T,64 nd]
-    Bn, T = t.shape[:2]
-    return t.view(Bn // nd, nd, T, 64).permute(0, 2, 1, 3).reshape(Bn // nd, T, 64 * nd)
+@functools.lru_cache(maxsize=256)
+def _value_block_plans(B, T, nd):
+    """Descriptors of the block copies (csrc/blocks.hip), one launch each way"""
+    D = 64 * nd
+    cut = ((B, nd, T), (T * D, 64, D))                       # [B,T,64 nd] -> [B nd,T,64]
+    repeat = ((B, nd, T), (T * 64, 0, 64))                   # [B,T,64] -> [B nd,T,64]
+    join = ((B, T, nd), (nd * T * 64, 64, T * 64))           # [B nd,T,64] -> [B,T,64 nd]
+    total = ((B, T), (nd * T * 64, 64), nd, T * 64)          # [B nd,T,64] -> [B,T,64], the sum over the blocks
+    return {"inputs": _lib.block_plan(repeat, repeat, cut), "outputs": _lib.block_plan(join),
+            "grads_in": _lib.block_plan(cut), "grads_out": _lib.block_plan(total, total, join)}
 
 
 def _dfw_forward_blocked(query, key, value, state, nd):
     """(outputs, final_state, what the backward needs: q and k repeated per block, delta and final state of the blocks)"""
     B, D, M = state.shape
-    qb, kb = _rows_repeated(query, nd), _rows_repeated(key, nd)
-    out_b, fin_b, delta_b = _dfw_forward(qb, kb, _rows_of_value_blocks(value, nd), state.view(B * nd, 64, M))
-    return _value_blocks_from_rows(out_b, nd), fin_b.view(B, D, M), (qb, kb, delta_b, fin_b)
+    T = value.shape[1]
+    plans = _value_block_plans(B, T, nd)
+    with _on_device(value.device):
+        qb, kb, vb = (value.new_empty((B * nd, T, 64)) for _ in range(3))
+        _lib.block_copy(plans["inputs"], (query, key, value), (qb, kb, vb))
+        out_b, fin_b, delta_b = _dfw_forward(qb, kb, vb, state.view(B * nd, 64, M))
+        outputs = torch.empty_like(value)
+        _lib.block_copy(plans["outputs"], (out_b,), (outputs,))
+    return outputs, fin_b.view(B, D, M), (qb, kb, delta_b, fin_b)
 
 
 def _dfw_backward_blocked(grad_output, grad_state, qb, kb, delta_b, fin_b, nd):
     Bn, T, M = qb.shape
     B = Bn // nd
-    d_qb, d_kb, d_vb, d_sb = _dfw_backward(_rows_of_value_blocks(grad_output, nd), grad_state.reshape(Bn, 64, M), qb, kb,
-                                           delta_b, fin_b)
-    return (d_qb.view(B, nd, T, M).sum(dim=1), d_kb.view(B, nd, T, M).sum(dim=1), _value_blocks_from_rows(d_vb, nd),
-            d_sb.view(B, 64 * nd, M))
+    plans = _value_block_plans(B, T, nd)
+    with _on_device(qb.device):
+        go_b = torch.empty_like(delta_b)
+        _lib.block_copy(plans["grads_in"], (grad_output,), (go_b,))
+        d_qb, d_kb, d_vb, d_sb = _dfw_backward(go_b, grad_state.reshape(Bn, 64, M), qb, kb, delta_b, fin_b)
+        d_q, d_k, d_v = qb.new_empty((B, T, M)), qb.new_empty((B, T, M)), qb.new_empty((B, T, 64 * nd))
+        _lib.block_copy(plans["grads_out"], (d_qb, d_kb, d_vb), (d_q, d_k, d_v))
+    return d_q, d_k, d_v, d_sb.view(B, 64 * nd, M)
 
 
 class DFWFunction(torch.autograd.Function):

@@ -53,7 +53,7 @@ def _host_hints_enabled():
 
 def _on_device(dev):
     """Make ``dev`` current for the allocations and the launch, without the cost of switching when it already is."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
+    if dev.type != "cuda" or dev.index is None or dev.index == torch.cuda.current_device():
         return contextlib.nullcontext()
     return torch.cuda.device(dev)
 
@@ -112,38 +112,54 @@ def _block_counts(value, query, flags):
 
 
 # Tensors are [B,T,W] or, with a head axis, [B,T,H,W]; states [B,D,K] or [B,H,D,K].  Block (i, j) of head h becomes
-# head (h * nd + i) * nk + j of the 64-wide call.
-def _value_blocks(t, nd, nk):
-    lead = t.shape[:-1]
-    return t.view(*lead, nd, 1, 64).expand(*lead, nd, nk, 64).reshape(lead[0], lead[1], -1, 64).contiguous()
+# head (h * nd + i) * nk + j of the 64-wide call.  The blocks of a call's tensors are cut in one launch and its results
+# put together in another (csrc/blocks.hip); what has only one block on the other side is a view and costs nothing.
+@functools.lru_cache(maxsize=256)
+def _block_plans(B, T, H, nd, nk):
+    lines, rows, D, K = B * T * H, B * H, 64 * nd, 64 * nk
+    value = ((lines, nd, nk), (D, 64, 0))
+    key = ((lines, nd, nk), (K, 0, 64))
+    state = ((rows, nd, nk, 64), (D * K, 64 * K, 64, K))
+    whole_state = ((rows, nd, 64, nk), (D * K, nk * 4096, 64, 4096))
+    key_sum = ((lines, nd), (nd * nk * 64, nk * 64), nk, 64)
+    value_sum = ((lines, nk), (nd * nk * 64, 64), nd, nk * 64)
+    inputs = [p for p, kept in ((value, nk > 1), (value, nk > 1), (key, nd > 1), (key, nd > 1), (key, nd > 1),
+                                (state, nk > 1)) if kept]
+    grads = [p for p, kept in ((key_sum, nk > 1), (key_sum, nk > 1), (value_sum, nd > 1), (value_sum, nd > 1),
+                               (value_sum, nd > 1), (whole_state, nk > 1)) if kept]
+    return {"inputs": _lib.block_plan(*inputs),
+            "outputs": _lib.block_plan(key_sum, whole_state) if nk > 1 else None,
+            "grads_in": _lib.block_plan(value, state) if nk > 1 else None,
+            "grads_out": _lib.block_plan(*grads)}
 
 
-def _key_blocks(t, nd, nk):
-    lead = t.shape[:-1]
-    return t.view(*lead, 1, nk, 64).expand(*lead, nd, nk, 64).reshape(lead[0], lead[1], -1, 64).contiguous()
+def _block_dims(value, blocks):
+    """(B, T, H, blocks along the value side, along the key side) of [B,T,W] or [B,T,H,W] tensors"""
+    return value.shape[0], value.shape[1], value.shape[2] if value.dim() == 4 else 1, blocks[0], blocks[1]
 
 
-def _state_blocks(s, nd, nk):
-    B = s.shape[0]
-    return s.view(B, -1, nd, 64, nk, 64).permute(0, 1, 2, 4, 3, 5).reshape(B, -1, 64, 64).contiguous()
+def _run_plan(plan, srcs, dsts, copied):
+    """dsts from srcs in one launch; an entry that is not ``copied`` is a view of its source, of the shape of dsts"""
+    outs, cs, cd = [], [], []
+    for s, shape, c in zip(srcs, dsts, copied):
+        if c:
+            t = torch.empty(shape, dtype=s.dtype, device=s.device)
+            cs.append(s)
+            cd.append(t)
+            outs.append(t)
+        else:
+            outs.append(s.view(shape))
+    if cs:
+        _lib.block_copy(plan, cs, cd)
+    return outs
 
 
-def _state_from_blocks(sb, nd, nk, like):
-    """back to the shape of ``like`` ([B,D,K] or [B,H,D,K])"""
-    B = sb.shape[0]
-    return sb.view(B, -1, nd, nk, 64, 64).permute(0, 1, 2, 4, 3, 5).reshape(like.shape)
-
-
-def _sum_key_blocks(tb, nd, nk, like):
-    """[B,T,heads of blocks,64] -> the shape of ``like`` ([B,T,D] or [B,T,H,D]): what the blocks of one row of
-    blocks hold adds up (fp32 accumulation)"""
-    B, T = tb.shape[:2]
-    return tb.view(B, T, -1, nd, nk, 64).sum(dim=4).reshape(like.shape)
-
-
-def _sum_value_blocks(tb, nd, nk, like):
-    B, T = tb.shape[:2]
-    return tb.view(B, T, -1, nd, nk, 64).sum(dim=3).reshape(like.shape)
+def _input_blocks(tensors, B, T, H, nd, nk):
+    """x, f, q, k, f_key [B,T,(H,)W] -> [B,T,H nd nk,64], state -> [B,H nd nk,64,64]"""
+    v, k = nk > 1, nd > 1
+    tok, st = (B, T, H * nd * nk, 64), (B, H * nd * nk, 64, 64)
+    with _on_device(tensors[0].device):
+        return _run_plan(_block_plans(B, T, H, nd, nk)["inputs"], tensors, (tok,) * 5 + (st,), (v, v, k, k, k, v))
 
 
 class _BlockedCall:
@@ -157,29 +173,30 @@ class _BlockedCall:
 
 
 def _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks):
-    nd, nk = blocks
-    tensors = (_value_blocks(value, nd, nk), _value_blocks(forget, nd, nk), _key_blocks(query, nd, nk),
-               _key_blocks(key, nd, nk), _key_blocks(f_key, nd, nk), _state_blocks(state, nd, nk))
+    dims = _block_dims(value, blocks)
+    tensors = _input_blocks((value, forget, query, key, f_key, state), *dims)
     out_b, nxt_b, ckpt, C, flags, hints = _lfw_forward(*tensors, need_grad, heads=True)
     kept = _BlockedCall(tensors, hints) if need_grad else None
-    return _sum_key_blocks(out_b, nd, nk, value), _state_from_blocks(nxt_b, nd, nk, state), ckpt, C, flags, kept
+    summed = blocks[1] > 1
+    with _on_device(value.device):
+        out, nxt = _run_plan(_block_plans(*dims)["outputs"], (out_b, nxt_b), (value.shape, state.shape), (summed, summed))
+    return out, nxt, ckpt, C, flags, kept
 
 
 def _lfw_backward_blocked(grad_output, grad_state, value, forget, query, key, f_key, state, ckpt, C, flags, kept, blocks):
-    """The adjoint of the copies is the sum over the blocks that share a channel."""
-    nd, nk = blocks
+    """The adjoint of the copies is the sum over the blocks that share a channel (fp32 sums)."""
+    B, T, H, nd, nk = dims = _block_dims(value, blocks)
     if isinstance(kept, _BlockedCall):
         tensors, hints = kept.tensors, kept.hints
     else:
-        tensors = (_value_blocks(value, nd, nk), _value_blocks(forget, nd, nk), _key_blocks(query, nd, nk),
-                   _key_blocks(key, nd, nk), _key_blocks(f_key, nd, nk), _state_blocks(state, nd, nk))
-        hints = None
-    d_xb, d_fb, d_qb, d_kb, d_fkb, d_sb = _lfw_backward(
-        _value_blocks(grad_output, nd, nk), _state_blocks(grad_state, nd, nk), *tensors, ckpt, C, flags, heads=True,
-        hints=hints)
-    return (_sum_key_blocks(d_xb, nd, nk, value), _sum_key_blocks(d_fb, nd, nk, value),
-            _sum_value_blocks(d_qb, nd, nk, query), _sum_value_blocks(d_kb, nd, nk, query),
-            _sum_value_blocks(d_fkb, nd, nk, query), _state_from_blocks(d_sb, nd, nk, state))
+        tensors, hints = _input_blocks((value, forget, query, key, f_key, state), *dims), None
+    plans = _block_plans(*dims)
+    v, k = nk > 1, nd > 1
+    with _on_device(value.device):
+        go_b, gs_b = _run_plan(plans["grads_in"], (grad_output, grad_state), (tensors[0].shape, tensors[5].shape), (v, v))
+        grads = _lfw_backward(go_b, gs_b, *tensors, ckpt, C, flags, heads=True, hints=hints)
+        return tuple(_run_plan(plans["grads_out"], grads, (value.shape, value.shape, query.shape, query.shape, query.shape,
+                                                           state.shape), (v, v, k, k, k, v)))
 
 
 def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False):
