@@ -14,9 +14,9 @@
 // them.  A row that is left to the recurrence over the whole sequence (lfw_xpar.hip) is walked by the workgroup of its
 // first chunk, chunk by chunk, with the state or the adjoint kept.
 //
-// B = 96, T = 1024: forward 77 us (51 us of VALU issue), backward 557 us (about 290 us of issue at two waves per SIMD: the
-// rest is waiting for a segment's inputs).  The per-step kernels over whole rows take 220 and 813 us, their bodies on
-// chunks 154 and 600 us.
+// B = 96, T = 1024: forward 77 us (51 us of VALU issue), backward 439 us (about 290 us of issue at two waves per SIMD;
+// 557 us before the inputs of a job were requested while the job before it ran).  The per-step kernels over whole rows
+// take 220 and 813 us, their bodies on chunks 154 and 600 us.
 // Tried and slower: rank-one terms on v_mfma_f32_4x4x1 (forward 115 us, backward 603), column vectors in scalar registers
 // (105 and 1145: every wave misses the scalar cache once per step and array).
 #include "lfw_chunk.hpp"
@@ -132,29 +132,27 @@ __device__ __forceinline__ void step(floatx4 (&out)[4], const floatx4 (&S)[4], f
 // G *= (column vector) (x) (row vector)
 __device__ __forceinline__ void scale_outer(floatx4 (&G)[4], float col, float row) {
     float g[16];
-#pragma unroll
-    for (int n = 0; n < 16; ++n) g[n] = G[n / 4][n % 4];
     asm("s_nop 1\n"
-        "v_mul_f32_dpp %0, %16, %0 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %1, %16, %1 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %2, %16, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %3, %16, %3 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %4, %16, %4 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %5, %16, %5 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %6, %16, %6 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %7, %16, %7 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %8, %16, %8 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %9, %16, %9 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %10, %16, %10 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %11, %16, %11 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %12, %16, %12 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %13, %16, %13 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %14, %16, %14 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-        "v_mul_f32_dpp %15, %16, %15 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-        : "+v"(g[0]), "+v"(g[1]), "+v"(g[2]), "+v"(g[3]), "+v"(g[4]), "+v"(g[5]), "+v"(g[6]), "+v"(g[7]), "+v"(g[8]), "+v"(g[9]), "+v"(g[10]), "+v"(g[11]), "+v"(g[12]), "+v"(g[13]), "+v"(g[14]), "+v"(g[15])
-        : "v"(col));
+        "v_mul_f32_dpp %0, %16, %17 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %1, %16, %17 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %2, %16, %17 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %3, %16, %17 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %4, %16, %17 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %5, %16, %17 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %6, %16, %17 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %7, %16, %17 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %8, %16, %17 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %9, %16, %17 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %10, %16, %17 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %11, %16, %17 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %12, %16, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %13, %16, %17 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %14, %16, %17 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+        "v_mul_f32_dpp %15, %16, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
+        : "=&v"(g[0]), "=&v"(g[1]), "=&v"(g[2]), "=&v"(g[3]), "=&v"(g[4]), "=&v"(g[5]), "=&v"(g[6]), "=&v"(g[7]), "=&v"(g[8]), "=&v"(g[9]), "=&v"(g[10]), "=&v"(g[11]), "=&v"(g[12]), "=&v"(g[13]), "=&v"(g[14]), "=&v"(g[15])
+        : "v"(col), "v"(row));
 #pragma unroll
-    for (int n = 0; n < 16; ++n) G[n / 4][n % 4] = g[n] * row;
+    for (int n = 0; n < 16; ++n) G[n / 4][n % 4] *= g[n];
 }
 
 __device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
@@ -268,29 +266,66 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
     const int cl = lane & 15;
     floatx4 S[4], G[4];
 
-    // S over the eight steps from t0
-    auto advance = [&](int t0) {
-        float va[XW_SEG], vf[XW_SEG], ka[XW_SEG], kf[XW_SEG];
-        load_steps(va, ra + t0 * ts, lane, ts, XW_SEG);
-        load_steps(vf, rf + t0 * ts, lane, ts, XW_SEG);
-        load_steps(ka, ca + t0 * ts, cl, ts, XW_SEG);
-        load_steps(kf, cf + t0 * ts, cl, ts, XW_SEG);
+    // A chunk is a list of jobs of up to eight steps: `ahead` that advance S to the start of the last block of 16 steps,
+    // then per block, last to first, an advance over its first half and the two halves in reverse (a last block of
+    // eight steps or fewer: one).  The gates and values of a job are requested while the job before it computes.
+    struct Job {
+        int t0, n, blk;
+        bool reverse, restart;               // restart: S is the state at the start of block blk
+    };
+    int tc = 0, len = 0, nblk = 0, ahead = 0, last_jobs = 0;
+    auto enter_chunk = [&](int c) {
+        tc = c * XP_CHUNK;
+        len = (int)min((int64_t)XP_CHUNK, p.T - tc);
+        nblk = (len + XW_BLOCK - 1) / XW_BLOCK;
+        ahead = 2 * (nblk - 1);
+        last_jobs = len - XW_BLOCK * (nblk - 1) > XW_SEG ? 3 : 1;
+    };
+    auto jobs = [&]() { return ahead + last_jobs + 3 * (nblk - 1); };
+    auto job = [&](int q) {
+        if (q < ahead) return Job{tc + XW_SEG * q, XW_SEG, q >> 1, false, q == 0};
+        const int r = q - ahead, o = r - last_jobs;
+        const int blk = r < last_jobs ? nblk - 1 : nblk - 2 - o / 3;
+        const int sub = r < last_jobs ? (last_jobs == 3 ? r : 2) : o % 3;
+        const int t0 = XW_BLOCK * blk + (sub == 1 ? XW_SEG : 0);
+        return Job{tc + t0, min(XW_SEG, len - t0), blk, sub != 0, sub != 1};
+    };
+    float va[XW_SEG], vf[XW_SEG], ka[XW_SEG], kf[XW_SEG];              // of the job that runs
+    float nva[XW_SEG], nvf[XW_SEG], nka[XW_SEG], nkf[XW_SEG];          // of the next one
+    int next_n = 0;
+    auto fetch = [&](const Job &b) {
+        load_steps(nva, ra + b.t0 * ts, lane, ts, b.n);
+        load_steps(nvf, rf + b.t0 * ts, lane, ts, b.n);
+        load_steps(nka, ca + b.t0 * ts, cl, ts, b.n);
+        load_steps(nkf, cf + b.t0 * ts, cl, ts, b.n);
+        next_n = b.n;
+    };
+    auto take = [&]() {
+        if (next_n < XW_SEG) {
+            pad_steps(nva, next_n, 0.f);
+            pad_steps(nvf, next_n, 1.f);
+            pad_steps(nka, next_n, 0.f);
+            pad_steps(nkf, next_n, 1.f);
+        }
 #pragma unroll
-        for (int j = 0; j < XW_SEG; ++j) step(S, S, ka[j], kf[j], va[j], vf[j]);
+        for (int j = 0; j < XW_SEG; ++j) {
+            va[j] = nva[j]; vf[j] = nvf[j]; ka[j] = nka[j]; kf[j] = nkf[j];
+        }
+    };
+
+    // S over the eight steps of a job
+    auto advance = [&](const Job &next) {
+        fetch(next);
+#pragma unroll
+        for (int j = 0; j < XW_SEG; ++j) {
+            settle(ka[j], kf[j], va[j], vf[j]);
+            step(S, S, ka[j], kf[j], va[j], vf[j]);
+            settle(S);
+        }
     };
     // The segment [t0, t0 + n): its states rebuilt from S, the adjoint back over them, the sums stored.
-    auto reverse = [&](int t0, int n) {
-        float va[XW_SEG], vf[XW_SEG], vu[XW_SEG], ka[XW_SEG], kf[XW_SEG], ku[XW_SEG];
-        load_steps(va, ra + t0 * ts, lane, ts, n);
-        load_steps(vf, rf + t0 * ts, lane, ts, n);
-        load_steps(ka, ca + t0 * ts, cl, ts, n);
-        load_steps(kf, cf + t0 * ts, cl, ts, n);
-        if (n < XW_SEG) {
-            pad_steps(va, n, 0.f);
-            pad_steps(vf, n, 1.f);
-            pad_steps(ka, n, 0.f);
-            pad_steps(kf, n, 1.f);
-        }
+    auto reverse = [&](int t0, int n, const Job &next) {
+        float vu[XW_SEG], ku[XW_SEG];
         floatx4 st[XW_SEG + 1][4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) st[0][q] = S[q];
@@ -310,6 +345,7 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
 #pragma unroll
         for (int j = XW_SEG - 1; j >= 0; --j) {
             settle(ku[j], kf[j], vu[j], vf[j]);
+            if (j == XW_SEG / 2) fetch(next);
             add_outer(G, ku[j], vu[j]);      // G_t = g_t (x) q_t + ...
             floatx4 w_[4];
             sm.part[0][j][w][lane] = dot(G, ka[j]);                                      // d_x / d_k
@@ -335,25 +371,28 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
     load_state<SIDE == 1>(G, g_end, lane, col0);
     for (int c = whole ? (int)p.NC - 1 : chunk; c >= chunk; --c) {
         const float *const s0 = (const float *)p.ckpt + (b * p.NC + c) * (XP_N * XP_N);
-        const int tc = c * XP_CHUNK, len = (int)min((int64_t)XP_CHUNK, p.T - tc), nblk = (len + XW_BLOCK - 1) / XW_BLOCK;
-        load_state<SIDE == 1>(S, s0, lane, col0);
-        for (int blk = 1; blk < nblk; ++blk) {           // to the start of the last block
-            advance(tc + XW_BLOCK * (blk - 1));
-            advance(tc + XW_BLOCK * (blk - 1) + XW_SEG);
-#pragma unroll
-            for (int u = 0; u < XW_COLS; ++u) sm.start[blk - 1][u][tid] = S[u / 4][u % 4];
-        }
-        for (int blk = nblk - 1; blk >= 0; --blk) {
-            const int t0 = tc + XW_BLOCK * blk, n = min(XW_BLOCK, tc + len - t0);
-            for (int half = n > XW_SEG ? 1 : 0; half >= 0; --half) {
-                if (blk == 0) {
+        enter_chunk(c);
+        const int njobs = jobs();
+        fetch(job(0));
+        for (int q = 0; q < njobs; ++q) {
+            const Job now = job(q), next = job(min(q + 1, njobs - 1));
+            take();
+            if (now.restart) {
+                if (now.blk == 0) {
                     load_state<SIDE == 1>(S, s0, lane, col0);
                 } else {
 #pragma unroll
-                    for (int u = 0; u < XW_COLS; ++u) S[u / 4][u % 4] = sm.start[blk - 1][u][tid];
+                    for (int u = 0; u < XW_COLS; ++u) S[u / 4][u % 4] = sm.start[now.blk - 1][u][tid];
                 }
-                if (half) advance(t0);
-                reverse(t0 + XW_SEG * half, min(n - XW_SEG * half, XW_SEG));
+            }
+            if (now.reverse) {
+                reverse(now.t0, now.n, next);
+            } else {
+                advance(next);
+                if (q < ahead && (q & 1)) {
+#pragma unroll
+                    for (int u = 0; u < XW_COLS; ++u) sm.start[q >> 1][u][tid] = S[u / 4][u % 4];
+                }
             }
         }
     }

@@ -75,7 +75,7 @@ def _dtype_code(dtype):
 
 # Where the chunk-parallel exact kernels (three launches per direction) take the place of the per-step ones (one launch
 # forward, two backward).  Forward + backward, per-step against chunk-parallel, microseconds: 96 rows of 64 x 64 float32,
-# 128 steps 180 / 192 (host-bound: the launches), 256 steps 264 / 216, 1024 steps 1005 / 673; 13 rows of 33 x 17 float16,
+# 128 steps 180 / 192 (host-bound: the launches), 256 steps 264 / 216, 1024 steps 1000 / 555; 13 rows of 33 x 17 float16,
 # 128 steps 177 / 195, 385 steps 338 / 193.  Many rows fill the chip by themselves: 512 rows of 64 x 64, 256 steps 872 /
 # 886; 1024 rows of 16 x 16 277 / 364.
 EXACT_CHUNKS_MIN_STEPS = 224
