@@ -104,7 +104,8 @@ extern "C" {
                                      side by side, for a checkpoint interval of 64 (a forward call without checkpoints:
                                      any).  Forward and backward need the workspace that t2fw_lfw_forward_workspace_bytes
                                      and t2fw_lfw_workspace_bytes report for these flags.  Rows with a gate of magnitude
-                                     above one are done step by step over the whole sequence in the same call.  More than
+                                     above one, an input above 2^58 or a state above 2^120 (infinities and NaN among
+                                     them) are done step by step over the whole sequence in the same call.  More than
                                      65536 rows x chunks: the flag is ignored. */
 
 int t2fw_abi_version(void);

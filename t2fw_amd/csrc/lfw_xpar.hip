@@ -13,9 +13,13 @@
 //   3  lfw_xpar_fwd_kernel / lfw_xpar_bwd_kernel: the recurrence itself, step by step, within each chunk; the last chunk's
 //      leaves the final state, the first one's d_s0.
 //
-// A row with a gate of magnitude above one (or NaN), or an increment that is not finite, is left to the recurrence over
-// the whole sequence: a product of one side's gates may then overflow where the product of both sides' does not.  The
-// workgroups of the row's first chunk do it in launch 3, the others of that row leave.
+// A row is left to the recurrence over the whole sequence where the sums could differ from it by more than rounding:
+//   * a gate of magnitude above one (or NaN): the product of one side's gates may overflow where the product of both
+//     sides' does not;
+//   * an input above XP_MAX_INPUT or a state above XP_MAX_STATE at a chunk's start or end (or NaN): with neither, no
+//     state within a chunk exceeds 2^120 + 64 * 2^116 < 2^123.  What the recurrence makes infinite it keeps infinite; an
+//     increment of decayed factors comes out finite, and infinity times a gate product that has underflowed is NaN.
+// The workgroups of the row's first chunk do it in launch 3, the others of that row leave.
 //
 // B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 24 + 19 + 77 us (220 per-step), backward 24 + 11 +
 // 439 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
@@ -33,6 +37,7 @@ namespace {
 
 constexpr int XI_THREADS = 512;
 constexpr int XLS = 68;                // row stride, in floats, of the token-major tiles [64][XLS]
+constexpr float XP_MAX_INPUT = 0x1p58f, XP_MAX_STATE = 0x1p120f;
 
 __device__ __forceinline__ int64_t uniform64(int64_t v) {
     const u32 lo = __builtin_amdgcn_readfirstlane((u32)(unsigned long long)v);
@@ -116,6 +121,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
             for (int j = 0; j < 4; ++j) {
                 const int t = 16 * m + 4 * kg + j;
                 const float a = (ch_ok && t < n_tok) ? to_acc(ra[m][j]) : 0.0f;
+                bad |= !(fabsf(a) <= XP_MAX_INPUT) ? 1 : 0;
                 tile[t * XLS + c] = a * (base * l[j]);
             }
         }
@@ -167,7 +173,10 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
         const int64_t DK = (int64_t)D * K, o = d * K + k;
         float S[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) S[e] = k + e < K ? to_acc(((const IO *)p.first)[b * DK + o + e]) : 0.0f;
+        for (int e = 0; e < 4; ++e) {
+            S[e] = k + e < K ? to_acc(((const IO *)p.first)[b * DK + o + e]) : 0.0f;
+            bad |= !(fabsf(S[e]) <= XP_MAX_STATE) ? 1 : 0;
+        }
         float *const st = p.ws.states + b * NC * (int64_t)(XP_N * XP_N) + d * XP_N + k;
         const float *const tots = p.ws.tots + b * NC * (int64_t)(2 * XP_N);
         IO *const ckpt = p.ckpt != nullptr ? (IO *)p.ckpt + b * NC * DK + o : nullptr;
@@ -194,8 +203,8 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
                 const float mv[4] = {m[u].x, m[u].y, m[u].z, m[u].w}, tv[4] = {tb[u].x, tb[u].y, tb[u].z, tb[u].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    bad |= (k + e >= K || fabsf(mv[e]) <= 3.402823466e38f) ? 0 : 1;
                     S[e] = S[e] * (ta[u] * tv[e]) + mv[e];
+                    bad |= (k + e >= K || fabsf(S[e]) <= XP_MAX_STATE) ? 0 : 1;
                 }
             }
         }

@@ -57,6 +57,51 @@ def test_unusual_gates_and_values(what, D, K, dtype):
     check_all((x, f, q, k, fk, s), go, gs, dtype)
 
 
+def _same_where_finite(got, want, what, tol):
+    got, want = got.detach().double().cpu(), want.detach().double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)), what
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)], want[torch.isinf(want)]), what
+    for g, w in zip(got, want):                            # row by row: one holds very large values
+        ok = torch.isfinite(w)
+        assert ((g - w)[ok].abs() <= tol[0] * w[ok].abs() + tol[1] * w[ok].abs().max()).all(), what
+
+
+@pytest.mark.parametrize("what", ["infinite states, fast decay", "a product overflows, then decays", "the state overflows between chunks"])
+@pytest.mark.parametrize("D,K,dtype", [(64, 64, F32), (20, 40, F32), (20, 40, BF16)])
+def test_infinities_as_step_by_step(what, D, K, dtype, monkeypatch):
+    """What the recurrence makes infinite stays so: the per-step kernels are the reference (sums differ in order only:
+    their tolerance, per row)."""
+    from t2fw_amd import LFWFunction
+    T = 200
+    x, f, q, k, fk, s, go, gs = make_config_inputs(3, T, D, K, dtype, seed=8, in_scale=0.5, state_std=0.5)
+    if what == "infinite states, fast decay":
+        s[1, 3, 5] = float("inf")
+        gs[1, 2, 2] = float("-inf")
+        f[1], fk[1] = 2.0 ** -6, 2.0 ** -6                 # a chunk's gate product is zero in fp32
+    elif what == "a product overflows, then decays":
+        f[1], fk[1] = 0.5, 0.5
+        x[1, 70, 3], k[1, 70, 5] = 1e30, 1e30
+        go[1, 120, 2], q[1, 120, 4] = 1e30, 1e30
+    else:
+        s[1, 3, 5] = 3e38
+        x[1, 10, 3], k[1, 10, 5] = 1e19, 1e19
+        f[1], fk[1] = 1.0, 1.0
+        f[1, 140:], fk[1, 140:] = 2.0 ** -6, 2.0 ** -6
+        x[1, :, 3] = x[1, :, 3].abs()
+        k[1, :, 5] = k[1, :, 5].abs()
+
+    def run(flags):
+        monkeypatch.setenv("T2FW_FLAGS", flags)
+        ins = [t.cuda().requires_grad_() for t in (x, f, q, k, fk, s)]
+        res = LFWFunction.apply(*ins)
+        return list(res) + list(torch.autograd.grad(res, ins, [go.cuda(), gs.cuda()]))
+
+    want = run("1")
+    assert not all(torch.isfinite(t).all() for t in want)
+    for n, g, w in zip(("outputs", "next_state") + NAMES, run("32"), want):
+        _same_where_finite(g, w, n, TOL[dtype])
+
+
 def test_nan_stays_in_its_row():
     from t2fw_amd import LFWFunction
     ins = [t.cuda() for t in make_config_inputs(3, 150, 64, 64, F32, seed=4)[:6]]
