@@ -18,8 +18,8 @@ namespace scan {
 // ------------------------------------------------------------------------------------
 // batch row b, tile of g.rows value channels.  KG: lanes per state row as a compile-time constant
 // (p.kg must equal it), which leaves the cross-lane sums without branches and the LDS strides as
-// immediates; 0 = take p.kg at run time.
-template <typename IO, int KPL, int KG>
+// immediates; 0 = take p.kg at run time.  TB: an upper bound of p.tb (fewer registers hold the block that is on its way).
+template <typename IO, int KPL, int KG, int TB = 1 << 30>
 __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b, int tile) {
     using Acc = typename AccOf<IO>::type;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -61,7 +61,7 @@ __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b
     };
 
     Prefetch<IO, 3, 2> pf;
-    block_load(pf, g, colp, rowp, b, T, 0, (int)(T < tb ? T : tb), K, D, d0, p.heads, col0, p.colw);
+    block_load<TB>(pf, g, colp, rowp, b, T, 0, (int)(T < tb ? T : tb), K, D, d0, p.heads, col0, p.colw);
 
     int until_ckpt = 0;          // steps until the next checkpoint is due
     int64_t chunk = 0;
@@ -72,11 +72,11 @@ __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b
         __syncthreads();                                   // previous block fully consumed
         // flush the previous block's outputs, then publish this block's inputs
         flush(n_prev, t_prev);
-        block_store<IO, Acc, 3, 2>(pf, g, colL, rowL, tb);
+        block_store<IO, Acc, 3, 2, TB>(pf, g, colL, rowL, tb);
         __syncthreads();
         if (t0 + tb < T) {
             const int64_t tn = t0 + tb;
-            block_load(pf, g, colp, rowp, b, T, tn, (int)(T - tn < tb ? T - tn : tb), K, D, d0, p.heads, col0, p.colw);
+            block_load<TB>(pf, g, colp, rowp, b, T, tn, (int)(T - tn < tb ? T - tn : tb), K, D, d0, p.heads, col0, p.colw);
         }
 #pragma unroll 4
         for (int tt = 0; tt < n; ++tt) {

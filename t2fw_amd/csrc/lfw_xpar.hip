@@ -19,10 +19,10 @@
 //   * an input above XP_MAX_INPUT or a state above XP_MAX_STATE at a chunk's start or end (or NaN): with neither, no
 //     state within a chunk exceeds 2^120 + 64 * 2^116 < 2^123.  What the recurrence makes infinite it keeps infinite; an
 //     increment of decayed factors comes out finite, and infinity times a gate product that has underflowed is NaN.
-// The workgroups of the row's first chunk do it in launch 3, the others of that row leave.
+// The workgroups of the row's first chunk (64 x 64 fp32: of the first four) do it in launch 3, the others of that row leave.
 //
-// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 24 + 19 + 77 us (220 per-step), backward 24 + 11 +
-// 439 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
+// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 25 + 19 + 70 us (220 per-step), backward 25 + 11 +
+// 440 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
 //
 // Replaces lfw_cuda_fwd_kernel, lfw_cuda_bwd_kernel and the einsums of the reference
 // (t2fw/csrc/lfw_kernel.cu:18-102, t2fw/csrc/lfw.cpp:45,84-93); semantics t2fw/torch.py:21-31.
@@ -214,6 +214,11 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
 }
 
 // ---- launch 3 -------------------------------------------------------------------------------------
+// Workgroups are numbered chunk by chunk, all rows of a chunk together, so that those that may have a whole row to do come
+// first and next to each other.  Numbered row by row, the ones with work were 16 chunks apart, all on the same one or two
+// dies and shader engines: 96 rows x 1024 steps with a gate above one in each, 32 x 32 fp32, forward + backward 2050 us
+// against 563 now and 752 on the per-step kernels; 64 x 64 7300, 1019, 992 (96 x 256 590, 277, 264; 16 x 1024 1430, 604,
+// 909).
 __device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
     const int4 v = *reinterpret_cast<const int4 *>(ws.row_flags + 4 * b);
     return __builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0;
@@ -221,8 +226,9 @@ __device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
 
 // One workgroup per (row, chunk, 16 value channels); base: the call over whole rows.
 template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_fwd_kernel(ScanFwdArgs base, XparScratch ws, int64_t NC) {
-    const int64_t item = blockIdx.x / base.ntiles, b = item / NC;
-    const int tile = (int)(blockIdx.x - item * base.ntiles), chunk = (int)(item - b * NC);
+    const int64_t pair = blockIdx.x / base.ntiles, b = pair % base.B;
+    const int tile = (int)(blockIdx.x - pair * base.ntiles), chunk = (int)(pair / base.B);
+    const int64_t item = b * NC + chunk;
     if (row_left(ws, b)) {
         if (chunk == 0) scan::fwd_scan_body_kg<IO, KPL, 16>(base, b, tile);
         return;
@@ -243,8 +249,9 @@ template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void 
 // One workgroup per (row, chunk, 16 channels of one side); KV, KK: columns per lane on the value and on the key side.
 template <typename IO, int KV, int KK> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_bwd_kernel(ScanBwdArgs base, XparScratch ws) {
     const int nd = ((int)base.D + 15) / 16, per = nd + ((int)base.K + 15) / 16;
-    const int64_t item = blockIdx.x / per, b = item / base.NC;
-    const int tile = (int)(blockIdx.x - item * per), chunk = (int)(item - b * base.NC);
+    const int64_t pair = blockIdx.x / per, b = pair % base.B;
+    const int tile = (int)(blockIdx.x - pair * per), chunk = (int)(pair / base.B);
+    const int64_t item = b * base.NC + chunk;
     ScanBwdArgs a = base;
     int64_t row = b;
     if (row_left(ws, b)) {

@@ -11,16 +11,19 @@
 //
 // Backward, per chunk: the states at steps 16, 32 and 48 (LDS) are rebuilt from the checkpoint, blocks of 16 steps are
 // visited last to first, and per half block the eight states are rebuilt into registers and the adjoint runs back over
-// them.  A row that is left to the recurrence over the whole sequence (lfw_xpar.hip) is walked by the workgroup of its
-// first chunk, chunk by chunk, with the state or the adjoint kept.
+// them.
 //
-// B = 96, T = 1024: forward 77 us (51 us of VALU issue), backward 439 us (about 290 us of issue at two waves per SIMD;
+// A row that is left to the recurrence over the whole sequence (lfw_xpar.hip) runs on the per-step bodies, a tile of 16
+// channels per workgroup: 226 and 780 us where all of 96 rows x 1024 steps are (per-step kernels 228 and 822; one
+// workgroup walking such a row in this file's layout: 335 and 1174).
+//
+// B = 96, T = 1024: forward 70 us (51 us of VALU issue), backward 440 us (about 290 us of issue at two waves per SIMD;
 // 557 us before the inputs of a job were requested while the job before it ran).  The per-step kernels over whole rows
 // take 220 and 813 us, their bodies on chunks 154 and 600 us.
 // Tried and slower: rank-one terms on v_mfma_f32_4x4x1 (forward 115 us, backward 603), column vectors in scalar registers
 // (105 and 1145: every wave misses the scalar cache once per step and array).
 #include "lfw_chunk.hpp"
-#include "lfw_scan.hpp"
+#include "lfw_scan_body.hpp"
 #include "lfw_xpar.hpp"
 
 namespace t2fw {
@@ -184,24 +187,55 @@ __device__ __forceinline__ void store_state(float *p, const floatx4 (&S)[4], int
         *reinterpret_cast<Float4 *>((p + col0 + 4 * q) + (unsigned)(row * XP_N)) = Float4{{S[q][0], S[q][1], S[q][2], S[q][3]}};
 }
 
+// ---- rows that are left ---------------------------------------------------------------------------
+constexpr int XW_LEFT_TB = 16;
+constexpr int XW_TILES = XP_N / 16;
+__device__ __forceinline__ void left_row_forward(const XparFwdArgs &p, int64_t b, int chunk) {
+    ScanFwdArgs s{};
+    s.x = p.x; s.f = p.f; s.q = p.q; s.k = p.k; s.f_key = p.f_key; s.s0 = p.s0;
+    s.out = p.out; s.next_state = p.next_state; s.ckpt = p.ckpt;
+    s.B = p.B; s.T = p.T; s.D = XP_N; s.K = XP_N; s.NC = p.NC;
+    s.C = XP_CHUNK; s.kg = 16; s.tb = XW_LEFT_TB; s.ntiles = XW_TILES; s.heads = p.heads;
+    for (int tile = chunk; tile < XW_TILES; tile += (int)p.NC)
+        scan::fwd_scan_body_kg<float, 4, 16, XW_LEFT_TB>(s, b, tile);
+}
+template <int SIDE> __device__ __forceinline__ void left_row_backward(const XparBwdArgs &p, int64_t b, int chunk) {
+    ScanBwdArgs s{};
+    s.g_out = p.g_out; s.g_state = p.g_state; s.x = p.x; s.f = p.f; s.q = p.q; s.k = p.k; s.f_key = p.f_key; s.ckpt = p.ckpt;
+    s.d_x = p.d_x; s.d_f = p.d_f; s.d_q = p.d_q; s.d_k = p.d_k; s.d_f_key = p.d_f_key; s.d_s0 = p.d_s0;
+    s.B = p.B; s.T = p.T; s.D = XP_N; s.K = XP_N; s.NC = p.NC;
+    s.C = XP_CHUNK; s.kg = 16; s.use_sub = 1; s.ntiles = XW_TILES; s.heads = p.heads;
+    for (int tile = chunk; tile < XW_TILES; tile += (int)p.NC)
+        scan::bwd_scan_body_kg<float, 4, SIDE, 16, 1>(s, b, tile);
+}
+
 // ---- forward --------------------------------------------------------------------------------------
-__global__ __launch_bounds__(XW_THREADS) void lfw_xpar64_fwd_kernel(XparFwdArgs p) {
-    __shared__ float part[2][XW_SEG][4][XP_N];
-    const int64_t item = blockIdx.x, b = item / p.NC;
-    const int chunk = (int)(item - b * p.NC);
+struct FwdSmem {
+    float part[2][XW_SEG][4][XP_N];
+};
+__global__ __launch_bounds__(XW_THREADS, 4) void lfw_xpar64_fwd_kernel(XparFwdArgs p) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    auto &part = reinterpret_cast<FwdSmem *>(smem_raw)->part;
+    const int64_t b = blockIdx.x % p.B;
+    const int chunk = (int)(blockIdx.x / p.B);
+    if (row_left(p.ws, b)) {
+        left_row_forward(p, b, chunk);
+        return;
+    }
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col0 = XW_COLS * w;
-    const bool whole = row_left(p.ws, b);
-    if (whole && chunk != 0) return;
-    const int T = (int)p.T, t_end = whole ? T : min(T, (chunk + 1) * XP_CHUNK);
+    const int T = (int)p.T;
+    int t_end = min(T, (chunk + 1) * XP_CHUNK);
+    // the compiler must not see that the loop below runs eight times at most: it would keep the addresses of its passes
+    // and need 134 registers, which leaves three waves per SIMD in the place of four
+    asm("" : "+s"(t_end));
     const int64_t ts = (int64_t)p.heads * XP_N, line0 = uniform64(row_first_token(b, p.T, p.heads)) * XP_N;
     const float *const x = (const float *)p.x + line0, *const f = (const float *)p.f + line0;
     const float *const k = (const float *)p.k + line0 + col0, *const fk = (const float *)p.f_key + line0 + col0;
     const int cl = lane & 15;
     const float *const q = (const float *)p.q + line0 + col0;
     float *const out = (float *)p.out + line0;
-    float *const ckpt = (float *)p.ckpt;
     floatx4 S[4];
-    load_state<false>(S, whole ? (const float *)p.s0 + b * (XP_N * XP_N) : p.ws.states + item * (XP_N * XP_N), lane, col0);
+    load_state<false>(S, p.ws.states + (b * p.NC + chunk) * (XP_N * XP_N), lane, col0);
     int buf = 0;
     float rx[XW_SEG], rf[XW_SEG], ck[XW_SEG], cf[XW_SEG], cq[XW_SEG];
     auto fetch = [&](int t0) {
@@ -222,8 +256,6 @@ __global__ __launch_bounds__(XW_THREADS) void lfw_xpar64_fwd_kernel(XparFwdArgs 
     fetch(t0);
     for (; t0 < t_end; t0 += XW_SEG, buf ^= 1) {
         const int n = min(XW_SEG, t_end - t0);
-        if (ckpt != nullptr && (t0 & (XP_CHUNK - 1)) == 0)
-            store_state(ckpt + (b * p.NC + (t0 / XP_CHUNK)) * (XP_N * XP_N), S, lane, col0);
         float cx[XW_SEG], cff[XW_SEG], kx[XW_SEG], kf[XW_SEG], kq[XW_SEG];
 #pragma unroll
         for (int j = 0; j < XW_SEG; ++j) {
@@ -254,7 +286,7 @@ struct BwdSmem {
 };
 static_assert(2 * sizeof(BwdSmem) <= 160 * 1024, "two workgroups must fit the LDS of one CU");
 
-template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdArgs &p, BwdSmem &sm, int64_t b, int chunk, bool whole) {
+template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdArgs &p, BwdSmem &sm, int64_t b, int chunk) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col0 = XW_COLS * w;
     const int64_t ts = (int64_t)p.heads * XP_N, line0 = uniform64(row_first_token(b, p.T, p.heads)) * XP_N;
     const float *const ra = (const float *)(SIDE ? p.k : p.x) + line0, *const rf = (const float *)(SIDE ? p.f_key : p.f) + line0;
@@ -367,32 +399,30 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
             }
     };
 
-    const float *const g_end = whole ? (const float *)p.g_state + b * (XP_N * XP_N) : p.ws.states + (b * p.NC + chunk) * (XP_N * XP_N);
-    load_state<SIDE == 1>(G, g_end, lane, col0);
-    for (int c = whole ? (int)p.NC - 1 : chunk; c >= chunk; --c) {
-        const float *const s0 = (const float *)p.ckpt + (b * p.NC + c) * (XP_N * XP_N);
-        enter_chunk(c);
-        const int njobs = jobs();
-        fetch(job(0));
-        for (int q = 0; q < njobs; ++q) {
-            const Job now = job(q), next = job(min(q + 1, njobs - 1));
-            take();
-            if (now.restart) {
-                if (now.blk == 0) {
-                    load_state<SIDE == 1>(S, s0, lane, col0);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < XW_COLS; ++u) S[u / 4][u % 4] = sm.start[now.blk - 1][u][tid];
-                }
-            }
-            if (now.reverse) {
-                reverse(now.t0, now.n, next);
+    const int64_t state = (b * p.NC + chunk) * (XP_N * XP_N);
+    load_state<SIDE == 1>(G, p.ws.states + state, lane, col0);
+    const float *const s0 = (const float *)p.ckpt + state;
+    enter_chunk(chunk);
+    const int njobs = jobs();
+    fetch(job(0));
+    for (int q = 0; q < njobs; ++q) {
+        const Job now = job(q), next = job(min(q + 1, njobs - 1));
+        take();
+        if (now.restart) {
+            if (now.blk == 0) {
+                load_state<SIDE == 1>(S, s0, lane, col0);
             } else {
-                advance(next);
-                if (q < ahead && (q & 1)) {
 #pragma unroll
-                    for (int u = 0; u < XW_COLS; ++u) sm.start[q >> 1][u][tid] = S[u / 4][u % 4];
-                }
+                for (int u = 0; u < XW_COLS; ++u) S[u / 4][u % 4] = sm.start[now.blk - 1][u][tid];
+            }
+        }
+        if (now.reverse) {
+            reverse(now.t0, now.n, next);
+        } else {
+            advance(next);
+            if (q < ahead && (q & 1)) {
+#pragma unroll
+                for (int u = 0; u < XW_COLS; ++u) sm.start[q >> 1][u][tid] = S[u / 4][u % 4];
             }
         }
     }
@@ -400,26 +430,36 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
 }
 
 __global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_kernel(XparBwdArgs p) {
-    __shared__ BwdSmem sm;
-    const int64_t item = blockIdx.x >> 1, b = item / p.NC;
-    const int chunk = (int)(item - b * p.NC);
-    const bool whole = row_left(p.ws, b);
-    if (whole && chunk != 0) return;
-    if ((blockIdx.x & 1) == 0)
-        backward_side<0>(p, sm, b, chunk, whole);
-    else
-        backward_side<1>(p, sm, b, chunk, whole);
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    BwdSmem &sm = *reinterpret_cast<BwdSmem *>(smem_raw);
+    const int64_t pair = blockIdx.x >> 1, b = pair % p.B;
+    const int chunk = (int)(pair / p.B);
+    if (row_left(p.ws, b)) {
+        if ((blockIdx.x & 1) == 0)
+            left_row_backward<0>(p, b, chunk);
+        else
+            left_row_backward<1>(p, b, chunk);
+    } else if ((blockIdx.x & 1) == 0) {
+        backward_side<0>(p, sm, b, chunk);
+    } else {
+        backward_side<1>(p, sm, b, chunk);
+    }
 }
 
 }  // namespace
 
 int xpar64_forward(const XparFwdArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL(lfw_xpar64_fwd_kernel, dim3((unsigned)(a.B * a.NC)), dim3(XW_THREADS), 0, stream, a);
+    const size_t left = scan_fwd_lds_bytes(XW_LEFT_TB, 16, 4, 16), smem = left > sizeof(FwdSmem) ? left : sizeof(FwdSmem);
+    hipLaunchKernelGGL(lfw_xpar64_fwd_kernel, dim3((unsigned)(a.B * a.NC)), dim3(XW_THREADS), smem, stream, a);
     return check_hip(hipGetLastError(), "lfw_xpar64_fwd_kernel launch");
 }
 
 int xpar64_backward(const XparBwdArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL(lfw_xpar64_bwd_kernel, dim3((unsigned)(2 * a.B * a.NC)), dim3(XW_THREADS), 0, stream, a);
+    const size_t left = scan_bwd_lds_bytes(scan::SegLen<4>::value, 16, 4, 16, XP_CHUNK, true);
+    const size_t smem = left > sizeof(BwdSmem) ? left : sizeof(BwdSmem);
+    const int rc = enable_lds(reinterpret_cast<const void *>(lfw_xpar64_bwd_kernel), (int)smem, "hipFuncSetAttribute(lfw_xpar64_bwd_kernel)");
+    if (rc) return rc;
+    hipLaunchKernelGGL(lfw_xpar64_bwd_kernel, dim3((unsigned)(2 * a.B * a.NC)), dim3(XW_THREADS), smem, stream, a);
     return check_hip(hipGetLastError(), "lfw_xpar64_bwd_kernel launch");
 }
 

@@ -57,6 +57,40 @@ def test_unusual_gates_and_values(what, D, K, dtype):
     check_all((x, f, q, k, fk, s), go, gs, dtype)
 
 
+@pytest.mark.parametrize("T", [40, 100, 250, 400])
+@pytest.mark.parametrize("D,K", [(64, 64), (33, 40)])
+def test_rows_left_next_to_others(T, D, K):
+    """Rows with a gate above one run step by step, on the workgroups of up to four of their chunks: one chunk to seven."""
+    x, f, q, k, fk, s, go, gs = make_config_inputs(5, T, D, K, F32, seed=T, in_scale=0.5, state_std=0.5)
+    f[1, T // 2, 3] = 1.25
+    fk[4, 0, 7] = 1.25
+    check_all((x, f, q, k, fk, s), go, gs, F32)
+
+
+def test_rows_left_take_no_longer_than_the_per_step_kernels(monkeypatch):
+    """Every row of 96 x 1024 steps has a gate above one.  Measured 1.03 times the per-step kernels' time; 7.4 times when
+    the workgroups that do such rows shared one die."""
+    from t2fw_amd import LFWFunction
+    ins = [t.cuda().requires_grad_() for t in make_config_inputs(96, 1024, 64, 64, F32, seed=2)[:6]]
+    with torch.no_grad():
+        ins[1][:, 500, 0] = 1.25
+    grads = [torch.ones(96, 1024, 64, device="cuda"), torch.ones(96, 64, 64, device="cuda")]
+
+    def fastest(flags):
+        monkeypatch.setenv("T2FW_FLAGS", flags)
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            torch.autograd.grad(LFWFunction.apply(*ins), ins, grads)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    assert fastest("32") < 2 * fastest("1")
+
+
 def _same_where_finite(got, want, what, tol):
     got, want = got.detach().double().cpu(), want.detach().double().cpu()
     assert torch.equal(torch.isnan(got), torch.isnan(want)), what
