@@ -106,7 +106,8 @@ extern "C" {
                                      and t2fw_lfw_workspace_bytes report for these flags.  Rows with a gate of magnitude
                                      above one, an input above 2^58 or a state above 2^120 (infinities and NaN among
                                      them) are done step by step over the whole sequence in the same call.  More than
-                                     65536 rows x chunks: the flag is ignored. */
+                                     65536 rows x chunks (1.11e9 bytes of workspace for 64 x 64 states): the flag is
+                                     ignored. */
 
 int t2fw_abi_version(void);
 const char *t2fw_last_error(void);

@@ -87,7 +87,8 @@ bool chunk_shape_ok(int64_t D, int64_t K, int32_t dtype, int32_t flags) {
 }
 
 // The chunk-parallel exact kernels (T2FW_FLAG_EXACT_CHUNKS) cover states of up to 64 x 64 that the 16-bit matrix-core
-// kernels do not take; the scratch is bounded (16 KB per row and chunk of 64 steps, 1 GB).
+// kernels do not take; the scratch is bounded (per row and chunk of 64 steps: the state and the gate products in fp32, both
+// widths rounded up to tiles of 16, 16.5 KB at most; 1.11e9 bytes in all).
 constexpr int64_t XPAR_MAX_ITEMS = 65536;
 int64_t xpar_chunks(int64_t T) { return T <= 0 ? 1 : (T + XP_CHUNK - 1) / XP_CHUNK; }
 bool xpar_ok(int64_t B, int64_t T, int64_t D, int64_t K, int32_t dtype, int32_t flags) {
@@ -95,18 +96,18 @@ bool xpar_ok(int64_t B, int64_t T, int64_t D, int64_t K, int32_t dtype, int32_t 
            dtype != T2FW_F64 && !chunk_shape_ok(D, K, dtype, flags) && B > 0 && T > 0 && B <= XPAR_MAX_ITEMS &&
            xpar_chunks(T) <= XPAR_MAX_ITEMS / B;
 }
-size_t xpar_workspace_bytes(int64_t B, int64_t T) {
-    const size_t items = (size_t)(B * xpar_chunks(T));
-    return items * (XP_N * XP_N * 4 + 2 * XP_N * 4) + (items * 4 + 255) / 256 * 256 + ((size_t)B * 16 + 255) / 256 * 256;
+size_t xpar_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K) {
+    const size_t items = (size_t)(B * xpar_chunks(T)), Dp = xp_padded(D), Kp = xp_padded(K);
+    return items * (Dp * Kp + Dp + Kp) * 4 + (items * 4 + 255) / 256 * 256 + ((size_t)B * 16 + 255) / 256 * 256;
 }
-XparScratch xpar_scratch(void *workspace, int64_t B, int64_t T) {
-    const size_t items = (size_t)(B * xpar_chunks(T));
+XparScratch xpar_scratch(void *workspace, int64_t B, int64_t T, int64_t D, int64_t K) {
+    const size_t items = (size_t)(B * xpar_chunks(T)), Dp = xp_padded(D), Kp = xp_padded(K);
     unsigned char *w = static_cast<unsigned char *>(workspace);
     XparScratch s;
     s.states = reinterpret_cast<float *>(w);
-    w += items * (XP_N * XP_N * 4);
+    w += items * (Dp * Kp * 4);
     s.tots = reinterpret_cast<float *>(w);
-    w += items * (2 * XP_N * 4);
+    w += items * ((Dp + Kp) * 4);
     s.chunk_flags = reinterpret_cast<int32_t *>(w);
     w += (items * 4 + 255) / 256 * 256;
     s.row_flags = reinterpret_cast<int32_t *>(w);
@@ -154,7 +155,7 @@ ParScratch par_scratch(int64_t B, int64_t T, int32_t C) {
 
 size_t forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32_t dtype, int32_t flags) {
     if (B > 0 && chunk_shape_ok(D, K, dtype, flags)) return 2 * row_flag_bytes(B);
-    if (xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T);
+    if (xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T, D, K);
     return 0;
 }
 
@@ -186,7 +187,7 @@ size_t backward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int3
         const size_t inner = par_ok(B, T, Cd, flags) ? par_scratch(B, T, Cd).total : 2 * row_flag_bytes(B);
         return Cd == C ? inner : dense_scratch(inner, B, T, Cd, elem_size(dtype)).total;
     }
-    if (C == XP_CHUNK && xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T);
+    if (C == XP_CHUNK && xpar_ok(B, T, D, K, dtype, flags)) return xpar_workspace_bytes(B, T, D, K);
     return 0;
 }
 
@@ -349,14 +350,14 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
         return chunk_forward(c, dtype, op, split, st);
     }
     if (xpar_ok(B, T, D, K, dtype, flags) && (ckpt == nullptr || C == XP_CHUNK) && T * heads < CHUNK_MAX_T) {
-        const size_t need = xpar_workspace_bytes(B, T);
+        const size_t need = xpar_workspace_bytes(B, T, D, K);
         if (workspace == nullptr || workspace_bytes < need)
             return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
         XparFwdArgs t{};
         t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.s0 = s0;
         t.out = out; t.next_state = next_state; t.ckpt = ckpt;
-        t.ws = xpar_scratch(workspace, B, T);
+        t.ws = xpar_scratch(workspace, B, T, D, K);
         t.B = B; t.T = T; t.NC = xpar_chunks(T);
         t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
         return xpar_forward(t, dtype, st);
@@ -500,14 +501,14 @@ static int lfw_backward_rows(const void *g_out, const void *g_state, const void 
         return chunk_backward(c, dtype, op, st);
     }
     if (C_given == XP_CHUNK && xpar_ok(B, T, D, K, dtype, flags) && T * heads < CHUNK_MAX_T) {
-        const size_t need = xpar_workspace_bytes(B, T);
+        const size_t need = xpar_workspace_bytes(B, T, D, K);
         if (workspace == nullptr || workspace_bytes < need)
             return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         if (!aligned16({workspace})) return fail(T2FW_ERR_MISALIGNED, "the workspace must be 16-byte aligned");
         XparBwdArgs t{};
         t.g_out = g_out; t.g_state = g_state; t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.ckpt = ckpt;
         t.d_x = d_x; t.d_f = d_f; t.d_q = d_q; t.d_k = d_k; t.d_f_key = d_f_key; t.d_s0 = d_s0;
-        t.ws = xpar_scratch(workspace, B, T);
+        t.ws = xpar_scratch(workspace, B, T, D, K);
         t.B = B; t.T = T; t.NC = a.NC;
         t.D = (int32_t)D; t.K = (int32_t)K; t.heads = (int32_t)heads;
         return xpar_backward(t, dtype, st);

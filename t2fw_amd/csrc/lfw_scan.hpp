@@ -16,9 +16,10 @@ struct ScanFwdArgs {
     // them: a pass with accumulate set adds its share to what the passes before it left in out.
     int64_t col0, colw;
     int32_t accumulate;
-    // Not null: the state before the first step comes from here (fp32, [64][64] whatever D and K) instead of s0, and
-    // next_state may be null: one chunk in the middle of a sequence (states of up to 64 x 64 only).
+    // Not null: the state before the first step comes from here (fp32, [D][K] with rows of s_stride elements) instead of
+    // s0, and next_state may be null: one chunk in the middle of a sequence (states of up to 64 x 64 only).
     const float *s_start;
+    int32_t s_stride;
 };
 
 struct ScanBwdArgs {
@@ -31,9 +32,10 @@ struct ScanBwdArgs {
     // side 1; colw = 0: all of them); with accumulate set the pass adds to the [.., T, .., D|K] gradients.
     int64_t col0, colw;
     int32_t accumulate;
-    // Not null: the adjoint of the state after the last step comes from here (fp32, [64][64] whatever D and K) instead
-    // of g_state, and d_s0 may be null: one chunk in the middle of a sequence (states of up to 64 x 64 only).
+    // Not null: the adjoint of the state after the last step comes from here (fp32, [D][K] with rows of g_stride elements)
+    // instead of g_state, and d_s0 may be null: one chunk in the middle of a sequence (states of up to 64 x 64 only).
     const float *g_end;
+    int32_t g_stride;
 };
 
 // Dynamic LDS, in bytes, that the scan bodies use for a 32-bit accumulator (lfw_scan_body.hpp): the kernels

@@ -46,7 +46,7 @@ __device__ __forceinline__ void fwd_scan_body_kg(const ScanFwdArgs &p, int64_t b
 #pragma unroll
     for (int j = 0; j < KPL; ++j)
         S[j] = !(row_ok && g.k0 + j < KW) ? Acc(0)
-               : p.s_start != nullptr     ? Acc(p.s_start[d * 64 + g.k0 + j])
+               : p.s_start != nullptr     ? Acc(p.s_start[d * p.s_stride + g.k0 + j])
                                           : to_acc(s0[(b * D + d) * K + col0 + g.k0 + j]);
 
     // outputs of a block of steps: written, or added to what the passes over other key channels left
@@ -187,7 +187,7 @@ __device__ __forceinline__ void bwd_scan_body_kg(const ScanBwdArgs &p, int64_t b
     if (p.g_end != nullptr) {
 #pragma unroll
         for (int j = 0; j < KPL; ++j)
-            G[j] = el_ok(j) ? Acc(p.g_end[SIDE == 0 ? row * 64 + g.k0 + j : (g.k0 + j) * 64 + row]) : Acc(0);
+            G[j] = el_ok(j) ? Acc(p.g_end[SIDE == 0 ? row * p.g_stride + g.k0 + j : (int64_t)(g.k0 + j) * p.g_stride + row]) : Acc(0);
     } else {
         const IO *gs = (const IO *)p.g_state + b * DK;
 #pragma unroll

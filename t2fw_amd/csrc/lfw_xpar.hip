@@ -63,7 +63,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
     const int chunk = (int)(item - b * p.NC);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int side = w >> 2, cb = w & 3, i = lane & 15, kg = lane >> 4, c = 16 * cb + i;
-    const int width = side ? p.K : p.D;
+    const int width = side ? p.K : p.D, Dp = xp_padded(p.D), Kp = xp_padded(p.K);
     const int n_tok = (int)min((int64_t)XP_CHUNK, p.T - (int64_t)chunk * XP_CHUNK);
     float *const VS = smem, *const KS = smem + XP_CHUNK * XLS;
     int bad = 0;
@@ -125,7 +125,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
                 tile[t * XLS + c] = a * (base * l[j]);
             }
         }
-        if (kg == 0) p.ws.tots[(item * 2 + side) * XP_N + c] = carry;
+        if (kg == 0) p.ws.tots[item * (Dp + Kp) + (side ? Dp : 0) + c] = carry;
     }
     const int any = __syncthreads_or(bad);
     if (tid == 0) p.ws.chunk_flags[item] = any;
@@ -154,7 +154,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
             }
             sum += m0 + m1;
         }
-        *reinterpret_cast<float4 *>(p.ws.states + item * (XP_N * XP_N) + (16 * db + i) * XP_N + 16 * kb + 4 * kg) =
+        *reinterpret_cast<float4 *>(p.ws.states + item * (Dp * Kp) + (16 * db + i) * Kp + 16 * kb + 4 * kg) =
             make_float4(sum[0], sum[1], sum[2], sum[3]);
     }
 }
@@ -166,7 +166,7 @@ constexpr int XC_THREADS = 256, XC_BATCH = 8;
 template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void lfw_xpar_chain_kernel(PassArgs p) {
     const int64_t b = blockIdx.x >> 2;
     const int idx = (blockIdx.x & 3) * XC_THREADS + threadIdx.x, d = idx >> 4, k = (idx & 15) * 4;
-    const int D = p.D, K = p.K, NC = (int)p.NC;
+    const int D = p.D, K = p.K, NC = (int)p.NC, Dp = xp_padded(D), Kp = xp_padded(K);
     int bad = 0;
     for (int c = threadIdx.x; c < NC; c += XC_THREADS) bad |= p.ws.chunk_flags[b * NC + c];
     if (d < D && k < K) {
@@ -177,8 +177,8 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
             S[e] = k + e < K ? to_acc(((const IO *)p.first)[b * DK + o + e]) : 0.0f;
             bad |= !(fabsf(S[e]) <= XP_MAX_STATE) ? 1 : 0;
         }
-        float *const st = p.ws.states + b * NC * (int64_t)(XP_N * XP_N) + d * XP_N + k;
-        const float *const tots = p.ws.tots + b * NC * (int64_t)(2 * XP_N);
+        float *const st = p.ws.states + b * NC * (int64_t)(Dp * Kp) + d * Kp + k;
+        const float *const tots = p.ws.tots + b * NC * (int64_t)(Dp + Kp);
         IO *const ckpt = p.ckpt != nullptr ? (IO *)p.ckpt + b * NC * DK + o : nullptr;
         for (int n0 = 0; n0 < NC; n0 += XC_BATCH) {
             float4 m[XC_BATCH], tb[XC_BATCH];
@@ -186,15 +186,15 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
 #pragma unroll
             for (int u = 0; u < XC_BATCH; ++u) {
                 const int n = min(n0 + u, NC - 1), c = BWD ? NC - 1 - n : n;
-                m[u] = *reinterpret_cast<const float4 *>(st + (int64_t)c * (XP_N * XP_N));
-                ta[u] = tots[c * 2 * XP_N + d];
-                tb[u] = *reinterpret_cast<const float4 *>(tots + c * 2 * XP_N + XP_N + k);
+                m[u] = *reinterpret_cast<const float4 *>(st + (int64_t)c * (Dp * Kp));
+                ta[u] = tots[c * (int64_t)(Dp + Kp) + d];
+                tb[u] = *reinterpret_cast<const float4 *>(tots + c * (int64_t)(Dp + Kp) + Dp + k);
             }
 #pragma unroll
             for (int u = 0; u < XC_BATCH; ++u) {
                 if (n0 + u >= NC) break;
                 const int c = BWD ? NC - 1 - (n0 + u) : n0 + u;
-                *reinterpret_cast<float4 *>(st + (int64_t)c * (XP_N * XP_N)) = make_float4(S[0], S[1], S[2], S[3]);
+                *reinterpret_cast<float4 *>(st + (int64_t)c * (Dp * Kp)) = make_float4(S[0], S[1], S[2], S[3]);
                 if (!BWD && ckpt != nullptr) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -241,7 +241,8 @@ template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void 
     a.out = (IO *)base.out + line * base.D;
     a.ckpt = nullptr;
     a.next_state = chunk == (int)NC - 1 ? (IO *)base.next_state + b * base.D * base.K : nullptr;
-    a.s_start = ws.states + item * (XP_N * XP_N);
+    a.s_stride = xp_padded(base.K);
+    a.s_start = ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
     a.T = min((int64_t)XP_CHUNK, base.T - (int64_t)chunk * XP_CHUNK);
     scan::fwd_scan_body_kg<IO, KPL, 16>(a, 0, tile);
 }
@@ -267,7 +268,8 @@ template <typename IO, int KV, int KK> __global__ __launch_bounds__(SCAN_THREADS
         a.d_q = (IO *)base.d_q + line * base.K; a.d_k = (IO *)base.d_k + line * base.K;
         a.d_f_key = (IO *)base.d_f_key + line * base.K;
         a.d_s0 = chunk == 0 ? (IO *)base.d_s0 + b * base.D * base.K : nullptr;
-        a.g_end = ws.states + item * (XP_N * XP_N);
+        a.g_stride = xp_padded(base.K);
+        a.g_end = ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
         a.T = min((int64_t)XP_CHUNK, base.T - (int64_t)chunk * XP_CHUNK);
         a.NC = 1;
         row = 0;

@@ -7,11 +7,13 @@
 namespace t2fw {
 
 constexpr int XP_CHUNK = 64;           // tokens per chunk, and between checkpoints
-constexpr int XP_N = 64;               // row stride of a chunk's state in the scratch
+constexpr int XP_N = 64;               // the widest state
+// A chunk's state in the scratch: [D][K], both rounded up to whole tiles of 16 channels.
+__host__ __device__ constexpr int xp_padded(int64_t width) { return (int)((width + 15) / 16 * 16); }
 
 struct XparScratch {
-    float *states;                     // [B * NC][64][64]: a chunk's increment, then the state (adjoint) entering it
-    float *tots;                       // [B * NC][2][64]: a chunk's gate products, value side and key side
+    float *states;                     // [B * NC][D][K], padded: a chunk's increment, then the state (adjoint) entering it
+    float *tots;                       // [B * NC][D + K], padded: a chunk's gate products, value side and key side
     int32_t *chunk_flags;              // [B * NC]
     int32_t *row_flags;                // [B][4]: the row is left to the recurrence over the whole sequence
 };
