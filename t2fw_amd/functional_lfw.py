@@ -46,6 +46,13 @@ def _sizes(rows, T, D, K, C, code, flags):
             lib.t2fw_lfw_workspace_bytes(rows, T, D, K, C, code, flags), tuple(regions))
 
 
+@functools.lru_cache(maxsize=256)
+def _forward_plan(rows, T, D, K, C, dtype, flags):
+    """The flags a forward call of this shape runs with (and its backward after it), then _sizes with these flags"""
+    flags = _exact_chunk_flags(rows, T, D, K, C, dtype, flags)
+    return (flags,) + _sizes(rows, T, D, K, C, _lib.DTYPE_CODE[dtype], flags)
+
+
 def _host_hints_enabled():
     """T2FW_HOST_HINTS=0 keeps every workspace in device memory (the backward then decides on the device)."""
     return os.environ.get("T2FW_HOST_HINTS", "1") != "0"
@@ -53,7 +60,7 @@ def _host_hints_enabled():
 
 def _on_device(dev):
     """Make ``dev`` current for the allocations and the launch, without the cost of switching when it already is."""
-    if dev.type != "cuda" or dev.index is None or dev.index == torch.cuda.current_device():
+    if dev.index is None or dev.index == torch.cuda.current_device():      # (host memory has no index)
         return contextlib.nullcontext()
     return torch.cuda.device(dev)
 
@@ -234,9 +241,8 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
         return _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
     lib = _lib.load()
     C = _ckpt_interval()
-    flags = _exact_chunk_flags(B * H, T, D, K, C, value.dtype, flags)
     dev = value.device
-    nc, ws_bytes, _, regions = _sizes(B * H, T, D, K, C, code, flags)
+    flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags)
     with _on_device(dev):
         outputs = torch.empty_like(value)
         next_state = torch.empty_like(state)
