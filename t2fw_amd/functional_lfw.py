@@ -47,9 +47,9 @@ def _sizes(rows, T, D, K, C, code, flags):
 
 
 @functools.lru_cache(maxsize=256)
-def _forward_plan(rows, T, D, K, C, dtype, flags):
+def _forward_plan(rows, T, D, K, C, dtype, flags, need_grad):
     """The flags a forward call of this shape runs with (and its backward after it), then _sizes with these flags"""
-    flags = _exact_chunk_flags(rows, T, D, K, C, dtype, flags)
+    flags = _exact_chunk_flags(rows, T, D, K, C, dtype, flags, need_grad)
     return (flags,) + _sizes(rows, T, D, K, C, _lib.DTYPE_CODE[dtype], flags)
 
 
@@ -81,21 +81,53 @@ def _dtype_code(dtype):
 
 
 # Where the chunk-parallel exact kernels (three launches per direction) take the place of the per-step ones (one launch
-# forward, two backward).  Forward + backward, per-step against chunk-parallel, microseconds: 96 rows of 64 x 64 float32,
-# 128 steps 180 / 192 (host-bound: the launches), 256 steps 264 / 216, 1024 steps 1000 / 555; 13 rows of 33 x 17 float16,
-# 128 steps 177 / 195, 385 steps 338 / 193.  Many rows fill the chip by themselves: 512 rows of 64 x 64, 256 steps 872 /
-# 886; 1024 rows of 16 x 16 277 / 364.
+# forward, two backward): where a sequence is long enough for the launches, and the rows are few enough that the per-step
+# kernels leave the chip idle.  Both sides in microseconds of GPU time, per-step / chunk-parallel.
+#   Steps, forward + backward: 96 rows of 64 x 64 float32, 128 steps 146 / 125 (a host that needs 180 for the launches:
+#     172 / 185), 224 steps 234 / 176, 1024 steps 992 / 541; 24 rows of 16 x 16, 224 steps 156 / 57 (such a host: 180 / 190).
+#   64 x 64 (float32; kernels of its own): 256 rows x 256 steps 497 / 372, forward alone 1.13 times as fast or more.  More
+#     rows would gain too (512 rows x 256 steps 918 / 739); the limit bounds the scratch.
+#   A width of 8 or less, where a workgroup of the per-step kernels takes several rows' worth of channels: 1024 rows of 8 x 8,
+#     224 steps 1341 / 345; 64 x 8 forward alone, 128 rows x 224 steps 1.17 times as fast, 160 rows 1.00, 256 rows 0.75.
+#   16 x 16: 384 rows x 224 steps 170 / 145, 512 rows 172 / 184, 768 rows 222 / 259, 1024 rows 248 / 332; x 448 steps 512 rows
+#     321 / 323, 640 rows 414 / 394, 768 rows 419 / 456.
+#   32 x 32: 384 rows x 224 steps 254 / 248, 512 rows 288 / 314.  33 x 17: 256 rows 257 / 250, 341 rows 288 / 325.
+#   63 x 63: 160 rows x 224 steps 313 / 300, 192 rows 332 / 363, 256 rows 457 / 459; x 1024 steps 256 rows 1.07 times as fast.
+#   Forward alone (one launch against three): up to 256 tiles of value channels 1.1 to 6 times as fast at every width; 384
+#     tiles 0.82 (16 x 16) to 1.07 (33 x 17) at 224 steps, 1.06 to 1.33 at 1024; 512 tiles 0.68 to 0.88, where the per-step
+#     kernel's workgroups come to two per CU; 640 and 768 tiles 1.02 to 1.48 from 448 steps on; 1024 tiles 0.72 to 1.0.
 EXACT_CHUNKS_MIN_STEPS = 224
-EXACT_CHUNKS_MAX_TILES = 1024          # rows x blocks of 16 channels
 
 
-def _exact_chunk_flags(rows, T, D, K, C, dtype, flags):
+def _exact_chunks_faster(rows, T, D, K, need_grad):
+    """Whether the chunk-parallel exact kernels take less time for ``rows`` states of D x K (up to 64 x 64) over T steps."""
+    if T < EXACT_CHUNKS_MIN_STEPS:
+        return False
+    if D == 64 and K == 64:
+        return rows <= 256
+    if not need_grad:
+        tiles = rows * -(-D // 16)
+        if K <= 8:
+            return tiles <= (1024 if D <= 16 else 512)
+        return tiles <= 256 or (T >= 1024 and tiles <= 384) or (T >= 448 and 512 < tiles <= 768)
+    narrow, wide = min(D, K), max(D, K)
+    tiles = rows * -(-wide // 16)
+    if narrow <= 8:
+        return tiles <= 1024
+    if wide <= 16:
+        return tiles <= (384 if T < 448 else 640)
+    if narrow <= 32:
+        return tiles <= 768
+    return tiles <= (640 if T < 448 else 1024)
+
+
+def _exact_chunk_flags(rows, T, D, K, C, dtype, flags, need_grad):
     """``flags`` of a call that the 16-bit matrix-core kernels do not take, with FLAG_EXACT_CHUNKS added where the
-    chunk-parallel exact kernels serve it (states of up to 64 x 64, checkpoints every 64 steps); a caller's own flags
-    stand."""
-    if flags != _lib.FLAG_AUTO or C != 64 or D > 64 or K > 64 or T < EXACT_CHUNKS_MIN_STEPS or dtype == torch.float64:
+    chunk-parallel exact kernels serve it (states of up to 64 x 64, checkpoints every 64 steps) and are faster; a caller's
+    own flags stand."""
+    if flags != _lib.FLAG_AUTO or C != 64 or D > 64 or K > 64 or dtype == torch.float64:
         return flags
-    if (D == 64 and K == 64 and dtype != torch.float32) or rows * -(-max(D, K) // 16) > EXACT_CHUNKS_MAX_TILES:
+    if (D == 64 and K == 64 and dtype != torch.float32) or not _exact_chunks_faster(rows, T, D, K, need_grad):
         return flags
     return flags | _lib.FLAG_EXACT_CHUNKS
 
@@ -242,7 +274,7 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
     lib = _lib.load()
     C = _ckpt_interval()
     dev = value.device
-    flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags)
+    flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags, need_grad)
     with _on_device(dev):
         outputs = torch.empty_like(value)
         next_state = torch.empty_like(state)
