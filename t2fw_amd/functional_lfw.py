@@ -54,8 +54,10 @@ def _forward_plan(rows, T, D, K, C, dtype, flags, need_grad):
 
 
 def _host_hints_enabled():
-    """T2FW_HOST_HINTS=0 keeps every workspace in device memory (the backward then decides on the device)."""
-    return os.environ.get("T2FW_HOST_HINTS", "1") != "0"
+    """T2FW_HOST_HINTS=0 keeps every workspace in device memory (the backward then decides on the device).  So does
+    torch.use_deterministic_algorithms: whether the hints are there when the backward is issued depends on the host's
+    pace, and for a batch with hinted rows the two backward kernels differ in the last bits."""
+    return os.environ.get("T2FW_HOST_HINTS", "1") != "0" and not torch.are_deterministic_algorithms_enabled()
 
 
 def _on_device(dev):

@@ -14,6 +14,10 @@ the backward call is issued, and pick the backward's flags without any synchroni
   * hints not there yet, or the stream is being captured into a graph -> the default call, which
     decides everything on the device.
 
+The three are equally accurate but not equal to the bit where rows are hinted, so which bits a training step
+gives then depends on the host's pace.  T2FW_HOST_HINTS=0 and torch.use_deterministic_algorithms(True) leave
+the choice to the device.
+
 The reference has a single path (t2fw/csrc/lfw.cpp:50-96); this module has no counterpart there.
 """
 import ctypes

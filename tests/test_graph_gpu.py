@@ -24,8 +24,12 @@ def make(B, T, seed, dtype=torch.float16, heads=None):
 
 
 @pytest.mark.parametrize("kind", ["folded", "heads", "flagged"])
-def test_replays_match_eager(kind):
+def test_replays_match_eager(kind, monkeypatch):
     from t2fw_amd import LFWFunction, LFWHeadsFunction
+    if kind == "flagged":
+        # a captured step leaves the choice of the backward kernel to the device; an eager step with a hinted row would
+        # take another one, equally accurate but not bit-equal, whenever the forward has completed in time
+        monkeypatch.setenv("T2FW_HOST_HINTS", "0")
     B, T = 6, 200
     heads = 3 if kind == "heads" else None
     fn = LFWHeadsFunction if heads else LFWFunction

@@ -245,3 +245,44 @@ def test_backward_before_the_hints_arrive_takes_the_default_path(monkeypatch):
     torch.autograd.backward([out, nxt], [go.cuda(), gs.cuda()])
     torch.cuda.synchronize()
     check((x, f, q, k, fk, s), go, gs, out, nxt, [t.grad for t in ins], torch.float16)
+
+
+def _one_row_of_six_hinted():
+    x, f, q, k, fk, s, go, gs = make_config_inputs(6, 200, 64, 64, torch.float16, seed=2, state_std=0.2)
+    f = f.clone()
+    f[2, 7, 5] = -0.0                   # outside [0, 1] to the kernels: redone exactly, and hinted
+    return (x, f, q, k, fk, s), go, gs
+
+
+def test_block_wise_backward_for_a_batch_with_one_hinted_row():
+    """the choice where the hints are there in time: the other rows come from the block-wise kernel too"""
+    from t2fw.functional_lfw import LFWFunction
+    inputs, go, gs = _one_row_of_six_hinted()
+    ins = [t.cuda().requires_grad_(True) for t in inputs]
+    out, nxt = LFWFunction.apply(*ins)
+    torch.cuda.synchronize()
+    grads = torch.autograd.grad([out, nxt], ins, [go.cuda(), gs.cuda()])
+    check(inputs, go, gs, out, nxt, grads, torch.float16)
+
+
+def test_deterministic_algorithms_give_the_same_bits_at_any_pace(monkeypatch):
+    """with the hints there when the backward is issued, and late"""
+    from t2fw.functional_lfw import LFWFunction
+    from t2fw_amd import path_hint
+    inputs, go, gs = _one_row_of_six_hinted()
+
+    def run():
+        ins = [t.cuda().requires_grad_(True) for t in inputs]
+        res = LFWFunction.apply(*ins)
+        torch.cuda.synchronize()
+        return list(res) + list(torch.autograd.grad(res, ins, [go.cuda(), gs.cuda()]))
+
+    torch.use_deterministic_algorithms(True)
+    try:
+        in_time = run()
+        monkeypatch.setattr(path_hint.ForwardHints, "hinted_rows", lambda self: None)
+        late = run()
+    finally:
+        torch.use_deterministic_algorithms(False)
+    for a, b in zip(in_time, late):
+        assert torch.equal(a, b)
