@@ -1,6 +1,6 @@
 """The chunk-parallel exact kernels of the decay rule (T2FW_FLAG_EXACT_CHUNKS: float32 tensors, widths of up to 64)
 against the float64 oracle, at the tolerance of the per-step kernels (TOL of test_lfw_gpu).  Sizes sit on the edges of the
-kernels' pieces (8, 16 and 64 steps, 16 and 32 channels)."""
+kernels' pieces (8, 16 and 64 steps, 16 and 32 channels, eight chunks of the chain)."""
 import pytest
 import torch
 
@@ -21,6 +21,8 @@ F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
 @pytest.mark.parametrize("B,T,D,K,dtype", [
     (1, 1, 64, 64, F32), (2, 7, 64, 64, F32), (2, 8, 64, 64, F32), (2, 9, 64, 64, F32), (2, 17, 64, 64, F32),
     (3, 64, 64, 64, F32), (2, 65, 64, 64, F32), (2, 127, 64, 64, F32), (2, 1000, 64, 64, F32), (2, 80, 1, 1, F32),
+    (2, 8 * 64, 64, 64, F32), (2, 8 * 64 + 1, 64, 64, F32), (2, 13 * 64 - 5, 64, 64, F32), (2, 17 * 64 + 2, 64, 64, F32),
+    (2, 8 * 64 + 1, 20, 40, F32), (2, 12 * 64, 40, 20, F32), (2, 15 * 64 - 1, 20, 40, F16), (1, 25 * 64 + 9, 9, 7, F32),
     (2, 80, 16, 17, F32), (1, 200, 63, 48, F32), (2, 65, 33, 64, F32), (2, 130, 64, 32, F32),
     (2, 150, 17, 5, F16), (2, 64, 64, 49, F16), (2, 150, 31, 32, BF16),
 ])
