@@ -39,12 +39,6 @@ constexpr int XI_THREADS = 512;
 constexpr int XLS = 68;                // row stride, in floats, of the token-major tiles [64][XLS]
 constexpr float XP_MAX_INPUT = 0x1p58f, XP_MAX_STATE = 0x1p120f;
 
-__device__ __forceinline__ int64_t uniform64(int64_t v) {
-    const u32 lo = __builtin_amdgcn_readfirstlane((u32)(unsigned long long)v);
-    const u32 hi = __builtin_amdgcn_readfirstlane((u32)((unsigned long long)v >> 32));
-    return (int64_t)(((unsigned long long)hi << 32) | lo);
-}
-
 // What launches 1 and 2 read and write; BWD swaps the arrays and the direction of the products.
 struct PassArgs {
     const void *val, *gate_val, *key, *gate_key;      // x f k f_key, or g_out f q f_key
@@ -219,11 +213,6 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
 // dies and shader engines: 96 rows x 1024 steps with a gate above one in each, 32 x 32 fp32, forward + backward 2050 us
 // against 563 now and 752 on the per-step kernels; 64 x 64 7300, 1019, 992 (96 x 256 590, 277, 264; 16 x 1024 1430, 604,
 // 909).
-__device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
-    const int4 v = *reinterpret_cast<const int4 *>(ws.row_flags + 4 * b);
-    return __builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0;
-}
-
 // One workgroup per (row, chunk, 16 value channels); base: the call over whole rows.
 template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_fwd_kernel(ScanFwdArgs base, XparScratch ws, int64_t NC) {
     const int64_t pair = blockIdx.x / base.ntiles, b = pair % base.B;

@@ -18,6 +18,19 @@ struct XparScratch {
     int32_t *row_flags;                // [B][4]: the row is left to the recurrence over the whole sequence
 };
 
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long long)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)v >> 32));
+    return (int64_t)(((unsigned long long)hi << 32) | lo);
+}
+
+// the row is left to the recurrence over the whole sequence
+__device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
+    const int4 v = *reinterpret_cast<const int4 *>(ws.row_flags + 4 * b);
+    return __builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0;
+}
+
 struct XparFwdArgs {
     const void *x, *f, *q, *k, *f_key, *s0;
     void *out, *next_state, *ckpt;     // ckpt may be null; else one state per chunk

@@ -33,13 +33,6 @@ constexpr int XW_THREADS = 256;
 constexpr int XW_COLS = 16;            // columns per wave
 constexpr int XW_SEG = 8;              // steps whose inputs, states and sums are in flight together
 
-// a value that is the same in every lane, moved to scalar registers
-__device__ __forceinline__ int64_t uniform64(int64_t v) {
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long long)v);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)v >> 32));
-    return (int64_t)(((unsigned long long)hi << 32) | lo);
-}
-
 // XW_SEG steps of one array, one value per lane.  p: the array at the segment's first step (wave-uniform), c: the lane's
 // channel; steps from n on are read from the last one (and replaced by pad_steps).
 __device__ __forceinline__ void load_steps(float (&r)[XW_SEG], const float *p, int c, int64_t ts, int n) {
@@ -156,11 +149,6 @@ __device__ __forceinline__ void scale_outer(floatx4 (&G)[4], float col, float ro
         : "v"(col), "v"(row));
 #pragma unroll
     for (int n = 0; n < 16; ++n) G[n / 4][n % 4] *= g[n];
-}
-
-__device__ __forceinline__ bool row_left(const XparScratch &ws, int64_t b) {
-    const int4 v = *reinterpret_cast<const int4 *>(ws.row_flags + 4 * b);
-    return __builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0;
 }
 
 // 16 consecutive columns of row `row` of a [64][64] state, or 16 rows of column `row` (TRANSPOSED); p, col0 wave-uniform,
