@@ -140,7 +140,7 @@ def _exact_chunk_flags(rows, T, D, K, C, dtype, flags, need_grad):
 # channels 64 i .. 64 i + 63 with key channels 64 j .. 64 j + 63 -- whose outputs add up over j.  For fp16 / bf16
 # tensors the blocks run as heads through the head-strided entry points, i.e. on the matrix-core
 # kernels, which take 64 x 64 states only; the exact per-step kernels that would otherwise serve such widths take
-# 4.1 ms for a forward + backward at B=24, T=1024, D=K=128 where the blocks take 0.24 ms.  The reference has one
+# 4.2 ms for a forward + backward at B=24, T=1024, D=K=128 where the blocks take 0.16 ms.  The reference has one
 # kernel for every shape (t2fw/csrc/lfw_kernel.cu:105-121).
 def _block_counts(value, query, flags):
     """(D / 64, K / 64) if tensors of these widths run as blocks, else None"""
@@ -349,7 +349,8 @@ class LFWFunction(torch.autograd.Function):
     Inputs are already gated (no sigmoid is applied here), as in the reference.
     fp16 / bf16 tensors with D = K = 64 run on the matrix-core kernels, those whose widths are other multiples
     of 64 as independent 64 x 64 blocks on the same kernels (``_block_counts`` above), everything else on the
-    exact kernels (per-step, or with the chunks of a row side by side: ``_exact_chunk_flags``); T2FW_FLAGS=1 keeps the exact kernels for every shape."""
+    exact kernels (per-step, or with the chunks of a row side by side: ``_exact_chunk_flags``); T2FW_FLAGS=1 keeps
+    the per-step kernels for every shape."""
 
     @staticmethod
     def forward(ctx, value, forget, query, key, f_key, state):
@@ -532,9 +533,9 @@ def lfw_apply_padded(value, forget, query, key, f_key, state):
     matrix-core kernels: the widths are padded up to the next multiple of 64 (values, keys, queries and the state
     with zeros, gates with ones -- the padded channels stay zero and add nothing), the padded tensors run as
     64 x 64 blocks (``LFWFunction.apply`` does that by itself for multiples of 64), and the results are cut back.
-    Correct for any width, and as expensive as the padded width: a 32 x 32 state costs what a 64 x 64 one costs,
-    which is still a quarter of the exact per-step kernels' time at B=96, T=1024.  An explicit choice of the
-    caller, because the results carry the matrix-core kernels' accuracy where ``LFWFunction.apply`` runs the exact
+    Correct for any width, and as expensive as the padded width: a 32 x 32 state costs what a 64 x 64 one costs
+    (forward + backward at B=96, T=1024: 201 us of GPU time where the exact kernels take 278; 33 x 17: 207 and
+    414).  An explicit choice of the caller, because the results carry the matrix-core kernels' accuracy where ``LFWFunction.apply`` runs the exact
     kernels for such widths.  Padding, cutting and their gradients are plain tensor operations."""
     assert value.dtype in (torch.float16, torch.bfloat16), "the matrix-core kernels take fp16 / bf16 tensors"
     assert value.shape == forget.shape and query.shape == key.shape and query.shape == f_key.shape
