@@ -11,7 +11,8 @@
 //   2  lfw_xpar_chain_kernel, elementwise: the chain over the chunks of a row; leaves the state at the START (the adjoint
 //      at the END) of every chunk in fp32 in place of the increments and writes the checkpoints.
 //   3  lfw_xpar_fwd_kernel / lfw_xpar_bwd_kernel: the recurrence itself, step by step, within each chunk; the last chunk's
-//      leaves the final state, the first one's d_s0.
+//      leaves the final state, the first one's d_s0.  64 x 64 fp32 (lfw_xpar64.hip): on fp64 matrix instructions where the
+//      gates allow it, and one more launch for the chunks where they don't.
 //
 // A row is left to the recurrence over the whole sequence where the sums could differ from it by more than rounding:
 //   * a gate of magnitude above one (or NaN): the product of one side's gates may overflow where the product of both
@@ -21,8 +22,8 @@
 //     increment of decayed factors comes out finite, and infinity times a gate product that has underflowed is NaN.
 // The workgroups of the row's first chunk (64 x 64 fp32: of the first four) do it in launch 3, the others of that row leave.
 //
-// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 25 + 19 + 70 us (220 per-step), backward 25 + 11 +
-// 440 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
+// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 31 + 19 + 56 + 4 us (220 per-step), backward 26 + 11 +
+// 160 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
 //
 // Replaces lfw_cuda_fwd_kernel, lfw_cuda_bwd_kernel and the einsums of the reference
 // (t2fw/csrc/lfw_kernel.cu:18-102, t2fw/csrc/lfw.cpp:45,84-93); semantics t2fw/torch.py:21-31.
@@ -37,7 +38,6 @@ namespace {
 
 constexpr int XI_THREADS = 512;
 constexpr int XLS = 68;                // row stride, in floats, of the token-major tiles [64][XLS]
-constexpr float XP_MAX_INPUT = 0x1p58f, XP_MAX_STATE = 0x1p120f;
 
 // What launches 1 and 2 read and write; BWD swaps the arrays and the direction of the products.
 struct PassArgs {
@@ -60,7 +60,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
     const int width = side ? p.K : p.D, Dp = xp_padded(p.D), Kp = xp_padded(p.K);
     const int n_tok = (int)min((int64_t)XP_CHUNK, p.T - (int64_t)chunk * XP_CHUNK);
     float *const VS = smem, *const KS = smem + XP_CHUNK * XLS;
-    int bad = 0;
+    int bad = 0, small = 0;
     if (16 * cb < width) {                       // wave-uniform
         const int64_t off = uniform64((row_first_token(b, p.T, p.heads) + (int64_t)chunk * XP_CHUNK * p.heads) * width);
         const IO *const gp = (const IO *)(side ? p.gate_key : p.gate_val) + off;
@@ -88,6 +88,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
             for (int j = 0; j < 4; ++j) {
                 g[j] = (ch_ok && 16 * m + 4 * kg + j < n_tok) ? to_acc(rg[m][j]) : 1.0f;
                 bad |= !(fabsf(g[j]) <= 1.0f) ? 1 : 0;
+                small |= !(g[j] >= XP_MM_MIN_GATE) ? 1 : 0;
             }
             float own;                           // product of the lane's four gates
             if (BWD) {                           // l: up to and with the token
@@ -121,8 +122,8 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XI_THREADS) void l
         }
         if (kg == 0) p.ws.tots[item * (Dp + Kp) + (side ? Dp : 0) + c] = carry;
     }
-    const int any = __syncthreads_or(bad);
-    if (tid == 0) p.ws.chunk_flags[item] = any;
+    const int any = __syncthreads_or(bad | small), left = any ? __syncthreads_or(bad) : 0;      // any: the same in every thread
+    if (tid == 0) p.ws.chunk_flags[item] = left ? XP_ROW_LEFT : any ? XP_CHUNK_STEPS : 0;
     // wave w: key channels of blocks kb, value channels of block db; a lane stores four consecutive k of its d
     const int db = w & 3;
     if (16 * db >= p.D) return;
@@ -162,7 +163,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
     const int idx = (blockIdx.x & 3) * XC_THREADS + threadIdx.x, d = idx >> 4, k = (idx & 15) * 4;
     const int D = p.D, K = p.K, NC = (int)p.NC, Dp = xp_padded(D), Kp = xp_padded(K);
     int bad = 0;
-    for (int c = threadIdx.x; c < NC; c += XC_THREADS) bad |= p.ws.chunk_flags[b * NC + c];
+    for (int c = threadIdx.x; c < NC; c += XC_THREADS) bad |= p.ws.chunk_flags[b * NC + c] & XP_ROW_LEFT;
     if (d < D && k < K) {
         const int64_t DK = (int64_t)D * K, o = d * K + k;
         float S[4];

@@ -8,6 +8,9 @@ namespace t2fw {
 
 constexpr int XP_CHUNK = 64;           // tokens per chunk, and between checkpoints
 constexpr int XP_N = 64;               // the widest state
+constexpr float XP_MAX_INPUT = 0x1p58f, XP_MAX_STATE = 0x1p120f;      // lfw_xpar.hip
+constexpr float XP_MM_MIN_GATE = 0x1p-20f;                             // lfw_xpar64_mm.hpp
+constexpr int XP_ROW_LEFT = 1, XP_CHUNK_STEPS = 2;                     // chunk_flags: a smaller gate (64 x 64 fp32: step by step)
 // A chunk's state in the scratch: [D][K], both rounded up to whole tiles of 16 channels.
 __host__ __device__ constexpr int xp_padded(int64_t width) { return (int)((width + 15) / 16 * 16); }
 

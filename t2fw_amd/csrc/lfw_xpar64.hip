@@ -1,30 +1,36 @@
-// Launch 3 of the chunk-parallel exact recurrence (lfw_xpar.hip) for fp32 tensors with 64 x 64 states: the same steps in
-// the same arithmetic, laid out so that almost every VALU instruction is one of the recurrence's own.
+// Launch 3 of the chunk-parallel exact recurrence (lfw_xpar.hip) for fp32 tensors with 64 x 64 states.
 //
-// One workgroup of four waves per (row, chunk) [backward: and side].  A lane is a row of the state (value channels;
-// key channels on the backward's key side), a wave holds 16 of the other side's channels ("columns") in registers; lane
-// l also holds the inputs of column l % 16, which DPP broadcasts within each row of 16 lanes as an operand of the
-// multiplications: neither LDS nor scalar registers carry the inputs.  A contraction over columns, S_t q_t and the like,
-// is lane-local; the four waves' shares meet in LDS, eight steps at a time.  A state element costs 4 VALU instructions
-// per step forward and 12.75 / 13.75 backward (value / key side: 3.75 + 3 to rebuild the states, the rest for the adjoint
-// and the sums), the per-step kernels' arithmetic without their cross-lane sums.
+// Chunks whose gates allow it run as products on fp64 matrix instructions (lfw_xpar64_mm.hpp), one workgroup of four
+// waves per (row, chunk) [backward: and side].  Everything else runs in one more launch (4 and 6 us where it finds nothing
+// to do; one kernel for both took no less, and 8 % more than the steps alone where every chunk has a zero gate): chunks
+// with a gate below 2^-20 or a gate product below 2^-400 step by step, a state in a workgroup's registers, and rows that are
+// left to the recurrence over the whole sequence on the per-step bodies.
 //
-// Backward, per chunk: the states at steps 16, 32 and 48 (LDS) are rebuilt from the checkpoint, blocks of 16 steps are
-// visited last to first, and per half block the eight states are rebuilt into registers and the adjoint runs back over
-// them.
+// B = 96, T = 1024, measured: forward 56 us, backward 160 us, against 70 and 439 us for the same chunks step by step.
+// Relative error against float64 (2-norm) 3.6e-8 outputs, 3.9e-8 gate gradients, 2.5e-8 states; step by step 8.5e-8, 1.03e-7
+// and 5.1e-8.  What bounds the backward: 248 matrix instructions of 27 ns per wave, 12 waves per SIMD, are 82 us; with the
+// matrix instructions taken out it takes 104 us, with the loads taken out 159 (fp64 vector instructions, 1200 per wave, do
+// not run beside fp64 matrix instructions).  Forms that were slower: tiles of 16 steps with the state carried over them
+// (operands in fp32: 199 us, twice the vector instructions); consecutive workgroups on chunks of one row in the place of
+// one chunk of all rows (181 us).
 //
-// A row that is left to the recurrence over the whole sequence (lfw_xpar.hip) runs on the per-step bodies, a tile of 16
-// channels per workgroup: 226 and 780 us where all of 96 rows x 1024 steps are (per-step kernels 228 and 822; one
-// workgroup walking such a row in this file's layout: 335 and 1174).
+// The steps: a lane is a row of the state (value channels; key channels on the backward's key side), a wave holds 16 of the
+// other side's channels ("columns") in registers; lane l also holds the inputs of column l % 16, which DPP broadcasts within
+// each row of 16 lanes as an operand of the multiplications: neither LDS nor scalar registers carry the inputs.  A
+// contraction over columns, S_t q_t and the like, is lane-local; the four waves' shares meet in LDS, eight steps at a time.
+// A state element costs 4 VALU instructions per step forward and 12.75 / 13.75 backward (value / key side: 3.75 + 3 to
+// rebuild the states, the rest for the adjoint and the sums), the per-step kernels' arithmetic without their cross-lane
+// sums.  Backward, per chunk: the states at steps 16, 32 and 48 (LDS) are rebuilt from the checkpoint, blocks of 16 steps
+// are visited last to first, and per half block the eight states are rebuilt into registers and the adjoint runs back over
+// them.  Tried and slower: rank-one terms on v_mfma_f32_4x4x1 (forward 115 us, backward 603), column vectors in scalar
+// registers (105 and 1145: every wave misses the scalar cache once per step and array).
 //
-// B = 96, T = 1024: forward 70 us (51 us of VALU issue), backward 440 us (about 290 us of issue at two waves per SIMD;
-// 557 us before the inputs of a job were requested while the job before it ran).  The per-step kernels over whole rows
-// take 220 and 813 us, their bodies on chunks 154 and 600 us.
-// Tried and slower: rank-one terms on v_mfma_f32_4x4x1 (forward 115 us, backward 603), column vectors in scalar registers
-// (105 and 1145: every wave misses the scalar cache once per step and array).
+// A row that is left runs a tile of 16 channels per workgroup: 226 and 780 us where all of 96 rows x 1024 steps are
+// (per-step kernels 228 and 822; one workgroup walking such a row in the layout of the steps: 335 and 1174).
 #include "lfw_chunk.hpp"
 #include "lfw_scan_body.hpp"
 #include "lfw_xpar.hpp"
+#include "lfw_xpar64_mm.hpp"
 
 namespace t2fw {
 namespace {
@@ -201,15 +207,8 @@ template <int SIDE> __device__ __forceinline__ void left_row_backward(const Xpar
 struct FwdSmem {
     float part[2][XW_SEG][4][XP_N];
 };
-__global__ __launch_bounds__(XW_THREADS, 4) void lfw_xpar64_fwd_kernel(XparFwdArgs p) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    auto &part = reinterpret_cast<FwdSmem *>(smem_raw)->part;
-    const int64_t b = blockIdx.x % p.B;
-    const int chunk = (int)(blockIdx.x / p.B);
-    if (row_left(p.ws, b)) {
-        left_row_forward(p, b, chunk);
-        return;
-    }
+__device__ __forceinline__ void forward_steps(const XparFwdArgs &p, FwdSmem &sm, int64_t b, int chunk) {
+    auto &part = sm.part;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col0 = XW_COLS * w;
     const int T = (int)p.T;
     int t_end = min(T, (chunk + 1) * XP_CHUNK);
@@ -264,6 +263,35 @@ __global__ __launch_bounds__(XW_THREADS, 4) void lfw_xpar64_fwd_kernel(XparFwdAr
         }
     }
     if (t_end == T) store_state((float *)p.next_state + b * (XP_N * XP_N), S, lane, col0);
+}
+
+// Both kernels of a direction number their workgroups chunk by chunk.  The first does the chunks that the matrix
+// instructions take and says which those were; the second does the others and the rows that are left.
+//
+// What the first says of a (row, chunk, side), in the place of the chunk's gate products, which launch 2 was the last to read.
+__device__ __forceinline__ int32_t *not_done(const XparScratch &ws, int64_t item, int side) {
+    return reinterpret_cast<int32_t *>(ws.tots + item * (2 * XP_N)) + side;
+}
+__global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_fwd_mm_kernel(XparFwdArgs p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int64_t b = blockIdx.x % p.B;
+    const int chunk = (int)(blockIdx.x / p.B);
+    const int64_t item = b * p.NC + chunk;
+    if (row_left(p.ws, b) || p.ws.chunk_flags[item] != 0) return;
+    mm::Smem &sm = *reinterpret_cast<mm::Smem *>(smem);
+    const bool done = (chunk + 1) * XP_CHUNK <= (int)p.T ? mm::forward_chunk<true>(p, sm, b, chunk) : mm::forward_chunk<false>(p, sm, b, chunk);
+    if (threadIdx.x == 0) *not_done(p.ws, item, 0) = done ? 0 : 1;
+}
+__global__ __launch_bounds__(XW_THREADS, 4) void lfw_xpar64_fwd_steps_kernel(XparFwdArgs p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int64_t b = blockIdx.x % p.B;
+    const int chunk = (int)(blockIdx.x / p.B);
+    const int64_t item = b * p.NC + chunk;
+    const int out_of_range = p.ws.chunk_flags[item], rejected = *not_done(p.ws, item, 0);      // requested together
+    if (row_left(p.ws, b))
+        left_row_forward(p, b, chunk);
+    else if ((out_of_range | rejected) != 0)
+        forward_steps(p, *reinterpret_cast<FwdSmem *>(smem), b, chunk);
 }
 
 // ---- backward -------------------------------------------------------------------------------------
@@ -417,12 +445,31 @@ template <int SIDE> __device__ __forceinline__ void backward_side(const XparBwdA
     if (SIDE == 0 && chunk == 0) store_state((float *)p.d_s0 + b * (XP_N * XP_N), G, lane, col0);
 }
 
-__global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_kernel(XparBwdArgs p) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    BwdSmem &sm = *reinterpret_cast<BwdSmem *>(smem_raw);
+__global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_mm_kernel(XparBwdArgs p) {
+    extern __shared__ __align__(16) unsigned char smem[];
     const int64_t pair = blockIdx.x >> 1, b = pair % p.B;
     const int chunk = (int)(pair / p.B);
-    if (row_left(p.ws, b)) {
+    const int64_t item = b * p.NC + chunk;
+    if (row_left(p.ws, b) || p.ws.chunk_flags[item] != 0) return;
+    mm::Smem &sm = *reinterpret_cast<mm::Smem *>(smem);
+    const bool full = (chunk + 1) * XP_CHUNK <= (int)p.T;
+    bool done;
+    if ((blockIdx.x & 1) == 0)
+        done = full ? mm::backward_chunk<0, true>(p, sm, b, chunk) : mm::backward_chunk<0, false>(p, sm, b, chunk);
+    else
+        done = full ? mm::backward_chunk<1, true>(p, sm, b, chunk) : mm::backward_chunk<1, false>(p, sm, b, chunk);
+    if (threadIdx.x == 0) *not_done(p.ws, item, blockIdx.x & 1) = done ? 0 : 1;
+}
+__global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_steps_kernel(XparBwdArgs p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int64_t pair = blockIdx.x >> 1, b = pair % p.B;
+    const int chunk = (int)(pair / p.B);
+    const int64_t item = b * p.NC + chunk;
+    const int out_of_range = p.ws.chunk_flags[item], rejected = *not_done(p.ws, item, blockIdx.x & 1);      // requested together
+    const bool left = row_left(p.ws, b);
+    if (!left && (out_of_range | rejected) == 0) return;
+    BwdSmem &sm = *reinterpret_cast<BwdSmem *>(smem);
+    if (left) {
         if ((blockIdx.x & 1) == 0)
             left_row_backward<0>(p, b, chunk);
         else
@@ -437,18 +484,25 @@ __global__ __launch_bounds__(XW_THREADS, 2) void lfw_xpar64_bwd_kernel(XparBwdAr
 }  // namespace
 
 int xpar64_forward(const XparFwdArgs &a, hipStream_t stream) {
+    const int rc = enable_lds(reinterpret_cast<const void *>(lfw_xpar64_fwd_mm_kernel), (int)sizeof(mm::Smem), "hipFuncSetAttribute(lfw_xpar64_fwd_mm_kernel)");
+    if (rc) return rc;
+    const dim3 grid((unsigned)(a.B * a.NC));
+    hipLaunchKernelGGL(lfw_xpar64_fwd_mm_kernel, grid, dim3(XW_THREADS), sizeof(mm::Smem), stream, a);
     const size_t left = scan_fwd_lds_bytes(XW_LEFT_TB, 16, 4, 16), smem = left > sizeof(FwdSmem) ? left : sizeof(FwdSmem);
-    hipLaunchKernelGGL(lfw_xpar64_fwd_kernel, dim3((unsigned)(a.B * a.NC)), dim3(XW_THREADS), smem, stream, a);
-    return check_hip(hipGetLastError(), "lfw_xpar64_fwd_kernel launch");
+    hipLaunchKernelGGL(lfw_xpar64_fwd_steps_kernel, grid, dim3(XW_THREADS), smem, stream, a);
+    return check_hip(hipGetLastError(), "lfw_xpar64 forward launches");
 }
 
 int xpar64_backward(const XparBwdArgs &a, hipStream_t stream) {
     const size_t left = scan_bwd_lds_bytes(scan::SegLen<4>::value, 16, 4, 16, XP_CHUNK, true);
     const size_t smem = left > sizeof(BwdSmem) ? left : sizeof(BwdSmem);
-    const int rc = enable_lds(reinterpret_cast<const void *>(lfw_xpar64_bwd_kernel), (int)smem, "hipFuncSetAttribute(lfw_xpar64_bwd_kernel)");
+    int rc = enable_lds(reinterpret_cast<const void *>(lfw_xpar64_bwd_mm_kernel), (int)sizeof(mm::Smem), "hipFuncSetAttribute(lfw_xpar64_bwd_mm_kernel)");
+    if (!rc) rc = enable_lds(reinterpret_cast<const void *>(lfw_xpar64_bwd_steps_kernel), (int)smem, "hipFuncSetAttribute(lfw_xpar64_bwd_steps_kernel)");
     if (rc) return rc;
-    hipLaunchKernelGGL(lfw_xpar64_bwd_kernel, dim3((unsigned)(2 * a.B * a.NC)), dim3(XW_THREADS), smem, stream, a);
-    return check_hip(hipGetLastError(), "lfw_xpar64_bwd_kernel launch");
+    const dim3 grid((unsigned)(2 * a.B * a.NC));
+    hipLaunchKernelGGL(lfw_xpar64_bwd_mm_kernel, grid, dim3(XW_THREADS), sizeof(mm::Smem), stream, a);
+    hipLaunchKernelGGL(lfw_xpar64_bwd_steps_kernel, grid, dim3(XW_THREADS), smem, stream, a);
+    return check_hip(hipGetLastError(), "lfw_xpar64 backward launches");
 }
 
 }  // namespace t2fw

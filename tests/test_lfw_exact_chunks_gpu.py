@@ -69,6 +69,47 @@ def test_rows_left_next_to_others(T, D, K):
     check_all((x, f, q, k, fk, s), go, gs, F32)
 
 
+@pytest.mark.parametrize("what,value", [("one gate", 2.0 ** -20), ("one gate", 2.0 ** -21), ("whole chunk", 2.0 ** -6.2),
+                                        ("whole chunk", 2.0 ** -6.3), ("every second gate", 2.0 ** -16), ("tiny gradients", 1e-30),
+                                        ("large value", 2.0 ** 57), ("large value", 2.0 ** 59), ("large state", 2.0 ** 121)])
+def test_limits_of_the_matrix_form(what, value):
+    """64 x 64 float32: on both sides of each limit of the products (a chunk beyond one runs step by step), with a chunk in
+    range and a ragged one next to it.  T = 150: chunks of 64, 64 and 22 steps."""
+    x, f, q, k, fk, s, go, gs = make_config_inputs(2, 150, 64, 64, F32, seed=11, in_scale=0.5, state_std=0.5)
+    if what == "one gate":
+        f[0, 70, 3] = fk[0, 140, 5] = fk[1, 0, 0] = value
+    elif what == "whole chunk":
+        f[0, 64:128, 7] = value
+        fk[1, 0:64, 9] = value
+    elif what == "every second gate":
+        f[0, ::2, 11] = fk[0, 1::2, 13] = value
+    elif what == "tiny gradients":
+        go[0], gs[0] = go[0] * value, gs[0] * value
+    elif what == "large value":
+        x[0, 80, 3] = value
+        q[1, 80, 3] = value
+    else:
+        s[0, 5, 6] = value
+        f[0, :, 5] = 0.5
+    check_all((x, f, q, k, fk, s), go, gs, F32)
+
+
+def test_error_of_the_matrix_form():
+    """Relative error (2-norm) against the float64 kernels: operands and sums are fp64, the products P are rounded to fp32
+    once and the result once (2.4e-8 each); checkpoints and the adjoint between chunks are fp32 sums of launch 1 (5e-8 of
+    what is left of them).  Step by step the gate gradients are at 1.0e-7."""
+    from t2fw_amd import LFWFunction
+    x, f, q, k, fk, s, go, gs = make_config_inputs(8, 300, 64, 64, F32, seed=12)
+
+    def run(dtype):
+        ins = [t.cuda().to(dtype).requires_grad_() for t in (x, f, q, k, fk, s)]
+        res = LFWFunction.apply(*ins)
+        return list(res) + list(torch.autograd.grad(res, ins, [go.cuda().to(dtype), gs.cuda().to(dtype)]))
+
+    for n, got, want in zip(("outputs", "next_state") + NAMES, run(F32), run(torch.float64)):
+        assert ((got.double() - want).norm() / want.norm()).item() < 6e-8, n
+
+
 def test_rows_left_take_no_longer_than_the_per_step_kernels(monkeypatch):
     """Every row of 96 x 1024 steps has a gate above one.  Measured 1.03 times the per-step kernels' time; 7.4 times when
     the workgroups that do such rows shared one die."""
