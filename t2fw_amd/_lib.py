@@ -5,12 +5,15 @@ loaded; stream handles from torch are then valid in the library.  There is no CP
 fallback: a missing library is an ImportError-like RuntimeError at first use.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch  # noqa: F401  (must be loaded before the HIP library)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libt2fw_hip.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_t2fw_host.so")
 
 ABI_VERSION = 3
 
@@ -81,6 +84,28 @@ def load():
     return lib
 
 
+_host = None
+
+
+def loaded():
+    """Whether the library is there already: a call that is an error is told so whether or not it can be loaded"""
+    return _lib is not None
+
+
+def host():
+    """The extension module that takes a call from tensors to the library in one step (csrc/host.cpp; once)"""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("t2fw: %s is missing -- build it with `python -m t2fw_amd.build`" % HOST_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_t2fw_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_t2fw_host", loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def check(rc):
     """Turn a nonzero return code into RuntimeError carrying the library's message."""
     if rc != 0:
@@ -90,6 +115,11 @@ def check(rc):
 
 def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+
+
+def current_stream(device):
+    """torch's current stream on ``device`` as an address"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def current_stream_handle(device):
@@ -112,16 +142,13 @@ def block_plan(*arrays):
 def block_copy(plan, srcs, dsts):
     """One launch of t2fw_block_copy on the current stream: dsts[i] from srcs[i] as ``plan`` (block_plan) says.
     Tensors in host memory (no kernel of this library takes them) are copied by torch."""
-    n = len(srcs)
-    descs = (BlockCopyDesc * n).from_buffer_copy(plan)
-    for d, s, t in zip(descs, srcs, dsts):
-        d.src, d.dst = s.data_ptr(), t.data_ptr()
     if not srcs[0].is_cuda:
+        descs = (BlockCopyDesc * len(srcs)).from_buffer_copy(plan)
         for d, s, t in zip(descs, srcs, dsts):
             view = s.as_strided((*d.size, d.terms, 64), (*d.stride, d.term_stride, 1))
             t.view(view.shape[:4] + (64,)).copy_(view.sum(dim=4))
         return
-    check(load().t2fw_block_copy(descs, n, DTYPE_CODE[srcs[0].dtype], current_stream_handle(srcs[0].device)))
+    host().block_copy(plan, srcs, dsts, DTYPE_CODE[srcs[0].dtype], current_stream(srcs[0].device))
 
 
 def cast_tensors(srcs, dsts, stream):

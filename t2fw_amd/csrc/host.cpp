@@ -1,0 +1,274 @@
+// The host side of a call, from torch tensors to the C ABI (include/t2fw_hip.h): checks, allocations and the launch in one
+// step.  The same through ctypes costs a Python operation per shape, type, pointer and output.  What the calls mean,
+// which kernels they ask for and what is an error stays in functional_lfw.py and functional_dfw.py.
+//
+// Host time of a call, 4 x 16 tokens of 64 x 64 fp16, ctypes / this: forward 29.5 / 19.1 us without gradients, a training step
+// 205 / 152 us (of which torch's own hand-over to a Python autograd function and back is 91), one generation step 14.6 / 8.0.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ATen.h>
+
+#include <vector>
+
+#include "../../include/t2fw_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+const Tensor &tensor(PyObject *o) {
+    TORCH_CHECK(THPVariable_Check(o), "t2fw: expected a tensor");
+    return THPVariable_Unpack(o);
+}
+int64_t integer(PyObject *o) {
+    const int64_t v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return v;
+}
+void *address(PyObject *o) {
+    void *v = PyLong_AsVoidPtr(o);
+    if (v == nullptr && PyErr_Occurred()) throw python_error();
+    return v;
+}
+void arguments(Py_ssize_t n, Py_ssize_t want) { TORCH_CHECK(n == want, "t2fw: ", n, " arguments, expected ", want); }
+void done(int rc) {
+    TORCH_CHECK_WITH(Error, rc == 0, "t2fw error ", rc, ": ", t2fw_last_error());
+}
+PyObject *wrapped(std::initializer_list<Tensor> ts) {
+    PyObject *t = PyTuple_New((Py_ssize_t)ts.size());
+    if (t == nullptr) throw python_error();
+    Py_ssize_t i = 0;
+    for (const Tensor &v : ts) {
+        PyObject *o = v.defined() ? THPVariable_Wrap(v) : Py_NewRef(Py_None);
+        if (o == nullptr) {
+            Py_DECREF(t);
+            throw python_error();
+        }
+        PyTuple_SET_ITEM(t, i++, o);
+    }
+    return t;
+}
+// The launches run without the interpreter's lock: they wait where the device's queue is full.
+template <typename F> int unlocked(F &&launch) {
+    pybind11::gil_scoped_release release;
+    return launch();
+}
+Tensor bytes_like(const Tensor &t, int64_t n) { return at::empty({n}, t.options().dtype(at::kByte)); }
+
+// lfw_shape(x, f, q, k, f_key, state, heads) -> (B, T, H, D, K), or None where a call on these is an error
+PyObject *lfw_shape(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 7);
+    for (int i = 0; i < 6; ++i)
+        if (!THPVariable_Check(a[i])) Py_RETURN_NONE;
+    const Tensor &x = tensor(a[0]), &q = tensor(a[2]), &s = tensor(a[5]);
+    const int64_t lead = a[6] == Py_True ? 3 : 2;
+    for (int i = 0; i < 6; ++i) {
+        const Tensor &t = tensor(a[i]);
+        if (!t.is_cuda() || !t.is_contiguous() || t.dim() != lead + 1 || t.scalar_type() != x.scalar_type()) Py_RETURN_NONE;
+    }
+    if (tensor(a[1]).sizes() != x.sizes() || tensor(a[3]).sizes() != q.sizes() || tensor(a[4]).sizes() != q.sizes()) Py_RETURN_NONE;
+    const int64_t B = x.size(0), T = x.size(1), H = lead == 3 ? x.size(2) : 1, D = x.size(lead), K = q.size(lead);
+    if (q.size(0) != B || q.size(1) != T || (lead == 3 && q.size(2) != H)) Py_RETURN_NONE;
+    if (s.size(0) != B || (lead == 3 && s.size(1) != H) || s.size(lead - 1) != D || s.size(lead) != K) Py_RETURN_NONE;
+    return Py_BuildValue("(LLLLL)", (long long)B, (long long)T, (long long)H, (long long)D, (long long)K);
+    END_HANDLE_TH_ERRORS
+}
+
+// lfw_forward(x, f, q, k, f_key, state, heads, checkpoints per row or -1 for none, C, dtype, flags, workspace address or 0, its bytes,
+// stream) -> (outputs, next_state, checkpoints or None); address 0: the workspace is allocated for the call
+PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 14);
+    const Tensor &x = tensor(a[0]), &f = tensor(a[1]), &q = tensor(a[2]), &k = tensor(a[3]), &fk = tensor(a[4]), &s = tensor(a[5]);
+    const bool heads = a[6] == Py_True;
+    const int64_t nc = integer(a[7]), ws_bytes = integer(a[12]);
+    const int32_t C = (int32_t)integer(a[8]), dtype = (int32_t)integer(a[9]), flags = (int32_t)integer(a[10]);
+    void *ws = address(a[11]), *const stream = address(a[13]);
+    const int64_t B = x.size(0), T = x.size(1), H = heads ? x.size(2) : 1, D = x.size(-1), K = q.size(-1);
+    const Tensor out = at::empty_like(x), next = at::empty_like(s);
+    Tensor ckpt, scratch;
+    if (nc >= 0) ckpt = at::empty({B * H, nc, D, K}, x.options());
+    if (ws == nullptr && ws_bytes > 0) {
+        scratch = bytes_like(x, ws_bytes);
+        ws = scratch.data_ptr();
+    }
+    void *const ck = ckpt.defined() ? ckpt.data_ptr() : nullptr;
+    done(unlocked([&] {
+        return heads ? t2fw_lfw_forward_heads(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
+                                              out.data_ptr(), next.data_ptr(), ck, B, T, H, D, K, C, dtype, flags, ws, ws_bytes, stream)
+                     : t2fw_lfw_forward(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
+                                        out.data_ptr(), next.data_ptr(), ck, B, T, D, K, C, dtype, flags, ws, ws_bytes, stream);
+    }));
+    return wrapped({out, next, ckpt});
+    END_HANDLE_TH_ERRORS
+}
+
+// lfw_backward_arguments(g_out, g_state, x, f, q, k, f_key, state, checkpoints, heads, C, dtype, flags, workspace bytes, stream)
+// -> ((d_x, d_f, d_q, d_k, d_f_key, d_state), arguments of t2fw_lfw_backward or t2fw_lfw_backward_heads, workspace or None).
+// The call itself is Python's: which kernels it asks for can be seen there.
+PyObject *lfw_backward_arguments(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 15);
+    const bool heads = a[9] == Py_True;
+    const Tensor &x = tensor(a[2]), &q = tensor(a[4]);
+    const int64_t ws_bytes = integer(a[13]);
+    Tensor grads[6], scratch;
+    for (int i = 0; i < 6; ++i) grads[i] = at::empty_like(tensor(a[2 + i]));
+    if (ws_bytes > 0) scratch = bytes_like(x, ws_bytes);
+    std::vector<long long> v;                      // addresses, sizes and options in the order of the C declaration
+    v.reserve(25);
+    for (int i = 0; i < 9; ++i) v.push_back((long long)(uintptr_t)tensor(a[i]).data_ptr());
+    for (const Tensor &g : grads) v.push_back((long long)(uintptr_t)g.data_ptr());
+    v.push_back(x.size(0));
+    v.push_back(x.size(1));
+    if (heads) v.push_back(x.size(2));
+    v.push_back(x.size(-1));
+    v.push_back(q.size(-1));
+    for (int i = 10; i < 13; ++i) v.push_back(integer(a[i]));
+    v.push_back(scratch.defined() ? (long long)(uintptr_t)scratch.data_ptr() : 0);
+    v.push_back(ws_bytes);
+    v.push_back((long long)(uintptr_t)address(a[14]));
+    pybind11::tuple args(v.size());
+    for (size_t i = 0; i < v.size(); ++i) {
+        PyObject *o = PyLong_FromLongLong(v[i]);
+        if (o == nullptr) throw python_error();
+        PyTuple_SET_ITEM(args.ptr(), (Py_ssize_t)i, o);
+    }
+    pybind11::object g = pybind11::reinterpret_steal<pybind11::object>(wrapped({grads[0], grads[1], grads[2], grads[3], grads[4], grads[5]}));
+    pybind11::object w = pybind11::reinterpret_steal<pybind11::object>(scratch.defined() ? THPVariable_Wrap(scratch) : Py_NewRef(Py_None));
+    return PyTuple_Pack(3, g.ptr(), args.ptr(), w.ptr());
+    END_HANDLE_TH_ERRORS
+}
+
+// lfw_step(x, f, q, k, f_key, state, out or None, inplace, stream) -> (out, state), or None where it is an error
+PyObject *lfw_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 9);
+    for (int i = 0; i < 6; ++i)
+        if (!THPVariable_Check(a[i])) Py_RETURN_NONE;
+    const Tensor &x = tensor(a[0]), &f = tensor(a[1]), &q = tensor(a[2]), &k = tensor(a[3]), &fk = tensor(a[4]), &s = tensor(a[5]);
+    for (int i = 0; i < 6; ++i) {
+        const Tensor &t = tensor(a[i]);
+        if (!t.is_cuda() || !t.is_contiguous() || t.dim() != (i == 5 ? 3 : 2) || t.scalar_type() != x.scalar_type()) Py_RETURN_NONE;
+    }
+    const int64_t B = x.size(0), D = x.size(1), K = q.size(1);
+    if (f.sizes() != x.sizes() || k.sizes() != q.sizes() || fk.sizes() != q.sizes() || q.size(0) != B || s.size(0) != B ||
+        s.size(1) != D || s.size(2) != K)
+        Py_RETURN_NONE;
+    int32_t dtype;
+    switch (x.scalar_type()) {
+        case at::kFloat: dtype = T2FW_F32; break;
+        case at::kHalf: dtype = T2FW_F16; break;
+        case at::kBFloat16: dtype = T2FW_BF16; break;
+        case at::kDouble: dtype = T2FW_F64; break;
+        default: Py_RETURN_NONE;
+    }
+    void *const stream = address(a[8]);
+    const Tensor out = a[6] == Py_None ? at::empty_like(x) : tensor(a[6]), next = a[7] == Py_True ? s : at::empty_like(s);
+    done(unlocked([&] {
+        return t2fw_lfw_step(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(), out.data_ptr(),
+                             next.data_ptr(), B, D, K, dtype, stream);
+    }));
+    return wrapped({out, next});
+    END_HANDLE_TH_ERRORS
+}
+
+// dfw_forward(q, k, v, state, dtype, flags, stream) -> (outputs, final_state, delta)
+PyObject *dfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 7);
+    const Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &s = tensor(a[3]);
+    const int32_t dtype = (int32_t)integer(a[4]), flags = (int32_t)integer(a[5]);
+    void *const stream = address(a[6]);
+    const Tensor out = at::empty_like(v), fin = at::empty_like(s), delta = at::empty_like(v);
+    done(unlocked([&] {
+        return t2fw_dfw_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), out.data_ptr(), fin.data_ptr(), delta.data_ptr(),
+                                v.size(0), v.size(1), v.size(2), q.size(2), dtype, flags, stream);
+    }));
+    return wrapped({out, fin, delta});
+    END_HANDLE_TH_ERRORS
+}
+
+// dfw_backward(g_out, g_state, q, k, delta, final_state, dtype, flags, stream) -> (d_q, d_k, d_v, d_state)
+PyObject *dfw_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 9);
+    const Tensor &go = tensor(a[0]), &gs = tensor(a[1]), &q = tensor(a[2]), &k = tensor(a[3]), &delta = tensor(a[4]), &fin = tensor(a[5]);
+    const int32_t dtype = (int32_t)integer(a[6]), flags = (int32_t)integer(a[7]);
+    void *const stream = address(a[8]);
+    const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(delta), ds = at::empty_like(fin);
+    done(unlocked([&] {
+        return t2fw_dfw_backward(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(), dq.data_ptr(),
+                                 dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), delta.size(0), delta.size(1), delta.size(2), q.size(2),
+                                 dtype, flags, stream);
+    }));
+    return wrapped({dq, dk, dv, ds});
+    END_HANDLE_TH_ERRORS
+}
+
+// gate_forward(f_logit, fk_logit, f or None, f_key or None, dtype, stream) -> (f, f_key)
+PyObject *gate_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 6);
+    const Tensor &lf = tensor(a[0]), &lk = tensor(a[1]);
+    const Tensor f = a[2] == Py_None ? at::empty_like(lf) : tensor(a[2]), fk = a[3] == Py_None ? at::empty_like(lk) : tensor(a[3]);
+    const int32_t dtype = (int32_t)integer(a[4]);
+    void *const stream = address(a[5]);
+    done(unlocked([&] {
+        return t2fw_gate_forward(lf.data_ptr(), lk.data_ptr(), f.data_ptr(), fk.data_ptr(), lf.numel(), lk.numel(), dtype, stream);
+    }));
+    return wrapped({f, fk});
+    END_HANDLE_TH_ERRORS
+}
+
+// gate_backward(d_f, d_f_key, f, f_key, dtype, stream): in place on the first two
+PyObject *gate_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 6);
+    const Tensor &df = tensor(a[0]), &dfk = tensor(a[1]), &f = tensor(a[2]), &fk = tensor(a[3]);
+    const int32_t dtype = (int32_t)integer(a[4]);
+    void *const stream = address(a[5]);
+    done(unlocked([&] {
+        return t2fw_gate_backward(df.data_ptr(), dfk.data_ptr(), f.data_ptr(), fk.data_ptr(), df.data_ptr(), dfk.data_ptr(), df.numel(),
+                                  dfk.numel(), dtype, stream);
+    }));
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+// block_copy(plan, sources, destinations, dtype, stream): plan is the bytes of the descriptors without their addresses
+PyObject *block_copy(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 5);
+    char *plan = nullptr;
+    Py_ssize_t len = 0;
+    if (PyBytes_AsStringAndSize(a[0], &plan, &len) != 0) throw python_error();
+    const Py_ssize_t count = PySequence_Size(a[1]);
+    TORCH_CHECK(count > 0 && count <= T2FW_BLOCK_COPY_MAX && PySequence_Size(a[2]) == count &&
+                    len == count * (Py_ssize_t)sizeof(t2fw_block_copy_desc), "t2fw: a plan of ", len, " bytes for ", count, " arrays");
+    t2fw_block_copy_desc d[T2FW_BLOCK_COPY_MAX];
+    memcpy(d, plan, (size_t)len);
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        pybind11::object src = pybind11::reinterpret_steal<pybind11::object>(PySequence_GetItem(a[1], i));
+        pybind11::object dst = pybind11::reinterpret_steal<pybind11::object>(PySequence_GetItem(a[2], i));
+        if (!src || !dst) throw python_error();
+        d[i].src = tensor(src.ptr()).data_ptr();
+        d[i].dst = tensor(dst.ptr()).data_ptr();
+    }
+    const int32_t dtype = (int32_t)integer(a[3]);
+    void *const stream = address(a[4]);
+    done(unlocked([&] { return t2fw_block_copy(d, (int32_t)count, dtype, stream); }));
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(lfw_shape), METHOD(lfw_forward), METHOD(lfw_backward_arguments), METHOD(dfw_forward), METHOD(dfw_backward),
+                         METHOD(lfw_step),
+                         METHOD(gate_forward), METHOD(gate_backward), METHOD(block_copy), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_t2fw_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__t2fw_host() { return PyModule_Create(&module); }

@@ -25,35 +25,18 @@ def _dfw_flags(dtype):
 
 def _dfw_forward(query, key, value, state):
     """The forward kernels on [B,T,M], [B,T,M], [B,T,D], [B,D,M]: (outputs, final_state, delta)"""
-    B, T, D = value.shape
-    M = query.shape[2]
-    lib = _lib.load()
     dev = value.device
     with _on_device(dev):
-        outputs = torch.empty_like(value)
-        final_state = torch.empty_like(state)
-        delta = torch.empty_like(value)
-        _lib.check(lib.t2fw_dfw_forward(
-            _lib.ptr(query), _lib.ptr(key), _lib.ptr(value), _lib.ptr(state), _lib.ptr(outputs),
-            _lib.ptr(final_state), _lib.ptr(delta), B, T, D, M, _dtype_code(value.dtype), _dfw_flags(value.dtype),
-            _lib.current_stream_handle(dev)))
-    return outputs, final_state, delta
+        return _lib.host().dfw_forward(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
+                                       _lib.current_stream(dev))
 
 
 def _dfw_backward(grad_output, grad_state, query, key, delta, final_state):
     """The backward kernels: (d_q, d_k, d_v, d_s), the order of t2fw/csrc/dfw_kernel.cu:557"""
-    B, T, D = delta.shape
-    M = query.shape[2]
-    lib = _lib.load()
     dev = delta.device
     with _on_device(dev):
-        d_q, d_k = torch.empty_like(query), torch.empty_like(key)
-        d_v, d_s = torch.empty_like(delta), torch.empty_like(final_state)
-        _lib.check(lib.t2fw_dfw_backward(
-            _lib.ptr(grad_output), _lib.ptr(grad_state), _lib.ptr(query), _lib.ptr(key), _lib.ptr(delta),
-            _lib.ptr(final_state), _lib.ptr(d_q), _lib.ptr(d_k), _lib.ptr(d_v), _lib.ptr(d_s),
-            B, T, D, M, _dtype_code(delta.dtype), _dfw_flags(delta.dtype), _lib.current_stream_handle(dev)))
-    return d_q, d_k, d_v, d_s
+        return _lib.host().dfw_backward(grad_output, grad_state, query, key, delta, final_state, _dtype_code(delta.dtype),
+                                        _dfw_flags(delta.dtype), _lib.current_stream(dev))
 
 
 # ---- value widths that are multiples of 64 (key width 64) as independent blocks -----------------------------

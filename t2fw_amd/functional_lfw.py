@@ -240,12 +240,9 @@ def _lfw_backward_blocked(grad_output, grad_state, value, forget, query, key, f_
                                                            state.shape), (v, v, k, k, k, v)))
 
 
-def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False):
-    """Checks as in t2fw/functional_lfw.py:42-49 and t2fw/csrc/lfw.cpp:24-26,36-41, then the forward
-    kernels.  heads=False: x,f [B,T,D]; q,k,f_key [B,T,K]; state [B,D,K].  heads=True: x,f [B,T,H,D];
-    q,k,f_key [B,T,H,K]; state [B,H,D,K].  Returns (outputs, next_state, ckpt or None, checkpoint
-    interval, flags, hints): ``hints`` is None, or the forward's verdict on which backward path the
-    gates allow, readable from the host once the forward has run (path_hint.py)."""
+def _checked_shape(value, forget, query, key, f_key, state, heads):
+    """(B, T, H, D, K) of a call, or the error that it is: checks as in t2fw/functional_lfw.py:42-49 and
+    t2fw/csrc/lfw.cpp:24-26,36-41 (``lfw_shape`` of csrc/host.cpp only tells whether there is one)"""
     assert value.shape == forget.shape
     assert query.shape == key.shape
     assert query.shape == f_key.shape
@@ -268,36 +265,34 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
             tuple(state.shape) != ((B, H, D, K) if heads else (B, D, K)):
         raise RuntimeError("t2fw: inconsistent shapes x %s, query %s, state %s"
                            % (tuple(value.shape), tuple(query.shape), tuple(state.shape)))
+    return B, T, H, D, K
+
+
+def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False):
+    """The checks, then the forward kernels.  heads=False: x,f [B,T,D]; q,k,f_key [B,T,K]; state [B,D,K].
+    heads=True: x,f [B,T,H,D]; q,k,f_key [B,T,H,K]; state [B,H,D,K].  Returns (outputs, next_state, ckpt or
+    None, checkpoint interval, flags, hints): ``hints`` is None, or the forward's verdict on which backward
+    path the gates allow, readable from the host once the forward has run (path_hint.py)."""
+    dims = _lib.host().lfw_shape(value, forget, query, key, f_key, state, heads) if _lib.loaded() else None
+    B, T, H, D, K = dims if dims is not None else _checked_shape(value, forget, query, key, f_key, state, heads)
     code = _dtype_code(value.dtype)
     flags = _flags()
     blocks = _block_counts(value, query, flags)
     if blocks is not None:
         return _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
-    lib = _lib.load()
+    host = _lib.host()
     C = _ckpt_interval()
     dev = value.device
     flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags, need_grad)
     with _on_device(dev):
-        outputs = torch.empty_like(value)
-        next_state = torch.empty_like(state)
-        ckpt = None
-        if need_grad:
-            ckpt = torch.empty((B * H, nc, D, K), dtype=value.dtype, device=dev)
         hints = None
+        ws_address = 0                                     # the workspace is allocated for the call
         if need_grad and ws_bytes and regions[3] and regions[5] and _host_hints_enabled() and ForwardHints.usable(dev):
             # a backward on the matrix cores will follow: the workspace goes to pinned host memory
             hints = ForwardHints(dev, ws_bytes, regions[2], regions[3], B * H)
-            ws_ptr = hints.workspace()[0]
-        else:
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-            ws_ptr = _lib.ptr(ws)
-        ptrs = (_lib.ptr(value), _lib.ptr(forget), _lib.ptr(query), _lib.ptr(key), _lib.ptr(f_key),
-                _lib.ptr(state), _lib.ptr(outputs), _lib.ptr(next_state), _lib.ptr(ckpt))
-        tail = (D, K, C, code, flags, ws_ptr, ws_bytes, _lib.current_stream_handle(dev))
-        if heads:
-            _lib.check(lib.t2fw_lfw_forward_heads(*ptrs, B, T, H, *tail))
-        else:
-            _lib.check(lib.t2fw_lfw_forward(*ptrs, B, T, *tail))
+            ws_address = hints.workspace()[0].value
+        outputs, next_state, ckpt = host.lfw_forward(value, forget, query, key, f_key, state, heads, nc if need_grad else -1, C, code,
+                                                     flags, ws_address, ws_bytes, _lib.current_stream(dev))
         if hints is not None:
             hints.launched()
     return outputs, next_state, ckpt, C, flags, hints
@@ -320,28 +315,17 @@ def _lfw_backward(grad_output, grad_state, value, forget, query, key, f_key, sta
     H = value.shape[2] if heads else 1
     D, K = value.shape[-1], query.shape[-1]
     code = _dtype_code(value.dtype)
-    lib = _lib.load()
+    host = _lib.host()
     dev = value.device
     if hints is not None:
         flags = choose_backward_flags(flags, hints.hinted_rows(), B * H)
     ws_bytes = _sizes(B * H, T, D, K, C, code, flags)[2]
     with _on_device(dev):
-        d_x = torch.empty_like(value)
-        d_f = torch.empty_like(forget)
-        d_q = torch.empty_like(query)
-        d_k = torch.empty_like(key)
-        d_fk = torch.empty_like(f_key)
-        d_s = torch.empty_like(state)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        ptrs = (_lib.ptr(grad_output), _lib.ptr(grad_state), _lib.ptr(value), _lib.ptr(forget),
-                _lib.ptr(query), _lib.ptr(key), _lib.ptr(f_key), _lib.ptr(state), _lib.ptr(ckpt),
-                _lib.ptr(d_x), _lib.ptr(d_f), _lib.ptr(d_q), _lib.ptr(d_k), _lib.ptr(d_fk), _lib.ptr(d_s))
-        tail = (D, K, C, code, flags, _lib.ptr(ws), ws_bytes, _lib.current_stream_handle(dev))
-        if heads:
-            _lib.check(lib.t2fw_lfw_backward_heads(*ptrs, B, T, H, *tail))
-        else:
-            _lib.check(lib.t2fw_lfw_backward(*ptrs, B, T, *tail))
-    return d_x, d_f, d_q, d_k, d_fk, d_s
+        grads, args, ws = host.lfw_backward_arguments(grad_output, grad_state, value, forget, query, key, f_key, state, ckpt, heads,
+                                                      C, code, flags, ws_bytes, _lib.current_stream(dev))
+        lib = _lib.load()
+        _lib.check((lib.t2fw_lfw_backward_heads if heads else lib.t2fw_lfw_backward)(*args))
+    return grads
 
 
 class LFWFunction(torch.autograd.Function):
@@ -376,25 +360,16 @@ def sigmoid_gates(f_logit, fk_logit, out_f=None, out_fk=None):
     for t, n in ((f_logit, "f_logit"), (fk_logit, "fk_logit")):
         _check_input(t, n)
     assert f_logit.dtype == fk_logit.dtype
-    lib = _lib.load()
     dev = f_logit.device
     with _on_device(dev):
-        f = torch.empty_like(f_logit) if out_f is None else out_f
-        fk = torch.empty_like(fk_logit) if out_fk is None else out_fk
-        _lib.check(lib.t2fw_gate_forward(_lib.ptr(f_logit), _lib.ptr(fk_logit), _lib.ptr(f), _lib.ptr(fk),
-                                         f_logit.numel(), fk_logit.numel(), _dtype_code(f_logit.dtype),
-                                         _lib.current_stream_handle(dev)))
-    return f, fk
+        return _lib.host().gate_forward(f_logit, fk_logit, out_f, out_fk, _dtype_code(f_logit.dtype), _lib.current_stream(dev))
 
 
 def _gate_backward_inplace(d_f, d_fk, forget, f_key):
     """d_f, d_fk: gate gradients on entry, logit gradients d_gate * gate * (1 - gate) on return."""
-    lib = _lib.load()
     dev = d_f.device
     with _on_device(dev):
-        _lib.check(lib.t2fw_gate_backward(_lib.ptr(d_f), _lib.ptr(d_fk), _lib.ptr(forget), _lib.ptr(f_key),
-                                          _lib.ptr(d_f), _lib.ptr(d_fk), d_f.numel(), d_fk.numel(),
-                                          _dtype_code(d_f.dtype), _lib.current_stream_handle(dev)))
+        _lib.host().gate_backward(d_f, d_fk, forget, f_key, _dtype_code(d_f.dtype), _lib.current_stream(dev))
 
 
 class LFWGatedFunction(torch.autograd.Function):
@@ -557,6 +532,12 @@ def lfw_step(x, f, query, key, f_key, state, out=None, inplace=True):
     state [B,D,K] updated in place when ``inplace``.  Returns (out [B,D], state).
     The reference does this through the T=1 forward (tests/benchmark.py:104-105), which
     allocates a new state tensor per step."""
+    if _lib.loaded() and x.is_cuda:
+        with _on_device(x.device):
+            done = _lib.host().lfw_step(x, f, query, key, f_key, state, out, bool(inplace), _lib.current_stream(x.device))
+        if done is not None:
+            return done
+    # which error it is, or what the step above leaves to the caller
     for t, n in ((x, "x"), (f, "f"), (query, "query"), (key, "key"), (f_key, "f_key"), (state, "state")):
         _check_input(t, n)
         assert t.dtype == x.dtype

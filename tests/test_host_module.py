@@ -1,0 +1,59 @@
+"""csrc/host.cpp: what it leaves to the Python checks, and calls that it must not take."""
+import pytest
+import torch
+
+
+def _host():
+    from t2fw_amd import _lib
+    return _lib.host()
+
+
+def _ins(B=2, T=3, D=4, K=5, device="cpu", dtype=torch.float32):
+    t = lambda *s: torch.ones(s, device=device, dtype=dtype)
+    return [t(B, T, D), t(B, T, D), t(B, T, K), t(B, T, K), t(B, T, K), t(B, D, K)]
+
+
+def test_host_memory_and_other_objects_are_left_to_the_python_checks():
+    assert _host().lfw_shape(*_ins(), False) is None
+    assert _host().lfw_shape(*_ins()[:5], None, False) is None
+    assert _host().lfw_step(*(t[:, 0] for t in _ins()[:5]), _ins()[5], None, True, 0) is None
+
+
+def test_calls_with_other_arguments_raise():
+    with pytest.raises(RuntimeError):
+        _host().lfw_shape(*_ins())
+    with pytest.raises(RuntimeError):
+        _host().block_copy(b"", (), (), 0, 0)
+    with pytest.raises(RuntimeError):
+        _host().block_copy(bytes(7), (torch.ones(64),), (torch.ones(64),), 0, 0)
+    with pytest.raises(RuntimeError):
+        _host().gate_forward(None, None, None, None, 0, 0)
+    with pytest.raises(TypeError):
+        _host().gate_forward(torch.ones(1), torch.ones(1), None, None, "0", 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [False, True])
+def test_shapes_that_fit_and_those_that_do_not(heads):
+    ins = _ins(device="cuda")
+    if heads:
+        ins = [t.unsqueeze(2) for t in ins[:5]] + [ins[5].unsqueeze(1)]
+    shape = lambda *a: _host().lfw_shape(*a, heads)
+    assert shape(*ins) == (2, 3, 1, 4, 5)
+    for i in range(6):
+        for other in (ins[i].half(), ins[i].cpu(), ins[i][:1], ins[i].unsqueeze(0), ins[i].transpose(0, 1), torch.cat([ins[i]] * 2, -1)[..., ::2]):
+            assert shape(*ins[:i], other, *ins[i + 1:]) is None, i
+
+
+@pytest.mark.gpu
+def test_step_returns_the_callers_tensors():
+    from t2fw_amd.functional_lfw import lfw_step
+    x, f, q, k, fk, s = [t[:, 0].contiguous() if t.dim() == 3 and i < 5 else t for i, t in enumerate(_ins(device="cuda"))]
+    out = torch.empty_like(x)
+    got, state = lfw_step(x, f, q, k, fk, s, out=out)
+    assert got is out and state is s
+    got, state = lfw_step(x, f, q, k, fk, s, inplace=False)
+    assert state is not s and torch.equal(s, torch.full_like(s, 2.0)) and torch.equal(state, torch.full_like(s, 3.0))
+    for bad in (dict(x=x[:1]), dict(f=f.half()), dict(state=s[:, :3])):
+        with pytest.raises((AssertionError, RuntimeError)):
+            lfw_step(**{**dict(x=x, f=f, query=q, key=k, f_key=fk, state=s), **bad})
