@@ -252,6 +252,24 @@ int t2fw_dfw_backward(const void *g_out, const void *g_state,
                       int32_t dtype, int32_t flags, void *stream);
 
 /*
+ * The same with M = 64 and D = 64 n (fp32, fp16, bf16; n >= 1) as n blocks of 64 value channels on the matrix cores: the rows
+ * of the state do not interact.  Arrays as above, 16-byte aligned, but d_q and d_k: [B, n, T, 64], each block's share
+ * of them (the gradients are the sums over n).  T2FW_ERR_UNSUPPORTED for other shapes, T * D >= 2^31 - 1 and
+ * T2FW_FLAG_FORCE_SCAN.
+ */
+int t2fw_dfw_forward_blocks(const void *q, const void *k, const void *v, const void *s0,
+                            void *out, void *final_state, void *delta,
+                            int64_t B, int64_t T, int64_t D, int64_t M,
+                            int32_t dtype, int32_t flags, void *stream);
+
+int t2fw_dfw_backward_blocks(const void *g_out, const void *g_state,
+                             const void *q, const void *k, const void *delta,
+                             const void *final_state,
+                             void *d_q, void *d_k, void *d_v, void *d_s0,
+                             int64_t B, int64_t T, int64_t D, int64_t M,
+                             int32_t dtype, int32_t flags, void *stream);
+
+/*
  * Conversion of `count` (<= 8) arrays of n[i] elements each between float32 and float16 / bfloat16 in one
  * launch (src_dtype -> dst_dtype, one of them T2FW_F32); arrays 16-byte aligned, `src`, `dst`, `n` host arrays.
  * No counterpart in the reference (one kernel serves every dtype there, lfw_kernel.cu:157-168): it is what a

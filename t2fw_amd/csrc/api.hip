@@ -590,7 +590,7 @@ int t2fw_dfw_forward(const void *q, const void *k, const void *v, const void *s0
     if ((rc = check_ptrs(ptrs, 5, es))) return rc;
     DfwFwdArgs a{};
     a.q = q; a.k = k; a.v = v; a.s0 = s0; a.out = out; a.final_state = final_state; a.delta = delta;
-    a.B = B; a.T = T; a.D = D; a.M = M;
+    a.B = B; a.T = T; a.D = D; a.M = M; a.blocks = 1;
     if (dfw_chunk_ok(D, M, dtype, flags) && T * CH_N < 0x7fffffffLL && aligned16({q, k, v, s0, out, final_state, delta}))
         return dfw_chunk_forward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, st);
     return dfw_forward(a, dtype, st);
@@ -621,11 +621,57 @@ int t2fw_dfw_backward(const void *g_out, const void *g_state, const void *q, con
     DfwBwdArgs a{};
     a.g_out = g_out; a.g_state = g_state; a.q = q; a.k = k; a.delta = delta; a.final_state = final_state;
     a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
-    a.B = B; a.T = T; a.D = D; a.M = M;
+    a.B = B; a.T = T; a.D = D; a.M = M; a.blocks = 1;
     if (dfw_chunk_ok(D, M, dtype, flags) && T * CH_N < 0x7fffffffLL &&
         aligned16({g_out, g_state, q, k, delta, final_state, d_q, d_k, d_v, d_s0}))
         return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, st);
     return dfw_backward(a, dtype, st);
+}
+
+// The value blocks of a call: 0 where it is an error (the message is set).
+static int dfw_blocks_of(int64_t B, int64_t T, int64_t D, int64_t M, int32_t dtype, int32_t flags) {
+    if (check_dims(B, T, D, M)) return 0;
+    if (M == 64 && D >= 64 && D % 64 == 0 && dfw_chunk_ok(64, M, dtype, flags) && T > 0 && T * D < 0x7fffffffLL &&
+        B * (D / 64) <= 0x1fffffffLL)
+        return (int)(D / 64);
+    fail(T2FW_ERR_UNSUPPORTED, "value blocks: T=%lld D=%lld M=%lld dtype %d flags %d", (long long)T, (long long)D, (long long)M, dtype, flags);
+    return 0;
+}
+
+int t2fw_dfw_forward_blocks(const void *q, const void *k, const void *v, const void *s0, void *out, void *final_state,
+                            void *delta, int64_t B, int64_t T, int64_t D, int64_t M, int32_t dtype, int32_t flags,
+                            void *stream) {
+    const size_t es = elem_size(dtype);
+    if (es == 0) return fail(T2FW_ERR_BAD_DTYPE, "unknown dtype code %d", dtype);
+    const int blocks = dfw_blocks_of(B, T, D, M, dtype, flags);
+    if (blocks == 0) return T2FW_ERR_UNSUPPORTED;
+    if (B == 0) return T2FW_OK;
+    const NamedPtr ptrs[] = {{"q", q}, {"k", k}, {"v", v}, {"s0", s0}, {"out", out}, {"final_state", final_state}, {"delta", delta}};
+    const int rc = check_ptrs(ptrs, 7, 16);
+    if (rc) return rc;
+    DfwFwdArgs a{};
+    a.q = q; a.k = k; a.v = v; a.s0 = s0; a.out = out; a.final_state = final_state; a.delta = delta;
+    a.B = B * blocks; a.T = T; a.D = D; a.M = M; a.blocks = blocks;
+    return dfw_chunk_forward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
+}
+
+int t2fw_dfw_backward_blocks(const void *g_out, const void *g_state, const void *q, const void *k, const void *delta,
+                             const void *final_state, void *d_q, void *d_k, void *d_v, void *d_s0, int64_t B, int64_t T,
+                             int64_t D, int64_t M, int32_t dtype, int32_t flags, void *stream) {
+    const size_t es = elem_size(dtype);
+    if (es == 0) return fail(T2FW_ERR_BAD_DTYPE, "unknown dtype code %d", dtype);
+    const int blocks = dfw_blocks_of(B, T, D, M, dtype, flags);
+    if (blocks == 0) return T2FW_ERR_UNSUPPORTED;
+    if (B == 0) return T2FW_OK;
+    const NamedPtr ptrs[] = {{"g_out", g_out}, {"g_state", g_state}, {"q", q}, {"k", k}, {"delta", delta},
+                             {"final_state", final_state}, {"d_q", d_q}, {"d_k", d_k}, {"d_v", d_v}, {"d_s0", d_s0}};
+    const int rc = check_ptrs(ptrs, 10, 16);
+    if (rc) return rc;
+    DfwBwdArgs a{};
+    a.g_out = g_out; a.g_state = g_state; a.q = q; a.k = k; a.delta = delta; a.final_state = final_state;
+    a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
+    a.B = B * blocks; a.T = T; a.D = D; a.M = M; a.blocks = blocks;
+    return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
 }
 
 int t2fw_cast(const void *const *src, void *const *dst, const int64_t *n, int32_t count, int32_t src_dtype,

@@ -245,13 +245,32 @@ template <bool SP> struct BlockInverse {
     __device__ __forceinline__ floatx4 acc_tm() const { return mma16(p2t, p1, floatx4{0.f, 0.f, 0.f, 0.f}); }
 };
 
+// ---- value blocks ----------------------------------------------------------------------------------------
+// The rows of the state do not interact: a state of 64 n value channels is n recurrences of 64 that share q and k.  Workgroup
+// row b is block b % n of batch row b / n; the value side's arrays are [B, T, 64 n] and are read and written in place.
+template <bool BLOCKS> struct DfwRow {
+    int64_t key, value;                            // elements before the row in q and k; before the row's block in v and its like
+    u32 vs;                                        // elements from a token to the next in those
+    __device__ __forceinline__ DfwRow(int64_t b, int64_t T, int blocks) {
+        if (BLOCKS) {
+            const int64_t row = b / blocks;
+            key = row * T * CH_N;
+            vs = (u32)(CH_N * blocks);
+            value = key * blocks + (b - row * blocks) * CH_N;
+        } else {
+            key = value = b * T * CH_N;
+            vs = CH_N;
+        }
+    }
+};
+
 // ---- staging of a [T, 64] array into tiles (one wave per array) ---------------------------------------
 // sixteen elements of one lane: token lane >> 2, channels 16 (lane & 3) .. + 15.  Rows at or past T read as zero.
 // Loads are issued unconditionally (rows at or past T are read from row T - 1 and zeroed when the tile is
 // built): a load inside a branch would make every later wait for a load a wait for all of them.
-template <typename E> __device__ __forceinline__ typename E::Raw16 load_tm(const typename E::elem *row0, int tok0, int T, int lane) {
+template <typename E> __device__ __forceinline__ typename E::Raw16 load_tm(const typename E::elem *row0, u32 ts, int tok0, int T, int lane) {
     const int t = min(tok0 + (lane >> 2), T - 1);
-    return E::load16(row0 + (size_t)t * CH_N + 16 * (lane & 3));
+    return E::load16(row0 + (size_t)t * ts + 16 * (lane & 3));
 }
 template <bool SP, typename E> __device__ __forceinline__ void store_tm(unsigned char *tile, int lane, const typename E::Raw16 &r, int tok0, int T, float sign = 1.f) {
     u16 *hi = reinterpret_cast<u16 *>(tile), *lo = reinterpret_cast<u16 *>(tile + TM_TILE);
@@ -291,6 +310,7 @@ template <int RAW_BLOCK, int ST_BLOCK, int NBLK> struct Ring {
 // for a load).  tok0_of(stage, bb): first token of a block (at or past T: a block of zeros).
 template <typename E> struct PrepJob {
     const typename E::elem *src;       // token 0 of the batch row
+    u32 ts;                 // elements from a token to the next
     int tm_off;             // byte offset of the token-major tile inside a block's raw tiles; < 0: the wave's scratch tile
     int cm_off;             // byte offset of the channel-major tile; < 0: none
     float sign;             // the token-major tile holds sign * src
@@ -307,7 +327,7 @@ __device__ __forceinline__ void prep_wave_jobs(unsigned char *smem, const PrepJo
 #pragma unroll
         for (int a = 0; a < NJOBS; ++a)
 #pragma unroll
-            for (int bb = 0; bb < NBLK; ++bb) regs[a][bb] = load_tm<E>(jobs[a].src, tok0_of(stage, bb), T, lane);
+            for (int bb = 0; bb < NBLK; ++bb) regs[a][bb] = load_tm<E>(jobs[a].src, jobs[a].ts, tok0_of(stage, bb), T, lane);
     };
     // stage `stage` out of `cur`; the loads of stage + SETS - 1 into `far` (the set that stage - 1 has left)
     auto stage_body = [&](int stage, auto &cur, auto &far) {

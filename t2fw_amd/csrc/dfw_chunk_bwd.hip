@@ -11,7 +11,8 @@
 //               and d_state.  Its chain per block is  G_end -> dU = Tm^T Bq^T g + (Tm^T K) G_end^T -> G_start,
 //               with Tm, Bq and K'' = Tm^T K prepared ahead by the matrix waves.
 //   key side    one workgroup per (row, half of the key channels): columns of S and of G in fp32 accumulators,
-//               both plain running sums (it reads d_value from the first launch); writes d_query and d_key.
+//               both plain running sums (it reads d_value from the first launch); writes d_query and d_key (with several
+//               value blocks the block's share of them).
 #include <type_traits>
 #include "common.hpp"
 #include "dfw_chunk.hpp"
@@ -67,13 +68,15 @@ template <bool SP> __device__ __forceinline__ void vs_structure_wave(unsigned ch
     }
 }
 
-template <bool SP, typename E> __device__ __forceinline__ void vs_slab_wave(const DfwBwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
+template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_slab_wave(const DfwBwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
     typedef typename E::elem elem;
     const int r = lane & 15, g = lane >> 4, d = d0 + r, T = (int)p.T, nblocks = nstages * DNB;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-    const elem *const go = reinterpret_cast<const elem *>(p.g_out) + b * p.T * CH_N;
-    elem *const d_v = reinterpret_cast<elem *>(p.d_v) + b * p.T * CH_N;
-    const u32 lane_off = (u32)(4 * g * CH_N + d);
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const u32 vs = row.vs;
+    const elem *const go = reinterpret_cast<const elem *>(p.g_out) + row.value;
+    elem *const d_v = reinterpret_cast<elem *>(p.d_v) + row.value;
+    const u32 lane_off = (u32)(4 * g) * vs + (u32)d;
     // G[j][e] = G[d][16 j + 4 g + e]
     floatx4 G[4];
     {
@@ -90,7 +93,7 @@ template <bool SP, typename E> __device__ __forceinline__ void vs_slab_wave(cons
         for (int bb = 0; bb < DNB; ++bb)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                x.x[bb][e] = go[(size_t)min(reverse_tok0(nblocks, DNB, stage, bb) + 4 * g + e, T - 1) * CH_N + d];
+                x.x[bb][e] = go[(size_t)min(reverse_tok0(nblocks, DNB, stage, bb) + 4 * g + e, T - 1) * vs + d];
     };
     // One stage.  FULL: every token of the stage is below T and the body has no branch.  (The waits that the
     // compiler places count outstanding memory operations along every path: a path that skips stores, or loads
@@ -115,10 +118,10 @@ template <bool SP, typename E> __device__ __forceinline__ void vs_slab_wave(cons
             const Sp4<SP> gb0 = cat(split4<SP>(G[0]), split4<SP>(G[1])), gb1 = cat(split4<SP>(G[2]), split4<SP>(G[3]));
             const floatx4 kg = mma32(KPP.acc_order(r, g, 1), gb1, mma32(KPP.acc_order(r, g, 0), gb0, zero));
             const floatx4 du = tbg + kg;
-            elem *const vb = d_v + (size_t)tok0 * CH_N;        // wave-uniform
+            elem *const vb = d_v + (size_t)tok0 * vs;        // wave-uniform
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (FULL || tok0 + 4 * g + e < T) vb[lane_off + e * CH_N] = E::e(du[e]);
+                if (FULL || tok0 + 4 * g + e < T) vb[lane_off + e * vs] = E::e(du[e]);
             // G += g^T Q - dU^T K
             const Sp2<SP> ndu = split4<SP>(-du);
 #pragma unroll
@@ -149,7 +152,7 @@ template <bool SP, typename E> __device__ __forceinline__ void vs_slab_wave(cons
 
 // blockIdx = half * rows_padded + row (rows_padded a multiple of 8: both halves of a row on one XCD).  Waves 0, 1:
 // slab waves, alone on SIMDs 0 and 1; waves 2, 3: matrix waves; waves 6, 7: prep waves; waves 4, 5 leave at once.
-template <bool SP, typename E> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_value_kernel(DfwBwdArgs p, int rows_padded) {
+template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_value_kernel(DfwBwdArgs p, int rows_padded) {
     typedef typename E::elem elem;
     extern __shared__ __align__(16) unsigned char smem[];
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
@@ -157,19 +160,20 @@ template <bool SP, typename E> __global__ __launch_bounds__(BW_THREADS) void dfw
     if (b >= p.B) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int T = (int)p.T, nstages = (T + DL * DNB - 1) / (DL * DNB), nblocks = nstages * DNB;
-    const elem *const k = reinterpret_cast<const elem *>(p.k) + b * p.T * CH_N;
-    const elem *const q = reinterpret_cast<const elem *>(p.q) + b * p.T * CH_N;
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const elem *const k = reinterpret_cast<const elem *>(p.k) + row.key;
+    const elem *const q = reinterpret_cast<const elem *>(p.q) + row.key;
     auto tok0_of = [=](int stage, int bb) { return reverse_tok0(nblocks, DNB, stage, bb); };
     static_assert(DNB == 2, "one matrix wave per block of a stage");
     if (wave < 2) {
-        vs_slab_wave<SP, E>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
+        vs_slab_wave<SP, E, BLOCKS>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
     } else if (wave < 4) {
         vs_structure_wave<SP>(smem, nstages, wave - 2, lane);
     } else if (wave == 6) {
-        const PrepJob<E> jobs[1] = {{k, VS_KT, VS_KC, 1.f, false}};
+        const PrepJob<E> jobs[1] = {{k, CH_N, VS_KT, VS_KC, 1.f, false}};
         prep_wave_jobs<VsRing, DNB, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
     } else if (wave == 7) {
-        const PrepJob<E> jobs[1] = {{q, VS_QT, VS_QC, 1.f, false}};
+        const PrepJob<E> jobs[1] = {{q, CH_N, VS_QT, VS_QC, 1.f, false}};
         prep_wave_jobs<VsRing, DNB, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
     }
 }
@@ -327,7 +331,7 @@ template <bool SP, typename E> __device__ __forceinline__ void ks_slab_wave(cons
 
 // Waves 0, 1: state waves (16 key channels each) and waves 4, 5: the adjoint waves of the same channels, on SIMDs 0
 // and 1; wave 2: matrix wave; waves 3, 6, 7: prep waves.
-template <bool SP, typename E> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_key_kernel(DfwBwdArgs p, int rows_padded) {
+template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_key_kernel(DfwBwdArgs p, int rows_padded) {
     typedef typename E::elem elem;
     extern __shared__ __align__(16) unsigned char smem[];
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
@@ -335,12 +339,12 @@ template <bool SP, typename E> __global__ __launch_bounds__(BW_THREADS) void dfw
     if (b >= p.B) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int T = (int)p.T, nstages = (T + DL - 1) / DL;
-    const int64_t row = b * p.T * CH_N;
-    const elem *const k = reinterpret_cast<const elem *>(p.k) + row;
-    const elem *const q = reinterpret_cast<const elem *>(p.q) + row;
-    const elem *const dl = reinterpret_cast<const elem *>(p.delta) + row;
-    const elem *const go = reinterpret_cast<const elem *>(p.g_out) + row;
-    const elem *const dv = reinterpret_cast<const elem *>(p.d_v) + row;
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const elem *const k = reinterpret_cast<const elem *>(p.k) + row.key;
+    const elem *const q = reinterpret_cast<const elem *>(p.q) + row.key;
+    const elem *const dl = reinterpret_cast<const elem *>(p.delta) + row.value;
+    const elem *const go = reinterpret_cast<const elem *>(p.g_out) + row.value;
+    const elem *const dv = reinterpret_cast<const elem *>(p.d_v) + row.value;
     auto tok0_of = [=](int stage, int bb) { return reverse_tok0(nstages, 1, stage, bb); };
     if (wave < 2) {
         ks_slab_wave<SP, E>(p, smem, b, 32 * half + 16 * wave, wave, nstages, lane);
@@ -349,22 +353,22 @@ template <bool SP, typename E> __global__ __launch_bounds__(BW_THREADS) void dfw
     } else if (wave == 2) {
         ks_structure_wave<SP>(smem, nstages, lane);
     } else if (wave == 3) {
-        const PrepJob<E> jobs[1] = {{dl, KS_DT, KS_NDC, 1.f, true}};
+        const PrepJob<E> jobs[1] = {{dl, row.vs, KS_DT, KS_NDC, 1.f, true}};
         prep_wave_jobs<KsRing, 1, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
     } else if (wave == 6) {
-        const PrepJob<E> jobs[2] = {{go, KS_GT, -1, 1.f, false}, {k, -1, KS_KC, 1.f, false}};
+        const PrepJob<E> jobs[2] = {{go, row.vs, KS_GT, -1, 1.f, false}, {k, CH_N, -1, KS_KC, 1.f, false}};
         prep_wave_jobs<KsRing, 1, 2, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, smem + KS_SCRATCH);
     } else if (wave == 7) {
-        const PrepJob<E> jobs[2] = {{dv, KS_NUT, -1, -1.f, false}, {q, -1, KS_QC, 1.f, false}};
+        const PrepJob<E> jobs[2] = {{dv, row.vs, KS_NUT, -1, -1.f, false}, {q, CH_N, -1, KS_QC, 1.f, false}};
         prep_wave_jobs<KsRing, 1, 2, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, smem + KS_SCRATCH + 2 * TM_TILE);
     }
 }
 
 }  // namespace
 
-template <bool SP, typename E> static int launch_backward(const DfwBwdArgs &a, hipStream_t stream) {
-    auto value_side = dfw_chunk_bwd_value_kernel<SP, E>;
-    auto key_side = dfw_chunk_bwd_key_kernel<SP, E>;
+template <bool SP, typename E, bool BLOCKS> static int launch_backward(const DfwBwdArgs &a, hipStream_t stream) {
+    auto value_side = dfw_chunk_bwd_value_kernel<SP, E, BLOCKS>;
+    auto key_side = dfw_chunk_bwd_key_kernel<SP, E, BLOCKS>;
     int rc = enable_lds(reinterpret_cast<const void *>(value_side), VsRing::SMEM, "hipFuncSetAttribute(delta-rule backward kernel, value side)");
     if (rc) return rc;
     if ((rc = enable_lds(reinterpret_cast<const void *>(key_side), KS_SMEM, "hipFuncSetAttribute(delta-rule backward kernel, key side)"))) return rc;
@@ -376,12 +380,13 @@ template <bool SP, typename E> static int launch_backward(const DfwBwdArgs &a, h
 }
 
 template <typename E> static int backward_of(const DfwBwdArgs &a, bool split_operands, hipStream_t stream) {
-    return split_operands ? launch_backward<true, E>(a, stream) : launch_backward<false, E>(a, stream);
+    if (a.blocks > 1) return split_operands ? launch_backward<true, E, true>(a, stream) : launch_backward<false, E, true>(a, stream);
+    return split_operands ? launch_backward<true, E, false>(a, stream) : launch_backward<false, E, false>(a, stream);
 }
 
 int dfw_chunk_backward(const DfwBwdArgs &a, int dtype, bool split_operands, hipStream_t stream) {
-    if (a.D != CH_N || a.M != CH_N) return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take D = M = 64");
-    if (a.T * CH_N >= 0x7fffffffLL || a.B > 0x1fffffffLL)
+    if (a.blocks < 1 || a.D != (int64_t)CH_N * a.blocks || a.M != CH_N) return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take M = 64 and D = 64 per block");
+    if (a.T * a.D >= 0x7fffffffLL || a.B > 0x1fffffffLL)
         return fail(T2FW_ERR_UNSUPPORTED, "B=%lld T=%lld is too large for the block-wise delta-rule kernels", (long long)a.B, (long long)a.T);
     switch (dtype) {
     case T2FW_F32: return backward_of<ElF32>(a, split_operands, stream);

@@ -74,15 +74,17 @@ template <bool SP> __device__ __forceinline__ void structure_wave(unsigned char 
     }
 }
 
-template <bool SP, typename E> __device__ __forceinline__ void slab_wave(const DfwFwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
+template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void slab_wave(const DfwFwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
     typedef typename E::elem elem;
     const int r = lane & 15, g = lane >> 4, d = d0 + r, T = (int)p.T;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     // token addresses: a wave-uniform base per block plus the lane's fixed offset (first token 4 g, channel d)
-    const elem *const v = reinterpret_cast<const elem *>(p.v) + b * p.T * CH_N;
-    elem *const out = reinterpret_cast<elem *>(p.out) + b * p.T * CH_N;
-    elem *const delta = reinterpret_cast<elem *>(p.delta) + b * p.T * CH_N;
-    const u32 lane_off = (u32)(4 * g * CH_N + d);
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const u32 vs = row.vs;
+    const elem *const v = reinterpret_cast<const elem *>(p.v) + row.value;
+    elem *const out = reinterpret_cast<elem *>(p.out) + row.value;
+    elem *const delta = reinterpret_cast<elem *>(p.delta) + row.value;
+    const u32 lane_off = (u32)(4 * g) * vs + (u32)d;
     // S[j][e] = S[d][16 j + 4 g + e]
     floatx4 S[4];
     {
@@ -100,7 +102,7 @@ template <bool SP, typename E> __device__ __forceinline__ void slab_wave(const D
 #pragma unroll
         for (int bb = 0; bb < DNB; ++bb)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x.x[bb][e] = v[(size_t)min((stage * DNB + bb) * DL + 4 * g + e, T - 1) * CH_N + d];
+            for (int e = 0; e < 4; ++e) x.x[bb][e] = v[(size_t)min((stage * DNB + bb) * DL + 4 * g + e, T - 1) * vs + d];
     };
     // One stage.  FULL: every token of the stage is below T, and the body is free of branches: the waits that
     // the compiler places count outstanding memory operations along every path, so a path that skips stores
@@ -127,12 +129,12 @@ template <bool SP, typename E> __device__ __forceinline__ void slab_wave(const D
             // O = Q S0^T + Bq Delta
             const floatx4 qs = mma32(QT.acc_order(r, g, 1), sb1, mma32(QT.acc_order(r, g, 0), sb0, zero));
             const floatx4 o = qs + mma16(st_load<SP>(st + FW_BQT, lane), dls, zero);
-            elem *const ob = out + (size_t)tok0 * CH_N, *const db = delta + (size_t)tok0 * CH_N;      // wave-uniform
+            elem *const ob = out + (size_t)tok0 * vs, *const db = delta + (size_t)tok0 * vs;      // wave-uniform
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (FULL || tok0 + 4 * g + e < T) {
-                    ob[lane_off + e * CH_N] = E::e(o[e]);
-                    db[lane_off + e * CH_N] = E::e(dl[e]);
+                    ob[lane_off + e * vs] = E::e(o[e]);
+                    db[lane_off + e * vs] = E::e(dl[e]);
                 }
             // S += Delta^T K
 #pragma unroll
@@ -167,7 +169,7 @@ template <bool SP, typename E> __device__ __forceinline__ void slab_wave(const D
 
 // blockIdx = half * rows_padded + row with rows_padded a multiple of 8: the two halves of a row land on the
 // same XCD and share its L2 for K and Q, which both read
-template <bool SP, typename E> __global__ __launch_bounds__(FW_THREADS) void dfw_chunk_fwd_kernel(DfwFwdArgs p, int rows_padded) {
+template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(FW_THREADS) void dfw_chunk_fwd_kernel(DfwFwdArgs p, int rows_padded) {
     typedef typename E::elem elem;
     extern __shared__ __align__(16) unsigned char smem[];
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
@@ -175,8 +177,9 @@ template <bool SP, typename E> __global__ __launch_bounds__(FW_THREADS) void dfw
     if (b >= p.B) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int T = (int)p.T, nstages = (T + DL * DNB - 1) / (DL * DNB);
-    const elem *const k = reinterpret_cast<const elem *>(p.k) + b * p.T * CH_N;
-    const elem *const q = reinterpret_cast<const elem *>(p.q) + b * p.T * CH_N;
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const elem *const k = reinterpret_cast<const elem *>(p.k) + row.key;
+    const elem *const q = reinterpret_cast<const elem *>(p.q) + row.key;
     // Every wave that stays executes nstages + 2 workgroup barriers.  Wave i runs on SIMD i % 4: the slab waves,
     // whose chain of dependent steps sets the kernel's duration, get SIMDs 0 and 1 to themselves (waves 4 and 5
     // leave at once; a workgroup barrier waits only for the waves that are left), the matrix waves and the
@@ -184,22 +187,22 @@ template <bool SP, typename E> __global__ __launch_bounds__(FW_THREADS) void dfw
     static_assert(DNB == 2, "one matrix wave per block of a stage");
     auto tok0_of = [](int stage, int bb) { return (stage * DNB + bb) * DL; };
     if (wave < 2)
-        slab_wave<SP, E>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
+        slab_wave<SP, E, BLOCKS>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
     else if (wave < 4)
         structure_wave<SP>(smem, nstages, wave - 2, lane);
     else if (wave == 6) {          // K: token-major, and channel-major derived from it
-        const PrepJob<E> jobs[1] = {{k, FW_KT, FW_KC, 1.f, false}};
+        const PrepJob<E> jobs[1] = {{k, CH_N, FW_KT, FW_KC, 1.f, false}};
         prep_wave_jobs<FwRing, DNB, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
     } else if (wave == 7) {        // Q: token-major
-        const PrepJob<E> jobs[1] = {{q, FW_QT, -1, 1.f, false}};
+        const PrepJob<E> jobs[1] = {{q, CH_N, FW_QT, -1, 1.f, false}};
         prep_wave_jobs<FwRing, DNB, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
     }
 }
 
 }  // namespace
 
-template <bool SP, typename E> static int launch_forward(const DfwFwdArgs &a, hipStream_t stream) {
-    auto kern = dfw_chunk_fwd_kernel<SP, E>;
+template <bool SP, typename E, bool BLOCKS> static int launch_forward(const DfwFwdArgs &a, hipStream_t stream) {
+    auto kern = dfw_chunk_fwd_kernel<SP, E, BLOCKS>;
     int rc = enable_lds(reinterpret_cast<const void *>(kern), FW_SMEM, "hipFuncSetAttribute(delta-rule forward kernel)");
     if (rc) return rc;
     const int rows_padded = (int)((a.B + 7) / 8 * 8);
@@ -208,12 +211,13 @@ template <bool SP, typename E> static int launch_forward(const DfwFwdArgs &a, hi
 }
 
 template <typename E> static int forward_of(const DfwFwdArgs &a, bool split_operands, hipStream_t stream) {
-    return split_operands ? launch_forward<true, E>(a, stream) : launch_forward<false, E>(a, stream);
+    if (a.blocks > 1) return split_operands ? launch_forward<true, E, true>(a, stream) : launch_forward<false, E, true>(a, stream);
+    return split_operands ? launch_forward<true, E, false>(a, stream) : launch_forward<false, E, false>(a, stream);
 }
 
 int dfw_chunk_forward(const DfwFwdArgs &a, int dtype, bool split_operands, hipStream_t stream) {
-    if (a.D != CH_N || a.M != CH_N) return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take D = M = 64");
-    if (a.T * CH_N >= 0x7fffffffLL || a.B > 0x1fffffffLL)
+    if (a.blocks < 1 || a.D != (int64_t)CH_N * a.blocks || a.M != CH_N) return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take M = 64 and D = 64 per block");
+    if (a.T * a.D >= 0x7fffffffLL || a.B > 0x1fffffffLL)
         return fail(T2FW_ERR_UNSUPPORTED, "B=%lld T=%lld is too large for the block-wise delta-rule kernels", (long long)a.B, (long long)a.T);
     switch (dtype) {
     case T2FW_F32: return forward_of<ElF32>(a, split_operands, stream);

@@ -10,6 +10,7 @@ struct DfwFwdArgs {
     void *out, *final_state, *delta;
     int64_t B, T, D, M;
     int32_t kg, tb, ntiles;
+    int32_t blocks;                    // matrix-core kernels: value blocks of 64 (at least 1); B counts (row, block) pairs
 };
 
 struct DfwBwdArgs {
@@ -17,12 +18,13 @@ struct DfwBwdArgs {
     void *d_q, *d_k, *d_v, *d_s0;
     int64_t B, T, D, M;
     int32_t kg, tb, ntiles;
+    int32_t blocks;                    // matrix-core kernels: value blocks of 64 (at least 1); B counts (row, block) pairs
 };
 
 int dfw_forward(const DfwFwdArgs &a, int dtype, hipStream_t stream);
 int dfw_backward(const DfwBwdArgs &a, int dtype, hipStream_t stream);
-// block-wise matrix-core kernels: D = M = 64, fp32 / fp16 / bf16 tensors, 16-byte aligned pointers (dfw_chunk_fwd.hip,
-// dfw_chunk_bwd.hip)
+// block-wise matrix-core kernels: M = 64, D = 64 `blocks` (each a recurrence of its own), fp32 / fp16 / bf16 tensors, 16-byte
+// aligned pointers (dfw_chunk_fwd.hip, dfw_chunk_bwd.hip)
 int dfw_chunk_forward(const DfwFwdArgs &a, int dtype, bool split_operands, hipStream_t stream);
 int dfw_chunk_backward(const DfwBwdArgs &a, int dtype, bool split_operands, hipStream_t stream);
 

@@ -207,6 +207,52 @@ PyObject *dfw_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// The value blocks' entry points take 16-byte aligned arrays
+bool aligned(std::initializer_list<Tensor> ts) {
+    for (const Tensor &t : ts)
+        if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) return false;
+    return true;
+}
+
+// dfw_forward_blocks(q, k, v, state, dtype, flags, stream) -> (outputs, final_state, delta), or None for arrays that
+// t2fw_dfw_forward_blocks does not take (empty, misaligned, very large)
+PyObject *dfw_forward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 7);
+    const Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &s = tensor(a[3]);
+    const int32_t dtype = (int32_t)integer(a[4]), flags = (int32_t)integer(a[5]);
+    void *const stream = address(a[6]);
+    const int64_t B = v.size(0), T = v.size(1), D = v.size(2);
+    if (B == 0 || T == 0 || T * D >= 0x7fffffffLL || B * (D / 64) > 0x1fffffffLL || !aligned({q, k, v, s})) Py_RETURN_NONE;
+    const Tensor out = at::empty_like(v), fin = at::empty_like(s), delta = at::empty_like(v);
+    done(unlocked([&] {
+        return t2fw_dfw_forward_blocks(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), out.data_ptr(), fin.data_ptr(),
+                                       delta.data_ptr(), B, T, D, q.size(2), dtype, flags, stream);
+    }));
+    return wrapped({out, fin, delta});
+    END_HANDLE_TH_ERRORS
+}
+
+// dfw_backward_blocks(g_out, g_state, q, k, delta, final_state, dtype, flags, stream) -> (d_q and d_k per block, d_v, d_state)
+PyObject *dfw_backward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    arguments(n, 9);
+    Tensor in[6];                                  // gradients, and what a caller's hooks give back, may lie anywhere
+    for (int i = 0; i < 6; ++i) in[i] = aligned({tensor(a[i])}) ? tensor(a[i]) : tensor(a[i]).clone();
+    const Tensor &go = in[0], &gs = in[1], &q = in[2], &k = in[3], &delta = in[4], &fin = in[5];
+    const int32_t dtype = (int32_t)integer(a[6]), flags = (int32_t)integer(a[7]);
+    void *const stream = address(a[8]);
+    const int64_t B = delta.size(0), T = delta.size(1), D = delta.size(2);
+    const Tensor dq = at::empty({B, D / 64, T, 64}, q.options()), dk = at::empty({B, D / 64, T, 64}, k.options());
+    const Tensor dv = at::empty_like(delta), ds = at::empty_like(fin);
+    done(unlocked([&] {
+        return t2fw_dfw_backward_blocks(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(),
+                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), B, T, D, q.size(2), dtype, flags, stream);
+    }));
+    return wrapped({dq, dk, dv, ds});
+    END_HANDLE_TH_ERRORS
+}
+
 // gate_forward(f_logit, fk_logit, f or None, f_key or None, dtype, stream) -> (f, f_key)
 PyObject *gate_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -266,6 +312,7 @@ PyObject *block_copy(PyObject *, PyObject *const *a, Py_ssize_t n) {
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(lfw_shape), METHOD(lfw_forward), METHOD(lfw_backward_arguments), METHOD(dfw_forward), METHOD(dfw_backward),
                          METHOD(lfw_step),
+                         METHOD(dfw_forward_blocks), METHOD(dfw_backward_blocks),
                          METHOD(gate_forward), METHOD(gate_backward), METHOD(block_copy), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_t2fw_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -42,8 +42,10 @@ def _dfw_backward(grad_output, grad_state, query, key, delta, final_state):
 # ---- value widths that are multiples of 64 (key width 64) as independent blocks -----------------------------
 # The rows of the state do not interact in the delta rule either: S[d, :] sees v[d], q, k only (the key side is
 # coupled through delta_t = v_t - S_{t-1} k_t, a sum over all of M, so only the value side can be cut).  A
-# [D, 64] state with D a multiple of 64 is D / 64 independent [64, 64] recurrences that share q and k; they run as
-# extra batch rows on the matrix-core kernels, which take D = M = 64 only.  d_query and d_key add up over the blocks.
+# [D, 64] state with D a multiple of 64 is D / 64 independent [64, 64] recurrences that share q and k.  The matrix-core
+# kernels read and write the value side's [B,T,D] arrays in place; d_query and d_key come per block and add up.  Arrays
+# that those kernels do not take (not 16-byte aligned, T * D of 2^31 and more) are cut into copies that run as extra
+# batch rows.  B=48, T=777, D=128 bf16, GPU time of a training step: 99 us, with copies 118 (kernels 85 and 78).
 def _value_block_count(value, query):
     D, M = value.shape[-1], query.shape[-1]
     if M != 64 or D % 64 or D <= 64 or value.dtype not in (torch.float32, torch.float16, torch.bfloat16):
@@ -61,16 +63,29 @@ def _value_block_plans(B, T, nd):
     repeat = ((B, nd, T), (T * 64, 0, 64))                   # [B,T,64] -> [B nd,T,64]
     join = ((B, T, nd), (nd * T * 64, 64, T * 64))           # [B nd,T,64] -> [B,T,64 nd]
     total = ((B, T), (nd * T * 64, 64), nd, T * 64)          # [B nd,T,64] -> [B,T,64], the sum over the blocks
-    return {"inputs": _lib.block_plan(repeat, repeat, cut), "outputs": _lib.block_plan(join),
-            "grads_in": _lib.block_plan(cut), "grads_out": _lib.block_plan(total, total, join)}
+    kept = ((B * T,), (64,))                                 # q and k as they are
+    return {"kept": _lib.block_plan(kept, kept), "inputs": _lib.block_plan(repeat, repeat, cut), "outputs": _lib.block_plan(join),
+            "grads_in": _lib.block_plan(cut), "grads_out": _lib.block_plan(total, total, join),
+            "key_grads": _lib.block_plan(total, total)}
 
 
-def _dfw_forward_blocked(query, key, value, state, nd):
-    """(outputs, final_state, what the backward needs: q and k repeated per block, delta and final state of the blocks)"""
+def _dfw_forward_blocked(query, key, value, state, nd, need_grad=True):
+    """(outputs, final_state, what the backward needs: q, k, delta and the final state, whole or of the blocks).  q and k
+    are kept as copies: a caller may change its own before the backward."""
     B, D, M = state.shape
     T = value.shape[1]
     plans = _value_block_plans(B, T, nd)
     with _on_device(value.device):
+        if value.is_cuda:
+            res = _lib.host().dfw_forward_blocks(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
+                                                 _lib.current_stream(value.device))
+            if res is not None:
+                outputs, final_state, delta = res
+                if not need_grad:
+                    return outputs, final_state, ()
+                q, k = torch.empty_like(query), torch.empty_like(key)
+                _lib.block_copy(plans["kept"], (query, key), (q, k))
+                return outputs, final_state, (q, k, delta, final_state)
         qb, kb, vb = (value.new_empty((B * nd, T, 64)) for _ in range(3))
         _lib.block_copy(plans["inputs"], (query, key, value), (qb, kb, vb))
         out_b, fin_b, delta_b = _dfw_forward(qb, kb, vb, state.view(B * nd, 64, M))
@@ -79,17 +94,24 @@ def _dfw_forward_blocked(query, key, value, state, nd):
     return outputs, fin_b.view(B, D, M), (qb, kb, delta_b, fin_b)
 
 
-def _dfw_backward_blocked(grad_output, grad_state, qb, kb, delta_b, fin_b, nd):
-    Bn, T, M = qb.shape
-    B = Bn // nd
+def _dfw_backward_blocked(grad_output, grad_state, q, k, delta, final_state, nd):
+    B, T, D = grad_output.shape
+    M = q.shape[2]
     plans = _value_block_plans(B, T, nd)
-    with _on_device(qb.device):
-        go_b = torch.empty_like(delta_b)
+    with _on_device(q.device):
+        if delta.shape[2] == D:                               # whole arrays: the kernels took them as they are
+            d_qb, d_kb, d_v, d_s = _lib.host().dfw_backward_blocks(grad_output, grad_state, q, k, delta, final_state,
+                                                                   _dtype_code(delta.dtype), _dfw_flags(delta.dtype),
+                                                                   _lib.current_stream(q.device))
+            d_q, d_k = torch.empty_like(q), torch.empty_like(k)
+            _lib.block_copy(plans["key_grads"], (d_qb, d_kb), (d_q, d_k))
+            return d_q, d_k, d_v, d_s
+        go_b = torch.empty_like(delta)
         _lib.block_copy(plans["grads_in"], (grad_output,), (go_b,))
-        d_qb, d_kb, d_vb, d_sb = _dfw_backward(go_b, grad_state.reshape(Bn, 64, M), qb, kb, delta_b, fin_b)
-        d_q, d_k, d_v = qb.new_empty((B, T, M)), qb.new_empty((B, T, M)), qb.new_empty((B, T, 64 * nd))
+        d_qb, d_kb, d_vb, d_sb = _dfw_backward(go_b, grad_state.reshape(B * nd, 64, M), q, k, delta, final_state)
+        d_q, d_k, d_v = q.new_empty((B, T, M)), q.new_empty((B, T, M)), q.new_empty((B, T, D))
         _lib.block_copy(plans["grads_out"], (d_qb, d_kb, d_vb), (d_q, d_k, d_v))
-    return d_q, d_k, d_v, d_sb.view(B, 64 * nd, M)
+    return d_q, d_k, d_v, d_sb.view(B, D, M)
 
 
 class DFWFunction(torch.autograd.Function):
@@ -118,7 +140,7 @@ class DFWFunction(torch.autograd.Function):
         _dtype_code(value.dtype)
         ctx.value_blocks = _value_block_count(value, query)
         if ctx.value_blocks:
-            outputs, final_state, kept = _dfw_forward_blocked(query, key, value, state, ctx.value_blocks)
+            outputs, final_state, kept = _dfw_forward_blocked(query, key, value, state, ctx.value_blocks, any(ctx.needs_input_grad))
             ctx.save_for_backward(*kept)
         else:
             outputs, final_state, delta = _dfw_forward(query, key, value, state)
