@@ -9,7 +9,8 @@
 //      products, no inverses: as many roundings per term as the recurrence has.  The sum over the 64 steps runs on fp32
 //      matrix instructions.
 //   2  lfw_xpar_chain_kernel, elementwise: the chain over the chunks of a row; leaves the state at the START (the adjoint
-//      at the END) of every chunk in fp32 in place of the increments and writes the checkpoints.
+//      at the END) of every chunk in fp32 in place of the increments and writes the checkpoints (64 x 64 fp32: those only,
+//      19 -> 16 us, where the call has them).
 //   3  lfw_xpar_fwd_kernel / lfw_xpar_bwd_kernel: the recurrence itself, step by step, within each chunk; the last chunk's
 //      leaves the final state, the first one's d_s0.  64 x 64 fp32 (lfw_xpar64.hip): on fp64 matrix instructions where the
 //      gates allow it, and one more launch for the chunks where they don't.
@@ -22,8 +23,8 @@
 //     increment of decayed factors comes out finite, and infinity times a gate product that has underflowed is NaN.
 // The workgroups of the row's first chunk (64 x 64 fp32: of the first four) do it in launch 3, the others of that row leave.
 //
-// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 31 + 19 + 56 + 4 us (220 per-step), backward 26 + 11 +
-// 160 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
+// B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 31 + 16 + 54 + 4 us (220 per-step), backward 26 + 11 +
+// 150 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
 //
 // Replaces lfw_cuda_fwd_kernel, lfw_cuda_bwd_kernel and the einsums of the reference
 // (t2fw/csrc/lfw_kernel.cu:18-102, t2fw/csrc/lfw.cpp:45,84-93); semantics t2fw/torch.py:21-31.
@@ -175,6 +176,8 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
         float *const st = p.ws.states + b * NC * (int64_t)(Dp * Kp) + d * Kp + k;
         const float *const tots = p.ws.tots + b * NC * (int64_t)(Dp + Kp);
         IO *const ckpt = p.ckpt != nullptr ? (IO *)p.ckpt + b * NC * DK + o : nullptr;
+        // 64 x 64 fp32 states are read from the checkpoints, where those are asked for (lfw_xpar64.hip)
+        const bool keep = !std::is_same<IO, float>::value || BWD || ckpt == nullptr || D != XP_N || K != XP_N;
         for (int n0 = 0; n0 < NC; n0 += XC_BATCH) {
             float4 m[XC_BATCH], tb[XC_BATCH];
             float ta[XC_BATCH];
@@ -189,7 +192,7 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
             for (int u = 0; u < XC_BATCH; ++u) {
                 if (n0 + u >= NC) break;
                 const int c = BWD ? NC - 1 - (n0 + u) : n0 + u;
-                *reinterpret_cast<float4 *>(st + (int64_t)c * (Dp * Kp)) = make_float4(S[0], S[1], S[2], S[3]);
+                if (keep) *reinterpret_cast<float4 *>(st + (int64_t)c * (Dp * Kp)) = make_float4(S[0], S[1], S[2], S[3]);
                 if (!BWD && ckpt != nullptr) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)

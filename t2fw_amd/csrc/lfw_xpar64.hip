@@ -2,17 +2,18 @@
 //
 // Chunks whose gates allow it run as products on fp64 matrix instructions (lfw_xpar64_mm.hpp), one workgroup of four
 // waves per (row, chunk) [backward: and side].  Everything else runs in one more launch (4 and 6 us where it finds nothing
-// to do; one kernel for both took no less, and 8 % more than the steps alone where every chunk has a zero gate): chunks
+// to do; one kernel for both was 3 % faster then, and 8 % slower than the steps alone where every chunk has a zero gate): chunks
 // with a gate below 2^-20 or a gate product below 2^-400 step by step, a state in a workgroup's registers, and rows that are
 // left to the recurrence over the whole sequence on the per-step bodies.
 //
-// B = 96, T = 1024, measured: forward 56 us, backward 160 us, against 70 and 439 us for the same chunks step by step.
-// Relative error against float64 (2-norm) 3.6e-8 outputs, 3.9e-8 gate gradients, 2.5e-8 states; step by step 8.5e-8, 1.03e-7
-// and 5.1e-8.  What bounds the backward: 248 matrix instructions of 27 ns per wave, 12 waves per SIMD, are 82 us; with the
-// matrix instructions taken out it takes 104 us, with the loads taken out 159 (fp64 vector instructions, 1200 per wave, do
-// not run beside fp64 matrix instructions).  Forms that were slower: tiles of 16 steps with the state carried over them
-// (operands in fp32: 199 us, twice the vector instructions); consecutive workgroups on chunks of one row in the place of
-// one chunk of all rows (181 us).
+// B = 96, T = 1024, measured: forward 54 us, backward 150 us, against 70 and 439 us for the same chunks step by step.
+// Relative error against float64 (2-norm) 4.0e-8 outputs, 4.6e-8 gate gradients, 2.5e-8 states; step by step 8.5e-8, 1.03e-7
+// and 5.1e-8.  What bounds the backward: the matrix instructions of a wave, 120 in fp64 (27 ns each) and 128 in fp32 (13.5),
+// are 60 us at 12 waves per SIMD, its fp64 vector instructions, which do not run beside fp64 matrix instructions, about 35,
+// and its 337 MB take 62 us at a large copy's rate; with two workgroups per CU these overlap in part.  Forms that were slower:
+// products with the states in fp64, too (backward 163, forward 56, state error 2.5e-8); tiles of 16 steps with the state
+// carried over them (operands in fp32: 199 us, twice the vector instructions); consecutive workgroups on chunks of one row in
+// the place of one chunk of all rows (181 us).
 //
 // The steps: a lane is a row of the state (value channels; key channels on the backward's key side), a wave holds 16 of the
 // other side's channels ("columns") in registers; lane l also holds the inputs of column l % 16, which DPP broadcasts within
@@ -222,7 +223,7 @@ __device__ __forceinline__ void forward_steps(const XparFwdArgs &p, FwdSmem &sm,
     const float *const q = (const float *)p.q + line0 + col0;
     float *const out = (float *)p.out + line0;
     floatx4 S[4];
-    load_state<false>(S, p.ws.states + (b * p.NC + chunk) * (XP_N * XP_N), lane, col0);
+    load_state<false>(S, mm::entering_state(p, b * p.NC + chunk), lane, col0);
     int buf = 0;
     float rx[XW_SEG], rf[XW_SEG], ck[XW_SEG], cf[XW_SEG], cq[XW_SEG];
     auto fetch = [&](int t0) {

@@ -8,12 +8,13 @@
 //             d_x_t = (x'_t + gs_t P[t,t]) / a_t;  d_k_t, d_q_t likewise from W (q', k': the two sides exchanged)
 //             f_t d_f_t = beta - sum_{r<t} (gs_r o'_r - xt_r x'_r),  beta = rowsum(Gh * S0) + sum_t gs_t (S0 qs_t)
 //
-// Precision.  Everything is fp64 but the inputs, S0 and G_end (fp32) and P and W, which are rounded to fp32 once.  The
-// running sum of the gate gradients cancels, but only against itself (both of its terms come from the same P), so what is
-// left of the cancellation is the rounding of fp64.
+// Precision.  What tokens share with tokens is fp64, but for P and W, which are rounded to fp32 once.  What they share with
+// S0 and G_end (Gh kt_t as a_63 times G_end with k_t times the gates after t) is an fp32 product in chains of 16 terms.  The
+// running sum of the gate gradients cancels, but only against itself: P's terms from the same P in fp64, the states' from
+// the same fp32 values, which enter beta and leave it again; what is left of the cancellation is the rounding of fp64.
 //
 // Range: gates in [MM_MIN_GATE, 1] with a product of at least MM_MIN_PRODUCT over the chunk, inputs of at most
-// XP_MAX_INPUT, states of at most XP_MAX_STATE (lfw_xpar.hpp): products of two scaled operands stay below 2^923 and factors
+// XP_MAX_INPUT (lfw_xpar.hpp), states and adjoints of at most MM_MAX_STATE: products of two scaled operands stay below 2^923 and factors
 // of both sides above 2^-800.  Chunks outside it run step by step (lfw_xpar64.hip); launch 1 sees single gates, this
 // workgroup the rest when it scales its operands.
 //
@@ -33,12 +34,16 @@ namespace mm {
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int MM_LS = 66;                          // row stride, in doubles, of the token-major operands [64][MM_LS]
+constexpr int MM_FS = 68;                          // row stride, in floats, of the fp32 operands [64][MM_FS]
 constexpr int MM_PS = 68;                          // a 16 x 16 product tile: element (t, s) at (s / 4) MM_PS + 4 t + s % 4
 constexpr float MM_MIN_GATE = XP_MM_MIN_GATE;
 constexpr double MM_MIN_PRODUCT = 0x1p-400;
+constexpr float MM_MAX_STATE = 0x1p40f;
 
 struct Smem {
-    double val[XP_CHUNK * MM_LS], adj[XP_CHUNK * MM_LS];     // other side's kt / xt and qs / gs
+    // other side's kt / xt and qs / gs; after the products of tokens with tokens, adj [and backward val] make room for what is
+    // multiplied with the states, in fp32 (state_operands)
+    double val[XP_CHUNK * MM_LS], adj[XP_CHUNK * MM_LS];
     double tot[XP_N];                              // other side's gate products over the chunk
     float pt[10][4 * MM_PS];                       // product tiles (m, n), n <= m, at m (m + 1) / 2 + n
     float diag[XP_CHUNK];
@@ -161,10 +166,12 @@ __device__ __forceinline__ double operand(float raw, double scale, Seen &seen) {
     return raw * scale;
 }
 
-// The other side's operands of the wave's channels -> LDS
-template <bool FULL>
-__device__ __forceinline__ bool stage_other(Smem &sm, const Lane<FULL> &ln, const float (&g)[4][4], const float (&v)[4][4], const float (&a)[4][4], Seen &seen) {
-    double carry = 1.0;
+// The other side's operands of the wave's channels -> LDS.  qf: the lane's qs / gs in fp32; kf (SUFFIX): its values times the
+// gates that follow them in the chunk.  Both are what multiplies a state: no factor is above one.
+template <bool FULL, bool SUFFIX>
+__device__ __forceinline__ bool stage_other(Smem &sm, const Lane<FULL> &ln, const float (&g)[4][4], const float (&v)[4][4], const float (&a)[4][4],
+                                            float (&qf)[4][4], float (&kf)[4][4], Seen &seen) {
+    double carry = 1.0, kept[4][4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         fence(seen);
@@ -172,9 +179,18 @@ __device__ __forceinline__ bool stage_other(Smem &sm, const Lane<FULL> &ln, cons
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int o = (16 * m + 4 * ln.kg + j) * MM_LS + ln.c;
-            sm.val[o] = operand(v[m][j], s.inv[j], seen);
-            sm.adj[o] = operand(a[m][j], s.pre[j], seen);
+            const double kt = operand(v[m][j], s.inv[j], seen), qs = operand(a[m][j], s.pre[j], seen);
+            sm.val[o] = kt;
+            sm.adj[o] = qs;
+            qf[m][j] = (float)qs;
+            if (SUFFIX) kept[m][j] = kt;
         }
+    }
+    if (SUFFIX) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) kf[m][j] = (float)(kept[m][j] * carry);
     }
     if (ln.kg == 0) sm.tot[ln.c] = carry;
     fence(seen);
@@ -212,18 +228,32 @@ template <bool INCL> __device__ __forceinline__ void product_tiles(Smem &sm, int
     }
 }
 
-// rows of tokens of tile m of an operand times the slab
-__device__ __forceinline__ doublex4 rows_times(const double *operand, int m, const doublex4 (&X)[4], int i, int kg) {
-    const double *const p = operand + (16 * m + mm_row(i)) * MM_LS + 4 * kg;
-    doublex4 a0 = {0., 0., 0., 0.}, a1 = a0;
+// fp32 operands into the place of fp64 ones that all waves are done with
+__device__ __forceinline__ float *state_operands(double *place) { return reinterpret_cast<float *>(place); }
+template <bool FULL> __device__ __forceinline__ void store_operands(float *tile, const Lane<FULL> &ln, const float (&v)[4][4]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-            a0 = mfma(p[16 * q + e], X[q][e], a0);
-            a1 = mfma(p[16 * q + e + 1], X[q][e + 1], a1);
-        }
-    return a0 + a1;
+        for (int j = 0; j < 4; ++j) tile[(16 * m + 4 * ln.kg + j) * MM_FS + ln.c] = v[m][j];
+}
+// rows of tokens of tile m of an fp32 operand times a slab of the state: v_mfma_f32_16x16x4_f32, half the time of the
+// fp64 form, whose rows come back as 4 kg + j.  Chains of 16 terms; nothing that cancels is made of these sums.
+__device__ __forceinline__ doublex4 rows_times(const float *tile, int m, const float (&X)[4][4], int i, int kg) {
+    const float *const p = tile + (16 * m + i) * MM_FS + 4 * kg;
+    floatx4 acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float4 v = ldv4(p + 16 * q);
+        const float av[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], X[q][e], q ? acc[e] : floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    }
+    const floatx4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    doublex4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = sum[j];
+    return o;
 }
 // o + P[m, n] w  (own tokens w of tile n)
 __device__ __forceinline__ doublex4 product_times(const Smem &sm, int m, int n, const double (&w)[4], doublex4 o, int i, int kg) {
@@ -241,13 +271,14 @@ __device__ __forceinline__ doublex4 product_transposed_times(const Smem &sm, int
     return x;
 }
 // X += sum over the chunk's tokens of (other side's operand) (x) (own tokens w), then times the chunk's products
-__device__ __forceinline__ void add_outer(doublex4 (&X)[4], const double *operand, const double (&w)[4][4], int i, int kg) {
+template <typename F, int STRIDE>
+__device__ __forceinline__ void add_outer(doublex4 (&X)[4], const F *operand, const double (&w)[4][4], int i, int kg) {
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) X[q] = mfma(operand[(16 * m + 4 * kg + e) * MM_LS + 16 * q + mm_row(i)], w[m][e], X[q]);
+            for (int q = 0; q < 4; ++q) X[q] = mfma(operand[(16 * m + 4 * kg + e) * STRIDE + 16 * q + mm_row(i)], w[m][e], X[q]);
 }
 __device__ __forceinline__ void scale(doublex4 (&X)[4], const double *tot, double own, int kg) {
 #pragma unroll
@@ -286,6 +317,11 @@ __device__ __forceinline__ bool any_bad(Smem &sm, int w, int lane, bool bad) {
     return __builtin_amdgcn_readfirstlane(sm.bad[0] | sm.bad[1] | sm.bad[2] | sm.bad[3]) != 0;
 }
 
+// fp32: the state entering a chunk is its checkpoint, where those are asked for
+__device__ __forceinline__ const float *entering_state(const XparFwdArgs &p, int64_t item) {
+    return (p.ckpt != nullptr ? (const float *)p.ckpt : p.ws.states) + item * (XP_N * XP_N);
+}
+
 // false: the chunk is out of range, nothing has been stored
 template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwdArgs &p, Smem &sm, int64_t b, int chunk) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -300,8 +336,9 @@ template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwd
     ln.load(oa, (const float *)p.q + line0, 0.0f);
     ln.load(g, (const float *)p.f + line0, 1.0f);
     ln.load(v, (const float *)p.x + line0, 0.0f);
-    load_slab<0>(s0, p.ws.states + (b * p.NC + chunk) * (XP_N * XP_N), ln.c, kg);
-    bool bad = stage_other<FULL>(sm, ln, og, ov, oa, seen);
+    load_slab<0>(s0, entering_state(p, b * p.NC + chunk), ln.c, kg);
+    float qf[4][4], unused[4][4];
+    bool bad = stage_other<FULL, false>(sm, ln, og, ov, oa, qf, unused, seen);
     double xt[4][4], first[4], carry = 1.0;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -313,17 +350,23 @@ template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwd
         }
         first[m] = s.pre[0];
     }
-    bad |= seen.out_of_range() || !(carry >= MM_MIN_PRODUCT);
+    float states = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) states += fabsf(s0[q][e]);
+    bad |= seen.out_of_range() || !(carry >= MM_MIN_PRODUCT) || !(states <= MM_MAX_STATE);
     if (any_bad(sm, w, lane, bad)) return false;
     product_tiles<true>(sm, w, i, kg, n_tok);
     __syncthreads();
-    doublex4 S[4];
-    widen(S, s0);
+    float *const qs = state_operands(sm.adj);
+    store_operands(qs, ln, qf);
+    __syncthreads();
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         if (!FULL && 16 * m >= n_tok) break;
         fence();
-        doublex4 o = rows_times(sm.adj, m, S, i, kg);
+        doublex4 o = rows_times(qs, m, s0, i, kg);
 #pragma unroll
         for (int n = 0; n <= m; ++n) o = product_times(sm, m, n, xt[n], o, i, kg);
         double pre[4];
@@ -334,7 +377,9 @@ template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwd
         ln.store((float *)p.out + line0, m, r);
     }
     if (chunk == (int)p.NC - 1) {
-        add_outer(S, sm.val, xt, i, kg);
+        doublex4 S[4];
+        widen(S, s0);
+        add_outer<double, MM_LS>(S, sm.val, xt, i, kg);
         scale(S, sm.tot, carry, kg);
         store_slab((float *)p.next_state + b * (XP_N * XP_N), S, ln.c, kg);
     }
@@ -358,7 +403,8 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
     ln.load(ra, (const float *)(SIDE ? p.q : p.g_out) + line0, 0.0f);
     load_slab<SIDE>(s0, (const float *)p.ckpt + state, ln.c, kg);
     load_slab<SIDE>(g_end, p.ws.states + state, ln.c, kg);
-    bool bad = stage_other<FULL>(sm, ln, og, ov, oa, seen);
+    float qf[4][4], kf[4][4];
+    bool bad = stage_other<FULL, true>(sm, ln, og, ov, oa, qf, kf, seen);
     double v[4][4], a[4][4], first[4], last[4], tot = 1.0;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -376,19 +422,21 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) states += fabsf(s0[q][e]);
-    bad |= seen.out_of_range() || !(tot >= MM_MIN_PRODUCT) || !(states <= XP_MAX_STATE);
+        for (int e = 0; e < 4; ++e) states += fabsf(s0[q][e]) + fabsf(g_end[q][e]);
+    bad |= seen.out_of_range() || !(tot >= MM_MIN_PRODUCT) || !(states <= MM_MAX_STATE);
     if (any_bad(sm, w, lane, bad)) return false;
     product_tiles<false>(sm, w, i, kg, n_tok);
     __syncthreads();
+    float *const qs = state_operands(sm.adj), *const ks = state_operands(sm.val);
+    store_operands(qs, ln, qf);
+    store_operands(ks, ln, kf);
+    __syncthreads();
     double du[4][4], beta = 0.0;
-    doublex4 X[4];
-    widen(X, s0);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         if (!FULL && 16 * m >= n_tok) break;
         fence();
-        doublex4 o = rows_times(sm.adj, m, X, i, kg);
+        doublex4 o = rows_times(qs, m, s0, i, kg);
 #pragma unroll
         for (int j = 0; j < 4; ++j) beta = fma(a[m][j], o[j], beta);
 #pragma unroll
@@ -408,16 +456,12 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
     }
     fence();
     {
-        doublex4 G[4];
-        widen(G, g_end);
-        scale(G, sm.tot, tot, kg);
+        double part = 0.0;                         // rowsum(Gh * S0)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                beta = fma(G[q][e], X[q][e], beta);
-                X[q][e] = G[q][e];
-            }
+            for (int e = 0; e < 4; ++e) part = fma((double)g_end[q][e] * s0[q][e], sm.tot[16 * q + 4 * kg + e], part);
+        beta = fma(part, tot, beta);
         const Pair r = rows16(beta), h = rows32(r.a + r.b);
         beta = h.a + h.b;                          // gate gradient of the tile's first token, times its gate
     }
@@ -425,7 +469,7 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
     for (int n = 0; n < 4; ++n) {
         if (!FULL && 16 * n >= n_tok) break;
         fence();
-        doublex4 x = rows_times(sm.val, n, X, i, kg);
+        doublex4 x = rows_times(ks, n, g_end, i, kg) * tot;
 #pragma unroll
         for (int m = n; m < 4; ++m)
             if (FULL || 16 * m < n_tok) x = product_transposed_times(sm, m, n, a[m], x, i, kg);
@@ -450,8 +494,11 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
         ln.store((float *)(SIDE ? p.d_f_key : p.d_f) + line0, n, dgt);
     }
     if (SIDE == 0 && chunk == 0) {
-        add_outer(X, sm.adj, a, i, kg);
-        store_slab((float *)p.d_s0 + b * (XP_N * XP_N), X, ln.c, kg);
+        doublex4 G[4];
+        widen(G, g_end);
+        scale(G, sm.tot, tot, kg);
+        add_outer<float, MM_FS>(G, qs, a, i, kg);
+        store_slab((float *)p.d_s0 + b * (XP_N * XP_N), G, ln.c, kg);
     }
     return true;
 }

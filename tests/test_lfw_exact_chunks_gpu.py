@@ -95,9 +95,10 @@ def test_limits_of_the_matrix_form(what, value):
 
 
 def test_error_of_the_matrix_form():
-    """Relative error (2-norm) against the float64 kernels: operands and sums are fp64, the products P are rounded to fp32
-    once and the result once (2.4e-8 each); checkpoints and the adjoint between chunks are fp32 sums of launch 1 (5e-8 of
-    what is left of them).  Step by step the gate gradients are at 1.0e-7."""
+    """Relative error (2-norm) against the float64 kernels: what tokens share with tokens is fp64 but for P, rounded to fp32
+    once, and the result is rounded once (2.4e-8 each); checkpoints, the adjoint between chunks and the products with them
+    are fp32 sums (8e-8 of the part that a chunk's first and last tokens have of them).  Step by step the gate gradients
+    are at 1.0e-7."""
     from t2fw_amd import LFWFunction
     x, f, q, k, fk, s, go, gs = make_config_inputs(8, 300, 64, 64, F32, seed=12)
 
