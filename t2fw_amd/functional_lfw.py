@@ -85,10 +85,10 @@ def _dtype_code(dtype):
 # Where the chunk-parallel exact kernels (three launches per direction) take the place of the per-step ones (one launch
 # forward, two backward): where a sequence is long enough for the launches, and the rows are few enough that the per-step
 # kernels leave the chip idle.  Both sides in microseconds of GPU time, per-step / chunk-parallel.
-#   Steps, forward + backward: 96 rows of 64 x 64 float32, 128 steps 146 / 125 (a host that needs 180 for the launches:
-#     172 / 185), 224 steps 234 / 176, 1024 steps 992 / 541; 24 rows of 16 x 16, 224 steps 156 / 57 (such a host: 180 / 190).
-#   64 x 64 (float32; kernels of its own): 256 rows x 256 steps 497 / 372, forward alone 1.13 times as fast or more.  More
-#     rows would gain too (512 rows x 256 steps 918 / 739); the limit bounds the scratch.
+#   Steps, forward + backward: 24 rows of 16 x 16, 224 steps 156 / 57 (a host that needs 180 for the launches: 180 / 190).
+#   64 x 64 (float32; kernels of its own, on matrix instructions): 96 rows, 128 steps 148 / 78 (as issued by such a host 148 / 154),
+#     224 steps 238 / 106, 1024 steps 1002 / 294; 256 rows x 256 steps 542 / 209, forward alone 123 / 76.  Fewer steps and more rows
+#     would gain too (512 rows x 256 steps 958 / 392); the limits bound the scratch and are those of the kernels before.
 #   A width of 8 or less, where a workgroup of the per-step kernels takes several rows' worth of channels: 1024 rows of 8 x 8,
 #     224 steps 1341 / 345; 64 x 8 forward alone, 128 rows x 224 steps 1.17 times as fast, 160 rows 1.00, 256 rows 0.75.
 #   16 x 16: 384 rows x 224 steps 170 / 145, 512 rows 172 / 184, 768 rows 222 / 259, 1024 rows 248 / 332; x 448 steps 512 rows
