@@ -87,6 +87,7 @@ def load():
 
 
 _host = None
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def loaded():
@@ -120,8 +121,16 @@ def ptr(t):
 
 
 def current_stream(device):
-    """torch's current stream on ``device`` as an address"""
+    """torch's current stream on ``device`` as an address.  (Under torch.compile's tracing there is none: an error, as
+    these calls cannot be traced.)"""
+    if torch.compiler.is_compiling():
+        return torch.cuda.current_stream(device).cuda_stream
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+def typed_like(tensors, models):
+    """``tensors`` as the tensor subclasses of ``models``, which is what torch.empty_like on them would have given"""
+    return tuple(t if type(m) in _PLAIN or t is None else t.as_subclass(type(m)) for t, m in zip(tensors, models))
 
 
 def current_stream_handle(device):

@@ -57,3 +57,35 @@ def test_step_returns_the_callers_tensors():
     for bad in (dict(x=x[:1]), dict(f=f.half()), dict(state=s[:, :3])):
         with pytest.raises((AssertionError, RuntimeError)):
             lfw_step(**{**dict(x=x, f=f, query=q, key=k, f_key=fk, state=s), **bad})
+
+
+class _Marked(torch.Tensor):
+    """a tensor subclass with torch's own behaviour"""
+
+
+@pytest.mark.gpu
+def test_results_keep_the_tensor_subclass_of_their_inputs():
+    from t2fw_amd import LFWFunction
+    from t2fw_amd.functional_dfw import DFWFunction
+    from t2fw_amd.functional_lfw import lfw_step, sigmoid_gates
+    ins = _ins(device="cuda")
+    marked = lambda ts: [t.as_subclass(_Marked) for t in ts]
+    assert [type(t) for t in LFWFunction.apply(*ins)] == [torch.Tensor] * 2
+    assert [type(t) for t in LFWFunction.apply(*marked(ins))] == [_Marked] * 2
+    assert [type(t) for t in sigmoid_gates(*marked(ins[1:3]))] == [_Marked] * 2
+    assert [type(t) for t in lfw_step(*marked([t[:, 0].contiguous() for t in ins[:5]] + ins[5:]))] == [_Marked] * 2
+    for D in (64, 128):
+        q, v, s = torch.ones(2, 3, 64, device="cuda"), torch.ones(2, 3, D, device="cuda"), torch.ones(2, D, 64, device="cuda")
+        assert [type(t) for t in DFWFunction.apply(*marked([q, q, v, s]))] == [_Marked] * 2
+    param = [torch.nn.Parameter(t) for t in ins]
+    assert [type(t) for t in LFWFunction.apply(*param)] == [torch.Tensor] * 2
+
+
+@pytest.mark.gpu
+def test_calls_are_not_traced():
+    """torch.compile finds no stream to trace these calls on, and says so"""
+    from t2fw_amd.functional_dfw import DFWFunction
+    q, v, s = torch.ones(2, 3, 64, device="cuda"), torch.ones(2, 3, 128, device="cuda"), torch.ones(2, 128, 64, device="cuda")
+    with pytest.raises(Exception):
+        torch.compile(lambda *a: DFWFunction.apply(*a), backend="eager")(q.requires_grad_(), q, v, s)
+    torch._dynamo.reset()
