@@ -130,7 +130,10 @@ def current_stream(device):
 
 def typed_like(tensors, models):
     """``tensors`` as the tensor subclasses of ``models``, which is what torch.empty_like on them would have given"""
-    return tuple(t if type(m) in _PLAIN or t is None else t.as_subclass(type(m)) for t, m in zip(tensors, models))
+    for m in models:
+        if type(m) not in _PLAIN:
+            return tuple(t if type(m) in _PLAIN else t.as_subclass(type(m)) for t, m in zip(tensors, models))
+    return tensors
 
 
 def current_stream_handle(device):

@@ -3,7 +3,7 @@
 // which kernels they ask for and what is an error stays in functional_lfw.py and functional_dfw.py.
 //
 // Host time of a call, 4 x 16 tokens of 64 x 64 fp16, ctypes / this: forward 29.5 / 19.1 us without gradients, a training step
-// 205 / 152 us (of which torch's own hand-over to a Python autograd function and back is 91), one generation step 14.6 / 8.0.
+// 205 / 152 us (of which torch's own hand-over to a Python autograd function and back is 91), one generation step 14.6 / 8.4.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
