@@ -13,7 +13,7 @@
 //      19 -> 16 us, where the call has them).
 //   3  lfw_xpar_fwd_kernel / lfw_xpar_bwd_kernel: the recurrence itself, step by step, within each chunk; the last chunk's
 //      leaves the final state, the first one's d_s0.  64 x 64 fp32 (lfw_xpar64.hip): on fp64 matrix instructions where the
-//      gates allow it, and one more launch for the chunks where they don't.
+//      gates and values allow it, and one more launch for the chunks where they don't.
 //
 // A row is left to the recurrence over the whole sequence where the sums could differ from it by more than rounding:
 //   * a gate of magnitude above one (or NaN): the product of one side's gates may overflow where the product of both

@@ -3,8 +3,8 @@
 // Chunks whose gates allow it run as products on fp64 matrix instructions (lfw_xpar64_mm.hpp), one workgroup of four
 // waves per (row, chunk) [backward: and side].  Everything else runs in one more launch (4 and 6 us where it finds nothing
 // to do; one kernel for both was 3 % faster then, and 8 % slower than the steps alone where every chunk has a zero gate): chunks
-// with a gate below 2^-20 or a gate product below 2^-400 step by step, a state in a workgroup's registers, and rows that are
-// left to the recurrence over the whole sequence on the per-step bodies.
+// with a gate below 2^-20 or a gate product below 2^-400, and those whose gate gradients have cancelled in the products, step by
+// step, a state in a workgroup's registers, and rows that are left to the recurrence over the whole sequence on the per-step bodies.
 //
 // B = 96, T = 1024, measured: forward 54 us, backward 150 us, against 70 and 439 us for the same chunks step by step.
 // Relative error against float64 (2-norm) 4.0e-8 outputs, 4.6e-8 gate gradients, 2.5e-8 states; step by step 8.5e-8, 1.03e-7
@@ -269,7 +269,7 @@ __device__ __forceinline__ void forward_steps(const XparFwdArgs &p, FwdSmem &sm,
 // Both kernels of a direction number their workgroups chunk by chunk.  The first does the chunks that the matrix
 // instructions take and says which those were; the second does the others and the rows that are left.
 //
-// What the first says of a (row, chunk, side), in the place of the chunk's gate products, which launch 2 was the last to read.
+// What the first says of a (row, chunk, side) (the second stores all results of those again), in the place of the chunk's gate products, which launch 2 was the last to read.
 __device__ __forceinline__ int32_t *not_done(const XparScratch &ws, int64_t item, int side) {
     return reinterpret_cast<int32_t *>(ws.tots + item * (2 * XP_N)) + side;
 }

@@ -11,12 +11,17 @@
 // Precision.  What tokens share with tokens is fp64, but for P and W, which are rounded to fp32 once.  What they share with
 // S0 and G_end (Gh kt_t as a_63 times G_end with k_t times the gates after t) is an fp32 product in chains of 16 terms.  The
 // running sum of the gate gradients cancels, but only against itself: P's terms from the same P in fp64, the states' from
-// the same fp32 values, which enter beta and leave it again; what is left of the cancellation is the rounding of fp64.
+// the same fp32 values, which enter beta and leave it again.  What is left of the cancellation is fp64 rounding of the LARGEST
+// term so far, measured 2^-50 of it; a value that the gates have forgotten, a token whose gates are small on both sides or
+// the end of the loss make the sum itself far smaller than that term.  MM_CANCELLED draws the line: a token of which less than
+// 2^-26 of the largest term is left ends the chunk's use of these products, so that the remainder stays below 2^-24 of every
+// gate gradient that is kept.  The measure of a token is the larger of f_t d_f_t and its own output's share of it, gs_t o'_t:
+// the sum over the other side's channels may vanish by chance, both rarely do (no chunk of 600 with normal gates).
 //
-// Range: gates in [MM_MIN_GATE, 1] with a product of at least MM_MIN_PRODUCT over the chunk, inputs of at most
+// Range: gates in [XP_MM_MIN_GATE, 1] with a product of at least MM_MIN_PRODUCT over the chunk, inputs of at most
 // XP_MAX_INPUT (lfw_xpar.hpp), states and adjoints of at most MM_MAX_STATE: products of two scaled operands stay below 2^923 and factors
 // of both sides above 2^-800.  Chunks outside it run step by step (lfw_xpar64.hip); launch 1 sees single gates, this
-// workgroup the rest when it scales its operands.
+// workgroup the rest when it scales its operands, and the cancellation when it has the gradients.
 //
 // Lane layout: v_mfma_f64_16x16x4_f64 takes A[i][kg] and B[kg][i] in lane (i = lane & 15, kg = lane >> 4) and returns
 // rows 4 j + kg of column i.  The rows of A are handed over in the order mm_row(i), which makes those rows 4 kg + j.
@@ -39,6 +44,7 @@ constexpr int MM_PS = 68;                          // a 16 x 16 product tile: el
 constexpr float MM_MIN_GATE = XP_MM_MIN_GATE;
 constexpr double MM_MIN_PRODUCT = 0x1p-400;
 constexpr float MM_MAX_STATE = 0x1p40f;
+constexpr unsigned MM_CANCELLED = 26u << 20;       // in the high word of a double: a factor of 2^26
 
 struct Smem {
     // other side's kt / xt and qs / gs; after the products of tokens with tokens, adj [and backward val] make room for what is
@@ -76,6 +82,10 @@ __device__ __forceinline__ doublex4 mfma(double a, double b, doublex4 c) {
 __device__ __forceinline__ float4 ldv4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 __device__ __forceinline__ constexpr int pt_index(int m, int n) { return m * (m + 1) / 2 + n; }
 
+// Magnitudes are compared by their high words.
+__device__ __forceinline__ unsigned magnitude(double v) {
+    return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
+}
 // {value of the even row of 16 lanes of each pair, of the odd one}, {of rows 0-1, of rows 2-3} (v the same in both rows)
 struct Pair { double a, b; };
 __device__ __forceinline__ double words(unsigned lo, unsigned hi) {
@@ -92,6 +102,15 @@ __device__ __forceinline__ Pair rows32(double v) {
     const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
     const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
     return {words(lo[0], hi[0]), words(lo[1], hi[1])};
+}
+struct PairU { unsigned a, b; };
+__device__ __forceinline__ PairU rows16(unsigned v) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {s[0], s[1]};
+}
+__device__ __forceinline__ PairU rows32(unsigned v) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {s[0], s[1]};
 }
 __device__ __forceinline__ double reciprocal(double v) {
     const double r = __builtin_amdgcn_rcp(v);
@@ -386,6 +405,7 @@ template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwd
     return true;
 }
 
+// false: the chunk is out of range, or its gate gradients have cancelled; results that have been stored are no good
 template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(const XparBwdArgs &p, Smem &sm, int64_t b, int chunk) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t line0 = uniform64(row_first_token(b, p.T, p.heads) + (int64_t)chunk * XP_CHUNK * p.heads) * XP_N;
@@ -432,13 +452,17 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
     store_operands(ks, ln, kf);
     __syncthreads();
     double du[4][4], beta = 0.0;
+    unsigned largest = 0;                          // of the terms of the gate gradients' running sum so far
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         if (!FULL && 16 * m >= n_tok) break;
         fence();
         doublex4 o = rows_times(qs, m, s0, i, kg);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) beta = fma(a[m][j], o[j], beta);
+        for (int j = 0; j < 4; ++j) {
+            beta = fma(a[m][j], o[j], beta);
+            largest = max(largest, magnitude(beta));
+        }
 #pragma unroll
         for (int n = 0; n <= m; ++n) o = product_times(sm, m, n, v[n], o, i, kg);
 #pragma unroll
@@ -464,7 +488,10 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
         beta = fma(part, tot, beta);
         const Pair r = rows16(beta), h = rows32(r.a + r.b);
         beta = h.a + h.b;                          // gate gradient of the tile's first token, times its gate
+        const PairU lr = rows16(largest), lh = rows32(max(lr.a, lr.b));
+        largest = max(max(lh.a, lh.b), magnitude(beta));
     }
+    bad = false;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
         if (!FULL && 16 * n >= n_tok) break;
@@ -479,18 +506,31 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
         reciprocals(inv, last[n], g[n]);
         float dv[4], dgt[4];
         double u[4];                               // what is gone after the lane's tokens up to and with the j-th
+        unsigned terms[4];                         // largest of those
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             dv[j] = (float)(fma(a[n][j], (double)dgv[j], x[j]) * inv[j]);
             u[j] = fma(-v[n][j], x[j], du[n][j]);
-            if (j > 0) u[j] += u[j - 1];
+            terms[j] = max(magnitude(du[n][j]), magnitude(u[j]));
+            if (j > 0) {
+                u[j] += u[j - 1];
+                terms[j] = max(terms[j], terms[j - 1]);
+            }
         }
         ln.store((float *)(SIDE ? p.d_k : p.d_x) + line0, n, dv);
         const Pair r = rows16(u[3]), h = rows32(r.a + r.b);
         const double first = beta - (((kg & 2) ? h.a : 0.0) + ((kg & 1) ? r.a : 0.0));
         beta -= h.a + h.b;
+        const PairU lr = rows16(terms[3]), lh = rows32(max(lr.a, lr.b));
+        const unsigned before = max(max(largest, (kg & 2) ? lh.a : 0u), (kg & 1) ? lr.a : 0u);
+        largest = max(largest, max(lh.a, lh.b));
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dgt[j] = (float)((j ? first - u[j - 1] : first) * reciprocal(g[n][j]));
+        for (int j = 0; j < 4; ++j) {
+            const double left = j ? first - u[j - 1] : first;
+            dgt[j] = (float)(left * reciprocal(g[n][j]));
+            const bool lost = max(magnitude(left), magnitude(du[n][j])) + MM_CANCELLED < (j ? max(before, terms[j - 1]) : before);
+            bad |= lost && ln.ok(n, j);
+        }
         ln.store((float *)(SIDE ? p.d_f_key : p.d_f) + line0, n, dgt);
     }
     if (SIDE == 0 && chunk == 0) {
@@ -500,7 +540,7 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
         add_outer<float, MM_FS>(G, qs, a, i, kg);
         store_slab((float *)p.d_s0 + b * (XP_N * XP_N), G, ln.c, kg);
     }
-    return true;
+    return !any_bad(sm, w, lane, bad);
 }
 
 }  // namespace mm

@@ -94,6 +94,70 @@ def test_limits_of_the_matrix_form(what, value):
     check_all((x, f, q, k, fk, s), go, gs, F32)
 
 
+def _gate_gradients(x, f, q, k, fk, s, go, gs):
+    """d_f and d_f_key in float64, and for each element the sum of the magnitudes of all products that it is made of"""
+    x, f, q, k, fk, S, go, G = (t.double() for t in (x, f, q, k, fk, s, go, gs))
+    T, A, H = x.shape[1], S.abs(), G.abs()
+    outer = lambda a, b: a.unsqueeze(2) * b.unsqueeze(1)
+    before = []
+    for t in range(T):
+        before.append((S, A))
+        w = outer(f[:, t], fk[:, t])
+        S, A = S * w + outer(x[:, t], k[:, t]), A * w + outer(x[:, t], k[:, t]).abs()
+    grads, sizes = [[], []], [[], []]
+    for t in reversed(range(T)):
+        g = outer(go[:, t], q[:, t])
+        G, H = G + g, H + g.abs()
+        for out, w in ((grads, G * before[t][0]), (sizes, H * before[t][1])):
+            out[0].append((w * fk[:, t].unsqueeze(1)).sum(2))
+            out[1].append((w * f[:, t].unsqueeze(2)).sum(1))
+        w = outer(f[:, t], fk[:, t])
+        G, H = G * w, H * w
+    back = lambda ts: torch.stack(ts[::-1], 1)
+    return [(back(grads[i]), back(sizes[i])) for i in range(2)]
+
+
+@pytest.mark.parametrize("what,value,gate,tokens", [
+    ("value", 1e6, 2.0 ** -20, 2), ("value", 1e9, 2.0 ** -20, 3), ("value", 1e10, 2.0 ** -20, 3), ("value", 1e12, 2.0 ** -20, 3),
+    ("value", 1e15, 2.0 ** -10, 8), ("value, both gates", 1e5, 2.0 ** -20, 2),
+    ("both gates", 1, 2.0 ** -20, 1), ("both gates", 1, 2.0 ** -17, 1), ("both gates", 1, 2.0 ** -12, 1), ("both gates", 1, 2.0 ** -20, 10),
+    ("step", 1e9, 0.1, 45), ("step", 1e12, 0.1, 45), ("step", 1e15, 0.1, 45), ("query", 1e12, 2.0 ** -10, 6),
+    ("loss ends", 0, 1, 1), ("loss ends, no state gradient", 0, 1, 1), ("no state", 0, 1, 1), ("as usual", 0, 1, 1)])
+def test_gate_gradients_element_by_element(what, value, gate, tokens):
+    """A large value that small gates make the state forget, tokens whose gates are small on both sides, a loss that ends within a
+    chunk: every gate gradient by itself, in units of the magnitudes that it is the sum of.  Bound: a product that is carried over n
+    steps is rounded 2 n times in fp32 (the gates' product and the state), 2^-24 each and independent; where one product outweighs the
+    rest that is sqrt(2 n) 2^-24, n up to 150, and twice that over so many elements.  The per-step kernels use 0.3 of it.  T = 150:
+    chunks of 64, 64 and 22 steps; the first and the last are out of the ordinary, in another row each."""
+    from t2fw_amd import LFWFunction
+    x, f, q, k, fk, s, go, gs = make_config_inputs(3, 150, 64, 64, F32, seed=21, in_scale=0.125, state_std=0.1)
+    for b, t in ((0, 5), (1, 130)):
+        later = slice(t + 1, t + 1 + min(tokens, 150 - t - 1)) if what == "step" else slice(t + 10, t + 10 + tokens)
+        if what.startswith("value"):
+            x[b, t, 3] = value
+            f[b, later, 3] = gate
+        if what.endswith("both gates"):
+            f[b, later], fk[b, later] = gate, gate
+        if what == "step":
+            x[b, t] *= value
+            f[b, later], fk[b, later] = gate, 0.5
+        if what == "query":
+            q[b, t + 9, 3] = value
+            fk[b, later, 3] = gate
+    if what.startswith("loss ends"):
+        go[0, 40:], go[1, 133:] = 0, 0
+        gs[:2] = 0 if "no state" in what else gs[:2] * 1e-12
+    if what == "no state":
+        s[:] = 0
+    want = _gate_gradients(x, f, q, k, fk, s, go, gs)
+    ins = [t.cuda().requires_grad_() for t in (x, f, q, k, fk, s)]
+    got = torch.autograd.grad(LFWFunction.apply(*ins), [ins[1], ins[4]], [go.cuda(), gs.cuda()])
+    for n, g, (w, size) in zip(("d_f", "d_f_key"), got, want):
+        used = ((g.double().cpu() - w).abs() / (2 * 300 ** 0.5 * 2.0 ** -24 * size).clamp_min(1e-40)).max().item()
+        print("%s %s: %.3g of the bound" % (what, n, used), flush=True)
+        assert used <= 1, n
+
+
 def test_error_of_the_matrix_form():
     """Relative error (2-norm) against the float64 kernels: what tokens share with tokens is fp64 but for P, rounded to fp32
     once, and the result is rounded once (2.4e-8 each); checkpoints, the adjoint between chunks and the products with them
