@@ -18,9 +18,11 @@
 // gate gradient that is kept.  The measure of a token is the larger of f_t d_f_t and its own output's share of it, gs_t o'_t:
 // the sum over the other side's channels may vanish by chance, both rarely do (no chunk of 600 with normal gates).
 //
-// Range: gates in [XP_MM_MIN_GATE, 1] with a product of at least MM_MIN_PRODUCT over the chunk, inputs of at most
-// XP_MAX_INPUT (lfw_xpar.hpp), states and adjoints of at most MM_MAX_STATE: products of two scaled operands stay below 2^923 and factors
-// of both sides above 2^-800.  Chunks outside it run step by step (lfw_xpar64.hip); launch 1 sees single gates, this
+// Range: gates in [XP_MM_MIN_GATE, 1] with a product of at least MM_MIN_PRODUCT over the chunk: products of two scaled operands
+// stay below 2^866 and factors of both sides above 2^-800.  Inputs, states and adjoints of at most MM_MAX_VALUE: where gate
+// products make P or an operand of the states underflow fp32, 2^-150 is lost, times a value or an element of a state.  At 2^30
+// that is 2^-24 of results of 2^-96 (with a limit of 2^58, values of 2^40 and queries and keys of 2^-50 gave outputs of 2^-95 that were wrong
+// altogether).  Chunks outside it run step by step (lfw_xpar64.hip); launch 1 sees single gates, this
 // workgroup the rest when it scales its operands, and the cancellation when it has the gradients.
 //
 // Lane layout: v_mfma_f64_16x16x4_f64 takes A[i][kg] and B[kg][i] in lane (i = lane & 15, kg = lane >> 4) and returns
@@ -43,7 +45,7 @@ constexpr int MM_FS = 68;                          // row stride, in floats, of 
 constexpr int MM_PS = 68;                          // a 16 x 16 product tile: element (t, s) at (s / 4) MM_PS + 4 t + s % 4
 constexpr float MM_MIN_GATE = XP_MM_MIN_GATE;
 constexpr double MM_MIN_PRODUCT = 0x1p-400;
-constexpr float MM_MAX_STATE = 0x1p40f;
+constexpr float MM_MAX_VALUE = 0x1p30f;
 constexpr unsigned MM_CANCELLED = 26u << 20;       // in the high word of a double: a factor of 2^26
 
 struct Smem {
@@ -67,7 +69,7 @@ struct Seen {
     unsigned gate = 0;
     float inputs = 0.0f;
     __device__ __forceinline__ bool out_of_range() const {
-        return gate > __float_as_uint(1.0f) - __float_as_uint(MM_MIN_GATE) || !(inputs <= XP_MAX_INPUT);
+        return gate > __float_as_uint(1.0f) - __float_as_uint(MM_MIN_GATE) || !(inputs <= MM_MAX_VALUE);
     }
 };
 // ... and the verdict on what has been looked at so far is taken, not put off with all values kept
@@ -374,7 +376,7 @@ template <bool FULL> __device__ __forceinline__ bool forward_chunk(const XparFwd
     for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int e = 0; e < 4; ++e) states += fabsf(s0[q][e]);
-    bad |= seen.out_of_range() || !(carry >= MM_MIN_PRODUCT) || !(states <= MM_MAX_STATE);
+    bad |= seen.out_of_range() || !(carry >= MM_MIN_PRODUCT) || !(states <= MM_MAX_VALUE);
     if (any_bad(sm, w, lane, bad)) return false;
     product_tiles<true>(sm, w, i, kg, n_tok);
     __syncthreads();
@@ -443,7 +445,7 @@ template <int SIDE, bool FULL> __device__ __forceinline__ bool backward_chunk(co
     for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int e = 0; e < 4; ++e) states += fabsf(s0[q][e]) + fabsf(g_end[q][e]);
-    bad |= seen.out_of_range() || !(tot >= MM_MIN_PRODUCT) || !(states <= MM_MAX_STATE);
+    bad |= seen.out_of_range() || !(tot >= MM_MIN_PRODUCT) || !(states <= MM_MAX_VALUE);
     if (any_bad(sm, w, lane, bad)) return false;
     product_tiles<false>(sm, w, i, kg, n_tok);
     __syncthreads();

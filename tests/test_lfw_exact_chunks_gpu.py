@@ -158,6 +158,31 @@ def test_gate_gradients_element_by_element(what, value, gate, tokens):
         assert used <= 1, n
 
 
+@pytest.mark.parametrize("value,small", [(2.0 ** 55, 2.0 ** -50), (2.0 ** 40, 2.0 ** -50), (2.0 ** 31, 2.0 ** -45), (2.0 ** 27, 2.0 ** -45), (1.0, 2.0 ** -45)])
+def test_outputs_of_small_queries_after_a_large_value(value, small):
+    """A value that key gates of 1/4 make the state forget, queries and keys so small that what is left of it is at the end of fp32's
+    range: every output by itself, in units of the magnitudes that it is the sum of (bound as in the test above)."""
+    from t2fw_amd import LFWFunction
+    x, f, q, k, fk, s, go, gs = make_config_inputs(2, 100, 64, 64, F32, seed=22, in_scale=1.0, state_std=0.0)
+    q, k = q * small, k * small
+    f[:] = 1
+    fk[:] = 0.9
+    fk[0, 6:36] = 0.25
+    x[0, 5] *= value
+    S = A = s.double()
+    want, size = [], []
+    for t in range(100):
+        w, xk = f[:, t].double().unsqueeze(2) * fk[:, t].double().unsqueeze(1), x[:, t].double().unsqueeze(2) * k[:, t].double().unsqueeze(1)
+        S, A = S * w + xk, A * w + xk.abs()
+        want.append((S @ q[:, t].double().unsqueeze(2)).squeeze(2))
+        size.append((A @ q[:, t].double().abs().unsqueeze(2)).squeeze(2))
+    with torch.no_grad():
+        got = LFWFunction.apply(*[t.cuda() for t in (x, f, q, k, fk, s)])[0].double().cpu()
+    used = ((got - torch.stack(want, 1)).abs() / (2 * 200 ** 0.5 * 2.0 ** -24 * torch.stack(size, 1))).max().item()
+    print("outputs: %.3g of the bound" % used, flush=True)
+    assert used <= 1
+
+
 def test_error_of_the_matrix_form():
     """Relative error (2-norm) against the float64 kernels: what tokens share with tokens is fp64 but for P, rounded to fp32
     once, and the result is rounded once (2.4e-8 each); checkpoints, the adjoint between chunks and the products with them
