@@ -87,7 +87,6 @@ def load():
 
 
 _host = None
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def loaded():
@@ -126,14 +125,6 @@ def current_stream(device):
     if torch.compiler.is_compiling():
         return torch.cuda.current_stream(device).cuda_stream
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
-
-
-def typed_like(tensors, models):
-    """``tensors`` as the tensor subclasses of ``models``, which is what torch.empty_like on them would have given"""
-    for m in models:
-        if type(m) not in _PLAIN:
-            return tuple(t if type(m) in _PLAIN else t.as_subclass(type(m)) for t, m in zip(tensors, models))
-    return tensors
 
 
 def current_stream_handle(device):

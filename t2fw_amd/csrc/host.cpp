@@ -53,6 +53,12 @@ template <typename F> int unlocked(F &&launch) {
     pybind11::gil_scoped_release release;
     return launch();
 }
+// torch.empty_like: a tensor subclass has its own
+Tensor empty_like(PyObject *o) {
+    if (THPVariable_CheckExact(o)) return at::empty_like(tensor(o));
+    const pybind11::object made = pybind11::module_::import("torch").attr("empty_like")(pybind11::handle(o));
+    return tensor(made.ptr());
+}
 Tensor bytes_like(const Tensor &t, int64_t n) { return at::empty({n}, t.options().dtype(at::kByte)); }
 
 // lfw_shape(x, f, q, k, f_key, state, heads) -> (B, T, H, D, K), or None where a call on these is an error
@@ -86,7 +92,7 @@ PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int32_t C = (int32_t)integer(a[8]), dtype = (int32_t)integer(a[9]), flags = (int32_t)integer(a[10]);
     void *ws = address(a[11]), *const stream = address(a[13]);
     const int64_t B = x.size(0), T = x.size(1), H = heads ? x.size(2) : 1, D = x.size(-1), K = q.size(-1);
-    const Tensor out = at::empty_like(x), next = at::empty_like(s);
+    const Tensor out = empty_like(a[0]), next = empty_like(a[5]);
     Tensor ckpt, scratch;
     if (nc >= 0) ckpt = at::empty({B * H, nc, D, K}, x.options());
     if (ws == nullptr && ws_bytes > 0) {
@@ -114,7 +120,7 @@ PyObject *lfw_backward_arguments(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const Tensor &x = tensor(a[2]), &q = tensor(a[4]);
     const int64_t ws_bytes = integer(a[13]);
     Tensor grads[6], scratch;
-    for (int i = 0; i < 6; ++i) grads[i] = at::empty_like(tensor(a[2 + i]));
+    for (int i = 0; i < 6; ++i) grads[i] = empty_like(a[2 + i]);
     if (ws_bytes > 0) scratch = bytes_like(x, ws_bytes);
     std::vector<long long> v;                      // addresses, sizes and options in the order of the C declaration
     v.reserve(25);
@@ -165,7 +171,7 @@ PyObject *lfw_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
         default: Py_RETURN_NONE;
     }
     void *const stream = address(a[8]);
-    const Tensor out = a[6] == Py_None ? at::empty_like(x) : tensor(a[6]), next = a[7] == Py_True ? s : at::empty_like(s);
+    const Tensor out = a[6] == Py_None ? empty_like(a[0]) : tensor(a[6]), next = a[7] == Py_True ? s : empty_like(a[5]);
     done(unlocked([&] {
         return t2fw_lfw_step(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(), out.data_ptr(),
                              next.data_ptr(), B, D, K, dtype, stream);
@@ -181,7 +187,7 @@ PyObject *dfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &s = tensor(a[3]);
     const int32_t dtype = (int32_t)integer(a[4]), flags = (int32_t)integer(a[5]);
     void *const stream = address(a[6]);
-    const Tensor out = at::empty_like(v), fin = at::empty_like(s), delta = at::empty_like(v);
+    const Tensor out = empty_like(a[2]), fin = empty_like(a[3]), delta = empty_like(a[2]);
     done(unlocked([&] {
         return t2fw_dfw_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), out.data_ptr(), fin.data_ptr(), delta.data_ptr(),
                                 v.size(0), v.size(1), v.size(2), q.size(2), dtype, flags, stream);
@@ -197,7 +203,7 @@ PyObject *dfw_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const Tensor &go = tensor(a[0]), &gs = tensor(a[1]), &q = tensor(a[2]), &k = tensor(a[3]), &delta = tensor(a[4]), &fin = tensor(a[5]);
     const int32_t dtype = (int32_t)integer(a[6]), flags = (int32_t)integer(a[7]);
     void *const stream = address(a[8]);
-    const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(delta), ds = at::empty_like(fin);
+    const Tensor dq = empty_like(a[2]), dk = empty_like(a[3]), dv = empty_like(a[4]), ds = empty_like(a[5]);
     done(unlocked([&] {
         return t2fw_dfw_backward(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(), dq.data_ptr(),
                                  dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), delta.size(0), delta.size(1), delta.size(2), q.size(2),
@@ -224,7 +230,7 @@ PyObject *dfw_forward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *const stream = address(a[6]);
     const int64_t B = v.size(0), T = v.size(1), D = v.size(2);
     if (B == 0 || T == 0 || T * D >= 0x7fffffffLL || B * (D / 64) > 0x1fffffffLL || !aligned({q, k, v, s})) Py_RETURN_NONE;
-    const Tensor out = at::empty_like(v), fin = at::empty_like(s), delta = at::empty_like(v);
+    const Tensor out = empty_like(a[2]), fin = empty_like(a[3]), delta = empty_like(a[2]);
     done(unlocked([&] {
         return t2fw_dfw_forward_blocks(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), out.data_ptr(), fin.data_ptr(),
                                        delta.data_ptr(), B, T, D, q.size(2), dtype, flags, stream);
@@ -244,7 +250,7 @@ PyObject *dfw_backward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *const stream = address(a[8]);
     const int64_t B = delta.size(0), T = delta.size(1), D = delta.size(2);
     const Tensor dq = at::empty({B, D / 64, T, 64}, q.options()), dk = at::empty({B, D / 64, T, 64}, k.options());
-    const Tensor dv = at::empty_like(delta), ds = at::empty_like(fin);
+    const Tensor dv = empty_like(a[4]), ds = empty_like(a[5]);
     done(unlocked([&] {
         return t2fw_dfw_backward_blocks(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(),
                                         dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), B, T, D, q.size(2), dtype, flags, stream);
@@ -258,7 +264,7 @@ PyObject *gate_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arguments(n, 6);
     const Tensor &lf = tensor(a[0]), &lk = tensor(a[1]);
-    const Tensor f = a[2] == Py_None ? at::empty_like(lf) : tensor(a[2]), fk = a[3] == Py_None ? at::empty_like(lk) : tensor(a[3]);
+    const Tensor f = a[2] == Py_None ? empty_like(a[0]) : tensor(a[2]), fk = a[3] == Py_None ? empty_like(a[1]) : tensor(a[3]);
     const int32_t dtype = (int32_t)integer(a[4]);
     void *const stream = address(a[5]);
     done(unlocked([&] {

@@ -27,18 +27,16 @@ def _dfw_forward(query, key, value, state):
     """The forward kernels on [B,T,M], [B,T,M], [B,T,D], [B,D,M]: (outputs, final_state, delta)"""
     dev = value.device
     with _on_device(dev):
-        res = _lib.host().dfw_forward(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
-                                      _lib.current_stream(dev))
-    return _lib.typed_like(res, (value, state, value))
+        return _lib.host().dfw_forward(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
+                                       _lib.current_stream(dev))
 
 
 def _dfw_backward(grad_output, grad_state, query, key, delta, final_state):
     """The backward kernels: (d_q, d_k, d_v, d_s), the order of t2fw/csrc/dfw_kernel.cu:557"""
     dev = delta.device
     with _on_device(dev):
-        res = _lib.host().dfw_backward(grad_output, grad_state, query, key, delta, final_state, _dtype_code(delta.dtype),
-                                       _dfw_flags(delta.dtype), _lib.current_stream(dev))
-    return _lib.typed_like(res, (query, key, delta, final_state))
+        return _lib.host().dfw_backward(grad_output, grad_state, query, key, delta, final_state, _dtype_code(delta.dtype),
+                                        _dfw_flags(delta.dtype), _lib.current_stream(dev))
 
 
 # ---- value widths that are multiples of 64 (key width 64) as independent blocks -----------------------------
@@ -82,7 +80,7 @@ def _dfw_forward_blocked(query, key, value, state, nd, need_grad=True):
             res = _lib.host().dfw_forward_blocks(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
                                                  _lib.current_stream(value.device))
             if res is not None:
-                outputs, final_state, delta = _lib.typed_like(res, (value, state, value))
+                outputs, final_state, delta = res
                 if not need_grad:
                     return outputs, final_state, ()
                 q, k = torch.empty_like(query), torch.empty_like(key)
@@ -107,7 +105,7 @@ def _dfw_backward_blocked(grad_output, grad_state, q, k, delta, final_state, nd)
                                                                    _lib.current_stream(q.device))
             d_q, d_k = torch.empty_like(q), torch.empty_like(k)
             _lib.block_copy(plans["key_grads"], (d_qb, d_kb), (d_q, d_k))
-            return (d_q, d_k) + _lib.typed_like((d_v, d_s), (delta, final_state))
+            return d_q, d_k, d_v, d_s
         go_b = torch.empty_like(delta)
         _lib.block_copy(plans["grads_in"], (grad_output,), (go_b,))
         d_qb, d_kb, d_vb, d_sb = _dfw_backward(go_b, grad_state.reshape(B * nd, 64, M), q, k, delta, final_state)

@@ -295,7 +295,6 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
                                                      flags, ws_address, ws_bytes, _lib.current_stream(dev))
         if hints is not None:
             hints.launched()
-    outputs, next_state = _lib.typed_like((outputs, next_state), (value, state))
     return outputs, next_state, ckpt, C, flags, hints
 
 
@@ -326,7 +325,7 @@ def _lfw_backward(grad_output, grad_state, value, forget, query, key, f_key, sta
                                                       C, code, flags, ws_bytes, _lib.current_stream(dev))
         lib = _lib.load()
         _lib.check((lib.t2fw_lfw_backward_heads if heads else lib.t2fw_lfw_backward)(*args))
-    return _lib.typed_like(grads, (value, forget, query, key, f_key, state))
+    return grads
 
 
 class LFWFunction(torch.autograd.Function):
@@ -363,8 +362,7 @@ def sigmoid_gates(f_logit, fk_logit, out_f=None, out_fk=None):
     assert f_logit.dtype == fk_logit.dtype
     dev = f_logit.device
     with _on_device(dev):
-        gates = _lib.host().gate_forward(f_logit, fk_logit, out_f, out_fk, _dtype_code(f_logit.dtype), _lib.current_stream(dev))
-    return _lib.typed_like(gates, (f_logit if out_f is None else out_f, fk_logit if out_fk is None else out_fk))
+        return _lib.host().gate_forward(f_logit, fk_logit, out_f, out_fk, _dtype_code(f_logit.dtype), _lib.current_stream(dev))
 
 
 def _gate_backward_inplace(d_f, d_fk, forget, f_key):
@@ -538,7 +536,7 @@ def lfw_step(x, f, query, key, f_key, state, out=None, inplace=True):
         with _on_device(x.device):
             done = _lib.host().lfw_step(x, f, query, key, f_key, state, out, bool(inplace), _lib.current_stream(x.device))
         if done is not None:
-            return _lib.typed_like(done, (x if out is None else out, state))
+            return done
     # which error it is, or what the step above leaves to the caller
     for t, n in ((x, "x"), (f, "f"), (query, "query"), (key, "key"), (f_key, "f_key"), (state, "state")):
         _check_input(t, n)

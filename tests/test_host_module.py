@@ -81,6 +81,49 @@ def test_results_keep_the_tensor_subclass_of_their_inputs():
     assert [type(t) for t in LFWFunction.apply(*param)] == [torch.Tensor] * 2
 
 
+class _Learned(torch.nn.Parameter):
+    """of torch's operations on it a plain tensor comes, as of any parameter"""
+
+
+class _Noted(torch.Tensor):
+    """a tensor subclass that hands something on through torch.empty_like"""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        res = super().__torch_function__(func, types, args, kwargs or {})
+        if func is torch.empty_like:
+            res.note = args[0].note
+        return res
+
+
+@pytest.mark.gpu
+def test_subclasses_through_torch_empty_like():
+    """What a call returns in the place of its own tensors is theirs, what it allocates is what torch.empty_like gives."""
+    from t2fw_amd import LFWFunction
+    from t2fw_amd.functional_dfw import DFWFunction
+    from t2fw_amd.functional_lfw import lfw_step, sigmoid_gates
+    ins = _ins(device="cuda")
+    step = [t[:, 0].contiguous().as_subclass(_Marked) for t in ins[:5]] + [ins[5].clone().as_subclass(_Marked)]
+    out, f, fk = torch.empty_like(step[0]), torch.empty_like(step[1]), torch.empty_like(step[4])
+    got, state = lfw_step(*step, out=out)
+    assert got is out and state is step[5]
+    got = sigmoid_gates(step[1], step[4], out_f=f, out_fk=fk)
+    assert got[0] is f and got[1] is fk
+    learned = [_Learned(t) for t in ins]
+    assert [type(t) for t in LFWFunction.apply(*learned)] == [torch.Tensor] * 2
+    assert [type(t) for t in lfw_step(*[_Learned(t.as_subclass(torch.Tensor)) for t in step], inplace=False)] == [torch.Tensor] * 2
+    noted = [t.as_subclass(_Noted) for t in ins]
+    for i, t in enumerate(noted):
+        t.note = i
+    assert [t.note for t in LFWFunction.apply(*noted)] == [0, 5]
+    for D in (64, 128):
+        q, v, s = torch.ones(2, 3, 64, device="cuda"), torch.ones(2, 3, D, device="cuda"), torch.ones(2, D, 64, device="cuda")
+        noted = [t.as_subclass(_Noted) for t in (q, q.clone(), v, s)]
+        for i, t in enumerate(noted):
+            t.note = i
+        assert [t.note for t in DFWFunction.apply(*noted)] == [2, 3]
+
+
 @pytest.mark.gpu
 def test_calls_are_not_traced():
     """torch.compile finds no stream to trace these calls on, and says so"""
