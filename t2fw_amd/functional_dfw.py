@@ -99,6 +99,10 @@ def _dfw_backward_blocked(grad_output, grad_state, q, k, delta, final_state, nd)
     M = q.shape[2]
     plans = _value_block_plans(B, T, nd)
     with _on_device(q.device):
+        if delta.shape[2] == D and _dfw_flags(delta.dtype) & _lib.FLAG_FORCE_SCAN:      # asked for since: its kernels take blocks
+            qb, kb, delta_b = (delta.new_empty((B * nd, T, 64)) for _ in range(3))
+            _lib.block_copy(plans["inputs"], (q, k, delta), (qb, kb, delta_b))
+            q, k, delta, final_state = qb, kb, delta_b, final_state.reshape(B * nd, 64, M)
         if delta.shape[2] == D:                               # whole arrays: the kernels took them as they are
             d_qb, d_kb, d_v, d_s = _lib.host().dfw_backward_blocks(grad_output, grad_state, q, k, delta, final_state,
                                                                    _dtype_code(delta.dtype), _dfw_flags(delta.dtype),

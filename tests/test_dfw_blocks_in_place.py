@@ -60,6 +60,26 @@ def test_queries_and_keys_may_change_before_the_backward():
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 33])
+def test_per_step_kernels_asked_for_between_forward_and_backward(dtype, T, monkeypatch):
+    """the backward reads T2FW_FLAGS for itself: the per-step kernels, on the blocks that the forward left whole"""
+    from t2fw_amd import functional_dfw as F
+    q, k, v, s, go, gs = [t.cuda() for t in make_inputs(2, T, 192, 64, dtype, seed=5)]
+    ins = [t.detach().requires_grad_(True) for t in (q, k, v, s)]
+    res = F.DFWFunction.apply(*ins)
+    kept = res[0].grad_fn.saved_tensors
+    monkeypatch.setenv("T2FW_FLAGS", "1")
+    got = torch.autograd.grad(res, ins, [go, gs])
+    cut = lambda t: t.view(2, T, 3, 64).transpose(1, 2).reshape(6, T, 64).contiguous()
+    rep = lambda t: t.unsqueeze(1).expand(2, 3, T, 64).reshape(6, T, 64).contiguous()
+    d_q, d_k, d_v, d_s = F._dfw_backward(cut(go), gs.view(6, 64, 64), rep(q), rep(k), cut(kept[2]), kept[3].view(6, 64, 64))
+    total = lambda t: sum(t.view(2, 3, T, 64).float().unbind(1)).to(dtype)
+    want = total(d_q), total(d_k), d_v.view(2, 3, T, 64).transpose(1, 2).reshape(2, T, 192), d_s.view(2, 192, 64)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
 def test_what_the_entry_points_refuse():
     from t2fw_amd import _lib
     lib = _lib.load()
