@@ -124,11 +124,51 @@ def test_subclasses_through_torch_empty_like():
         assert [t.note for t in DFWFunction.apply(*noted)] == [2, 3]
 
 
-@pytest.mark.gpu
-def test_calls_are_not_traced():
-    """torch.compile finds no stream to trace these calls on, and says so"""
+def _traced_calls():
+    from t2fw_amd import LFWFunction, LFWHeadsFunction
     from t2fw_amd.functional_dfw import DFWFunction
-    q, v, s = torch.ones(2, 3, 64, device="cuda"), torch.ones(2, 3, 128, device="cuda"), torch.ones(2, 128, 64, device="cuda")
-    with pytest.raises(Exception):
-        torch.compile(lambda *a: DFWFunction.apply(*a), backend="eager")(q.requires_grad_(), q, v, s)
+    from t2fw_amd.functional_lfw import LFWGatedFunction, lfw_step, sigmoid_gates
+    ones = lambda *s, dtype=torch.float32: torch.ones(s, device="cuda", dtype=dtype)
+    delta = lambda D: [ones(2, 3, 64), ones(2, 3, 64), ones(2, 3, D), ones(2, D, 64)]
+    lfw = _ins(device="cuda")
+    return {
+        "LFWFunction": (LFWFunction.apply, lfw),
+        "LFWFunction, matrix cores": (LFWFunction.apply, _ins(2, 70, 64, 64, "cuda", torch.float16)),
+        "LFWFunction, blocks": (LFWFunction.apply, _ins(2, 3, 128, 64, "cuda", torch.float16)),
+        "LFWGatedFunction": (LFWGatedFunction.apply, lfw),
+        "LFWHeadsFunction": (LFWHeadsFunction.apply, [t.unsqueeze(2) for t in lfw[:5]] + [lfw[5].unsqueeze(1)]),
+        "lfw_step": (lfw_step, [t[:, 0].contiguous() for t in lfw[:5]] + [lfw[5]]),
+        "sigmoid_gates": (sigmoid_gates, [lfw[1], lfw[4]]),
+        "DFWFunction": (DFWFunction.apply, delta(64)),
+        "DFWFunction, blocks": (DFWFunction.apply, delta(128)),
+        "DFWFunction, per step": (DFWFunction.apply, delta(5)),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("loaded", [False, True])
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("name", ["LFWFunction", "LFWFunction, matrix cores", "LFWFunction, blocks", "LFWGatedFunction", "LFWHeadsFunction",
+                                  "lfw_step", "sigmoid_gates", "DFWFunction", "DFWFunction, blocks", "DFWFunction, per step"])
+def test_calls_are_not_traced(name, grad, loaded, monkeypatch):
+    """What torch.compile makes of a call that runs by itself, before and after the library is loaded: an error of its tracing,
+    as these calls can't be traced (no stream is known there, and the host module and ctypes are closed to it).  The host
+    module isn't reached while a call is traced."""
+    from t2fw_amd import _lib
+    call, ins = _traced_calls()[name]
+    fn = lambda *a: call(*a)
+    if grad and name not in ("lfw_step", "sigmoid_gates"):
+        ins[0].requires_grad_()
+    for t in fn(*ins):
+        assert t.is_cuda
+    torch.cuda.synchronize()
+    monkeypatch.setattr(_lib, "loaded", lambda: loaded)
     torch._dynamo.reset()
+    try:
+        with pytest.raises(torch._dynamo.exc.Unsupported, match="Dynamo does not know how to trace"):
+            torch.compile(fn, backend="eager", fullgraph=True)(*ins)
+        torch._dynamo.reset()
+        with pytest.raises(AttributeError, match="'torch.Stream' object has no attribute 'cuda_stream'"):
+            torch.compile(fn, backend="eager")(*ins)
+    finally:
+        torch._dynamo.reset()
