@@ -69,31 +69,6 @@ def test_rows_left_next_to_others(T, D, K):
     check_all((x, f, q, k, fk, s), go, gs, F32)
 
 
-@pytest.mark.parametrize("what,value", [("one gate", 2.0 ** -20), ("one gate", 2.0 ** -21), ("whole chunk", 2.0 ** -6.2),
-                                        ("whole chunk", 2.0 ** -6.3), ("every second gate", 2.0 ** -16), ("tiny gradients", 1e-30),
-                                        ("large value", 2.0 ** 57), ("large value", 2.0 ** 59), ("large state", 2.0 ** 121)])
-def test_limits_of_the_matrix_form(what, value):
-    """64 x 64 float32: on both sides of each limit of the products (a chunk beyond one runs step by step), with a chunk in
-    range and a ragged one next to it.  T = 150: chunks of 64, 64 and 22 steps."""
-    x, f, q, k, fk, s, go, gs = make_config_inputs(2, 150, 64, 64, F32, seed=11, in_scale=0.5, state_std=0.5)
-    if what == "one gate":
-        f[0, 70, 3] = fk[0, 140, 5] = fk[1, 0, 0] = value
-    elif what == "whole chunk":
-        f[0, 64:128, 7] = value
-        fk[1, 0:64, 9] = value
-    elif what == "every second gate":
-        f[0, ::2, 11] = fk[0, 1::2, 13] = value
-    elif what == "tiny gradients":
-        go[0], gs[0] = go[0] * value, gs[0] * value
-    elif what == "large value":
-        x[0, 80, 3] = value
-        q[1, 80, 3] = value
-    else:
-        s[0, 5, 6] = value
-        f[0, :, 5] = 0.5
-    check_all((x, f, q, k, fk, s), go, gs, F32)
-
-
 def _gate_gradients(x, f, q, k, fk, s, go, gs):
     """d_f and d_f_key in float64, and for each element the sum of the magnitudes of all products that it is made of"""
     x, f, q, k, fk, S, go, G = (t.double() for t in (x, f, q, k, fk, s, go, gs))
@@ -117,19 +92,59 @@ def _gate_gradients(x, f, q, k, fk, s, go, gs):
     return [(back(grads[i]), back(sizes[i])) for i in range(2)]
 
 
+def check_gate_gradients(x, f, q, k, fk, s, go, gs):
+    """Every gate gradient by itself, in units of the magnitudes that it is the sum of.  Bound: a product that is carried over n
+    steps is rounded 2 n times in fp32 (the gates' product and the state), 2^-24 each and independent; where one product outweighs the
+    rest that is sqrt(2 n) 2^-24, n up to 150, and twice that over so many elements.  The per-step kernels use 0.3 of it."""
+    from t2fw_amd import LFWFunction
+    assert x.shape[1] <= 150
+    want = _gate_gradients(x, f, q, k, fk, s, go, gs)
+    ins = [t.cuda().requires_grad_() for t in (x, f, q, k, fk, s)]
+    got = torch.autograd.grad(LFWFunction.apply(*ins), [ins[1], ins[4]], [go.cuda(), gs.cuda()])
+    for n, g, (w, size) in zip(("d_f", "d_f_key"), got, want):
+        used = ((g.double().cpu() - w).abs() / (2 * 300 ** 0.5 * 2.0 ** -24 * size).clamp_min(1e-40)).max().item()
+        print("%s: %.3g of the bound" % (n, used), flush=True)
+        assert used <= 1, n
+
+
+@pytest.mark.parametrize("what,value", [("one gate", 2.0 ** -20), ("one gate", 2.0 ** -21), ("whole chunk", 2.0 ** -6.2),
+                                        ("whole chunk", 2.0 ** -6.3), ("every second gate", 2.0 ** -16), ("tiny gradients", 1e-30),
+                                        ("large value", 2.0 ** 29), ("large value", 2.0 ** 31), ("large value", 2.0 ** 57), ("large value", 2.0 ** 59),
+                                        ("large state", 2.0 ** 29), ("large state", 2.0 ** 31), ("large state", 2.0 ** 121)])
+def test_limits_of_the_matrix_form(what, value):
+    """64 x 64 float32: on both sides of each limit of the products (a chunk beyond one runs step by step, a row with inputs beyond
+    2^58 or states beyond 2^120 over the whole sequence), with a chunk in range and a ragged one next to it.  T = 150: chunks of 64,
+    64 and 22 steps."""
+    x, f, q, k, fk, s, go, gs = make_config_inputs(2, 150, 64, 64, F32, seed=11, in_scale=0.5, state_std=0.5)
+    if what == "one gate":
+        f[0, 70, 3] = fk[0, 140, 5] = fk[1, 0, 0] = value
+    elif what == "whole chunk":
+        f[0, 64:128, 7] = value
+        fk[1, 0:64, 9] = value
+    elif what == "every second gate":
+        f[0, ::2, 11] = fk[0, 1::2, 13] = value
+    elif what == "tiny gradients":
+        go[0], gs[0] = go[0] * value, gs[0] * value
+    elif what == "large value":
+        x[0, 80, 3] = value
+        q[1, 80, 3] = value
+    else:
+        s[0, 5, 6] = value
+        f[0, :, 5] = 0.5
+    check_all((x, f, q, k, fk, s), go, gs, F32)
+    check_gate_gradients(x, f, q, k, fk, s, go, gs)
+
+
 @pytest.mark.parametrize("what,value,gate,tokens", [
     ("value", 1e6, 2.0 ** -20, 2), ("value", 1e9, 2.0 ** -20, 3), ("value", 1e10, 2.0 ** -20, 3), ("value", 1e12, 2.0 ** -20, 3),
     ("value", 1e15, 2.0 ** -10, 8), ("value, both gates", 1e5, 2.0 ** -20, 2),
     ("both gates", 1, 2.0 ** -20, 1), ("both gates", 1, 2.0 ** -17, 1), ("both gates", 1, 2.0 ** -12, 1), ("both gates", 1, 2.0 ** -20, 10),
     ("step", 1e9, 0.1, 45), ("step", 1e12, 0.1, 45), ("step", 1e15, 0.1, 45), ("query", 1e12, 2.0 ** -10, 6),
-    ("loss ends", 0, 1, 1), ("loss ends, no state gradient", 0, 1, 1), ("no state", 0, 1, 1), ("as usual", 0, 1, 1)])
+    ("loss ends", 0, 1, 1), ("loss ends, no state gradient", 0, 1, 1), ("no state", 0, 1, 1), ("gates of all sizes", 0, 1, 1),
+    ("as usual", 0, 1, 1)])
 def test_gate_gradients_element_by_element(what, value, gate, tokens):
     """A large value that small gates make the state forget, tokens whose gates are small on both sides, a loss that ends within a
-    chunk: every gate gradient by itself, in units of the magnitudes that it is the sum of.  Bound: a product that is carried over n
-    steps is rounded 2 n times in fp32 (the gates' product and the state), 2^-24 each and independent; where one product outweighs the
-    rest that is sqrt(2 n) 2^-24, n up to 150, and twice that over so many elements.  The per-step kernels use 0.3 of it.  T = 150:
-    chunks of 64, 64 and 22 steps; the first and the last are out of the ordinary, in another row each."""
-    from t2fw_amd import LFWFunction
+    chunk.  T = 150: chunks of 64, 64 and 22 steps; the first and the last are out of the ordinary, in another row each."""
     x, f, q, k, fk, s, go, gs = make_config_inputs(3, 150, 64, 64, F32, seed=21, in_scale=0.125, state_std=0.1)
     for b, t in ((0, 5), (1, 130)):
         later = slice(t + 1, t + 1 + min(tokens, 150 - t - 1)) if what == "step" else slice(t + 10, t + 10 + tokens)
@@ -149,13 +164,9 @@ def test_gate_gradients_element_by_element(what, value, gate, tokens):
         gs[:2] = 0 if "no state" in what else gs[:2] * 1e-12
     if what == "no state":
         s[:] = 0
-    want = _gate_gradients(x, f, q, k, fk, s, go, gs)
-    ins = [t.cuda().requires_grad_() for t in (x, f, q, k, fk, s)]
-    got = torch.autograd.grad(LFWFunction.apply(*ins), [ins[1], ins[4]], [go.cuda(), gs.cuda()])
-    for n, g, (w, size) in zip(("d_f", "d_f_key"), got, want):
-        used = ((g.double().cpu() - w).abs() / (2 * 300 ** 0.5 * 2.0 ** -24 * size).clamp_min(1e-40)).max().item()
-        print("%s %s: %.3g of the bound" % (what, n, used), flush=True)
-        assert used <= 1, n
+    if what == "gates of all sizes":             # 1/64 to 63/64, one per channel
+        f[:] = fk[:] = torch.linspace(1 / 64, 63 / 64, 64)
+    check_gate_gradients(x, f, q, k, fk, s, go, gs)
 
 
 @pytest.mark.parametrize("value,small", [(2.0 ** 55, 2.0 ** -50), (2.0 ** 40, 2.0 ** -50), (2.0 ** 31, 2.0 ** -45), (2.0 ** 27, 2.0 ** -45), (1.0, 2.0 ** -45)])
