@@ -50,12 +50,12 @@ def _compile_host():
     import torch
     from torch.utils.cpp_extension import include_paths
     obj = os.path.join(OBJ_DIR, "host.o")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-w", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
            "-I" + sysconfig.get_paths()["include"]] + ["-isystem" + i for i in include_paths()] + ["-c", HOST_SRC, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed for %s:\n%s" % (HOST_SRC, r.stderr))
-    return obj
+    return obj, r.stderr
 
 
 def _link_host(obj):
@@ -74,8 +74,8 @@ def build(verbose=False):
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         host = ex.submit(_compile_host)
         results = list(ex.map(_compile, srcs))
-        host_obj = host.result()
-    for obj, err in results:
+        host_result = host.result()
+    for obj, err in results + [host_result]:
         if verbose and err.strip():
             print(err, file=sys.stderr)
     objs = [o for o, _ in results]
@@ -83,7 +83,7 @@ def build(verbose=False):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
-    _link_host(host_obj)
+    _link_host(host_result[0])
     return LIB_PATH
 
 
