@@ -88,7 +88,7 @@ def _dtype_code(dtype):
 #   Steps, forward + backward: 24 rows of 16 x 16, 224 steps 156 / 57 (a host that needs 180 for the launches: 180 / 190).
 #   64 x 64 (float32; kernels of its own, on matrix instructions): 96 rows, 128 steps 148 / 78 (as issued by such a host 148 / 154),
 #     224 steps 238 / 106, 1024 steps 1002 / 294; 256 rows x 256 steps 542 / 209, forward alone 123 / 76.  Fewer steps and more rows
-#     would gain too (512 rows x 256 steps 958 / 392); the limits bound the scratch and are those of the kernels before.
+#     would gain too (512 rows x 256 steps 958 / 392): the limits were measured for the step-by-step kernels that these replaced.
 #   A width of 8 or less, where a workgroup of the per-step kernels takes several rows' worth of channels: 1024 rows of 8 x 8,
 #     224 steps 1341 / 345; 64 x 8 forward alone, 128 rows x 224 steps 1.17 times as fast, 160 rows 1.00, 256 rows 0.75.
 #   16 x 16: 384 rows x 224 steps 170 / 145, 512 rows 172 / 184, 768 rows 222 / 259, 1024 rows 248 / 332; x 448 steps 512 rows
