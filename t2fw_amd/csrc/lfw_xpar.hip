@@ -24,7 +24,7 @@
 // The workgroups of the row's first chunk (64 x 64 fp32: of the first four) do it in launch 3, the others of that row leave.
 //
 // B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 31 + 16 + 54 + 4 us (220 per-step), backward 26 + 11 +
-// 150 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
+// 154 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
 //
 // Replaces lfw_cuda_fwd_kernel, lfw_cuda_bwd_kernel and the einsums of the reference
 // (t2fw/csrc/lfw_kernel.cu:18-102, t2fw/csrc/lfw.cpp:45,84-93); semantics t2fw/torch.py:21-31.

@@ -6,7 +6,7 @@
 // with a gate below 2^-20 or a gate product below 2^-400, and those whose gate gradients have cancelled in the products, step by
 // step, a state in a workgroup's registers, and rows that are left to the recurrence over the whole sequence on the per-step bodies.
 //
-// B = 96, T = 1024, measured: forward 54 us, backward 150 us, against 70 and 439 us for the same chunks step by step.
+// B = 96, T = 1024, measured: forward 53 us, backward 154 us, against 70 and 439 us for the same chunks step by step.
 // Relative error against float64 (2-norm) 4.0e-8 outputs, 4.6e-8 gate gradients, 2.5e-8 states; step by step 8.5e-8, 1.03e-7
 // and 5.1e-8.  What bounds the backward: the matrix instructions of a wave, 120 in fp64 (27 ns each) and 128 in fp32 (13.5),
 // are 60 us at 12 waves per SIMD, its fp64 vector instructions, which do not run beside fp64 matrix instructions, about 35,
@@ -269,7 +269,8 @@ __device__ __forceinline__ void forward_steps(const XparFwdArgs &p, FwdSmem &sm,
 // Both kernels of a direction number their workgroups chunk by chunk.  The first does the chunks that the matrix
 // instructions take and says which those were; the second does the others and the rows that are left.
 //
-// What the first says of a (row, chunk, side) (the second stores all results of those again), in the place of the chunk's gate products, which launch 2 was the last to read.
+// What the first says of a (row, chunk, side), in the place of the chunk's gate products, which launch 2 was the last to read.
+// All results of those not done are stored again by the second.
 __device__ __forceinline__ int32_t *not_done(const XparScratch &ws, int64_t item, int side) {
     return reinterpret_cast<int32_t *>(ws.tots + item * (2 * XP_N)) + side;
 }
