@@ -270,6 +270,22 @@ int t2fw_dfw_backward_blocks(const void *g_out, const void *g_state,
                              int32_t dtype, int32_t flags, void *stream);
 
 /*
+ * The same backward with d_q and d_k whole, [B,T,64], the sums over the blocks (each share rounded to the tensors' type before it is
+ * added).  `workspace`: device memory, 16-byte aligned, of as many elements as 2 n arrays of [B,T,64], not read across calls.  The query is 0 where the
+ * entry point does not take a call (T2FW_ERR_UNSUPPORTED): other shapes, T2FW_FLAG_FORCE_SCAN, and fp16 / bf16 tensors without
+ * T2FW_FLAG_BF16_OPERANDS.
+ */
+size_t t2fw_dfw_backward_sums_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t M,
+                                              int32_t dtype, int32_t flags);
+int t2fw_dfw_backward_sums(const void *g_out, const void *g_state,
+                           const void *q, const void *k, const void *delta,
+                           const void *final_state,
+                           void *d_q, void *d_k, void *d_v, void *d_s0,
+                           int64_t B, int64_t T, int64_t D, int64_t M,
+                           int32_t dtype, int32_t flags,
+                           void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Conversion of `count` (<= 8) arrays of n[i] elements each between float32 and float16 / bfloat16 in one
  * launch (src_dtype -> dst_dtype, one of them T2FW_F32); arrays 16-byte aligned, `src`, `dst`, `n` host arrays.
  * No counterpart in the reference (one kernel serves every dtype there, lfw_kernel.cu:157-168): it is what a

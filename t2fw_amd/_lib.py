@@ -60,6 +60,8 @@ SIGNATURES = {
     "t2fw_dfw_backward": (ctypes.c_int, [_vp] * 10 + [_i64] * 4 + [_i32, _i32, _vp]),
     "t2fw_dfw_forward_blocks": (ctypes.c_int, [_vp] * 7 + [_i64] * 4 + [_i32, _i32, _vp]),
     "t2fw_dfw_backward_blocks": (ctypes.c_int, [_vp] * 10 + [_i64] * 4 + [_i32, _i32, _vp]),
+    "t2fw_dfw_backward_sums_workspace_bytes": (_sz, [_i64] * 4 + [_i32, _i32]),
+    "t2fw_dfw_backward_sums": (ctypes.c_int, [_vp] * 10 + [_i64] * 4 + [_i32, _i32, _vp, _sz, _vp]),
 }
 
 _lib = None

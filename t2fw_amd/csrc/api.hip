@@ -623,8 +623,13 @@ int t2fw_dfw_backward(const void *g_out, const void *g_state, const void *q, con
     a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
     a.B = B; a.T = T; a.D = D; a.M = M; a.blocks = 1;
     if (dfw_chunk_ok(D, M, dtype, flags) && T * CH_N < 0x7fffffffLL &&
-        aligned16({g_out, g_state, q, k, delta, final_state, d_q, d_k, d_v, d_s0}))
+        aligned16({g_out, g_state, q, k, delta, final_state, d_q, d_k, d_v, d_s0})) {
+        if (dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0)) {
+            a.states = d_q;
+            a.adjoints = d_k;
+        }
         return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, st);
+    }
     return dfw_backward(a, dtype, st);
 }
 
@@ -671,6 +676,47 @@ int t2fw_dfw_backward_blocks(const void *g_out, const void *g_state, const void 
     a.g_out = g_out; a.g_state = g_state; a.q = q; a.k = k; a.delta = delta; a.final_state = final_state;
     a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
     a.B = B * blocks; a.T = T; a.D = D; a.M = M; a.blocks = blocks;
+    if (blocks == 1 && dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0)) {
+        a.states = d_q;
+        a.adjoints = d_k;
+    }
+    return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
+}
+
+// Where the key side runs in chunks: what t2fw_dfw_backward_sums needs for the edges of several blocks' chunks.
+size_t t2fw_dfw_backward_sums_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t M, int32_t dtype, int32_t flags) {
+    const size_t es = elem_size(dtype);
+    if (B <= 0 || T <= 0 || M != 64 || D < 64 || D % 64 != 0 || !dfw_chunk_ok(64, M, dtype, flags) || check_dims(B, T, D, M) ||
+        T * D >= 0x7fffffffLL || B * (D / 64) > 0x1fffffffLL || B * ((T + CH_N - 1) / CH_N) > 0x7fffffffLL ||
+        !dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0))
+        return 0;
+    return 2 * (size_t)(B * T * D) * es;
+}
+
+int t2fw_dfw_backward_sums(const void *g_out, const void *g_state, const void *q, const void *k, const void *delta,
+                           const void *final_state, void *d_q, void *d_k, void *d_v, void *d_s0, int64_t B, int64_t T,
+                           int64_t D, int64_t M, int32_t dtype, int32_t flags, void *workspace, size_t workspace_bytes,
+                           void *stream) {
+    const size_t es = elem_size(dtype);
+    if (es == 0) return fail(T2FW_ERR_BAD_DTYPE, "unknown dtype code %d", dtype);
+    int rc = check_dims(B, T, D, M);
+    if (rc) return rc;
+    if (B == 0) return T2FW_OK;
+    const size_t need = t2fw_dfw_backward_sums_workspace_bytes(B, T, D, M, dtype, flags);
+    if (need == 0)
+        return fail(T2FW_ERR_UNSUPPORTED, "sums over value blocks: B=%lld T=%lld D=%lld M=%lld dtype %d flags %d", (long long)B, (long long)T,
+                    (long long)D, (long long)M, dtype, flags);
+    if (workspace_bytes < need) return fail(T2FW_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    const NamedPtr ptrs[] = {{"g_out", g_out}, {"g_state", g_state}, {"q", q}, {"k", k}, {"delta", delta}, {"final_state", final_state},
+                             {"d_q", d_q}, {"d_k", d_k}, {"d_v", d_v}, {"d_s0", d_s0}, {"workspace", workspace}};
+    if ((rc = check_ptrs(ptrs, 11, 16))) return rc;
+    DfwBwdArgs a{};
+    a.g_out = g_out; a.g_state = g_state; a.q = q; a.k = k; a.delta = delta; a.final_state = final_state;
+    a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
+    a.blocks = (int32_t)(D / 64);
+    a.B = B * a.blocks; a.T = T; a.D = D; a.M = M;
+    a.states = workspace;
+    a.adjoints = static_cast<char *>(workspace) + need / 2;
     return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
 }
 

@@ -62,10 +62,9 @@ struct ElF32 {
         }
     }
     // four consecutive elements, 16-byte aligned
-    static __device__ __forceinline__ floatx4 load4(const elem *p) {
-        const float4 t = *reinterpret_cast<const float4 *>(p);
-        return floatx4{t.x, t.y, t.z, t.w};
-    }
+    typedef float4 Raw4;
+    static __device__ __forceinline__ floatx4 floats(const Raw4 &t) { return floatx4{t.x, t.y, t.z, t.w}; }
+    static __device__ __forceinline__ floatx4 load4(const elem *p) { return floats(*reinterpret_cast<const Raw4 *>(p)); }
     static __device__ __forceinline__ void store4(elem *p, const floatx4 &v) {
         *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
     }
@@ -92,11 +91,13 @@ template <typename IOE> struct El16 {          // IOE = Fp16 or Bf16 (lfw_chunk.
         }
     }
     // four consecutive elements, 8-byte aligned
-    static __device__ __forceinline__ floatx4 load4(const elem *p) {
+    typedef uint2 Raw4;
+    static __device__ __forceinline__ floatx4 floats(const Raw4 &t) {
         float o[4];
-        unpack4<IOE>(*reinterpret_cast<const uint2 *>(p), o);
+        unpack4<IOE>(t, o);
         return floatx4{o[0], o[1], o[2], o[3]};
     }
+    static __device__ __forceinline__ floatx4 load4(const elem *p) { return floats(*reinterpret_cast<const Raw4 *>(p)); }
     static __device__ __forceinline__ void store4(elem *p, const floatx4 &v) { *reinterpret_cast<uint2 *>(p) = packq<IOE>(v[0], v[1], v[2], v[3]); }
 };
 
@@ -263,6 +264,24 @@ template <bool BLOCKS> struct DfwRow {
         }
     }
 };
+
+// ---- states and adjoints at chunk edges -------------------------------------------------------------------
+// The value side of the backward leaves the state before each whole chunk of 64 tokens and the adjoint after it as the split operands
+// that the key side's chunks read, in the order of its own accumulators: piece ((plane * 4 + d / 16) * 2 + h) * 64 + lane of 16
+// bytes holds, of row d = 16 (d / 16) + r, the channels 32 h + 4 g .. + 3 and 32 h + 16 + 4 g .. + 3 (plane 0: heads; with SP, 1:
+// remainders).  Every store is a contiguous KB: rows of the matrix, 32 bytes of 16 of them per store, cost the value side 11 of 64 us
+// (B = 96, T = 1024, fp32).
+constexpr int DCH = 64;                        // tokens of a chunk
+constexpr int DCH_PIECES = CH_N * CH_N / 8;    // 16-byte pieces of a plane
+template <bool SP> __device__ __forceinline__ void store_edge(void *edge, int tile, int lane, const floatx4 (&v)[4]) {
+    uint4 *const p = reinterpret_cast<uint4 *>(edge) + tile * 128 + lane;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const Sp4<SP> s = cat(split4<SP>(v[2 * h]), split4<SP>(v[2 * h + 1]));
+        p[64 * h] = s.hi;
+        if constexpr (SP) p[DCH_PIECES + 64 * h] = s.lo;
+    }
+}
 
 // ---- staging of a [T, 64] array into tiles (one wave per array) ---------------------------------------
 // sixteen elements of one lane: token lane >> 2, channels 16 (lane & 3) .. + 15.  Rows at or past T read as zero.

@@ -10,9 +10,11 @@
 //   value side  one workgroup per (row, half of the value channels): G rows in fp32 accumulators; writes d_value
 //               and d_state.  Its chain per block is  G_end -> dU = Tm^T Bq^T g + (Tm^T K) G_end^T -> G_start,
 //               with Tm, Bq and K'' = Tm^T K prepared ahead by the matrix waves.
-//   key side    one workgroup per (row, half of the key channels): columns of S and of G in fp32 accumulators,
-//               both plain running sums (it reads d_value from the first launch); writes d_query and d_key (with several
-//               value blocks the block's share of them).
+//               Two more waves walk the state backwards, and both leave what the key side's chunks start from.
+//   key side    reads d_value and writes d_query and d_key, a workgroup per chunk of 64 tokens (dfw_key.hip).  Where an edge
+//               of a chunk does not fit the chunk's results (16-bit tensors with split operands), and for the shares of
+//               several value blocks (t2fw_dfw_backward_blocks), the sequential form below: one workgroup per (row,
+//               half of the key channels), columns of S and of G in fp32 accumulators, both plain running sums.
 #include <type_traits>
 #include "common.hpp"
 #include "dfw_chunk.hpp"
@@ -30,11 +32,49 @@ constexpr int VS_KT = 0, VS_QT = VS_KT + 2 * TM_TILE, VS_KC = VS_QT + 2 * TM_TIL
               VS_RAW_BLOCK = VS_QC + 2 * CM_TILE;
 constexpr int VS_KPP = 0, VS_TM = VS_KPP + 2 * TM_TILE, VS_BQ = VS_TM + 2 * ST_TILE, VS_ST_BLOCK = VS_BQ + 2 * ST_TILE;
 using VsRing = Ring<VS_RAW_BLOCK, VS_ST_BLOCK, DNB>;
-static_assert(VsRing::SMEM <= 160 * 1024, "value-side tiles exceed the LDS of one CU");
+// The slab waves hand the adjoint at a chunk's edge to the state waves, which store it: per wave the pieces of store_edge.
+constexpr int VS_HAND_WAVE = 2 * 2 * 64 * 16, VS_HAND = VsRing::SMEM, VS_SMEM = VS_HAND + 2 * VS_HAND_WAVE;
+static_assert(VS_SMEM <= 160 * 1024, "value-side tiles exceed the LDS of one CU");
 
 // first token of block `bb` of a stage when the blocks are visited last to first
 __device__ __forceinline__ int reverse_tok0(int nblocks, int nblk_per_stage, int stage, int bb) {
     return (nblocks - 1 - (stage * nblk_per_stage + bb)) * DL;
+}
+
+// The stages of a wave whose loads run one stage ahead (x: those of stage 0; y: the other register set).  The blocks are visited
+// last to first, so only stage 0 can hold tokens at or past T; `full` says that a stage has none.  With EDGES the stages
+// that end where a chunk of two stages begins are told apart: the first of them, the last (the sequence's first chunk) and
+// those between.  All of this is known at compile time: the waits that the compiler places count outstanding memory
+// operations along every path, and a path that skips stores, or loads still pending where a loop is entered, would make each
+// stage wait for the stores of the stage before.
+enum Edge { EDGE_NONE, EDGE_FIRST, EDGE_INNER, EDGE_LAST };
+template <bool EDGES, typename F, typename R> __device__ __forceinline__ void visit_stages(F &&stage_body, int nstages, R &x, R &y) {
+    const std::false_type no{};
+    const std::true_type yes{};
+    const std::integral_constant<int, EDGE_NONE> none{};
+    const std::integral_constant<int, EDGES ? EDGE_FIRST : EDGE_NONE> first{};
+    const std::integral_constant<int, EDGES ? EDGE_INNER : EDGE_NONE> inner{};
+    const std::integral_constant<int, EDGES ? EDGE_LAST : EDGE_NONE> last{};
+    static_assert(DCH == 2 * DNB * DL, "a chunk is two stages");
+    int stage = 1;
+    if (nstages & 1) {
+        stage_body(no, first, 0, x, y);
+    } else {
+        stage_body(no, none, 0, x, y);
+        wait_vmem_all();
+        stage_body(yes, first, 1, y, x);
+        y = x;
+        stage = 2;
+    }
+    wait_vmem_all();
+    for (; stage + 2 < nstages + (EDGES ? 0 : 1); stage += 2) {
+        stage_body(yes, none, stage, y, x);
+        stage_body(yes, inner, stage + 1, x, y);
+    }
+    if (EDGES && stage < nstages) {
+        stage_body(yes, none, stage, y, x);
+        stage_body(yes, last, stage + 1, x, y);
+    }
 }
 
 template <bool SP> __device__ __forceinline__ void vs_structure_wave(unsigned char *smem, int nstages, int bb, int lane) {
@@ -68,7 +108,75 @@ template <bool SP> __device__ __forceinline__ void vs_structure_wave(unsigned ch
     }
 }
 
-template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_slab_wave(const DfwBwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
+// Where the edges of whole chunk c of a row (or of a row's value block) lie: at its tokens in the key side's [T, 64] results, which the
+// workgroup that reads them writes afterwards.
+template <typename E> __device__ __forceinline__ void *edge_at(void *base, int64_t b, int64_t T, int c) {
+    return reinterpret_cast<typename E::elem *>(base) + (b * T + (int64_t)c * DCH) * CH_N;
+}
+
+// The state walked backwards by 16 value channels, for the key side's chunks: S before each whole chunk goes to `states`, and the
+// adjoint after it, which the slab wave of the same channels leaves in LDS, to `adjoints`.  (Stored by the slab wave itself it cost
+// the kernel 8 of 63 us at B = 96, T = 1024, fp32: loads return in order with the stores before them.)
+template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_state_wave(const DfwBwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
+    typedef typename E::elem elem;
+    const int r = lane & 15, g = lane >> 4, d = d0 + r, T = (int)p.T, nblocks = nstages * DNB;
+    const DfwRow<BLOCKS> row(b, p.T, p.blocks);
+    const u32 vs = row.vs;
+    const elem *const dl = reinterpret_cast<const elem *>(p.delta) + row.value;
+    floatx4 S[4];           // S[j][e] = S[d][16 j + 4 g + e]
+    {
+        const elem *fs = reinterpret_cast<const elem *>(p.final_state) + (b * CH_N + d) * CH_N + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[j] = E::load4(fs + 16 * j);
+    }
+    struct Raw {
+        elem x[DNB][4];
+    };
+    auto load = [&](Raw &x, int stage) {
+#pragma unroll
+        for (int bb = 0; bb < DNB; ++bb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                x.x[bb][e] = dl[(size_t)min(reverse_tok0(nblocks, DNB, stage, bb) + 4 * g + e, T - 1) * vs + d];
+    };
+    auto stage_body = [&](auto full, auto edge, int stage, Raw &cur, Raw &nxt) {
+        constexpr bool FULL = decltype(full)::value;
+        constexpr int EDGE = decltype(edge)::value;
+        load(nxt, min(stage + 1, nstages - 1));
+        static_assert(DNB == 2, "the two blocks of a stage make one 32-deep product");
+        Sp2<SP> nds[DNB];
+#pragma unroll
+        for (int bb = 0; bb < DNB; ++bb) {
+            const int tok0 = reverse_tok0(nblocks, DNB, stage, bb);
+            floatx4 nd;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) nd[e] = (FULL || tok0 + 4 * g + e < T) ? -E::f(cur.x[bb][e]) : 0.f;
+            nds[bb] = split4<SP>(nd);
+        }
+        const CmTile<SP> K0(VsRing::raw(smem, stage, 0) + VS_KC), K1(VsRing::raw(smem, stage, 1) + VS_KC);
+        const Sp4<SP> ns = cat(nds[0], nds[1]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[j] = mma32(cat(K0.tokens(16 * j + r, g), K1.tokens(16 * j + r, g)), ns, S[j]);
+        if constexpr (EDGE != EDGE_NONE) {
+            const int c = (nstages - 1 - stage) >> 1;              // the chunk that begins here
+            if constexpr (EDGE != EDGE_FIRST) {                    // the adjoint after it, which the slab wave left a stage ago
+                const uint4 *const hand = reinterpret_cast<const uint4 *>(smem + VS_HAND + ((d0 >> 4) & 1) * VS_HAND_WAVE) + lane;
+                uint4 *const to = reinterpret_cast<uint4 *>(edge_at<E>(p.adjoints, b, p.T, c)) + (d0 >> 4) * 128 + lane;
+#pragma unroll
+                for (int i = 0; i < (SP ? 4 : 2); ++i) to[(i >> 1) * DCH_PIECES + (i & 1) * 64] = hand[64 * i];
+            }
+            if (EDGE != EDGE_FIRST || (c + 1) * DCH <= T) store_edge<SP>(edge_at<E>(p.states, b, p.T, c), d0 >> 4, lane, S);
+        }
+        __syncthreads();
+    };
+    Raw a, c;
+    load(a, 0);
+    __syncthreads();
+    __syncthreads();
+    visit_stages<true>(stage_body, nstages, a, c);
+}
+
+template <bool SP, typename E, bool BLOCKS, bool EDGES> __device__ __forceinline__ void vs_slab_wave(const DfwBwdArgs &p, unsigned char *smem, int64_t b, int d0, int nstages, int lane) {
     typedef typename E::elem elem;
     const int r = lane & 15, g = lane >> 4, d = d0 + r, T = (int)p.T, nblocks = nstages * DNB;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -95,11 +203,11 @@ template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_s
             for (int e = 0; e < 4; ++e)
                 x.x[bb][e] = go[(size_t)min(reverse_tok0(nblocks, DNB, stage, bb) + 4 * g + e, T - 1) * vs + d];
     };
-    // One stage.  FULL: every token of the stage is below T and the body has no branch.  (The waits that the
-    // compiler places count outstanding memory operations along every path: a path that skips stores, or loads
-    // still pending where the loop is entered, would make each stage wait for the stores of the stage before.)
-    auto stage_body = [&](auto full, int stage, GRaw &graw, GRaw &gnxt) {
+    if (EDGES && T % DCH == 0) store_edge<SP>(edge_at<E>(p.adjoints, b, p.T, T / DCH - 1), d0 >> 4, lane, G);
+    // One stage.  FULL: every token of the stage is below T and the body has no branch.
+    auto stage_body = [&](auto full, auto edge, int stage, GRaw &graw, GRaw &gnxt) {
         constexpr bool FULL = decltype(full)::value;
+        constexpr int EDGE = decltype(edge)::value;
         load_g(gnxt, min(stage + 1, nstages - 1));
 #pragma unroll
         for (int bb = 0; bb < DNB; ++bb) {
@@ -116,6 +224,16 @@ template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_s
             const floatx4 bg = mma16(st_load<SP>(st + VS_BQ, lane), gs, zero);
             const floatx4 tbg = mma16(st_load<SP>(st + VS_TM, lane), split4<SP>(bg), zero);
             const Sp4<SP> gb0 = cat(split4<SP>(G[0]), split4<SP>(G[1])), gb1 = cat(split4<SP>(G[2]), split4<SP>(G[3]));
+            if constexpr (EDGES && FULL && EDGE == EDGE_NONE)
+                if (bb == 0) {                                // G at the edge that the stage before ended at
+                    uint4 *const hand = reinterpret_cast<uint4 *>(smem + VS_HAND + ((d0 >> 4) & 1) * VS_HAND_WAVE) + lane;
+                    hand[0] = gb0.hi;
+                    hand[64] = gb1.hi;
+                    if constexpr (SP) {
+                        hand[128] = gb0.lo;
+                        hand[192] = gb1.lo;
+                    }
+                }
             const floatx4 kg = mma32(KPP.acc_order(r, g, 1), gb1, mma32(KPP.acc_order(r, g, 0), gb0, zero));
             const floatx4 du = tbg + kg;
             elem *const vb = d_v + (size_t)tok0 * vs;        // wave-uniform
@@ -136,23 +254,16 @@ template <bool SP, typename E, bool BLOCKS> __device__ __forceinline__ void vs_s
     load_g(g_a, 0);
     __syncthreads();        // ticks 0 and 1: the prep and matrix waves fill the pipeline
     __syncthreads();
-    // the blocks are visited last to first: only stage 0 can hold tokens at or past T
-    stage_body(std::false_type{}, 0, g_a, g_b);
-    wait_vmem_all();
-    int stage = 1;
-    for (; stage + 2 <= nstages; stage += 2) {
-        stage_body(std::true_type{}, stage, g_b, g_a);
-        stage_body(std::true_type{}, stage + 1, g_a, g_b);
-    }
-    if (stage < nstages) stage_body(std::true_type{}, stage, g_b, g_a);
+    visit_stages<EDGES>(stage_body, nstages, g_a, g_b);
     elem *ds0 = reinterpret_cast<elem *>(p.d_s0) + (b * CH_N + d) * CH_N + 4 * g;
 #pragma unroll
     for (int j = 0; j < 4; ++j) E::store4(ds0 + 16 * j, G[j]);
 }
 
 // blockIdx = half * rows_padded + row (rows_padded a multiple of 8: both halves of a row on one XCD).  Waves 0, 1:
-// slab waves, alone on SIMDs 0 and 1; waves 2, 3: matrix waves; waves 6, 7: prep waves; waves 4, 5 leave at once.
-template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_value_kernel(DfwBwdArgs p, int rows_padded) {
+// slab waves, on SIMDs 0 and 1; waves 2, 3: matrix waves; waves 6, 7: prep waves; waves 4, 5, on the slab waves' SIMDs: state waves
+// (EDGES) or nothing.
+template <bool SP, typename E, bool BLOCKS, bool EDGES> __global__ __launch_bounds__(BW_THREADS) void dfw_chunk_bwd_value_kernel(DfwBwdArgs p, int rows_padded) {
     typedef typename E::elem elem;
     extern __shared__ __align__(16) unsigned char smem[];
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
@@ -166,9 +277,11 @@ template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THRE
     auto tok0_of = [=](int stage, int bb) { return reverse_tok0(nblocks, DNB, stage, bb); };
     static_assert(DNB == 2, "one matrix wave per block of a stage");
     if (wave < 2) {
-        vs_slab_wave<SP, E, BLOCKS>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
+        vs_slab_wave<SP, E, BLOCKS, EDGES>(p, smem, b, 32 * half + 16 * wave, nstages, lane);
     } else if (wave < 4) {
         vs_structure_wave<SP>(smem, nstages, wave - 2, lane);
+    } else if (EDGES && wave < 6) {
+        vs_state_wave<SP, E, BLOCKS>(p, smem, b, 32 * half + 16 * (wave - 4), nstages, lane);
     } else if (wave == 6) {
         const PrepJob<E> jobs[1] = {{k, CH_N, VS_KT, VS_KC, 1.f, false}};
         prep_wave_jobs<VsRing, DNB, 1, SP, 3, E>(smem, jobs, T, nstages, lane, tok0_of, nullptr);
@@ -366,17 +479,31 @@ template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THRE
 
 }  // namespace
 
-template <bool SP, typename E, bool BLOCKS> static int launch_backward(const DfwBwdArgs &a, hipStream_t stream) {
-    auto value_side = dfw_chunk_bwd_value_kernel<SP, E, BLOCKS>;
-    auto key_side = dfw_chunk_bwd_key_kernel<SP, E, BLOCKS>;
-    int rc = enable_lds(reinterpret_cast<const void *>(value_side), VsRing::SMEM, "hipFuncSetAttribute(delta-rule backward kernel, value side)");
+template <bool SP, typename E, bool BLOCKS, bool EDGES> static int launch_value_side(const DfwBwdArgs &a, hipStream_t stream) {
+    auto value_side = dfw_chunk_bwd_value_kernel<SP, E, BLOCKS, EDGES>;
+    const int rc = enable_lds(reinterpret_cast<const void *>(value_side), VS_SMEM, "hipFuncSetAttribute(delta-rule backward kernel, value side)");
     if (rc) return rc;
-    if ((rc = enable_lds(reinterpret_cast<const void *>(key_side), KS_SMEM, "hipFuncSetAttribute(delta-rule backward kernel, key side)"))) return rc;
     const int rows_padded = (int)((a.B + 7) / 8 * 8);
-    hipLaunchKernelGGL(value_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), VsRing::SMEM, stream, a, rows_padded);
-    if ((rc = check_hip(hipGetLastError(), "dfw_chunk_bwd_value_kernel launch"))) return rc;
-    hipLaunchKernelGGL(key_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), KS_SMEM, stream, a, rows_padded);
-    return check_hip(hipGetLastError(), "dfw_chunk_bwd_key_kernel launch");
+    hipLaunchKernelGGL(value_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), VS_SMEM, stream, a, rows_padded);
+    return check_hip(hipGetLastError(), "dfw_chunk_bwd_value_kernel launch");
+}
+
+template <bool SP, typename E, bool BLOCKS> static int launch_backward(const DfwBwdArgs &a, hipStream_t stream) {
+    constexpr bool CHUNKS = dfw_key_chunks_ok(sizeof(typename E::elem), SP);
+    if constexpr (CHUNKS)
+        if (a.states) return launch_value_side<SP, E, BLOCKS, true>(a, stream);
+    if constexpr (CHUNKS && !BLOCKS) {
+        return fail(T2FW_ERR_UNSUPPORTED, "the key side runs in chunks for this type");       // not reached: d_q and d_k take the edges
+    } else {
+        if (a.states) return fail(T2FW_ERR_UNSUPPORTED, "16-bit tensors with split operands have no chunks of the key side");
+        int rc = launch_value_side<SP, E, BLOCKS, false>(a, stream);
+        if (rc) return rc;
+        auto key_side = dfw_chunk_bwd_key_kernel<SP, E, BLOCKS>;
+        if ((rc = enable_lds(reinterpret_cast<const void *>(key_side), KS_SMEM, "hipFuncSetAttribute(delta-rule backward kernel, key side)"))) return rc;
+        const int rows_padded = (int)((a.B + 7) / 8 * 8);
+        hipLaunchKernelGGL(key_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), KS_SMEM, stream, a, rows_padded);
+        return check_hip(hipGetLastError(), "dfw_chunk_bwd_key_kernel launch");
+    }
 }
 
 template <typename E> static int backward_of(const DfwBwdArgs &a, bool split_operands, hipStream_t stream) {
@@ -388,12 +515,14 @@ int dfw_chunk_backward(const DfwBwdArgs &a, int dtype, bool split_operands, hipS
     if (a.blocks < 1 || a.D != (int64_t)CH_N * a.blocks || a.M != CH_N) return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take M = 64 and D = 64 per block");
     if (a.T * a.D >= 0x7fffffffLL || a.B > 0x1fffffffLL)
         return fail(T2FW_ERR_UNSUPPORTED, "B=%lld T=%lld is too large for the block-wise delta-rule kernels", (long long)a.B, (long long)a.T);
+    int rc;
     switch (dtype) {
-    case T2FW_F32: return backward_of<ElF32>(a, split_operands, stream);
-    case T2FW_F16: return backward_of<El16<Fp16>>(a, split_operands, stream);
-    case T2FW_BF16: return backward_of<El16<Bf16>>(a, split_operands, stream);
+    case T2FW_F32: rc = backward_of<ElF32>(a, split_operands, stream); break;
+    case T2FW_F16: rc = backward_of<El16<Fp16>>(a, split_operands, stream); break;
+    case T2FW_BF16: rc = backward_of<El16<Bf16>>(a, split_operands, stream); break;
     default: return fail(T2FW_ERR_UNSUPPORTED, "the block-wise delta-rule kernels take fp32, fp16 and bf16 tensors");
     }
+    return rc || !a.states ? rc : dfw_key_chunks(a, dtype, split_operands, stream);
 }
 
 }  // namespace t2fw

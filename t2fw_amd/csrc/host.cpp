@@ -239,7 +239,8 @@ PyObject *dfw_forward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// dfw_backward_blocks(g_out, g_state, q, k, delta, final_state, dtype, flags, stream) -> (d_q and d_k per block, d_v, d_state)
+// dfw_backward_blocks(g_out, g_state, q, k, delta, final_state, dtype, flags, stream) -> (d_q, d_k, d_v, d_state); d_q and d_k
+// [B, n, T, 64], per block, where t2fw_dfw_backward_sums does not take the call
 PyObject *dfw_backward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arguments(n, 9);
@@ -249,8 +250,18 @@ PyObject *dfw_backward_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int32_t dtype = (int32_t)integer(a[6]), flags = (int32_t)integer(a[7]);
     void *const stream = address(a[8]);
     const int64_t B = delta.size(0), T = delta.size(1), D = delta.size(2);
-    const Tensor dq = at::empty({B, D / 64, T, 64}, q.options()), dk = at::empty({B, D / 64, T, 64}, k.options());
     const Tensor dv = empty_like(a[4]), ds = empty_like(a[5]);
+    const size_t ws_bytes = t2fw_dfw_backward_sums_workspace_bytes(B, T, D, q.size(2), dtype, flags);
+    if (ws_bytes > 0) {
+        const Tensor dq = empty_like(a[2]), dk = empty_like(a[3]), scratch = bytes_like(delta, (int64_t)ws_bytes);
+        done(unlocked([&] {
+            return t2fw_dfw_backward_sums(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(),
+                                            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), B, T, D, q.size(2), dtype, flags,
+                                            scratch.data_ptr(), ws_bytes, stream);
+        }));
+        return wrapped({dq, dk, dv, ds});
+    }
+    const Tensor dq = at::empty({B, D / 64, T, 64}, q.options()), dk = at::empty({B, D / 64, T, 64}, k.options());
     done(unlocked([&] {
         return t2fw_dfw_backward_blocks(go.data_ptr(), gs.data_ptr(), q.data_ptr(), k.data_ptr(), delta.data_ptr(), fin.data_ptr(),
                                         dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), B, T, D, q.size(2), dtype, flags, stream);

@@ -107,6 +107,8 @@ def _dfw_backward_blocked(grad_output, grad_state, q, k, delta, final_state, nd)
             d_qb, d_kb, d_v, d_s = _lib.host().dfw_backward_blocks(grad_output, grad_state, q, k, delta, final_state,
                                                                    _dtype_code(delta.dtype), _dfw_flags(delta.dtype),
                                                                    _lib.current_stream(q.device))
+            if d_qb.dim() == 3:
+                return d_qb, d_kb, d_v, d_s
             d_q, d_k = torch.empty_like(q), torch.empty_like(k)
             _lib.block_copy(plans["key_grads"], (d_qb, d_kb), (d_q, d_k))
             return d_q, d_k, d_v, d_s
