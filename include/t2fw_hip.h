@@ -285,6 +285,9 @@ int t2fw_dfw_backward_sums(const void *g_out, const void *g_state,
                            int32_t dtype, int32_t flags,
                            void *workspace, size_t workspace_bytes, void *stream);
 
+/* hipEventRecord, for a caller that goes from its tensors to the launch and the event after it in one step. */
+int t2fw_record_event(void *event, void *stream);
+
 /*
  * Conversion of `count` (<= 8) arrays of n[i] elements each between float32 and float16 / bfloat16 in one
  * launch (src_dtype -> dst_dtype, one of them T2FW_F32); arrays 16-byte aligned, `src`, `dst`, `n` host arrays.

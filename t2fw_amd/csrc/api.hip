@@ -720,6 +720,10 @@ int t2fw_dfw_backward_sums(const void *g_out, const void *g_state, const void *q
     return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
 }
 
+int t2fw_record_event(void *event, void *stream) {
+    return check_hip(hipEventRecord(static_cast<hipEvent_t>(event), static_cast<hipStream_t>(stream)), "hipEventRecord");
+}
+
 int t2fw_cast(const void *const *src, void *const *dst, const int64_t *n, int32_t count, int32_t src_dtype,
               int32_t dst_dtype, void *stream) {
     if (count < 0 || count > CAST_MAX_TENSORS) return fail(T2FW_ERR_BAD_SHAPE, "t2fw_cast takes 0 to %d arrays, got %d", CAST_MAX_TENSORS, count);

@@ -78,14 +78,10 @@ def _dfw_forward_blocked(query, key, value, state, nd, need_grad=True):
     with _on_device(value.device):
         if value.is_cuda:
             res = _lib.host().dfw_forward_blocks(query, key, value, state, _dtype_code(value.dtype), _dfw_flags(value.dtype),
-                                                 _lib.current_stream(value.device))
+                                                 _lib.current_stream(value.device), plans["kept"] if need_grad else None)
             if res is not None:
-                outputs, final_state, delta = res
-                if not need_grad:
-                    return outputs, final_state, ()
-                q, k = torch.empty_like(query), torch.empty_like(key)
-                _lib.block_copy(plans["kept"], (query, key), (q, k))
-                return outputs, final_state, (q, k, delta, final_state)
+                outputs, final_state, delta, q, k = res
+                return outputs, final_state, (q, k, delta, final_state) if need_grad else ()
         qb, kb, vb = (value.new_empty((B * nd, T, 64)) for _ in range(3))
         _lib.block_copy(plans["inputs"], (query, key, value), (qb, kb, vb))
         out_b, fin_b, delta_b = _dfw_forward(qb, kb, vb, state.view(B * nd, 64, M))

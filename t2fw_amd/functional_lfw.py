@@ -181,6 +181,11 @@ def _block_dims(value, blocks):
 
 def _run_plan(plan, srcs, dsts, copied):
     """dsts from srcs in one launch; an entry that is not ``copied`` is a view of its source, of the shape of dsts"""
+    if srcs[0].is_cuda:
+        outs = _lib.host().blocks_of(plan, tuple(srcs), tuple(dsts), tuple(copied), _dtype_code(srcs[0].dtype),
+                                     _lib.current_stream(srcs[0].device))
+        if outs is not None:
+            return outs
     outs, cs, cd = [], [], []
     for s, shape, c in zip(srcs, dsts, copied):
         if c:
@@ -268,33 +273,39 @@ def _checked_shape(value, forget, query, key, f_key, state, heads):
     return B, T, H, D, K
 
 
-def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False):
+def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False, logits=False):
     """The checks, then the forward kernels.  heads=False: x,f [B,T,D]; q,k,f_key [B,T,K]; state [B,D,K].
     heads=True: x,f [B,T,H,D]; q,k,f_key [B,T,H,K]; state [B,H,D,K].  Returns (outputs, next_state, ckpt or
     None, checkpoint interval, flags, hints): ``hints`` is None, or the forward's verdict on which backward
-    path the gates allow, readable from the host once the forward has run (path_hint.py)."""
+    path the gates allow, readable from the host once the forward has run (path_hint.py).  logits=True: ``forget`` and
+    ``f_key`` are gate logits, and the gates follow what is returned."""
     dims = _lib.host().lfw_shape(value, forget, query, key, f_key, state, heads) if _lib.loaded() else None
     B, T, H, D, K = dims if dims is not None else _checked_shape(value, forget, query, key, f_key, state, heads)
     code = _dtype_code(value.dtype)
     flags = _flags()
     blocks = _block_counts(value, query, flags)
     if blocks is not None:
-        return _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
+        if logits:
+            forget, f_key = sigmoid_gates(forget, f_key)
+        res = _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
+        return (*res, forget, f_key) if logits else res
     host = _lib.host()
     C = _ckpt_interval()
     dev = value.device
     flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags, need_grad)
     with _on_device(dev):
         hints = None
-        ws_address = 0                                     # the workspace is allocated for the call
+        ws_address = event = 0                             # the workspace is allocated for the call
         if need_grad and ws_bytes and regions[3] and regions[5] and _host_hints_enabled() and ForwardHints.usable(dev):
             # a backward on the matrix cores will follow: the workspace goes to pinned host memory
             hints = ForwardHints(dev, ws_bytes, regions[2], regions[3], B * H)
-            ws_address = hints.workspace()[0].value
-        outputs, next_state, ckpt = host.lfw_forward(value, forget, query, key, f_key, state, heads, nc if need_grad else -1, C, code,
-                                                     flags, ws_address, ws_bytes, _lib.current_stream(dev))
+            ws_address, event = hints.workspace()[0].value, hints.event()
+        outputs, next_state, ckpt, *gates = host.lfw_forward(value, forget, query, key, f_key, state, heads, nc if need_grad else -1, C, code,
+                                                             flags, ws_address, ws_bytes, _lib.current_stream(dev), logits, event)
         if hints is not None:
             hints.launched()
+    if logits:
+        return outputs, next_state, ckpt, C, flags, hints, *gates
     return outputs, next_state, ckpt, C, flags, hints
 
 
@@ -372,6 +383,14 @@ def _gate_backward_inplace(d_f, d_fk, forget, f_key):
         _lib.host().gate_backward(d_f, d_fk, forget, f_key, _dtype_code(d_f.dtype), _lib.current_stream(dev))
 
 
+def _lfw_forward_logits(value, f_logit, query, key, fk_logit, state, need_grad, heads):
+    """_lfw_forward on gate logits.  Where the call is an error, the gates come first, which may be one by themselves."""
+    if _lib.loaded() and value.dtype != torch.float64 and _lib.host().lfw_shape(value, f_logit, query, key, fk_logit, state, heads) is not None:
+        return _lfw_forward(value, f_logit, query, key, fk_logit, state, need_grad, heads, True)
+    forget, f_key = sigmoid_gates(f_logit, fk_logit)
+    return (*_lfw_forward(value, forget, query, key, f_key, state, need_grad, heads), forget, f_key)
+
+
 class LFWGatedFunction(torch.autograd.Function):
     """``LFWFunction`` on gate *logits*: f = sigmoid(f_logit), f_key = sigmoid(fk_logit) are computed
     by one streaming kernel for both gates, the gates (not the logits) are kept for backward, and
@@ -383,9 +402,9 @@ class LFWGatedFunction(torch.autograd.Function):
     def forward(ctx, value, f_logit, query, key, fk_logit, state):
         assert value.shape == f_logit.shape and query.shape == fk_logit.shape
         assert f_logit.dtype == value.dtype and fk_logit.dtype == value.dtype
-        forget, f_key = sigmoid_gates(f_logit, fk_logit)
         need_grad = any(ctx.needs_input_grad)
-        outputs, next_state, ckpt, C, flags, hints = _lfw_forward(value, forget, query, key, f_key, state, need_grad)
+        outputs, next_state, ckpt, C, flags, hints, forget, f_key = _lfw_forward_logits(value, f_logit, query, key, fk_logit, state, need_grad,
+                                                                                        False)
         if need_grad:
             ctx.save_for_backward(value, forget, query, key, f_key, state, ckpt)
             ctx.ckpt_interval = C
@@ -418,10 +437,12 @@ class LFWHeadsFunction(torch.autograd.Function):
         if logits:
             assert value.shape == forget.shape and query.shape == f_key.shape
             assert forget.dtype == value.dtype and f_key.dtype == value.dtype
-            forget, f_key = sigmoid_gates(forget, f_key)
         need_grad = any(ctx.needs_input_grad)
-        outputs, next_state, ckpt, C, flags, hints = _lfw_forward(value, forget, query, key, f_key, state, need_grad,
-                                                                  heads=True)
+        if logits:
+            outputs, next_state, ckpt, C, flags, hints, forget, f_key = _lfw_forward_logits(value, forget, query, key, f_key, state, need_grad,
+                                                                                            True)
+        else:
+            outputs, next_state, ckpt, C, flags, hints = _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=True)
         if need_grad:
             ctx.save_for_backward(value, forget, query, key, f_key, state, ckpt)
             ctx.ckpt_interval = C

@@ -64,7 +64,7 @@ def count_hinted_rows(hints, rows):
 class _Slot:
     """One pinned workspace: the tensor that owns it, the address the GPU sees it under, a view of its
     hint region and the event recorded after the last launch that writes it."""
-    __slots__ = ("buf", "dptr", "view", "event")
+    __slots__ = ("buf", "dptr", "view", "event", "handle")
 
 
 class _PinnedPool:
@@ -90,6 +90,8 @@ class _PinnedPool:
                                                                   ctypes.byref(slot.dptr)))
         slot.view = slot.buf.numpy()[hint_offset:hint_offset + 4 * hint_count].view(np.int32)
         slot.event = torch.cuda.Event()
+        slot.event.record()                     # there is no handle before; the stream is that of the call that follows
+        slot.handle = slot.event.cuda_event
         return slot
 
     def release(self, key, slot):
@@ -121,9 +123,12 @@ class ForwardHints:
     def workspace(self):
         return self.slot.dptr, self.nbytes
 
+    def event(self):
+        """The handle of the event that the forward call records on its stream after the launch."""
+        return self.slot.handle
+
     def launched(self):
-        """Call right after the forward launch, on the launch stream."""
-        self.slot.event.record(torch.cuda.current_stream(self.device))
+        """Call after the forward call, which has recorded the event."""
         self.launched_ = True
 
     def hinted_rows(self):
