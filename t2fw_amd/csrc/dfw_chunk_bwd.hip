@@ -52,28 +52,39 @@ template <bool EDGES, typename F, typename R> __device__ __forceinline__ void vi
     const std::false_type no{};
     const std::true_type yes{};
     const std::integral_constant<int, EDGE_NONE> none{};
-    const std::integral_constant<int, EDGES ? EDGE_FIRST : EDGE_NONE> first{};
-    const std::integral_constant<int, EDGES ? EDGE_INNER : EDGE_NONE> inner{};
-    const std::integral_constant<int, EDGES ? EDGE_LAST : EDGE_NONE> last{};
-    static_assert(DCH == 2 * DNB * DL, "a chunk is two stages");
-    int stage = 1;
-    if (nstages & 1) {
-        stage_body(no, first, 0, x, y);
-    } else {
+    if constexpr (!EDGES) {
         stage_body(no, none, 0, x, y);
         wait_vmem_all();
-        stage_body(yes, first, 1, y, x);
-        y = x;
-        stage = 2;
-    }
-    wait_vmem_all();
-    for (; stage + 2 < nstages + (EDGES ? 0 : 1); stage += 2) {
-        stage_body(yes, none, stage, y, x);
-        stage_body(yes, inner, stage + 1, x, y);
-    }
-    if (EDGES && stage < nstages) {
-        stage_body(yes, none, stage, y, x);
-        stage_body(yes, last, stage + 1, x, y);
+        int stage = 1;
+        for (; stage + 2 <= nstages; stage += 2) {
+            stage_body(yes, none, stage, y, x);
+            stage_body(yes, none, stage + 1, x, y);
+        }
+        if (stage < nstages) stage_body(yes, none, stage, y, x);
+    } else {
+        const std::integral_constant<int, EDGE_FIRST> first{};
+        const std::integral_constant<int, EDGE_INNER> inner{};
+        const std::integral_constant<int, EDGE_LAST> last{};
+        static_assert(DCH == 2 * DNB * DL, "a chunk is two stages");
+        int stage = 1;
+        if (nstages & 1) {
+            stage_body(no, first, 0, x, y);
+        } else {
+            stage_body(no, none, 0, x, y);
+            wait_vmem_all();
+            stage_body(yes, first, 1, y, x);
+            y = x;
+            stage = 2;
+        }
+        wait_vmem_all();
+        for (; stage + 2 < nstages; stage += 2) {
+            stage_body(yes, none, stage, y, x);
+            stage_body(yes, inner, stage + 1, x, y);
+        }
+        if (stage < nstages) {
+            stage_body(yes, none, stage, y, x);
+            stage_body(yes, last, stage + 1, x, y);
+        }
     }
 }
 
@@ -481,10 +492,11 @@ template <bool SP, typename E, bool BLOCKS> __global__ __launch_bounds__(BW_THRE
 
 template <bool SP, typename E, bool BLOCKS, bool EDGES> static int launch_value_side(const DfwBwdArgs &a, hipStream_t stream) {
     auto value_side = dfw_chunk_bwd_value_kernel<SP, E, BLOCKS, EDGES>;
-    const int rc = enable_lds(reinterpret_cast<const void *>(value_side), VS_SMEM, "hipFuncSetAttribute(delta-rule backward kernel, value side)");
+    constexpr int smem = EDGES ? VS_SMEM : VsRing::SMEM;
+    const int rc = enable_lds(reinterpret_cast<const void *>(value_side), smem, "hipFuncSetAttribute(delta-rule backward kernel, value side)");
     if (rc) return rc;
     const int rows_padded = (int)((a.B + 7) / 8 * 8);
-    hipLaunchKernelGGL(value_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), VS_SMEM, stream, a, rows_padded);
+    hipLaunchKernelGGL(value_side, dim3(2u * (unsigned)rows_padded), dim3(BW_THREADS), smem, stream, a, rows_padded);
     return check_hip(hipGetLastError(), "dfw_chunk_bwd_value_kernel launch");
 }
 
