@@ -224,6 +224,21 @@ int t2fw_lfw_backward_heads(const void *g_out, const void *g_state,
                             void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The forward of few rows of many steps with the chunks of 64 steps of a row side by side: as t2fw_lfw_forward_heads (H = 1:
+ * t2fw_lfw_forward), with `scratch`, device memory, 16-byte aligned, of t2fw_lfw_forward_scratch_bytes; not read across calls.
+ * The query (checkpoints: whether ckpt will be given) is 0 where the call is t2fw_lfw_forward_heads' own: other widths and types,
+ * any flag, checkpoints at another C than 64, and wherever the sequential kernel is the faster one.  The scratch may then be null.
+ */
+size_t t2fw_lfw_forward_scratch_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int64_t K, int32_t C,
+                                      int32_t dtype, int32_t flags, int32_t checkpoints);
+int t2fw_lfw_forward_scratch(const void *x, const void *f, const void *q, const void *k, const void *f_key,
+                             const void *s0, void *out, void *next_state, void *ckpt,
+                             int64_t B, int64_t T, int64_t H, int64_t D, int64_t K,
+                             int32_t C, int32_t dtype, int32_t flags,
+                             void *workspace, size_t workspace_bytes,
+                             void *scratch, size_t scratch_bytes, void *stream);
+
+/*
  * One generation step (T = 1) that may update the state in place
  * (next_state == s0 is allowed).  x,f,out [B,D]; q,k,f_key [B,K].
  */

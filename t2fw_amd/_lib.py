@@ -51,6 +51,8 @@ SIGNATURES = {
     "t2fw_lfw_backward": (ctypes.c_int, [_vp] * 15 + [_i64] * 4 + [_i32] * 3 + [_vp, _sz, _vp]),
     "t2fw_lfw_forward_heads": (ctypes.c_int, [_vp] * 9 + [_i64] * 5 + [_i32] * 3 + [_vp, _sz, _vp]),
     "t2fw_lfw_backward_heads": (ctypes.c_int, [_vp] * 15 + [_i64] * 5 + [_i32] * 3 + [_vp, _sz, _vp]),
+    "t2fw_lfw_forward_scratch_bytes": (_sz, [_i64] * 5 + [_i32] * 4),
+    "t2fw_lfw_forward_scratch": (ctypes.c_int, [_vp] * 9 + [_i64] * 5 + [_i32] * 3 + [_vp, _sz, _vp, _sz, _vp]),
     "t2fw_lfw_step": (ctypes.c_int, [_vp] * 8 + [_i64] * 3 + [_i32, _vp]),
     "t2fw_record_event": (ctypes.c_int, [_vp, _vp]),
     "t2fw_cast": (ctypes.c_int, [ctypes.POINTER(ctypes.c_void_p)] * 2 + [ctypes.POINTER(ctypes.c_int64), _i32, _i32, _i32, _vp]),

@@ -159,6 +159,35 @@ size_t forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32
     return 0;
 }
 
+// The chunk-parallel forward: per row and chunk of 64 tokens what it adds to the state (fp32), the state before it (bf16), gate
+// products and a flag; a verdict per row.
+int64_t par_fwd_chunks(int64_t T) { return (T + 63) / 64; }
+struct ParFwdScratch {
+    size_t states, vecs, chunk_flags, declined, total;       // byte offsets; the increments come first
+};
+ParFwdScratch par_fwd_scratch(int64_t B, int64_t T) {
+    const size_t items = (size_t)(B * par_fwd_chunks(T));
+    ParFwdScratch s;
+    s.states = items * (CH_N * CH_N * 4);
+    s.vecs = s.states + items * (CH_N * CH_N * 2);
+    s.chunk_flags = s.vecs + items * (PF_NVEC * CH_N * 4);
+    s.declined = s.chunk_flags + (items * 4 + 255) / 256 * 256;
+    s.total = s.declined + ((size_t)B * 4 + 255) / 256 * 256;
+    return s;
+}
+// Where it takes less time than the sequential kernel, whose time is 4 + 1.4 us per chunk of a row whatever the rows (up to 128);
+// the four launches here take about 20 us to issue and run, 10 + 0.02 per chunk + 0.1 per chunk of a row.  Sequential / chunks, us,
+// forwards one after the other: 4 x 512 14.8 / 21.1, 4 x 1024 25.8 / 21.1, 4 x 4096 92 / 25, 8 x 8192 178 / 44, 16 x 1024 26 / 19, 16 x 4096 92 / 36,
+// 32 x 1024 26 / 22, 32 x 4096 93 / 55, 48 x 1024 26.5 / 25.9, 48 x 2048 49 / 41, 64 x 1024 27 / 32, 64 x 4096 93 / 95, 96 x 1024 27 / 43.
+// With checkpoints a backward follows (8 + 0.035 per chunk), and where host time of about 170 us bounds the step, three more
+// launches lose 10 of it: only where the step's kernels take longer than that.
+bool par_fwd_faster(int64_t B, int64_t T, bool checkpoints) {
+    if (B < 1 || B > 56 || T >= CHUNK_MAX_T) return false;
+    const int64_t c = par_fwd_chunks(T);
+    if (c < 14 || B * c > PAR_FWD_MAX_ITEMS || (60 - B) * c < 310) return false;
+    return !checkpoints || (137 + 7 * B / 2) * c > 18000;
+}
+
 // Checkpoint intervals that are a multiple of 32 other than 32 and 64 (the forward takes them, the backward
 // kernels do not): the backward call first runs the forward kernel once more at an interval the backward takes,
 // into checkpoints of its own in the workspace, and then proceeds as for that interval.
@@ -293,7 +322,7 @@ int t2fw_lfw_flag_regions(int64_t B, int64_t T, int64_t D, int64_t K, int32_t C,
 static int lfw_forward_rows(const void *x, const void *f, const void *q, const void *k, const void *f_key,
                             const void *s0, void *out, void *next_state, void *ckpt, int64_t B, int64_t T,
                             int64_t heads, int64_t D, int64_t K, int32_t C, int32_t dtype, int32_t flags,
-                            void *workspace, size_t workspace_bytes, void *stream) {
+                            void *workspace, size_t workspace_bytes, void *stream, void *scratch = nullptr) {
     const size_t es = elem_size(dtype);
     if (es == 0) return fail(T2FW_ERR_BAD_DTYPE, "unknown dtype code %d", dtype);
     int rc = check_dims(B, T, D, K);
@@ -347,6 +376,22 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
         const int cus = compute_units();
         if (cus < 0) return fail(T2FW_ERR_HIP, "could not read the device's compute-unit count");
         const bool split = 2 * chunk_rows_padded(B) <= cus;
+        if (scratch != nullptr) {
+            const ParFwdScratch ps = par_fwd_scratch(B, T);
+            unsigned char *const at = static_cast<unsigned char *>(scratch);
+            ParFwdArgs t{};
+            t.x = x; t.f = f; t.q = q; t.k = k; t.f_key = f_key; t.s0 = s0;
+            t.out = out; t.next_state = next_state; t.ckpt = ckpt;
+            t.incr = reinterpret_cast<float *>(at);
+            t.states = reinterpret_cast<uint16_t *>(at + ps.states);
+            t.vecs = reinterpret_cast<float *>(at + ps.vecs);
+            t.chunk_flags = reinterpret_cast<int32_t *>(at + ps.chunk_flags);
+            t.declined = reinterpret_cast<int32_t *>(at + ps.declined);
+            t.row_flags = c.row_flags; t.par_hint = c.par_hint;
+            t.B = B; t.T = T; t.NC = par_fwd_chunks(T); t.heads = (int32_t)heads;
+            if ((rc = par_forward(t, dtype, st))) return rc;
+            c.row_select = t.declined;
+        }
         return chunk_forward(c, dtype, op, split, st);
     }
     if (xpar_ok(B, T, D, K, dtype, flags) && (ckpt == nullptr || C == XP_CHUNK) && T * heads < CHUNK_MAX_T) {
@@ -369,6 +414,29 @@ static int check_heads(int64_t B, int64_t H) {
     if (B < 0 || H < 1 || H > 65536) return fail(T2FW_ERR_BAD_SHAPE, "B=%lld must be non-negative and H=%lld in [1, 65536]", (long long)B, (long long)H);
     if ((long double)B * (long double)H > 4.0e18L) return fail(T2FW_ERR_BAD_SHAPE, "B*H is too large");
     return T2FW_OK;
+}
+
+size_t t2fw_lfw_forward_scratch_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int64_t K, int32_t C, int32_t dtype, int32_t flags,
+                                      int32_t checkpoints) {
+    if (B <= 0 || T <= 0 || H < 1 || H > 65536 || B > PAR_FWD_MAX_ITEMS || flags != 0 || (checkpoints && C != 64) ||
+        !chunk_shape_ok(D, K, dtype, flags) || T >= CHUNK_MAX_T || T * H >= CHUNK_MAX_T || !par_fwd_faster(B * H, T, checkpoints != 0))
+        return 0;
+    return par_fwd_scratch(B * H, T).total;
+}
+
+int t2fw_lfw_forward_scratch(const void *x, const void *f, const void *q, const void *k, const void *f_key, const void *s0, void *out,
+                             void *next_state, void *ckpt, int64_t B, int64_t T, int64_t H, int64_t D, int64_t K, int32_t C, int32_t dtype,
+                             int32_t flags, void *workspace, size_t workspace_bytes, void *scratch, size_t scratch_bytes, void *stream) {
+    int rc = check_heads(B, H);
+    if (rc) return rc;
+    const size_t need = t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt != nullptr);
+    if (need > 0 && aligned16({x, f, q, k, f_key, s0, out, next_state, ckpt})) {
+        if (scratch == nullptr || scratch_bytes < need)
+            return fail(T2FW_ERR_WORKSPACE, "scratch of %zu bytes needed, %zu given", need, scratch_bytes);
+        if (!aligned16({scratch})) return fail(T2FW_ERR_MISALIGNED, "the scratch must be 16-byte aligned");
+    }
+    return lfw_forward_rows(x, f, q, k, f_key, s0, out, next_state, ckpt, B * H, T, H, D, K, C, dtype, flags, workspace, workspace_bytes,
+                            stream, need > 0 ? scratch : nullptr);
 }
 
 int t2fw_lfw_forward(const void *x, const void *f, const void *q, const void *k, const void *f_key,

@@ -105,12 +105,18 @@ PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         ws = scratch.data_ptr();
     }
     void *const ck = ckpt.defined() ? ckpt.data_ptr() : nullptr;
+    const size_t extra = t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt.defined());
+    Tensor chunks;
+    if (extra > 0) chunks = bytes_like(x, (int64_t)extra);
     done(unlocked([&] {
         if (logits) {
             const int rc = t2fw_gate_forward(lf.data_ptr(), lk.data_ptr(), f.data_ptr(), fk.data_ptr(), lf.numel(), lk.numel(), dtype, stream);
             if (rc) return rc;
         }
-        const int rc = heads ? t2fw_lfw_forward_heads(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
+        const int rc = extra > 0 ? t2fw_lfw_forward_scratch(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
+                                                            out.data_ptr(), next.data_ptr(), ck, B, T, H, D, K, C, dtype, flags, ws, ws_bytes,
+                                                            chunks.data_ptr(), extra, stream)
+                     : heads ? t2fw_lfw_forward_heads(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
                                               out.data_ptr(), next.data_ptr(), ck, B, T, H, D, K, C, dtype, flags, ws, ws_bytes, stream)
                      : t2fw_lfw_forward(x.data_ptr(), f.data_ptr(), q.data_ptr(), k.data_ptr(), fk.data_ptr(), s.data_ptr(),
                                         out.data_ptr(), next.data_ptr(), ck, B, T, D, K, C, dtype, flags, ws, ws_bytes, stream);

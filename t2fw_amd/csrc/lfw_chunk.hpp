@@ -35,6 +35,7 @@ struct ChunkFwdArgs {
     int64_t B, T, NC;
     int32_t C;                         // checkpoint interval, multiple of 32
     int32_t heads;                     // 1: rows are [T, 64] slabs; H > 1: row b is head b % H of a [B / H, T, H, 64] tensor
+    const int32_t *row_select;         // null: every row; else only rows b with row_select[b] != 0 (the others' flags stand)
     // rows the chunked form cannot take are redone in place with the exact scan (0: only reported);
     // launch geometry of that scan for a 64 x 64 state (set by chunk_forward)
     int32_t redo, scan_kg, scan_tb, scan_ntiles;

@@ -525,11 +525,13 @@ __device__ __forceinline__ void fwd_redo_if_flagged(const ChunkFwdArgs &p, unsig
     }
 }
 
-template <typename IOE, typename OPE, bool HEADS>
+// SELECT: only the rows that p.row_select names (a template parameter, as the test alone costs a call without it 0.2 us)
+template <typename IOE, typename OPE, bool HEADS, bool SELECT>
 __global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int64_t b = blockIdx.x;
+    if (SELECT && p.row_select[b] == 0) return;
     // every wave executes exactly ceil(number of steps / 2) workgroup barriers
     if (tid < 256) {
         fwd_matrix_waves<IOE, OPE, HEADS>(p, smem, tid, b, 0, b, true);
@@ -549,13 +551,14 @@ __global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs
 // 8, so that the two halves of a row land on the same XCD and share its L2 for the key-side
 // inputs both of them read.  Each half reports flagged rows in a slot of its own (the value-side
 // gates it checks are its own 32 channels): row_flags[row] and row_flags[rows_padded + row].
-template <typename IOE, typename OPE, bool HEADS>
+template <typename IOE, typename OPE, bool HEADS, bool SELECT>
 __global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(ChunkFwdArgs p, int rows_padded) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
     const int64_t b = (int)blockIdx.x - half * rows_padded;
     if (b >= p.B) return;
+    if (SELECT && p.row_select[b] == 0) return;
     const int64_t slot = (int64_t)half * rows_padded + b;
     // waves: 0, 1 matrix; 2..5 key side (block, token half); 6, 7 value side (block; a lane takes
     // one of the half's 32 channels and one token half).  SIMD i runs waves i and i + 4.
@@ -572,24 +575,30 @@ __global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(Ch
     fwd_redo_if_flagged<IOE>(p, smem, tid, b, half * (p.scan_ntiles / 2), (half + 1) * (p.scan_ntiles / 2));
 }
 
-template <typename IOE, typename OPE, bool HEADS> int launch(const ChunkFwdArgs &a, bool split, hipStream_t stream) {
+template <typename IOE, typename OPE, bool HEADS, bool SELECT> int launch_rows(const ChunkFwdArgs &a, bool split, hipStream_t stream) {
     if (a.B > 0x1fffffffLL) return fail(T2FW_ERR_UNSUPPORTED, "B=%lld is too large", (long long)a.B);
     if (a.heads < 1 || a.T * a.heads >= CHUNK_MAX_T)
         return fail(T2FW_ERR_UNSUPPORTED, "T=%lld with %d heads is too long for 32-bit row offsets", (long long)a.T, a.heads);
     // more than 64 KB of dynamic LDS has to be enabled per function (and per device)
     if (split) {
-        auto kern = lfw_fwd_chunk_half_kernel<IOE, OPE, HEADS>;
+        auto kern = lfw_fwd_chunk_half_kernel<IOE, OPE, HEADS, SELECT>;
         int rc = enable_lds(reinterpret_cast<const void *>(kern), FWD_SMEM, "hipFuncSetAttribute(forward chunk kernel, two workgroups per row)");
         if (rc) return rc;
         const int rows_padded = (int)chunk_rows_padded(a.B);
         hipLaunchKernelGGL(kern, dim3(2u * (unsigned)rows_padded), dim3(FWD_THREADS_HALF), FWD_SMEM, stream, a, rows_padded);
         return check_hip(hipGetLastError(), "lfw_fwd_chunk_half_kernel launch");
     }
-    auto kern = lfw_fwd_chunk_kernel<IOE, OPE, HEADS>;
+    auto kern = lfw_fwd_chunk_kernel<IOE, OPE, HEADS, SELECT>;
     int rc = enable_lds(reinterpret_cast<const void *>(kern), FWD_SMEM, "hipFuncSetAttribute(forward chunk kernel)");
     if (rc) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)a.B), dim3(FWD_THREADS), FWD_SMEM, stream, a);
     return check_hip(hipGetLastError(), "lfw_fwd_chunk_kernel launch");
+}
+
+template <typename IOE, typename OPE, bool HEADS> int launch(const ChunkFwdArgs &a, bool split, hipStream_t stream) {
+    if constexpr (std::is_same<OPE, Bf16>::value)
+        if (a.row_select != nullptr) return launch_rows<IOE, OPE, HEADS, true>(a, split, stream);
+    return launch_rows<IOE, OPE, HEADS, false>(a, split, stream);
 }
 
 }  // namespace

@@ -57,6 +57,23 @@ struct ParBwdArgs {
 
 int par_backward(const ParBwdArgs &a, int dtype, hipStream_t stream);
 
+// Forward, three launches (lfw_par_fwd.hip); the rows that it leaves in `declined` are the caller's to redo.
+constexpr int PF_NVEC = 4;             // per (row, chunk): totA, totB, refA, refB, [64] floats each
+constexpr int64_t PAR_FWD_MAX_ITEMS = 16384;       // rows x chunks: 420 MB of scratch
+struct ParFwdArgs {
+    const void *x, *f, *q, *k, *f_key, *s0;
+    void *out, *next_state, *ckpt;     // ckpt may be null, else at intervals of 64
+    float *incr;                       // scratch [B, NC, 64, 64]: what a chunk adds to the state
+    uint16_t *states;                  // scratch [B, NC, 64, 64] bf16: the state before it, scaled to its middle
+    float *vecs;                       // scratch [B, NC, PF_NVEC, 64]
+    int32_t *chunk_flags;              // scratch [B * NC]
+    int32_t *declined;                 // scratch [B]: 1 for rows whose results are not valid
+    int32_t *row_flags, *par_hint;     // as in ChunkFwdArgs: cleared
+    int64_t B, T, NC;                  // NC: chunks of 64
+    int32_t heads;                     // as in ChunkFwdArgs
+};
+int par_forward(const ParFwdArgs &a, int dtype, hipStream_t stream);
+
 #if defined(__HIPCC__)
 namespace par {
 
@@ -207,12 +224,12 @@ __device__ __forceinline__ void load_tokens(RawTokens<NT> &r, const u16 *ubase, 
 // what the sweeps produce (lfw_par_bwd.hip), with an absolute error of fp32 rounding (2^-24) of the
 // terms that cancel in it, and d_gate = that / gate with the floored gate is then good to 2^-12 of those
 // terms.  (d_gate at a step does not depend on the step's own gate, so the floored gate gives the right
-// value.)
-template <typename IOE, int NT, bool FULL, bool MID>
+// value.)  The forward asks for its own floor, 2^-24.
+template <typename IOE, int NT, bool FULL, bool MID, u16 FLOOR = IOE::BWD_FLOOR_BITS>
 __device__ __forceinline__ void gate_scan(LaneChunk<NT> &lc, float (&gate)[NT][4], const RawTokens<NT> &raw, int kg,
                                           int n_left) {
     us2 mx = {0, 0};
-    const us2 floor_bits = {IOE::BWD_FLOOR_BITS, IOE::BWD_FLOOR_BITS};
+    const us2 floor_bits = {FLOOR, FLOOR};
 #pragma unroll
     for (int m = 0; m < NT; ++m)
 #pragma unroll
@@ -223,7 +240,7 @@ __device__ __forceinline__ void gate_scan(LaneChunk<NT> &lc, float (&gate)[NT][4
                 if (!(16 * m + 2 * jj + 1 < n_left)) bits.y = IOE::ONE_BITS;
             }
             mx = __builtin_elementwise_max(mx, bits);      // > bits(1.0): above one, negative, NaN
-            bits = __builtin_elementwise_max(bits, floor_bits);      // gates in [0, 2^-12) count as 2^-12
+            bits = __builtin_elementwise_max(bits, floor_bits);      // gates in [0, floor) count as the floor
             gate[m][2 * jj] = IOE::to_f32(bits.x);
             gate[m][2 * jj + 1] = IOE::to_f32(bits.y);
         }
@@ -296,13 +313,13 @@ template <int NT> __device__ __forceinline__ void store_cm(u16 *tile, int c, int
 // MFMA result tile (rows 4 kg + j, column i) -> 16-bit A/B operand of a 16-deep contraction over its
 // rows, keeping rows < column (LOWER: strictly below the diagonal of the transposed tile, i.e.
 // row index < column index) or rows > column, or everything
-enum { KEEP_ALL = 0, KEEP_ROW_LT_COL = 1, KEEP_ROW_GT_COL = 2 };
+enum { KEEP_ALL = 0, KEEP_ROW_LT_COL = 1, KEEP_ROW_GT_COL = 2, KEEP_ROW_LE_COL = 3 };
 template <int KEEP> __device__ __forceinline__ uint2 mask_pack(const floatx4 &t, int i, int kg) {
     float v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int row = 4 * kg + j;
-        const bool keep = KEEP == KEEP_ALL || (KEEP == KEEP_ROW_LT_COL ? row < i : row > i);
+        const bool keep = KEEP == KEEP_ALL || (KEEP == KEEP_ROW_LT_COL ? row < i : KEEP == KEEP_ROW_LE_COL ? row <= i : row > i);
         v[j] = keep ? t[j] : 0.0f;
     }
     return packq<Bf16>(v[0], v[1], v[2], v[3]);
