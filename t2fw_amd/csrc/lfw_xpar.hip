@@ -10,7 +10,7 @@
 //      matrix instructions.
 //   2  lfw_xpar_chain_kernel, elementwise: the chain over the chunks of a row; leaves the state at the START (the adjoint
 //      at the END) of every chunk in fp32 in place of the increments and writes the checkpoints (64 x 64 fp32: those only,
-//      19 -> 16 us, where the call has them).
+//      19 -> 16 us, where the call has them).  Small calls do without it (chain_in_place).
 //   3  lfw_xpar_fwd_kernel / lfw_xpar_bwd_kernel: the recurrence itself, step by step, within each chunk; the last chunk's
 //      leaves the final state, the first one's d_s0.  64 x 64 fp32 (lfw_xpar64.hip): on fp64 matrix instructions where the
 //      gates and values allow it, and one more launch for the chunks where they don't.
@@ -24,7 +24,7 @@
 // The workgroups of the row's first chunk (64 x 64 fp32: of the first four) do it in launch 3, the others of that row leave.
 //
 // B = 96, T = 1024, 64 x 64 fp32 (launch 3 in lfw_xpar64.hip): forward 31 + 16 + 54 + 4 us (220 per-step), backward 26 + 11 +
-// 154 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16: 6 + 5 + 14 us (76) and 6 + 4 + 33 us (251).
+// 154 + 6 us (813).  13 rows, T = 385, 33 x 17 fp16, without launch 2: 6 + 20 us (76) and 6 + 38 us (251).
 //
 // Replaces lfw_cuda_fwd_kernel, lfw_cuda_bwd_kernel and the einsums of the reference
 // (t2fw/csrc/lfw_kernel.cu:18-102, t2fw/csrc/lfw.cpp:45,84-93); semantics t2fw/torch.py:21-31.
@@ -211,18 +211,62 @@ template <typename IO, bool BWD> __global__ __launch_bounds__(XC_THREADS) void l
     if (threadIdx.x == 0) p.ws.row_flags[blockIdx.x] = any;
 }
 
+// Small calls without launch 2: every workgroup of launch 3 goes through its row's whole chain itself, all elements of the state in
+// the same order (the verdict on a row is on all of them), and keeps the state at its own chunk's edge in LDS, [Dp][Kp] floats.
+// The row's verdict.  What bounds it: one memory latency per batch of a thread's element (chain_is_in_place).  Three elements
+// at a time were no faster (33 x 17: 72 us in the place of 71), with the gate products in LDS slower (75).
+template <typename IO, bool BWD>
+__device__ __forceinline__ bool chain_in_place(const XparScratch &ws, const void *first, int D, int K, int NC, int64_t b, int chunk, float *edge) {
+    const int Dp = xp_padded(D), Kp = xp_padded(K), tid = threadIdx.x;
+    int bad = 0;
+    for (int c = tid; c < NC; c += SCAN_THREADS) bad |= ws.chunk_flags[b * NC + c] & XP_ROW_LEFT;
+    const float *const st = ws.states + b * NC * (int64_t)(Dp * Kp), *const tots = ws.tots + b * NC * (int64_t)(Dp + Kp);
+    for (int o = tid; o < Dp * Kp; o += SCAN_THREADS) {
+        const int d = o / Kp, k = o - d * Kp;
+        if (d >= D || k >= K) continue;
+        float S = to_acc(((const IO *)first)[(b * D + d) * K + k]);
+        bad |= !(fabsf(S) <= XP_MAX_STATE) ? 1 : 0;
+        for (int n0 = 0; n0 < NC; n0 += XC_BATCH) {
+            float m[XC_BATCH], ta[XC_BATCH], tb[XC_BATCH];
+#pragma unroll
+            for (int u = 0; u < XC_BATCH; ++u) {
+                const int n = min(n0 + u, NC - 1), c = BWD ? NC - 1 - n : n;
+                m[u] = st[c * (Dp * Kp) + o];
+                ta[u] = tots[c * (Dp + Kp) + d];
+                tb[u] = tots[c * (Dp + Kp) + Dp + k];
+            }
+#pragma unroll
+            for (int u = 0; u < XC_BATCH; ++u) {
+                if (n0 + u >= NC) break;
+                if ((BWD ? NC - 1 - (n0 + u) : n0 + u) == chunk) edge[o] = S;
+                S = S * (ta[u] * tb[u]) + m[u];
+                bad |= fabsf(S) <= XP_MAX_STATE ? 0 : 1;
+            }
+        }
+    }
+    return __syncthreads_or(bad) != 0;
+}
+
 // ---- launch 3 -------------------------------------------------------------------------------------
+// IN_PLACE: without launch 2 (chain_in_place; the state lies behind the body's LDS, `edge` bytes from its start).
 // Workgroups are numbered chunk by chunk, all rows of a chunk together, so that those that may have a whole row to do come
 // first and next to each other.  Numbered row by row, the ones with work were 16 chunks apart, all on the same one or two
 // dies and shader engines: 96 rows x 1024 steps with a gate above one in each, 32 x 32 fp32, forward + backward 2050 us
 // against 563 now and 752 on the per-step kernels; 64 x 64 7300, 1019, 992 (96 x 256 590, 277, 264; 16 x 1024 1430, 604,
 // 909).
 // One workgroup per (row, chunk, 16 value channels); base: the call over whole rows.
-template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_fwd_kernel(ScanFwdArgs base, XparScratch ws, int64_t NC) {
+template <typename IO, int KPL, bool IN_PLACE> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_fwd_kernel(ScanFwdArgs base, XparScratch ws, int64_t NC, int edge) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    float *const entering = reinterpret_cast<float *>(smem_raw + edge);
     const int64_t pair = blockIdx.x / base.ntiles, b = pair % base.B;
     const int tile = (int)(blockIdx.x - pair * base.ntiles), chunk = (int)(pair / base.B);
     const int64_t item = b * NC + chunk;
-    if (row_left(ws, b)) {
+    bool left;
+    if constexpr (IN_PLACE)
+        left = chain_in_place<IO, false>(ws, base.s0, (int)base.D, (int)base.K, (int)NC, b, chunk, entering);
+    else
+        left = row_left(ws, b);
+    if (left) {
         if (chunk == 0) scan::fwd_scan_body_kg<IO, KPL, 16>(base, b, tile);
         return;
     }
@@ -232,23 +276,37 @@ template <typename IO, int KPL> __global__ __launch_bounds__(SCAN_THREADS) void 
     a.q = (const IO *)base.q + line * base.K; a.k = (const IO *)base.k + line * base.K;
     a.f_key = (const IO *)base.f_key + line * base.K;
     a.out = (IO *)base.out + line * base.D;
+    if constexpr (IN_PLACE) {
+        if (base.ckpt != nullptr) {
+            const int D = (int)base.D, K = (int)base.K, rows = min(16, D - 16 * tile);
+            IO *const to = (IO *)base.ckpt + (item * D + 16 * tile) * K;
+            for (int o = threadIdx.x; o < rows * K; o += SCAN_THREADS) to[o] = from_acc<IO>(entering[(16 * tile + o / K) * xp_padded(K) + o % K]);
+        }
+    }
     a.ckpt = nullptr;
     a.next_state = chunk == (int)NC - 1 ? (IO *)base.next_state + b * base.D * base.K : nullptr;
     a.s_stride = xp_padded(base.K);
-    a.s_start = ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
+    a.s_start = IN_PLACE ? entering : ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
     a.T = min((int64_t)XP_CHUNK, base.T - (int64_t)chunk * XP_CHUNK);
     scan::fwd_scan_body_kg<IO, KPL, 16>(a, 0, tile);
 }
 
 // One workgroup per (row, chunk, 16 channels of one side); KV, KK: columns per lane on the value and on the key side.
-template <typename IO, int KV, int KK> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_bwd_kernel(ScanBwdArgs base, XparScratch ws) {
+template <typename IO, int KV, int KK, bool IN_PLACE> __global__ __launch_bounds__(SCAN_THREADS) void lfw_xpar_bwd_kernel(ScanBwdArgs base, XparScratch ws, int edge) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    float *const entering = reinterpret_cast<float *>(smem_raw + edge);
     const int nd = ((int)base.D + 15) / 16, per = nd + ((int)base.K + 15) / 16;
     const int64_t pair = blockIdx.x / per, b = pair % base.B;
     const int tile = (int)(blockIdx.x - pair * per), chunk = (int)(pair / base.B);
     const int64_t item = b * base.NC + chunk;
     ScanBwdArgs a = base;
     int64_t row = b;
-    if (row_left(ws, b)) {
+    bool left;
+    if constexpr (IN_PLACE)
+        left = chain_in_place<IO, true>(ws, base.g_state, (int)base.D, (int)base.K, (int)base.NC, b, chunk, entering);
+    else
+        left = row_left(ws, b);
+    if (left) {
         if (chunk != 0) return;
     } else {
         const int64_t line = row_first_token(b, base.T, base.heads) + (int64_t)chunk * XP_CHUNK * base.heads;
@@ -262,7 +320,7 @@ template <typename IO, int KV, int KK> __global__ __launch_bounds__(SCAN_THREADS
         a.d_f_key = (IO *)base.d_f_key + line * base.K;
         a.d_s0 = chunk == 0 ? (IO *)base.d_s0 + b * base.D * base.K : nullptr;
         a.g_stride = xp_padded(base.K);
-        a.g_end = ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
+        a.g_end = IN_PLACE ? entering : ws.states + item * (xp_padded(base.D) * xp_padded(base.K));
         a.T = min((int64_t)XP_CHUNK, base.T - (int64_t)chunk * XP_CHUNK);
         a.NC = 1;
         row = 0;
@@ -273,10 +331,21 @@ template <typename IO, int KV, int KK> __global__ __launch_bounds__(SCAN_THREADS
         scan::bwd_scan_body_kg<IO, KV, 1, 16, 1>(a, row, tile - nd);
 }
 
-template <typename IO, bool BWD> int entering_states(const PassArgs &p, int64_t B, hipStream_t stream) {
+// Whether `tiles` workgroups per (row, chunk) go through the chain themselves: few batches of loads per thread, and not too much
+// to read in all.  GPU time of forward + backward, fp16, with launch 2 / in place, us: 1 x 230 of 9 x 5 57 / 52, 16 x 1024 of
+// 16 x 8 66 / 57, 64 x 512 of 16 x 16 73 / 66, 13 x 385 of 33 x 17 (six batches) 69 / 71, beyond the line 16 x 512 of 63 x 32 (eight) 77 / 81.
+// The host issues two launches fewer of six, which is what bounds such a step: 16 x 700 of 16 x 8 157 / 146, 16 x 300 of 20 x 10
+// 156 / 148, 13 x 385 of 33 x 17 158 / 146.
+constexpr int64_t XC_IN_PLACE_READS = 5 << 20;             // floats
+bool chain_is_in_place(int64_t B, int64_t NC, int D, int K, int tiles) {
+    const int64_t state = (int64_t)xp_padded(D) * xp_padded(K);
+    return state / SCAN_THREADS * ((NC + XC_BATCH - 1) / XC_BATCH) <= 6 && B * NC * tiles <= XC_IN_PLACE_READS / (NC * state);
+}
+
+template <typename IO, bool BWD> int entering_states(const PassArgs &p, int64_t B, bool in_place, hipStream_t stream) {
     hipLaunchKernelGGL((lfw_xpar_incr_kernel<IO, BWD>), dim3((unsigned)(B * p.NC)), dim3(XI_THREADS), 0, stream, p);
     const int rc = check_hip(hipGetLastError(), "lfw_xpar_incr_kernel launch");
-    if (rc) return rc;
+    if (rc || in_place) return rc;
     hipLaunchKernelGGL((lfw_xpar_chain_kernel<IO, BWD>), dim3((unsigned)(4 * B)), dim3(XC_THREADS), 0, stream, p);
     return check_hip(hipGetLastError(), "lfw_xpar_chain_kernel launch");
 }
@@ -286,9 +355,11 @@ template <typename IO> int forward(const XparFwdArgs &a, hipStream_t stream) {
     p.val = a.x; p.gate_val = a.f; p.key = a.k; p.gate_key = a.f_key;
     p.first = a.s0; p.ckpt = a.ckpt;
     p.ws = a.ws; p.T = a.T; p.NC = a.NC; p.D = a.D; p.K = a.K; p.heads = a.heads;
-    const int rc = entering_states<IO, false>(p, a.B, stream);
+    const bool own = std::is_same<IO, float>::value && a.D == XP_N && a.K == XP_N;      // kernels of its own, which read the chain's results
+    const bool in_place = !own && chain_is_in_place(a.B, a.NC, a.D, a.K, (a.D + 15) / 16);
+    const int rc = entering_states<IO, false>(p, a.B, in_place, stream);
     if (rc) return rc;
-    if (std::is_same<IO, float>::value && a.D == XP_N && a.K == XP_N) return xpar64_forward(a, stream);
+    if (own) return xpar64_forward(a, stream);
     const int kpl = a.K <= 32 ? 2 : 4, tb = 32;
     ScanFwdArgs s{};
     s.x = a.x; s.f = a.f; s.q = a.q; s.k = a.k; s.f_key = a.f_key; s.s0 = a.s0;
@@ -296,11 +367,10 @@ template <typename IO> int forward(const XparFwdArgs &a, hipStream_t stream) {
     s.B = a.B; s.T = a.T; s.D = a.D; s.K = a.K; s.NC = a.ckpt != nullptr ? a.NC : 1;
     s.C = a.ckpt != nullptr ? XP_CHUNK : 1; s.kg = 16; s.tb = tb; s.ntiles = (a.D + 15) / 16; s.heads = a.heads;
     const dim3 grid((unsigned)(a.B * a.NC * s.ntiles));
-    const size_t smem = scan_fwd_lds_bytes(tb, 16, kpl, 16);
-    if (kpl == 2)
-        hipLaunchKernelGGL((lfw_xpar_fwd_kernel<IO, 2>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws, a.NC);
-    else
-        hipLaunchKernelGGL((lfw_xpar_fwd_kernel<IO, 4>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws, a.NC);
+    const size_t body = (scan_fwd_lds_bytes(tb, 16, kpl, 16) + 15) / 16 * 16, smem = body + (in_place ? 4 * xp_padded(a.D) * xp_padded(a.K) : 0);
+    auto kern = in_place ? (kpl == 2 ? lfw_xpar_fwd_kernel<IO, 2, true> : lfw_xpar_fwd_kernel<IO, 4, true>)
+                         : (kpl == 2 ? lfw_xpar_fwd_kernel<IO, 2, false> : lfw_xpar_fwd_kernel<IO, 4, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(SCAN_THREADS), smem, stream, s, a.ws, a.NC, (int)body);
     return check_hip(hipGetLastError(), "lfw_xpar_fwd_kernel launch");
 }
 
@@ -309,24 +379,26 @@ template <typename IO> int backward(const XparBwdArgs &a, hipStream_t stream) {
     p.val = a.g_out; p.gate_val = a.f; p.key = a.q; p.gate_key = a.f_key;
     p.first = a.g_state;
     p.ws = a.ws; p.T = a.T; p.NC = a.NC; p.D = a.D; p.K = a.K; p.heads = a.heads;
-    const int rc = entering_states<IO, true>(p, a.B, stream);
+    const bool own = std::is_same<IO, float>::value && a.D == XP_N && a.K == XP_N;
+    const bool in_place = !own && chain_is_in_place(a.B, a.NC, a.D, a.K, (a.D + 15) / 16 + (a.K + 15) / 16);
+    const int rc = entering_states<IO, true>(p, a.B, in_place, stream);
     if (rc) return rc;
-    if (std::is_same<IO, float>::value && a.D == XP_N && a.K == XP_N) return xpar64_backward(a, stream);
+    if (own) return xpar64_backward(a, stream);
     ScanBwdArgs s{};
     s.g_out = a.g_out; s.g_state = a.g_state; s.x = a.x; s.f = a.f; s.q = a.q; s.k = a.k; s.f_key = a.f_key; s.ckpt = a.ckpt;
     s.d_x = a.d_x; s.d_f = a.d_f; s.d_q = a.d_q; s.d_k = a.d_k; s.d_f_key = a.d_f_key; s.d_s0 = a.d_s0;
     s.B = a.B; s.T = a.T; s.D = a.D; s.K = a.K; s.NC = a.NC; s.C = XP_CHUNK; s.kg = 16; s.use_sub = 1; s.heads = a.heads;
     const dim3 grid((unsigned)(a.B * a.NC * ((a.D + 15) / 16 + (a.K + 15) / 16)));
     const int kv = a.D <= 32 ? 2 : 4, kk = a.K <= 32 ? 2 : 4;
-    const size_t smem = scan_bwd_lds_bytes(scan::SegLen<4>::value, 16, kv > kk ? kv : kk, 16, XP_CHUNK, true);
-    if (kv == 4 && kk == 4)
-        hipLaunchKernelGGL((lfw_xpar_bwd_kernel<IO, 4, 4>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws);
-    else if (kv == 4)
-        hipLaunchKernelGGL((lfw_xpar_bwd_kernel<IO, 4, 2>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws);
-    else if (kk == 4)
-        hipLaunchKernelGGL((lfw_xpar_bwd_kernel<IO, 2, 4>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws);
-    else
-        hipLaunchKernelGGL((lfw_xpar_bwd_kernel<IO, 2, 2>), grid, dim3(SCAN_THREADS), smem, stream, s, a.ws);
+    const size_t body = (scan_bwd_lds_bytes(scan::SegLen<4>::value, 16, kv > kk ? kv : kk, 16, XP_CHUNK, true) + 15) / 16 * 16;
+    const size_t smem = body + (in_place ? 4 * xp_padded(a.D) * xp_padded(a.K) : 0);
+    auto pick = [&](auto flag) {
+        constexpr bool IN = decltype(flag)::value;
+        return kv == 4 ? (kk == 4 ? lfw_xpar_bwd_kernel<IO, 4, 4, IN> : lfw_xpar_bwd_kernel<IO, 4, 2, IN>)
+                       : (kk == 4 ? lfw_xpar_bwd_kernel<IO, 2, 4, IN> : lfw_xpar_bwd_kernel<IO, 2, 2, IN>);
+    };
+    auto kern = in_place ? pick(std::true_type{}) : pick(std::false_type{});
+    hipLaunchKernelGGL(kern, grid, dim3(SCAN_THREADS), smem, stream, s, a.ws, (int)body);
     return check_hip(hipGetLastError(), "lfw_xpar_bwd_kernel launch");
 }
 
