@@ -390,7 +390,7 @@ static int lfw_forward_rows(const void *x, const void *f, const void *q, const v
             t.row_flags = c.row_flags; t.par_hint = c.par_hint;
             t.B = B; t.T = T; t.NC = par_fwd_chunks(T); t.heads = (int32_t)heads;
             if ((rc = par_forward(t, dtype, st))) return rc;
-            c.row_select = t.declined;
+            return chunk_forward(c, dtype, op, split, st, t.declined);
         }
         return chunk_forward(c, dtype, op, split, st);
     }

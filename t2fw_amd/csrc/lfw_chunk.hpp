@@ -35,7 +35,6 @@ struct ChunkFwdArgs {
     int64_t B, T, NC;
     int32_t C;                         // checkpoint interval, multiple of 32
     int32_t heads;                     // 1: rows are [T, 64] slabs; H > 1: row b is head b % H of a [B / H, T, H, 64] tensor
-    const int32_t *row_select;         // null: every row; else only rows b with row_select[b] != 0 (the others' flags stand)
     // rows the chunked form cannot take are redone in place with the exact scan (0: only reported);
     // launch geometry of that scan for a 64 x 64 state (set by chunk_forward)
     int32_t redo, scan_kg, scan_tb, scan_ntiles;
@@ -59,7 +58,8 @@ struct ChunkBwdArgs {
 __host__ __device__ inline int64_t chunk_rows_padded(int64_t B) { return (B + 7) / 8 * 8; }
 
 // op: 0 = bf16 operands, 1 = fp16 operands (fp16 I/O only); split: two workgroups per batch row
-int chunk_forward(const ChunkFwdArgs &a, int dtype, int op, bool split, hipStream_t stream);
+// row_select: null for every row, else (bf16 operands) only rows b with row_select[b] != 0; the others' flags stand
+int chunk_forward(const ChunkFwdArgs &a, int dtype, int op, bool split, hipStream_t stream, const int32_t *row_select = nullptr);
 // two workgroups per batch row (one per side of the state)
 int chunk_backward(const ChunkBwdArgs &a, int dtype, int op, hipStream_t stream);
 constexpr int64_t CHUNK_MAX_T = 1 << 24;      // the kernels address a batch row with 32-bit offsets: T * heads must stay below this

@@ -525,13 +525,14 @@ __device__ __forceinline__ void fwd_redo_if_flagged(const ChunkFwdArgs &p, unsig
     }
 }
 
-// SELECT: only the rows that p.row_select names (a template parameter, as the test alone costs a call without it 0.2 us)
+// SELECT: only the rows that row_select names.  (A parameter of the template and the last of the kernel: as a test at run time, or as
+// a field of the arguments, it cost every call 0.2 to 0.4 us of 26.5.)
 template <typename IOE, typename OPE, bool HEADS, bool SELECT>
-__global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs p) {
+__global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs p, const int32_t *row_select) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int64_t b = blockIdx.x;
-    if (SELECT && p.row_select[b] == 0) return;
+    if (SELECT && row_select[b] == 0) return;
     // every wave executes exactly ceil(number of steps / 2) workgroup barriers
     if (tid < 256) {
         fwd_matrix_waves<IOE, OPE, HEADS>(p, smem, tid, b, 0, b, true);
@@ -552,13 +553,13 @@ __global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs
 // inputs both of them read.  Each half reports flagged rows in a slot of its own (the value-side
 // gates it checks are its own 32 channels): row_flags[row] and row_flags[rows_padded + row].
 template <typename IOE, typename OPE, bool HEADS, bool SELECT>
-__global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(ChunkFwdArgs p, int rows_padded) {
+__global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(ChunkFwdArgs p, int rows_padded, const int32_t *row_select) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
     const int64_t b = (int)blockIdx.x - half * rows_padded;
     if (b >= p.B) return;
-    if (SELECT && p.row_select[b] == 0) return;
+    if (SELECT && row_select[b] == 0) return;
     const int64_t slot = (int64_t)half * rows_padded + b;
     // waves: 0, 1 matrix; 2..5 key side (block, token half); 6, 7 value side (block; a lane takes
     // one of the half's 32 channels and one token half).  SIMD i runs waves i and i + 4.
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(Ch
     fwd_redo_if_flagged<IOE>(p, smem, tid, b, half * (p.scan_ntiles / 2), (half + 1) * (p.scan_ntiles / 2));
 }
 
-template <typename IOE, typename OPE, bool HEADS, bool SELECT> int launch_rows(const ChunkFwdArgs &a, bool split, hipStream_t stream) {
+template <typename IOE, typename OPE, bool HEADS, bool SELECT> int launch_rows(const ChunkFwdArgs &a, bool split, hipStream_t stream, const int32_t *row_select) {
     if (a.B > 0x1fffffffLL) return fail(T2FW_ERR_UNSUPPORTED, "B=%lld is too large", (long long)a.B);
     if (a.heads < 1 || a.T * a.heads >= CHUNK_MAX_T)
         return fail(T2FW_ERR_UNSUPPORTED, "T=%lld with %d heads is too long for 32-bit row offsets", (long long)a.T, a.heads);
@@ -585,25 +586,25 @@ template <typename IOE, typename OPE, bool HEADS, bool SELECT> int launch_rows(c
         int rc = enable_lds(reinterpret_cast<const void *>(kern), FWD_SMEM, "hipFuncSetAttribute(forward chunk kernel, two workgroups per row)");
         if (rc) return rc;
         const int rows_padded = (int)chunk_rows_padded(a.B);
-        hipLaunchKernelGGL(kern, dim3(2u * (unsigned)rows_padded), dim3(FWD_THREADS_HALF), FWD_SMEM, stream, a, rows_padded);
+        hipLaunchKernelGGL(kern, dim3(2u * (unsigned)rows_padded), dim3(FWD_THREADS_HALF), FWD_SMEM, stream, a, rows_padded, row_select);
         return check_hip(hipGetLastError(), "lfw_fwd_chunk_half_kernel launch");
     }
     auto kern = lfw_fwd_chunk_kernel<IOE, OPE, HEADS, SELECT>;
     int rc = enable_lds(reinterpret_cast<const void *>(kern), FWD_SMEM, "hipFuncSetAttribute(forward chunk kernel)");
     if (rc) return rc;
-    hipLaunchKernelGGL(kern, dim3((unsigned)a.B), dim3(FWD_THREADS), FWD_SMEM, stream, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)a.B), dim3(FWD_THREADS), FWD_SMEM, stream, a, row_select);
     return check_hip(hipGetLastError(), "lfw_fwd_chunk_kernel launch");
 }
 
-template <typename IOE, typename OPE, bool HEADS> int launch(const ChunkFwdArgs &a, bool split, hipStream_t stream) {
+template <typename IOE, typename OPE, bool HEADS> int launch(const ChunkFwdArgs &a, bool split, hipStream_t stream, const int32_t *row_select) {
     if constexpr (std::is_same<OPE, Bf16>::value)
-        if (a.row_select != nullptr) return launch_rows<IOE, OPE, HEADS, true>(a, split, stream);
-    return launch_rows<IOE, OPE, HEADS, false>(a, split, stream);
+        if (row_select != nullptr) return launch_rows<IOE, OPE, HEADS, true>(a, split, stream, row_select);
+    return launch_rows<IOE, OPE, HEADS, false>(a, split, stream, nullptr);
 }
 
 }  // namespace
 
-int chunk_forward(const ChunkFwdArgs &args, int dtype, int op, bool split, hipStream_t stream) {
+int chunk_forward(const ChunkFwdArgs &args, int dtype, int op, bool split, hipStream_t stream, const int32_t *row_select) {
     ChunkFwdArgs a = args;
     {   // geometry of the exact scan for a 64 x 64 state, as lfw_scan.hip chooses it
         const ScanGeom g = scan_geometry(CH_N);
@@ -623,12 +624,12 @@ int chunk_forward(const ChunkFwdArgs &args, int dtype, int op, bool split, hipSt
     }
     if (a.heads == 1) {
         if (dtype == T2FW_F16)
-            return op == 1 ? launch<Fp16, Fp16, false>(a, split, stream) : launch<Fp16, Bf16, false>(a, split, stream);
-        if (dtype == T2FW_BF16) return launch<Bf16, Bf16, false>(a, split, stream);
+            return op == 1 ? launch<Fp16, Fp16, false>(a, split, stream, row_select) : launch<Fp16, Bf16, false>(a, split, stream, row_select);
+        if (dtype == T2FW_BF16) return launch<Bf16, Bf16, false>(a, split, stream, row_select);
     } else {
         if (dtype == T2FW_F16)
-            return op == 1 ? launch<Fp16, Fp16, true>(a, split, stream) : launch<Fp16, Bf16, true>(a, split, stream);
-        if (dtype == T2FW_BF16) return launch<Bf16, Bf16, true>(a, split, stream);
+            return op == 1 ? launch<Fp16, Fp16, true>(a, split, stream, row_select) : launch<Fp16, Bf16, true>(a, split, stream, row_select);
+        if (dtype == T2FW_BF16) return launch<Bf16, Bf16, true>(a, split, stream, row_select);
     }
     return fail(T2FW_ERR_UNSUPPORTED, "the chunked kernels take fp16 or bf16 tensors");
 }
