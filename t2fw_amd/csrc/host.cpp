@@ -91,7 +91,13 @@ PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     arguments(n, 16);
     const Tensor &x = tensor(a[0]), &q = tensor(a[2]), &k = tensor(a[3]), &s = tensor(a[5]);
     const bool heads = a[6] == Py_True, logits = a[14] == Py_True;
-    const Tensor &lf = tensor(a[1]), &lk = tensor(a[4]), f = logits ? empty_like(a[1]) : lf, fk = logits ? empty_like(a[4]) : lk;
+    const Tensor &lf = tensor(a[1]), &lk = tensor(a[4]);
+    Tensor made_f, made_fk;
+    if (logits) {
+        made_f = empty_like(a[1]);
+        made_fk = empty_like(a[4]);
+    }
+    const Tensor &f = logits ? made_f : lf, &fk = logits ? made_fk : lk;
     void *const event = address(a[15]);
     const int64_t nc = integer(a[7]), ws_bytes = integer(a[12]);
     const int32_t C = (int32_t)integer(a[8]), dtype = (int32_t)integer(a[9]), flags = (int32_t)integer(a[10]);

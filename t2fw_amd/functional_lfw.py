@@ -60,10 +60,13 @@ def _host_hints_enabled():
     return os.environ.get("T2FW_HOST_HINTS", "1") != "0" and not torch.are_deterministic_algorithms_enabled()
 
 
+_AS_IT_IS = contextlib.nullcontext()      # may be entered any number of times, by any thread
+
+
 def _on_device(dev):
     """Make ``dev`` current for the allocations and the launch, without the cost of switching when it already is."""
     if dev.index is None or dev.index == torch.cuda.current_device():      # (host memory has no index)
-        return contextlib.nullcontext()
+        return _AS_IT_IS
     return torch.cuda.device(dev)
 
 
@@ -279,7 +282,8 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
     None, checkpoint interval, flags, hints): ``hints`` is None, or the forward's verdict on which backward
     path the gates allow, readable from the host once the forward has run (path_hint.py).  logits=True: ``forget`` and
     ``f_key`` are gate logits, and the gates follow what is returned."""
-    dims = _lib.host().lfw_shape(value, forget, query, key, f_key, state, heads) if _lib.loaded() else None
+    host = _lib.host() if _lib.loaded() else None
+    dims = host.lfw_shape(value, forget, query, key, f_key, state, heads) if host is not None else None
     B, T, H, D, K = dims if dims is not None else _checked_shape(value, forget, query, key, f_key, state, heads)
     code = _dtype_code(value.dtype)
     flags = _flags()
@@ -289,7 +293,8 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
             forget, f_key = sigmoid_gates(forget, f_key)
         res = _lfw_forward_blocked(value, forget, query, key, f_key, state, need_grad, blocks)
         return (*res, forget, f_key) if logits else res
-    host = _lib.host()
+    if host is None:
+        host = _lib.host()
     C = _ckpt_interval()
     dev = value.device
     flags, nc, ws_bytes, _, regions = _forward_plan(B * H, T, D, K, C, value.dtype, flags, need_grad)
@@ -300,12 +305,13 @@ def _lfw_forward(value, forget, query, key, f_key, state, need_grad, heads=False
             # a backward on the matrix cores will follow: the workspace goes to pinned host memory
             hints = ForwardHints(dev, ws_bytes, regions[2], regions[3], B * H)
             ws_address, event = hints.workspace()[0].value, hints.event()
-        outputs, next_state, ckpt, *gates = host.lfw_forward(value, forget, query, key, f_key, state, heads, nc if need_grad else -1, C, code,
-                                                             flags, ws_address, ws_bytes, _lib.current_stream(dev), logits, event)
+        res = host.lfw_forward(value, forget, query, key, f_key, state, heads, nc if need_grad else -1, C, code, flags, ws_address, ws_bytes,
+                               _lib.current_stream(dev), logits, event)
         if hints is not None:
             hints.launched()
     if logits:
-        return outputs, next_state, ckpt, C, flags, hints, *gates
+        return *res[:3], C, flags, hints, *res[3:]
+    outputs, next_state, ckpt = res
     return outputs, next_state, ckpt, C, flags, hints
 
 
