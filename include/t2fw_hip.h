@@ -81,10 +81,11 @@ extern "C" {
                                      what it cannot take); the caller reads the flags
                                      from the workspace (nonzero = that row's results are not
                                      valid; t2fw_lfw_flag_regions says where they are) and redoes
-                                     those rows with T2FW_FLAG_FORCE_SCAN, or knows its gates are in
-                                     range: a forward call whose hints (below) are all zero proves
-                                     that for the backward call on the same gates.  Saves the
-                                     backward's extra launch.                                     */
+                                     those rows with T2FW_FLAG_FORCE_SCAN, or knows its gates and
+                                     values are in range: a forward call whose hints (below) are all
+                                     zero proves that of the gates, and finite fp16 values always are
+                                     (bf16 values may not be: a row whose results are not finite is
+                                     flagged too).  Saves the backward's extra launch.            */
 
 #define T2FW_FLAG_BLOCKWISE 8     /* matrix-core path, backward: the block-wise kernel (16-step blocks in one
                                      pass per batch row; takes 16-step gate products down to 2^-100)
@@ -130,9 +131,11 @@ size_t t2fw_lfw_forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t
  *   [0],[1]  forward verdicts: nonzero = the matrix-core form could not take the row (it has been redone
  *            exactly unless T2FW_FLAG_NO_FIXUP was given);
  *   [2],[3]  forward hints for the backward call on the same gates: all zero = the chunk-parallel
- *            backward will flag no row, so that call may be given T2FW_FLAG_NO_FIXUP; many nonzero =
- *            most rows would be declined and redone, and T2FW_FLAG_BLOCKWISE is the faster path
- *            (a gate outside [0, 1] or a 16-step gate product below 2^-40 sets a row's hint);
+ *            backward will flag no row for its gates, so that call on finite fp16 tensors may be given
+ *            T2FW_FLAG_NO_FIXUP; many nonzero = most rows would be declined and redone, and
+ *            T2FW_FLAG_BLOCKWISE is the faster path (a gate outside [0, 1] or a 16-step gate product below
+ *            2^-40 sets a row's hint; t2fw_lfw_forward_scratch: only in rows that have a gate outside
+ *            [0, 1], a product below 2^-80 over the 32 steps of half a chunk, or a result that is not finite);
  *   [4],[5]  backward verdicts, as [0],[1].
  * A region a path does not write has zero entries (exact kernels: all three).  The workspace may be
  * any memory the GPU can write, pinned host memory included: a caller that wants to steer the

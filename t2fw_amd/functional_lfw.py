@@ -335,7 +335,7 @@ def _lfw_backward(grad_output, grad_state, value, forget, query, key, f_key, sta
     host = _lib.host()
     dev = value.device
     if hints is not None:
-        flags = choose_backward_flags(flags, hints.hinted_rows(), B * H)
+        flags = choose_backward_flags(flags, hints.hinted_rows(), B * H, value.dtype == torch.float16)
     ws_bytes = _sizes(B * H, T, D, K, C, code, flags)[2]
     with _on_device(dev):
         grads, args, ws = host.lfw_backward_arguments(grad_output, grad_state, value, forget, query, key, f_key, state, ckpt, heads,

@@ -9,13 +9,17 @@ The forward call already looks at every gate; it leaves one hint per batch row i
 hints as soon as the forward call has completed on the GPU, which in a training step is long before
 the backward call is issued, and pick the backward's flags without any synchronisation:
 
-  * no row hinted          -> T2FW_FLAG_NO_FIXUP (the extra launch is skipped; no row can be flagged)
+  * no row hinted          -> float16 tensors: T2FW_FLAG_NO_FIXUP (the extra launch is skipped: the gates give no row
+    reason to be declined, and finite float16 values are too small for an intermediate to leave the range of
+    its type).  bfloat16 tensors keep it: the hints are about the gates alone, and the kernels also decline a row
+    for a result that is not finite, which values of a size that bfloat16 holds can bring about with any gates.
   * enough rows hinted     -> T2FW_FLAG_BLOCKWISE (see ``choose_backward_flags``)
   * hints not there yet, or the stream is being captured into a graph -> the default call, which
     decides everything on the device.
 
 The three are equally accurate but not equal to the bit where rows are hinted, so which bits a training step
-gives then depends on the host's pace.  T2FW_HOST_HINTS=0 and torch.use_deterministic_algorithms(True) leave
+gives then depends on the host's pace; and without the extra launch an infinity or a NaN among float16 tensors
+reaches the results of the whole chunk around it.  T2FW_HOST_HINTS=0 and torch.use_deterministic_algorithms(True) leave
 the choice to the device.
 
 The reference has a single path (t2fw/csrc/lfw.cpp:50-96); this module has no counterpart there.
@@ -40,15 +44,16 @@ def _rounds(rows):
     return -(-rows // BLOCKWISE_ROWS_PER_ROUND)
 
 
-def choose_backward_flags(flags, hinted_rows, rows):
+def choose_backward_flags(flags, hinted_rows, rows, small_values=True):
     """Flags for the backward call, given the caller's ``flags``, the number of rows the forward call
-    hinted (None: unknown) and the number of batch rows.  Pure function of its arguments."""
+    hinted (None: unknown), the number of batch rows and whether the tensors' type keeps values small enough for
+    the gates to be the only reason to decline a row (float16).  Pure function of its arguments."""
     if hinted_rows is None or rows <= 0:
         return flags
     if flags & (_lib.FLAG_FORCE_SCAN | _lib.FLAG_FP16_OPERANDS | _lib.FLAG_BLOCKWISE | _lib.FLAG_NO_FIXUP):
         return flags                                   # the caller chose a path
     if hinted_rows == 0:
-        return flags | _lib.FLAG_NO_FIXUP
+        return flags | _lib.FLAG_NO_FIXUP if small_values else flags
     chunk_parallel = PAR_US_PER_ROW * rows + BLOCKWISE_US_PER_ROUND * _rounds(hinted_rows)
     blockwise = BLOCKWISE_US_PER_ROUND * _rounds(rows)
     return flags | _lib.FLAG_BLOCKWISE if blockwise <= chunk_parallel else flags
