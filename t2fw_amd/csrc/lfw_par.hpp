@@ -58,13 +58,13 @@ struct ParBwdArgs {
 int par_backward(const ParBwdArgs &a, int dtype, hipStream_t stream);
 
 // Forward, three launches (lfw_par_fwd.hip); the rows that it leaves in `declined` are the caller's to redo.
-constexpr int PF_NVEC = 4;             // per (row, chunk): totA, totB, refA, refB, [64] floats each
+constexpr int PF_NVEC = 4;             // per (row, chunk): totA, totB, refB, [64] floats each (1 KB apart)
 constexpr int64_t PAR_FWD_MAX_ITEMS = 16384;       // rows x chunks: 420 MB of scratch
 struct ParFwdArgs {
     const void *x, *f, *q, *k, *f_key, *s0;
     void *out, *next_state, *ckpt;     // ckpt may be null, else at intervals of 64
     float *incr;                       // scratch [B, NC, 64, 64]: what a chunk adds to the state
-    uint16_t *states;                  // scratch [B, NC, 64, 64] bf16: the state before it, scaled to its middle
+    uint16_t *states;                  // scratch [B, NC, 64, 64] bf16: the state before it, scaled to its middle on the key side
     float *vecs;                       // scratch [B, NC, PF_NVEC, 64]
     int32_t *chunk_flags;              // scratch [B * NC]
     int32_t *declined;                 // scratch [B]: 1 for rows whose results are not valid
@@ -225,7 +225,11 @@ __device__ __forceinline__ void load_tokens(RawTokens<NT> &r, const u16 *ubase, 
 // terms that cancel in it, and d_gate = that / gate with the floored gate is then good to 2^-12 of those
 // terms.  (d_gate at a step does not depend on the step's own gate, so the floored gate gives the right
 // value.)  The forward asks for its own floor, 2^-24.
-template <typename IOE, int NT, bool FULL, bool MID, u16 FLOOR = IOE::BWD_FLOOR_BITS>
+//
+// POW2 (with MID): the origin is pow2_below(ref) instead of ref, so that what is scaled to it, the state above all, is scaled
+// without a rounding.
+__device__ __forceinline__ float pow2_below(float v) { return __uint_as_float(__float_as_uint(v) & 0x7f800000u); }
+template <typename IOE, int NT, bool FULL, bool MID, u16 FLOOR = IOE::BWD_FLOOR_BITS, bool POW2 = false>
 __device__ __forceinline__ void gate_scan(LaneChunk<NT> &lc, float (&gate)[NT][4], const RawTokens<NT> &raw, int kg,
                                           int n_left) {
     us2 mx = {0, 0};
@@ -256,7 +260,7 @@ __device__ __forceinline__ void gate_scan(LaneChunk<NT> &lc, float (&gate)[NT][4
         carry *= s.all;
         if (m == NT / 2 - 1) {
             lc.ref = carry;
-            if (MID) carry = 1.0f;
+            if (MID) carry = POW2 ? carry * __uint_as_float(0x7f000000u - __float_as_uint(pow2_below(carry))) : 1.0f;
         }
         if (m >= NT / 2) second *= s.all;
 #pragma unroll
@@ -265,7 +269,7 @@ __device__ __forceinline__ void gate_scan(LaneChunk<NT> &lc, float (&gate)[NT][4
     lc.tot = MID ? lc.ref * second : carry;
     lc.sfx = second;
     if (MID) {
-        const float r = __builtin_amdgcn_rcpf(lc.ref);
+        const float r = POW2 ? __uint_as_float(0x7f000000u - __float_as_uint(pow2_below(lc.ref))) : __builtin_amdgcn_rcpf(lc.ref);
 #pragma unroll
         for (int m = 0; m < NT / 2; ++m) {
             lc.off[m] *= r;
@@ -304,6 +308,17 @@ __device__ __forceinline__ void scale_pack(uint2 (&p)[NT], const float (&v)[NT][
         p[m] = packq<Bf16>(v[m][0] * s[m][0], v[m][1] * s[m][1], v[m][2] * s[m][2], v[m][3] * s[m][3]);
 }
 
+// ... and what that rounded off, packed in the same way
+__device__ __forceinline__ uint2 pack_rest(const uint2 &hi, float a, float b, float c, float d) {
+    return packq<Bf16>(a - Bf16::to_f32((u16)(hi.x & 0xffffu)), b - Bf16::to_f32((u16)(hi.x >> 16)), c - Bf16::to_f32((u16)(hi.y & 0xffffu)),
+                       d - Bf16::to_f32((u16)(hi.y >> 16)));
+}
+template <int NT>
+__device__ __forceinline__ void scale_pack_rest(uint2 (&p)[NT], const uint2 (&hi)[NT], const float (&v)[NT][4], const float (&s)[NT][4]) {
+#pragma unroll
+    for (int m = 0; m < NT; ++m) p[m] = pack_rest(hi[m], v[m][0] * s[m][0], v[m][1] * s[m][1], v[m][2] * s[m][2], v[m][3] * s[m][3]);
+}
+
 // the lane's packed tokens -> its channel's row of a channel-major tile
 template <int NT> __device__ __forceinline__ void store_cm(u16 *tile, int c, int kg, const uint2 (&p)[NT]) {
 #pragma unroll
@@ -314,14 +329,18 @@ template <int NT> __device__ __forceinline__ void store_cm(u16 *tile, int c, int
 // rows, keeping rows < column (LOWER: strictly below the diagonal of the transposed tile, i.e.
 // row index < column index) or rows > column, or everything
 enum { KEEP_ALL = 0, KEEP_ROW_LT_COL = 1, KEEP_ROW_GT_COL = 2, KEEP_ROW_LE_COL = 3 };
-template <int KEEP> __device__ __forceinline__ uint2 mask_pack(const floatx4 &t, int i, int kg) {
-    float v[4];
+template <int KEEP> __device__ __forceinline__ floatx4 mask(const floatx4 &t, int i, int kg) {
+    floatx4 v;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int row = 4 * kg + j;
         const bool keep = KEEP == KEEP_ALL || (KEEP == KEEP_ROW_LT_COL ? row < i : KEEP == KEEP_ROW_LE_COL ? row <= i : row > i);
         v[j] = keep ? t[j] : 0.0f;
     }
+    return v;
+}
+template <int KEEP> __device__ __forceinline__ uint2 mask_pack(const floatx4 &t, int i, int kg) {
+    const floatx4 v = mask<KEEP>(t, i, kg);
     return packq<Bf16>(v[0], v[1], v[2], v[3]);
 }
 
