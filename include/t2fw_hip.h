@@ -231,6 +231,7 @@ int t2fw_lfw_backward_heads(const void *g_out, const void *g_state,
  * t2fw_lfw_forward), with `scratch`, device memory, 16-byte aligned, of t2fw_lfw_forward_scratch_bytes; not read across calls.
  * The query (checkpoints: whether ckpt will be given) is 0 where the call is t2fw_lfw_forward_heads' own: other widths and types,
  * any flag, checkpoints at another C than 64, and wherever the sequential kernel is the faster one.  The scratch may then be null.
+ * No result may overlap an input: rows that the form cannot take are done again from the inputs.
  */
 size_t t2fw_lfw_forward_scratch_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int64_t K, int32_t C,
                                       int32_t dtype, int32_t flags, int32_t checkpoints);

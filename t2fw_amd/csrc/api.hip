@@ -160,7 +160,7 @@ size_t forward_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t K, int32
 }
 
 // The chunk-parallel forward: per row and chunk of 64 tokens what it adds to the state (fp32), the state before it (bf16), gate
-// products and a flag; a verdict per row.
+// products and a flag; two verdicts per row.
 int64_t par_fwd_chunks(int64_t T) { return (T + 63) / 64; }
 struct ParFwdScratch {
     size_t states, vecs, chunk_flags, declined, total;       // byte offsets; the increments come first
@@ -172,7 +172,7 @@ ParFwdScratch par_fwd_scratch(int64_t B, int64_t T) {
     s.vecs = s.states + items * (CH_N * CH_N * 2);
     s.chunk_flags = s.vecs + items * (PF_NVEC * CH_N * 4);
     s.declined = s.chunk_flags + (items * 4 + 255) / 256 * 256;
-    s.total = s.declined + ((size_t)B * 4 + 255) / 256 * 256;
+    s.total = s.declined + ((size_t)B * 8 + 255) / 256 * 256;
     return s;
 }
 // Where it takes less time than the sequential kernel, whose time is 4 + 1.4 us per chunk of a row whatever the rows (up to 128);

@@ -58,7 +58,7 @@ struct ChunkBwdArgs {
 __host__ __device__ inline int64_t chunk_rows_padded(int64_t B) { return (B + 7) / 8 * 8; }
 
 // op: 0 = bf16 operands, 1 = fp16 operands (fp16 I/O only); split: two workgroups per batch row
-// row_select: null for every row, else (bf16 operands) only rows b with row_select[b] != 0; the others' flags stand
+// row_select: null for every row, else (bf16 operands) only rows b with row_select[b] or row_select[B + b] != 0; the others' flags stand
 int chunk_forward(const ChunkFwdArgs &a, int dtype, int op, bool split, hipStream_t stream, const int32_t *row_select = nullptr);
 // two workgroups per batch row (one per side of the state)
 int chunk_backward(const ChunkBwdArgs &a, int dtype, int op, hipStream_t stream);

@@ -532,7 +532,7 @@ __global__ __launch_bounds__(FWD_THREADS) void lfw_fwd_chunk_kernel(ChunkFwdArgs
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int64_t b = blockIdx.x;
-    if (SELECT && row_select[b] == 0) return;
+    if (SELECT && (row_select[b] | row_select[p.B + b]) == 0) return;
     // every wave executes exactly ceil(number of steps / 2) workgroup barriers
     if (tid < 256) {
         fwd_matrix_waves<IOE, OPE, HEADS>(p, smem, tid, b, 0, b, true);
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(FWD_THREADS_HALF) void lfw_fwd_chunk_half_kernel(Ch
     const int half = (int)blockIdx.x >= rows_padded ? 1 : 0;
     const int64_t b = (int)blockIdx.x - half * rows_padded;
     if (b >= p.B) return;
-    if (SELECT && row_select[b] == 0) return;
+    if (SELECT && (row_select[b] | row_select[p.B + b]) == 0) return;
     const int64_t slot = (int64_t)half * rows_padded + b;
     // waves: 0, 1 matrix; 2..5 key side (block, token half); 6, 7 value side (block; a lane takes
     // one of the half's 32 channels and one token half).  SIMD i runs waves i and i + 4.

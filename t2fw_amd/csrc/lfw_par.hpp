@@ -67,7 +67,8 @@ struct ParFwdArgs {
     uint16_t *states;                  // scratch [B, NC, 64, 64] bf16: the state before it, scaled to its middle on the key side
     float *vecs;                       // scratch [B, NC, PF_NVEC, 64]
     int32_t *chunk_flags;              // scratch [B * NC]
-    int32_t *declined;                 // scratch [B]: 1 for rows whose results are not valid
+    int32_t *declined;                 // scratch [2, B]: 1 for rows whose results are not valid, by the gates and states (launches 1, 2)
+                                       // and by the outputs (launch 3, which reads the former)
     int32_t *row_flags, *par_hint;     // as in ChunkFwdArgs: cleared
     int64_t B, T, NC;                  // NC: chunks of 64
     int32_t heads;                     // as in ChunkFwdArgs

@@ -104,7 +104,7 @@ template <typename IOE, bool HEADS> __global__ __launch_bounds__(PAR_THREADS) vo
     const int any_bad = __syncthreads_or((int)lc.bad);
     if (tid == 0) {
         p.chunk_flags[item] = any_bad ? 1 : 0;
-        if (chunk == 0) p.declined[b] = 0;
+        if (chunk == 0) p.declined[b] = p.declined[p.B + b] = 0;
     }
     // this wave's two tiles of the increment: rows d = 16 db + 4 kg + j, column k = 16 kb + i
     const u16 *const XH = reinterpret_cast<const u16 *>(smem), *const KH = reinterpret_cast<const u16 *>(smem + CM_BYTES),
@@ -252,7 +252,7 @@ template <typename IOE, bool HEADS, bool FULL> __device__ __forceinline__ void o
         store_cm<NT>(QS, c, kg, qs);
     }
     *reinterpret_cast<uint4 *>(S0 + (tid >> 3) * CMS + (tid & 7) * 8) = state;
-    if (__builtin_amdgcn_readfirstlane(declined)) return;          // uniform over the workgroup
+    if (__builtin_amdgcn_readfirstlane(declined)) return;          // uniform over the workgroup: nothing in this launch writes it
     __syncthreads();
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     // tile (m, n), n <= m, of P at m (m + 1) / 2 + n: element [t = 16 m + i][s = 16 n + 4 kg + j] in lane (i, kg), s <= t
@@ -293,7 +293,7 @@ template <typename IOE, bool HEADS, bool FULL> __device__ __forceinline__ void o
             }
         }
     }
-    if (!(chk == 0.0f)) p.declined[b] = 1;
+    if (!(chk == 0.0f)) p.declined[p.B + b] = 1;
 }
 
 template <typename IOE, bool HEADS> __global__ __launch_bounds__(PAR_THREADS, 4) void lfw_par_fwd_out_kernel(ParFwdArgs p) {
