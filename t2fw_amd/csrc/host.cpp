@@ -111,9 +111,15 @@ PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         ws = scratch.data_ptr();
     }
     void *const ck = ckpt.defined() ? ckpt.data_ptr() : nullptr;
-    const size_t extra = t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt.defined());
+    size_t extra = t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt.defined());
     Tensor chunks;
-    if (extra > 0) chunks = bytes_like(x, (int64_t)extra);
+    if (extra > 0) {
+        try {
+            chunks = bytes_like(x, (int64_t)extra);
+        } catch (const c10::OutOfMemoryError &) {        // up to 420 MB, which the sequential kernel does without
+            extra = 0;
+        }
+    }
     done(unlocked([&] {
         if (logits) {
             const int rc = t2fw_gate_forward(lf.data_ptr(), lk.data_ptr(), f.data_ptr(), fk.data_ptr(), lf.numel(), lk.numel(), dtype, stream);
