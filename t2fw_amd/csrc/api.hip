@@ -179,8 +179,10 @@ ParFwdScratch par_fwd_scratch(int64_t B, int64_t T) {
 // the four launches here take about 20 us to issue and run, 10 + 0.02 per chunk + 0.1 per chunk of a row.  Sequential / chunks, us,
 // forwards one after the other: 4 x 512 14.8 / 21.1, 4 x 1024 25.8 / 21.1, 4 x 4096 92 / 25, 8 x 8192 178 / 44, 16 x 1024 26 / 19, 16 x 4096 92 / 36,
 // 32 x 1024 26 / 22, 32 x 4096 93 / 55, 48 x 1024 26.5 / 25.9, 48 x 2048 49 / 41, 64 x 1024 27 / 32, 64 x 4096 93 / 95, 96 x 1024 27 / 43.
-// With checkpoints a backward follows (8 + 0.035 per chunk), and where host time of about 170 us bounds the step, three more
-// launches lose 10 of it: only where the step's kernels take longer than that.
+// With checkpoints a backward follows (8 + 0.035 per chunk), and where the host bounds the step, at about 160 us, the allocation and
+// three more launches only cost: 8 x 1024 to 32 x 2048 153..157 -> 156..162 us one after the other, 178..181 -> 204..211 each by
+// itself.  So there only where the step's kernels take longer than that (32 x 4096 170 -> 158).  The line is the host's: replayed from
+// a graph, or on a faster host, shorter steps would gain too (16 x 1024 7 us of the forward).
 bool par_fwd_faster(int64_t B, int64_t T, bool checkpoints) {
     if (B < 1 || B > 56 || T >= CHUNK_MAX_T) return false;
     const int64_t c = par_fwd_chunks(T);

@@ -111,7 +111,8 @@ PyObject *lfw_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         ws = scratch.data_ptr();
     }
     void *const ck = ckpt.defined() ? ckpt.data_ptr() : nullptr;
-    size_t extra = t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt.defined());
+    // whether the chunks of a row run side by side depends on the call (its rows, with or without gradients), and the bits with it
+    size_t extra = at::globalContext().deterministicAlgorithms() ? 0 : t2fw_lfw_forward_scratch_bytes(B, T, H, D, K, C, dtype, flags, ckpt.defined());
     Tensor chunks;
     if (extra > 0) {
         try {

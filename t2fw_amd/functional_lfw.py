@@ -351,7 +351,12 @@ class LFWFunction(torch.autograd.Function):
     fp16 / bf16 tensors with D = K = 64 run on the matrix-core kernels, those whose widths are other multiples
     of 64 as independent 64 x 64 blocks on the same kernels (``_block_counts`` above), everything else on the
     exact kernels (per-step, or with the chunks of a row side by side: ``_exact_chunk_flags``); T2FW_FLAGS=1 keeps
-    the per-step kernels for every shape."""
+    the per-step kernels for every shape.
+
+    Which kernels run depends on the whole call: the number of rows and steps, and whether gradients are wanted.  The
+    results of a row are then equal to rounding and not to the bit, for instance the first pass of activation
+    checkpointing, which has no gradients, and its recomputation, which does.  torch.use_deterministic_algorithms(True) keeps
+    the forward of 16-bit 64 x 64 states (and of blocks of them) on one kernel, whose bits depend on the row alone."""
 
     @staticmethod
     def forward(ctx, value, forget, query, key, f_key, state):
