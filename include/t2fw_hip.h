@@ -256,8 +256,9 @@ int t2fw_lfw_step(const void *x, const void *f, const void *q, const void *k,
  * s0,final_state,g_state,d_s0 [B,D,M].  Replaces dfw.cpp:27-39 / :41-64.
  * D = M = 64 with fp32, fp16 or bf16 tensors and 16-byte aligned pointers runs on the matrix cores in blocks of
  * 16 steps (flags: T2FW_FLAG_BF16_OPERANDS above); everything else, or T2FW_FLAG_FORCE_SCAN, the exact
- * per-step kernels.  The backward keeps states in the memory of d_q and d_k until it writes the results there:
- * they must not overlap any other array of the call.
+ * per-step kernels.  The backward keeps states in the memory of d_q and d_k until it writes the results there; where
+ * those overlap another array of the call a slower form runs, as far as the overlap allows a result (d_q in the place of q
+ * and d_k in that of k do).
  */
 int t2fw_dfw_forward(const void *q, const void *k, const void *v, const void *s0,
                      void *out, void *final_state, void *delta,

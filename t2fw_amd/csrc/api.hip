@@ -666,6 +666,19 @@ int t2fw_dfw_forward(const void *q, const void *k, const void *v, const void *s0
     return dfw_forward(a, dtype, st);
 }
 
+// Gives the key side's chunks the memory of d_q and d_k for their edges, unless a caller has put other arrays there: what is
+// still read then would be overwritten, and the key side runs as one sequential pass.
+static void dfw_edges_in_results(DfwBwdArgs &a, size_t es, int32_t flags) {
+    if (!dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0)) return;
+    const int64_t key = a.B * a.T * CH_N * (int64_t)es, value = key, state = a.B * CH_N * CH_N * (int64_t)es;
+    for (void *d : {a.d_q, a.d_k})
+        if (meets_any({d, key}, {{a.g_out, value}, {a.g_state, state}, {a.q, key}, {a.k, key}, {a.delta, value}, {a.final_state, state},
+                                 {a.d_v, value}, {a.d_s0, state}, {d == a.d_q ? a.d_k : a.d_q, key}}))
+            return;
+    a.states = a.d_q;
+    a.adjoints = a.d_k;
+}
+
 int t2fw_dfw_backward(const void *g_out, const void *g_state, const void *q, const void *k, const void *delta,
                       const void *final_state, void *d_q, void *d_k, void *d_v, void *d_s0, int64_t B, int64_t T,
                       int64_t D, int64_t M, int32_t dtype, int32_t flags, void *stream) {
@@ -694,10 +707,7 @@ int t2fw_dfw_backward(const void *g_out, const void *g_state, const void *q, con
     a.B = B; a.T = T; a.D = D; a.M = M; a.blocks = 1;
     if (dfw_chunk_ok(D, M, dtype, flags) && T * CH_N < 0x7fffffffLL &&
         aligned16({g_out, g_state, q, k, delta, final_state, d_q, d_k, d_v, d_s0})) {
-        if (dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0)) {
-            a.states = d_q;
-            a.adjoints = d_k;
-        }
+        dfw_edges_in_results(a, es, flags);
         return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, st);
     }
     return dfw_backward(a, dtype, st);
@@ -746,10 +756,7 @@ int t2fw_dfw_backward_blocks(const void *g_out, const void *g_state, const void 
     a.g_out = g_out; a.g_state = g_state; a.q = q; a.k = k; a.delta = delta; a.final_state = final_state;
     a.d_q = d_q; a.d_k = d_k; a.d_v = d_v; a.d_s0 = d_s0;
     a.B = B * blocks; a.T = T; a.D = D; a.M = M; a.blocks = blocks;
-    if (blocks == 1 && dfw_key_chunks_ok(es, (flags & T2FW_FLAG_BF16_OPERANDS) == 0)) {
-        a.states = d_q;
-        a.adjoints = d_k;
-    }
+    if (blocks == 1) dfw_edges_in_results(a, es, flags);
     return dfw_chunk_backward(a, dtype, (flags & T2FW_FLAG_BF16_OPERANDS) == 0, static_cast<hipStream_t>(stream));
 }
 

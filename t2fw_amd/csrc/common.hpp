@@ -9,6 +9,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/t2fw_hip.h"
 
@@ -22,6 +23,21 @@ int check_hip(hipError_t e, const char *what);
 // Allows `kernel` to be launched with up to `bytes` of dynamic LDS (more than 64 KB has to be enabled per
 // function and device); the runtime is asked once per (kernel, device).
 int enable_lds(const void *kernel, int bytes, const char *what);
+
+// Arrays of a call that a caller may have put in one place, where a form of the kernels needs them apart
+struct Span {
+    const void *at;
+    int64_t bytes;
+    bool meets(const Span &o) const {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(at), b = reinterpret_cast<uintptr_t>(o.at);
+        return at != nullptr && o.at != nullptr && a < b + (uintptr_t)o.bytes && b < a + (uintptr_t)bytes;
+    }
+};
+inline bool meets_any(const Span &first, std::initializer_list<Span> others) {
+    for (const Span &o : others)
+        if (first.meets(o)) return true;
+    return false;
+}
 
 // ----------------------------------------------------------------------------------
 // layout of the [.., T, .., width] tensors: batch rows are either contiguous [T, width] slabs

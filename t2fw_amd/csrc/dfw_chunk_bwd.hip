@@ -12,8 +12,8 @@
 //               with Tm, Bq and K'' = Tm^T K prepared ahead by the matrix waves.
 //               Two more waves walk the state backwards, and both leave what the key side's chunks start from.
 //   key side    reads d_value and writes d_query and d_key, a workgroup per chunk of 64 tokens (dfw_key.hip).  Where an edge
-//               of a chunk does not fit the chunk's results (16-bit tensors with split operands), and for the shares of
-//               several value blocks (t2fw_dfw_backward_blocks), the sequential form below: one workgroup per (row,
+//               of a chunk does not fit the chunk's results (16-bit tensors with split operands) or a caller has put other arrays
+//               in their place, and for the shares of several value blocks (t2fw_dfw_backward_blocks), the sequential form below: one workgroup per (row,
 //               half of the key channels), columns of S and of G in fp32 accumulators, both plain running sums.
 #include <type_traits>
 #include "common.hpp"
@@ -505,7 +505,7 @@ template <bool SP, typename E, bool BLOCKS> static int launch_backward(const Dfw
     if constexpr (CHUNKS)
         if (a.states) return launch_value_side<SP, E, BLOCKS, true>(a, stream);
     if constexpr (CHUNKS && !BLOCKS) {
-        return fail(T2FW_ERR_UNSUPPORTED, "the key side runs in chunks for this type");       // not reached: d_q and d_k take the edges
+        return launch_backward<SP, E, true>(a, stream);          // rare: the form for several blocks serves one
     } else {
         if (a.states) return fail(T2FW_ERR_UNSUPPORTED, "16-bit tensors with split operands have no chunks of the key side");
         int rc = launch_value_side<SP, E, BLOCKS, false>(a, stream);

@@ -342,22 +342,6 @@ bool chain_is_in_place(int64_t B, int64_t NC, int D, int K, int tiles) {
     return state / SCAN_THREADS * ((NC + XC_BATCH - 1) / XC_BATCH) <= 6 && B * NC * tiles <= XC_IN_PLACE_READS / (NC * state);
 }
 
-// Without launch 2 every workgroup of launch 3 reads the state (adjoint) that the row starts from, while others write results: those
-// must not lie where it does (next_state in the place of s0, d_s0 in that of g_state).
-struct Span {
-    const void *at;
-    int64_t bytes;
-    bool meets(const Span &o) const {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(at), b = reinterpret_cast<uintptr_t>(o.at);
-        return at != nullptr && o.at != nullptr && a < b + (uintptr_t)o.bytes && b < a + (uintptr_t)bytes;
-    }
-};
-bool meets_any(const Span &first, std::initializer_list<Span> results) {
-    for (const Span &r : results)
-        if (first.meets(r)) return true;
-    return false;
-}
-
 template <typename IO, bool BWD> int entering_states(const PassArgs &p, int64_t B, bool in_place, hipStream_t stream) {
     hipLaunchKernelGGL((lfw_xpar_incr_kernel<IO, BWD>), dim3((unsigned)(B * p.NC)), dim3(XI_THREADS), 0, stream, p);
     const int rc = check_hip(hipGetLastError(), "lfw_xpar_incr_kernel launch");
@@ -372,6 +356,8 @@ template <typename IO> int forward(const XparFwdArgs &a, hipStream_t stream) {
     p.first = a.s0; p.ckpt = a.ckpt;
     p.ws = a.ws; p.T = a.T; p.NC = a.NC; p.D = a.D; p.K = a.K; p.heads = a.heads;
     const bool own = std::is_same<IO, float>::value && a.D == XP_N && a.K == XP_N;      // kernels of its own, which read the chain's results
+    // without launch 2 every workgroup of launch 3 reads the state that the row starts from while others write results, which must
+    // not lie where it does (next_state in the place of s0); the same for the adjoint in the backward
     const int64_t es = sizeof(IO), state = a.B * a.D * a.K * es;
     const bool in_place = !own && chain_is_in_place(a.B, a.NC, a.D, a.K, (a.D + 15) / 16) &&
                           !meets_any({a.s0, state}, {{a.next_state, state}, {a.out, a.B * a.T * a.D * es}, {a.ckpt, state * a.NC}});
