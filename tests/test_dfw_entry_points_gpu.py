@@ -62,3 +62,28 @@ def test_shares_and_sums_of_several_value_blocks(dtype, flags, B, T, n):
     for name, g, r in zip(NAMES, sums, refs):
         assert_close(g, r, dtype, name, tol=tol)
     assert torch.equal(sums[2], grads[2]) and torch.equal(sums[3], grads[3])
+
+
+@pytest.mark.parametrize("dtype,flags", [m for m in MODES if m[0] == torch.float32 or m[1]])
+def test_error_of_the_sums_against_that_of_the_shares(dtype, flags):
+    """d_query and d_key against float64: the key side's chunks (the sums) no worse than its sequential form (the shares, rounded each
+    and added up), where operands are single bf16 numbers as well; 1 % is what the two scatter by, in either direction"""
+    from t2fw_amd import _lib
+    from t2fw_amd.functional_dfw import DFWFunction
+    lib, P, code, (B, T, n) = _lib.load(), _lib.ptr, _lib.DTYPE_CODE[dtype], (24, 777, 2)
+    D = 64 * n
+    q, k, v, s, go, gs = [t.cuda() for t in make_inputs(B, T, D, 64, dtype, seed=6)]
+    st = _lib.current_stream_handle(v.device)
+    out, delta, fin = torch.empty_like(v), torch.empty_like(v), torch.empty_like(s)
+    _lib.check(lib.t2fw_dfw_forward_blocks(P(q), P(k), P(v), P(s), P(out), P(fin), P(delta), B, T, D, 64, code, flags, st))
+    shares = [q.new_empty((B, n, T, 64)), q.new_empty((B, n, T, 64)), torch.empty_like(v), torch.empty_like(s)]
+    _lib.check(lib.t2fw_dfw_backward_blocks(P(go), P(gs), P(q), P(k), P(delta), P(fin), *[P(t) for t in shares], B, T, D, 64, code, flags, st))
+    size = lib.t2fw_dfw_backward_sums_workspace_bytes(B, T, D, 64, code, flags)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    sums = [torch.empty_like(t) for t in (q, k, v, s)]
+    _lib.check(lib.t2fw_dfw_backward_sums(P(go), P(gs), P(q), P(k), P(delta), P(fin), *[P(t) for t in sums], B, T, D, 64, code, flags, P(ws), size, st))
+    ins = [t.double().requires_grad_() for t in (q, k, v, s)]
+    want = torch.autograd.grad(DFWFunction.apply(*ins), ins, (go.double(), gs.double()))
+    for i in range(2):
+        err = lambda t: ((t.double() - want[i]).norm() / want[i].norm()).item()
+        assert err(sums[i]) <= 1.01 * err(shares[i].float().sum(1).to(dtype)), (i, err(sums[i]), err(shares[i].float().sum(1).to(dtype)))
