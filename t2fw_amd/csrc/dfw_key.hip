@@ -5,8 +5,8 @@
 //   d_key   = X1^T Q + Delta G - dU S0 + (X2 + X2^T) K             X2[t][s] = -dU_t . delta_s  (s < t)
 // is the block form of 16 with longer sums.  Workgroup = (row, chunk), wave w = tokens 16 w .. 16 w + 15 and all 64 key channels: its
 // rows of X1, X1^T and X2 + X2^T come out of the products as ready operands (the accumulator tile of X^T is the operand "rows of
-// X") and never leave its registers.  Two phases share the LDS, so that two workgroups (four with single operands) fit a CU
-// and one loads while the other computes: first Delta, g and -dU as [64][72] tiles, then K, Q, S0 and G; everything is
+// X") and never leave its registers.  Two phases share the LDS, so that two workgroups (with single operands three, of one value
+// block of 16-bit tensors four) fit a CU and one loads while the other computes: first Delta, g and -dU as [64][72] tiles, then K, Q, S0 and G; everything is
 // loaded up front, 16 bytes per lane, whole token rows at a time.
 //
 // Value blocks (several recurrences that share q and k): the workgroup does them one after the other and adds their
@@ -14,7 +14,9 @@
 // their own.
 //
 // What bounds it: memory.  B = 96, T = 1024, fp32: 5 arrays and two 64 x 64 edges per chunk in, two arrays out, 226 MB in 42 us, 5.4
-// TB/s, the rate of a large copy.  The sequential key side (two workgroups per row, 64 dependent blocks) took 72 us for it; the
+// TB/s, the rate of a large copy.  Error of d_query and d_key against float64, sequential key side / here: fp32 4.5e-6 / 3.6e-6 and
+// 6.7e-6 / 5.9e-6; bf16 with single operands 2.8e-3 / 2.5e-3 and 2.89e-3 / 2.89e-3 (a result is off by what its operands are rounded by,
+// a score of two tokens where it was the state that holds one of them).  The sequential key side (two workgroups per row, 64 dependent blocks) took 72 us for it; the
 // edges cost the value side 8 us (50 -> 58) and the whole training step goes from 164 to 150 us.  B = 48, T = 777, two value blocks
 // of bf16: 32 -> 20 us here, a launch less (6 us), value side 25 -> 31.
 #include "common.hpp"
@@ -62,8 +64,6 @@ template <bool SP> struct Tile64 {
     }
 };
 
-// RAGGED: the last chunk of a sequence that ends within it.  Its edges have no place among its tokens' results: the adjoint after it
-// is the final state's own, the state before it comes from the final state by one more product, S0 = S_end - Delta^T K.
 // c + a b with the remainders' product too: the matrix cores have the time, and it takes out what the sums of 64 tokens in the place of
 // 16 add to the error
 template <bool SP> __device__ __forceinline__ floatx4 mma(const Sp4<SP> &a, const Sp4<SP> &b, floatx4 c) {
@@ -71,6 +71,8 @@ template <bool SP> __device__ __forceinline__ floatx4 mma(const Sp4<SP> &a, cons
     return mma32(a, b, c);
 }
 
+// RAGGED: the last chunk of a sequence that ends within it.  Its edges have no place among its tokens' results: the adjoint after it
+// is the final state's own, the state before it comes from the final state by one more product, S0 = S_end - Delta^T K.
 template <bool SP, typename E, bool BLOCKS, bool RAGGED> __device__ __forceinline__ void key_chunk(const DfwBwdArgs &p, u16 *lds, int64_t brow, int c) {
     typedef typename E::elem elem;
     typedef typename E::Raw4 Raw4;

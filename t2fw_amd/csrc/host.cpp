@@ -4,8 +4,8 @@
 //
 // Host time of a call, 4 x 16 tokens of 64 x 64 fp16, ctypes / this: forward 29.5 / 19.1 us without gradients, a training step
 // 205 / 152 us (of which torch's own hand-over to a Python autograd function and back is 91), one generation step 14.6 / 8.4.
-// Gates, event and block copies with their results in the same step as the launch: a training step on gate logits 180 / 172, of 128-wide
-// heads 252 / 225.
+// Gates, event and block copies with their results in the same step as the launch: a training step on gate logits (8 x 1000 tokens, 12
+// heads, bf16) 181 / 168, of 128-wide heads (24 x 1024, fp16) 260 / 219.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>

@@ -332,10 +332,14 @@ template <typename IO, int KV, int KK, bool IN_PLACE> __global__ __launch_bounds
 }
 
 // Whether `tiles` workgroups per (row, chunk) go through the chain themselves: few batches of loads per thread, and not too much
-// to read in all.  GPU time of forward + backward, fp16, with launch 2 / in place, us: 1 x 230 of 9 x 5 57 / 52, 16 x 1024 of
-// 16 x 8 66 / 57, 64 x 512 of 16 x 16 73 / 66, 13 x 385 of 33 x 17 (six batches) 69 / 71, beyond the line 16 x 512 of 63 x 32 (eight) 77 / 81.
-// The host issues two launches fewer of six, which is what bounds such a step: 16 x 700 of 16 x 8 157 / 146, 16 x 300 of 20 x 10
-// 156 / 148, 13 x 385 of 33 x 17 158 / 146.
+// to read in all.  Two measures, with launch 2 / in place, us:
+//   GPU time of forward + backward, fp16: 1 x 230 of 9 x 5 57 / 52, 16 x 1024 of 16 x 8 66 / 57, 64 x 512 of 16 x 16 73 / 66, 13 x 385 of
+//   33 x 17 (six batches) 69 / 71, 16 x 512 of 63 x 32 (eight) 77 / 81.  Forwards one after the other: 13 x 385 of 33 x 17 24.6 / 24.5,
+//   6 x 512 of 63 x 32 24.7 / 26.8.
+//   A training step as issued, which the host bounds and which has two launches fewer of six: 16 x 700 of 16 x 8 151 / 141, 13 x 385 of
+//   33 x 17 149 / 135, 6 x 512 of 63 x 32 153 / 141, 4 x 448 of 63 x 63 (sixteen batches) 150 / 141.
+// The line lies at six batches, where a forward by itself breaks even: there a step that the host does not bound (replayed from a
+// graph) loses 2 us of GPU time and one that it does gains 12; beyond it every forward would lose.
 constexpr int64_t XC_IN_PLACE_READS = 5 << 20;             // floats
 bool chain_is_in_place(int64_t B, int64_t NC, int D, int K, int tiles) {
     const int64_t state = (int64_t)xp_padded(D) * xp_padded(K);
