@@ -1,5 +1,5 @@
-"""Delta rule, value widths 64 n read and written in place by the matrix-core kernels (t2fw_dfw_forward_blocks,
-t2fw_dfw_backward_blocks): the bits of the same kernels on copies of the blocks, at the edges of their blocks of 16 and
+"""Delta rule, value widths 64 n read and written in place by the matrix-core kernels (t2fw_dfw_forward_blocks, and
+t2fw_dfw_backward_sums or, for float16 tensors, t2fw_dfw_backward_blocks): the bits of the same kernels on copies of the blocks, at the edges of their blocks of 16 and
 stages of 32 steps, and the arrays that they leave to the copies."""
 import pytest
 import torch
